@@ -52,16 +52,18 @@ struct LatticeArgs {
     double r, M, g;
 };
 
-// Full Wilson operator on one site for the four components of `v` (SoA planes).
-// Load functor ld(i, c) returns component c at flat site i.
-template <bool DAG, typename Load>
+// Spinor forms (NC planes of two reals per site, see ycn_device.hpp): NC = 4, complex
+// components; NC = 2, the packed real form of the fermion force.
+// Full Wilson operator on one site for the NC planes of `v`.
+// Load functor ld(i, c) returns plane c at flat site i.
+template <int NC, bool DAG, typename Load>
 __device__ __forceinline__ void wilson_site(const LatticeArgs &L, const WilsonCoef &w, double phi, int s, Load ld,
-                                            double2 o[4]) {
+                                            double2 o[NC]) {
     const int t = s / L.Nx, x = s - t * L.Nx;
     const Nbr n = neighbours(t, x, L.Nt, L.Nx);
     const double d = w.two_r_plus_m + w.g * phi;
 #pragma unroll
-    for (int f = 0; f < 4; f += 2) {
+    for (int f = 0; f < NC; f += 2) {
         wilson_flavour<DAG, double2>(w, d, ld(s, f), ld(s, f + 1), ld(n.tf, f), ld(n.tf, f + 1), n.sf, ld(n.tb, f),
                                      ld(n.tb, f + 1), n.sb, ld(n.xf, f), ld(n.xf, f + 1), ld(n.xb, f),
                                      ld(n.xb, f + 1), o[f], o[f + 1]);
@@ -71,20 +73,27 @@ __device__ __forceinline__ void wilson_site(const LatticeArgs &L, const WilsonCo
 // ---------------------------------------------------------------------------
 // plain Dirac apply: out = D in / D^dag in (DiracOP::applyD, Dirac.cu:23-47)
 // ---------------------------------------------------------------------------
-template <bool DAG>
+template <int NC, bool DAG>
 __global__ void __launch_bounds__(kNT)
 k_dirac(LatticeArgs L, const double *__restrict__ phi, const double2 *__restrict__ in, double2 *__restrict__ out) {
     const int s = blockIdx.x * kNT + threadIdx.x;
     if (s >= L.V) return;
     const int sys = blockIdx.y;
     const size_t V = L.V;
-    const double2 *v = in + (size_t)sys * 4 * V;
+    const double2 *v = in + (size_t)sys * NC * V;
     const WilsonCoef w = make_coef(L.r, L.M, L.g);
-    double2 o[4];
-    wilson_site<DAG>(L, w, phi[(size_t)(sys / L.nNoise) * V + s], s, [&](int i, int c) { return v[c * V + i]; }, o);
-    double2 *q = out + (size_t)sys * 4 * V;
+    double2 o[NC];
+    wilson_site<NC, DAG>(L, w, phi[(size_t)(sys / L.nNoise) * V + s], s, [&](int i, int c) { return v[c * V + i]; }, o);
+    double2 *q = out + (size_t)sys * NC * V;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) q[c * V + s] = o[c];
+    for (int c = 0; c < NC; ++c) q[c * V + s] = o[c];
+}
+
+// (1, 1, 0, 0) at site 0: in both forms the first members of planes 0 and 1
+__global__ void __launch_bounds__(kNT) k_point_source(int V, int planes, double2 *__restrict__ eta) {
+    const int s = blockIdx.x * kNT + threadIdx.x;
+    if (s >= V) return;
+    for (int c = 0; c < planes; ++c) eta[(size_t)c * V + s] = make_double2(s == 0 && c < 2 ? 1.0 : 0.0, 0.0);
 }
 
 __global__ void k_set_int(int *p, int v) {
@@ -312,7 +321,7 @@ __global__ void __launch_bounds__(kNT) k_fin_fcg(const double2 *__restrict__ par
 // FP64 CG kernels
 // ---------------------------------------------------------------------------
 // setup: eta (generated or given) -> b; x = 0; r = b; p0 = p1 = b; partial |b|^2
-template <bool GEN>
+template <int NC, bool GEN>
 __global__ void __launch_bounds__(kNT)
 k_cg_setup(LatticeArgs L, const uint64_t *__restrict__ seeds, uint32_t streamBase, uint64_t step,
            double2 *__restrict__ eta, double2 *__restrict__ x, double2 *__restrict__ r, double2 *__restrict__ p0,
@@ -321,20 +330,20 @@ k_cg_setup(LatticeArgs L, const uint64_t *__restrict__ seeds, uint32_t streamBas
     const int sys = blockIdx.y;
     const size_t V = L.V;
     const int s = blockIdx.x * kNT + threadIdx.x;
-    const size_t off = (size_t)sys * 4 * V;
+    const size_t off = (size_t)sys * NC * V;
     double2 acc = make_double2(0.0, 0.0);
     if (s < L.V) {
-        double2 b[4];
+        double2 b[NC];
         if (GEN) {
-            eta_site(seeds, streamBase, step, sys, L.nNoise, s, b);
+            eta_planes<NC>(seeds, streamBase, step, sys, L.nNoise, s, b);
 #pragma unroll
-            for (int c = 0; c < 4; ++c) eta[off + c * V + s] = b[c];
+            for (int c = 0; c < NC; ++c) eta[off + c * V + s] = b[c];
         } else {
 #pragma unroll
-            for (int c = 0; c < 4; ++c) b[c] = eta[off + c * V + s];
+            for (int c = 0; c < NC; ++c) b[c] = eta[off + c * V + s];
         }
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
+        for (int c = 0; c < NC; ++c) {
             const size_t i = off + c * V + s;
             x[i] = make_double2(0.0, 0.0);
             r[i] = b[c];
@@ -348,7 +357,7 @@ k_cg_setup(LatticeArgs L, const uint64_t *__restrict__ seeds, uint32_t streamBas
 }
 
 // cg_a: p' = r + beta p_old (written at own site), t = D1 p'
-template <bool DAG1>
+template <int NC, bool DAG1>
 __global__ void __launch_bounds__(kNT)
 k_cg_a(LatticeArgs L, const double *__restrict__ phi, const CgState *__restrict__ st, const double2 *__restrict__ r,
        const double2 *__restrict__ pold, double2 *__restrict__ pnew, double2 *__restrict__ t) {
@@ -357,26 +366,26 @@ k_cg_a(LatticeArgs L, const double *__restrict__ phi, const CgState *__restrict_
     const int s = blockIdx.x * kNT + threadIdx.x;
     if (s >= L.V) return;
     const double beta = st[sys].beta;
-    const size_t V = L.V, off = (size_t)sys * 4 * V;
+    const size_t V = L.V, off = (size_t)sys * NC * V;
     const double2 *rr = r + off, *po = pold + off;
     auto ld = [&](int i, int c) {
         const double2 a = rr[c * V + i], b = po[c * V + i];
         return make_double2(a.x + beta * b.x, a.y + beta * b.y);
     };
 #pragma unroll
-    for (int c = 0; c < 4; ++c) pnew[off + c * V + s] = ld(s, c);
+    for (int c = 0; c < NC; ++c) pnew[off + c * V + s] = ld(s, c);
     const WilsonCoef w = make_coef(L.r, L.M, L.g);
-    double2 o[4];
-    wilson_site<DAG1>(L, w, phi[(size_t)(sys / L.nNoise) * V + s], s, ld, o);
+    double2 o[NC];
+    wilson_site<NC, DAG1>(L, w, phi[(size_t)(sys / L.nNoise) * V + s], s, ld, o);
 #pragma unroll
-    for (int c = 0; c < 4; ++c) t[off + c * V + s] = o[c];
+    for (int c = 0; c < NC; ++c) t[off + c * V + s] = o[c];
 }
 
 // FP32 two-stencil pair for lattices that no fused FP32 tile divides (mixed precision on
 // any lattice).  cg_a32: p' = r + beta p_old in FP32 (written at the own site; the hop
 // reads the same FP32 values at the neighbours), t = D1 p'; cg_b32: Ap = D2 t, partial
 // <p', Ap>.  The hop arithmetic runs in FP64 on the FP32 vectors and FP32 field.
-template <bool DAG1>
+template <int NC, bool DAG1>
 __global__ void __launch_bounds__(kNT)
 k_cg_a32(LatticeArgs L, const float *__restrict__ phi, const CgState *__restrict__ st, const float2 *__restrict__ r,
          const float2 *__restrict__ pold, float2 *__restrict__ pnew, float2 *__restrict__ t) {
@@ -385,7 +394,7 @@ k_cg_a32(LatticeArgs L, const float *__restrict__ phi, const CgState *__restrict
     const int s = blockIdx.x * kNT + threadIdx.x;
     if (s >= L.V) return;
     const float beta = (float)st[sys].beta;
-    const size_t V = L.V, off = (size_t)sys * 4 * V;
+    const size_t V = L.V, off = (size_t)sys * NC * V;
     const float2 *rr = r + off, *po = pold + off;
     auto pf = [&](int i, int c) {
         const float2 a = rr[c * V + i], b = po[c * V + i];
@@ -396,15 +405,15 @@ k_cg_a32(LatticeArgs L, const float *__restrict__ phi, const CgState *__restrict
         return make_double2((double)v.x, (double)v.y);
     };
 #pragma unroll
-    for (int c = 0; c < 4; ++c) pnew[off + c * V + s] = pf(s, c);
+    for (int c = 0; c < NC; ++c) pnew[off + c * V + s] = pf(s, c);
     const WilsonCoef w = make_coef(L.r, L.M, L.g);
-    double2 o[4];
-    wilson_site<DAG1>(L, w, (double)phi[(size_t)(sys / L.nNoise) * V + s], s, ld, o);
+    double2 o[NC];
+    wilson_site<NC, DAG1>(L, w, (double)phi[(size_t)(sys / L.nNoise) * V + s], s, ld, o);
 #pragma unroll
-    for (int c = 0; c < 4; ++c) t[off + c * V + s] = make_float2((float)o[c].x, (float)o[c].y);
+    for (int c = 0; c < NC; ++c) t[off + c * V + s] = make_float2((float)o[c].x, (float)o[c].y);
 }
 
-template <bool DAG2>
+template <int NC, bool DAG2>
 __global__ void __launch_bounds__(kNT)
 k_cg_b32(LatticeArgs L, const float *__restrict__ phi, const CgState *__restrict__ st, const float2 *__restrict__ t,
          const float2 *__restrict__ p, float2 *__restrict__ Ap, double2 *__restrict__ part) {
@@ -412,32 +421,32 @@ k_cg_b32(LatticeArgs L, const float *__restrict__ phi, const CgState *__restrict
     const int sys = blockIdx.y;
     if (st[sys].done) return;
     const int s = blockIdx.x * kNT + threadIdx.x;
-    const size_t V = L.V, off = (size_t)sys * 4 * V;
+    const size_t V = L.V, off = (size_t)sys * NC * V;
     double2 acc = make_double2(0.0, 0.0);
     if (s < L.V) {
         const float2 *tv = t + off;
         const WilsonCoef w = make_coef(L.r, L.M, L.g);
-        double2 o[4];
-        wilson_site<DAG2>(L, w, (double)phi[(size_t)(sys / L.nNoise) * V + s], s,
+        double2 o[NC];
+        wilson_site<NC, DAG2>(L, w, (double)phi[(size_t)(sys / L.nNoise) * V + s], s,
                           [&](int i, int c) {
                               const float2 v = tv[c * V + i];
                               return make_double2((double)v.x, (double)v.y);
                           },
                           o);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
+        for (int c = 0; c < NC; ++c) {
             const float2 a = make_float2((float)o[c].x, (float)o[c].y);
             Ap[off + c * V + s] = a;
             const float2 pv = p[off + c * V + s];
-            acc = cadd(acc, cdotc(make_double2((double)pv.x, (double)pv.y), make_double2((double)a.x, (double)a.y)));
+            acc = cadd(acc, pdot<NC>(make_double2((double)pv.x, (double)pv.y), make_double2((double)a.x, (double)a.y)));
         }
     }
     acc = block_sum2<kNT>(acc, lds);
     if (threadIdx.x == 0) part[(size_t)sys * gridDim.x + blockIdx.x] = acc;
 }
 
-// cg_b: Ap = D2 t; partial <p', Ap>// cg_b: Ap = D2 t; partial <p', Ap>
-template <bool DAG2>
+// cg_b: Ap = D2 t; partial <p', Ap>
+template <int NC, bool DAG2>
 __global__ void __launch_bounds__(kNT)
 k_cg_b(LatticeArgs L, const double *__restrict__ phi, const CgState *__restrict__ st, const double2 *__restrict__ t,
        const double2 *__restrict__ p, double2 *__restrict__ Ap, double2 *__restrict__ part) {
@@ -445,18 +454,18 @@ k_cg_b(LatticeArgs L, const double *__restrict__ phi, const CgState *__restrict_
     const int sys = blockIdx.y;
     if (st[sys].done) return;
     const int s = blockIdx.x * kNT + threadIdx.x;
-    const size_t V = L.V, off = (size_t)sys * 4 * V;
+    const size_t V = L.V, off = (size_t)sys * NC * V;
     double2 acc = make_double2(0.0, 0.0);
     if (s < L.V) {
         const double2 *tv = t + off;
         const WilsonCoef w = make_coef(L.r, L.M, L.g);
-        double2 o[4];
-        wilson_site<DAG2>(L, w, phi[(size_t)(sys / L.nNoise) * V + s], s,
+        double2 o[NC];
+        wilson_site<NC, DAG2>(L, w, phi[(size_t)(sys / L.nNoise) * V + s], s,
                           [&](int i, int c) { return tv[c * V + i]; }, o);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
+        for (int c = 0; c < NC; ++c) {
             Ap[off + c * V + s] = o[c];
-            acc = cadd(acc, cdotc(p[off + c * V + s], o[c]));
+            acc = cadd(acc, pdot<NC>(p[off + c * V + s], o[c]));
         }
     }
     acc = block_sum2<kNT>(acc, lds);
@@ -465,6 +474,7 @@ k_cg_b(LatticeArgs L, const double *__restrict__ phi, const CgState *__restrict_
 
 // cg_c: x += alpha p'; r -= alpha Ap; partial |r|^2.  All loads are issued before
 // any store so each thread keeps 16 loads in flight.
+template <int NC>
 __global__ void __launch_bounds__(kNT)
 k_cg_c(int V_, const CgState *__restrict__ st, double2 *__restrict__ x, double2 *__restrict__ r,
        const double2 *__restrict__ p, const double2 *__restrict__ Ap, double2 *__restrict__ part) {
@@ -472,13 +482,13 @@ k_cg_c(int V_, const CgState *__restrict__ st, double2 *__restrict__ x, double2 
     const int sys = blockIdx.y;
     if (st[sys].done) return;
     const int s = blockIdx.x * kNT + threadIdx.x;
-    const size_t V = V_, off = (size_t)sys * 4 * V;
+    const size_t V = V_, off = (size_t)sys * NC * V;
     const double2 al = st[sys].alpha;
     double2 acc = make_double2(0.0, 0.0);
     if (s < V_) {
-        double2 xv[4], rv[4], pv[4], av[4];
+        double2 xv[NC], rv[NC], pv[NC], av[NC];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
+        for (int c = 0; c < NC; ++c) {
             const size_t i = off + c * V + s;
             xv[c] = x[i];
             rv[c] = r[i];
@@ -486,10 +496,10 @@ k_cg_c(int V_, const CgState *__restrict__ st, double2 *__restrict__ x, double2 
             av[c] = Ap[i];
         }
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
+        for (int c = 0; c < NC; ++c) {
             const size_t i = off + c * V + s;
-            x[i] = cadd(xv[c], cmul(al, pv[c]));
-            const double2 rn = csub(rv[c], cmul(al, av[c]));
+            x[i] = cadd(xv[c], pscale<NC>(al, pv[c]));
+            const double2 rn = csub(rv[c], pscale<NC>(al, av[c]));
             r[i] = rn;
             acc.x += rn.x * rn.x + rn.y * rn.y;
         }
@@ -499,24 +509,24 @@ k_cg_c(int V_, const CgState *__restrict__ st, double2 *__restrict__ x, double2 
 }
 
 // true residual, part 1: t = D1 x
-template <bool DAG1>
+template <int NC, bool DAG1>
 __global__ void __launch_bounds__(kNT)
 k_true_a(LatticeArgs L, const double *__restrict__ phi, const double2 *__restrict__ x, double2 *__restrict__ t) {
     const int s = blockIdx.x * kNT + threadIdx.x;
     if (s >= L.V) return;
     const int sys = blockIdx.y;
-    const size_t V = L.V, off = (size_t)sys * 4 * V;
+    const size_t V = L.V, off = (size_t)sys * NC * V;
     const double2 *xv = x + off;
     const WilsonCoef w = make_coef(L.r, L.M, L.g);
-    double2 o[4];
-    wilson_site<DAG1>(L, w, phi[(size_t)(sys / L.nNoise) * V + s], s, [&](int i, int c) { return xv[c * V + i]; }, o);
+    double2 o[NC];
+    wilson_site<NC, DAG1>(L, w, phi[(size_t)(sys / L.nNoise) * V + s], s, [&](int i, int c) { return xv[c * V + i]; }, o);
 #pragma unroll
-    for (int c = 0; c < 4; ++c) t[off + c * V + s] = o[c];
+    for (int c = 0; c < NC; ++c) t[off + c * V + s] = o[c];
 }
 
 // true residual, part 2: res = b - D2 t -> r (FP64) or, for the mixed solver, rs
 // (FP32); partial |res|^2.  The mixed solver skips systems that are already final.
-template <bool DAG2, bool MIXED>
+template <int NC, bool DAG2, bool MIXED>
 __global__ void __launch_bounds__(kNT)
 k_true_b(LatticeArgs L, const double *__restrict__ phi, const CgState *__restrict__ st, const double2 *__restrict__ b,
          const double2 *__restrict__ t, double2 *__restrict__ r, float2 *__restrict__ rs, double2 *__restrict__ part) {
@@ -524,16 +534,16 @@ k_true_b(LatticeArgs L, const double *__restrict__ phi, const CgState *__restric
     const int sys = blockIdx.y;
     if (MIXED && st[sys].final_) return;
     const int s = blockIdx.x * kNT + threadIdx.x;
-    const size_t V = L.V, off = (size_t)sys * 4 * V;
+    const size_t V = L.V, off = (size_t)sys * NC * V;
     double2 acc = make_double2(0.0, 0.0);
     if (s < L.V) {
         const double2 *tv = t + off;
         const WilsonCoef w = make_coef(L.r, L.M, L.g);
-        double2 o[4];
-        wilson_site<DAG2>(L, w, phi[(size_t)(sys / L.nNoise) * V + s], s,
+        double2 o[NC];
+        wilson_site<NC, DAG2>(L, w, phi[(size_t)(sys / L.nNoise) * V + s], s,
                           [&](int i, int c) { return tv[c * V + i]; }, o);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
+        for (int c = 0; c < NC; ++c) {
             const double2 res = csub(b[off + c * V + s], o[c]);
             if (MIXED)
                 rs[off + c * V + s] = make_float2((float)res.x, (float)res.y);
@@ -548,6 +558,7 @@ k_true_b(LatticeArgs L, const double *__restrict__ phi, const CgState *__restric
 
 // drift_x = fac/nNoise * sum_j Re sum_k conj((D y_j)_xk) eta_j,xk
 // (FermionicDrift.cu:69 applyD Normal + computeDrift :83-100)
+template <int NC>
 __global__ void __launch_bounds__(kNT)
 k_drift(LatticeArgs L, const double *__restrict__ phi, const double2 *__restrict__ y, const double2 *__restrict__ eta,
         double *__restrict__ drift, double fac) {
@@ -559,21 +570,24 @@ k_drift(LatticeArgs L, const double *__restrict__ phi, const double2 *__restrict
     const double ph = phi[(size_t)rep * V + s];
     double acc = 0.0;
     for (int j = 0; j < L.nNoise; ++j) {
-        const size_t off = ((size_t)rep * L.nNoise + j) * 4 * V;
+        const size_t off = ((size_t)rep * L.nNoise + j) * NC * V;
         const double2 *yv = y + off;
-        double2 o[4];
-        wilson_site<false>(L, w, ph, s, [&](int i, int c) { return yv[c * V + i]; }, o);
-        double2 sm = cdotc(o[0], eta[off + s]);
-        sm = cadd(sm, cdotc(o[1], eta[off + V + s]));
-        sm = cadd(sm, cdotc(o[2], eta[off + 2 * V + s]));
-        sm = cadd(sm, cdotc(o[3], eta[off + 3 * V + s]));
-        acc += sm.x;
+        double2 o[NC];
+        wilson_site<NC, false>(L, w, ph, s, [&](int i, int c) { return yv[c * V + i]; }, o);
+        double sm = 0.0;   // Re conj(chi) eta, the same sum in both forms
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            const double2 e = eta[off + c * V + s];
+            sm += o[c].x * e.x + o[c].y * e.y;
+        }
+        acc += sm;
     }
     drift[(size_t)rep * V + s] = (L.nNoise == 1) ? fac * acc : fac * acc / (double)L.nNoise;
 }
 
 // corr[t] = sum_x sum_k Re psi (gpuTimeSlices_spinors, reductions.cu:176-191);
 // one block per time slice, fixed-order block reduction.
+template <int NC>
 __global__ void __launch_bounds__(kNT)
 k_spinor_slices(const double2 *__restrict__ psi, int Nt, int Nx, double *__restrict__ out) {
     __shared__ double2 lds[kNT / kWave];
@@ -582,7 +596,10 @@ k_spinor_slices(const double2 *__restrict__ psi, int Nt, int Nx, double *__restr
     double2 acc = make_double2(0.0, 0.0);
     for (int x = threadIdx.x; x < Nx; x += kNT) {
         const size_t s = (size_t)t * Nx + x;
-        acc.x += psi[s].x + psi[V + s].x + psi[2 * V + s].x + psi[3 * V + s].x;
+        if (NC == 4)
+            acc.x += psi[s].x + psi[V + s].x + psi[2 * V + s].x + psi[3 * V + s].x;
+        else
+            acc.x += psi[s].x + psi[V + s].x + psi[s].y + psi[V + s].y;
     }
     acc = block_sum2<kNT>(acc, lds);
     if (threadIdx.x == 0) out[t] = acc.x;
@@ -602,7 +619,7 @@ k_to_f32(const double *__restrict__ a, float *__restrict__ b, int64_t n, const i
     if (copy) copy[i] = v;
 }
 
-template <bool GEN>
+template <int NC, bool GEN>
 __global__ void __launch_bounds__(kNT)
 k_mp_setup(LatticeArgs L, const uint64_t *__restrict__ seeds, uint32_t streamBase, uint64_t step,
            double2 *__restrict__ eta, double2 *__restrict__ x, float2 *__restrict__ xs, float2 *__restrict__ rs,
@@ -611,20 +628,20 @@ k_mp_setup(LatticeArgs L, const uint64_t *__restrict__ seeds, uint32_t streamBas
     const int sys = blockIdx.y;
     const size_t V = L.V;
     const int s = blockIdx.x * kNT + threadIdx.x;
-    const size_t off = (size_t)sys * 4 * V;
+    const size_t off = (size_t)sys * NC * V;
     double2 acc = make_double2(0.0, 0.0);
     if (s < L.V) {
-        double2 b[4];
+        double2 b[NC];
         if (GEN) {
-            eta_site(seeds, streamBase, step, sys, L.nNoise, s, b);
+            eta_planes<NC>(seeds, streamBase, step, sys, L.nNoise, s, b);
 #pragma unroll
-            for (int c = 0; c < 4; ++c) eta[off + c * V + s] = b[c];
+            for (int c = 0; c < NC; ++c) eta[off + c * V + s] = b[c];
         } else {
 #pragma unroll
-            for (int c = 0; c < 4; ++c) b[c] = eta[off + c * V + s];
+            for (int c = 0; c < NC; ++c) b[c] = eta[off + c * V + s];
         }
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
+        for (int c = 0; c < NC; ++c) {
             const size_t i = off + c * V + s;
             const float2 bs = make_float2((float)b[c].x, (float)b[c].y);
             x[i] = make_double2(0.0, 0.0);
@@ -640,6 +657,7 @@ k_mp_setup(LatticeArgs L, const uint64_t *__restrict__ seeds, uint32_t streamBas
 }
 
 // FP32 update: xs += alpha p', rs -= alpha Ap; partial |rs|^2 accumulated in FP64
+template <int NC>
 __global__ void __launch_bounds__(kNT)
 k_mp_update(int V_, const CgState *__restrict__ st, float2 *__restrict__ xs, float2 *__restrict__ rs,
             const float2 *__restrict__ p, const float2 *__restrict__ Ap, double2 *__restrict__ part) {
@@ -647,14 +665,14 @@ k_mp_update(int V_, const CgState *__restrict__ st, float2 *__restrict__ xs, flo
     const int sys = blockIdx.y;
     if (st[sys].done) return;
     const int s = blockIdx.x * kNT + threadIdx.x;
-    const size_t V = V_, off = (size_t)sys * 4 * V;
+    const size_t V = V_, off = (size_t)sys * NC * V;
     const double2 ad = st[sys].alpha;
-    const float ax = (float)ad.x, ay = (float)ad.y;
+    const float ax = (float)ad.x, ay = NC == 4 ? (float)ad.y : 0.f;   // packed: alpha is real
     double2 acc = make_double2(0.0, 0.0);
     if (s < V_) {
-        float2 xv[4], rv[4], pv[4], av[4];
+        float2 xv[NC], rv[NC], pv[NC], av[NC];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
+        for (int c = 0; c < NC; ++c) {
             const size_t i = off + c * V + s;
             xv[c] = xs[i];
             rv[c] = rs[i];
@@ -663,7 +681,7 @@ k_mp_update(int V_, const CgState *__restrict__ st, float2 *__restrict__ xs, flo
         }
         float prr = 0.f;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
+        for (int c = 0; c < NC; ++c) {
             const size_t i = off + c * V + s;
             float2 xn, rn;
             xn.x = xv[c].x + (ax * pv[c].x - ay * pv[c].y);
@@ -681,22 +699,23 @@ k_mp_update(int V_, const CgState *__restrict__ st, float2 *__restrict__ xs, flo
 }
 
 // reliable update, part 1: x += xs (FP64), xs = 0
+template <int NC>
 __global__ void __launch_bounds__(kNT)
 k_mp_accum(int V_, const CgState *__restrict__ st, double2 *__restrict__ x, float2 *__restrict__ xs) {
     const int sys = blockIdx.y;
     if (st[sys].final_) return;
     const int s = blockIdx.x * kNT + threadIdx.x;
     if (s >= V_) return;
-    const size_t V = V_, off = (size_t)sys * 4 * V;
-    float2 d[4];
-    double2 xv[4];
+    const size_t V = V_, off = (size_t)sys * NC * V;
+    float2 d[NC];
+    double2 xv[NC];
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
+    for (int c = 0; c < NC; ++c) {
         d[c] = xs[off + c * V + s];
         xv[c] = x[off + c * V + s];
     }
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
+    for (int c = 0; c < NC; ++c) {
         x[off + c * V + s] = make_double2(xv[c].x + (double)d[c].x, xv[c].y + (double)d[c].y);
         xs[off + c * V + s] = make_float2(0.f, 0.f);
     }
@@ -716,6 +735,13 @@ static LatticeArgs largs(const Ctx &c) {
     L.g = c.p.g;
     return L;
 }
+
+template <int NC>
+static int mp_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, uint32_t streamBase, uint64_t step,
+                    SolveStats *st);
+template <int NC>
+static int fp64_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, uint32_t streamBase, uint64_t step,
+                      SolveStats *st);
 
 static dim3 site_grid(const Ctx &c, int nsys) { return dim3((c.V + kNT - 1) / kNT, nsys); }
 static int site_blocks(const Ctx &c) { return (c.V + kNT - 1) / kNT; }
@@ -777,9 +803,9 @@ int dirac_apply(Ctx &c, const double *phi_dev, const double2 *in, double2 *out, 
     const LatticeArgs L = largs(c);
     prof_before(c, PK_DIRAC, (double)nsys * c.V * (2 * 64 + 8));
     if (dagger)
-        hipLaunchKernelGGL(k_dirac<true>, site_grid(c, nsys), dim3(kNT), 0, c.stream, L, phi_dev, in, out);
+        hipLaunchKernelGGL((k_dirac<4, true>), site_grid(c, nsys), dim3(kNT), 0, c.stream, L, phi_dev, in, out);
     else
-        hipLaunchKernelGGL(k_dirac<false>, site_grid(c, nsys), dim3(kNT), 0, c.stream, L, phi_dev, in, out);
+        hipLaunchKernelGGL((k_dirac<4, false>), site_grid(c, nsys), dim3(kNT), 0, c.stream, L, phi_dev, in, out);
     prof_after(c, PK_DIRAC);
     YCN_HIP(hipGetLastError());
     return YCN_OK;
@@ -788,6 +814,7 @@ int dirac_apply(Ctx &c, const double *phi_dev, const double2 *in, double2 *out, 
 // p' = r + beta p_old, Ap = A p' and the partials of <p', Ap>: the fused LDS kernel
 // with tile `tile` (>= 0) or the two-stencil pair cg_a + cg_b (tile = -1).  Returns
 // the number of partials per system.
+template <int NC>
 static int launch_normal_op(Ctx &c, const LatticeArgs &L, const double *phi, int nsys, int mtype, int parity,
                             int tile) {
     const double2 *pold = c.pv[parity];
@@ -795,34 +822,35 @@ static int launch_normal_op(Ctx &c, const LatticeArgs &L, const double *phi, int
     const bool dag1 = (mtype != YCN_DAGGER);
     if (tile >= 0) {
         // compulsory traffic: read r, p_old, phi; write p', Ap  (4S + P per site)
-        prof_before(c, PK_NORMAL_OP, (double)nsys * c.V * (4 * 64 + 8));
-        launch_fused<double>(c, tile, nsys, dag1, phi, c.cg_d, (const double2 *)c.r, pold, pnew, c.Ap, c.partials);
+        prof_before(c, PK_NORMAL_OP, (double)nsys * c.V * (4 * NC * 16 + 8));
+        launch_fused<double, NC>(c, tile, nsys, dag1, phi, c.cg_d, (const double2 *)c.r, pold, pnew, c.Ap, c.partials);
         prof_after(c, PK_NORMAL_OP);
         return fused_args(c, kTiles64[tile].TT, kTiles64[tile].TX).tilesPerSys;
     }
     const dim3 g = site_grid(c, nsys);
     // cg_a + cg_b: read r, p_old, phi, write p', t; read t, p', phi, write Ap  (7S + 2P)
-    prof_before(c, PK_NORMAL_OP, (double)nsys * c.V * (7 * 64 + 16));
+    prof_before(c, PK_NORMAL_OP, (double)nsys * c.V * (7 * NC * 16 + 16));
     if (!dag1) {
-        hipLaunchKernelGGL(k_cg_a<false>, g, dim3(kNT), 0, c.stream, L, phi, (const CgState *)c.cg_d,
+        hipLaunchKernelGGL((k_cg_a<NC, false>), g, dim3(kNT), 0, c.stream, L, phi, (const CgState *)c.cg_d,
                            (const double2 *)c.r, pold, pnew, c.t);
-        hipLaunchKernelGGL(k_cg_b<true>, g, dim3(kNT), 0, c.stream, L, phi, (const CgState *)c.cg_d,
+        hipLaunchKernelGGL((k_cg_b<NC, true>), g, dim3(kNT), 0, c.stream, L, phi, (const CgState *)c.cg_d,
                            (const double2 *)c.t, (const double2 *)pnew, c.Ap, c.partials);
     } else {
-        hipLaunchKernelGGL(k_cg_a<true>, g, dim3(kNT), 0, c.stream, L, phi, (const CgState *)c.cg_d,
+        hipLaunchKernelGGL((k_cg_a<NC, true>), g, dim3(kNT), 0, c.stream, L, phi, (const CgState *)c.cg_d,
                            (const double2 *)c.r, pold, pnew, c.t);
-        hipLaunchKernelGGL(k_cg_b<false>, g, dim3(kNT), 0, c.stream, L, phi, (const CgState *)c.cg_d,
+        hipLaunchKernelGGL((k_cg_b<NC, false>), g, dim3(kNT), 0, c.stream, L, phi, (const CgState *)c.cg_d,
                            (const double2 *)c.t, (const double2 *)pnew, c.Ap, c.partials);
     }
     prof_after(c, PK_NORMAL_OP);
     return site_blocks(c);
 }
 
+template <int NC>
 static void launch_iteration(Ctx &c, const LatticeArgs &L, const double *phi, int nsys, int mtype, int parity) {
-    const int nb = launch_normal_op(c, L, phi, nsys, mtype, parity, c.tile64);
+    const int nb = launch_normal_op<NC>(c, L, phi, nsys, mtype, parity, c.tile64);
     hipLaunchKernelGGL(k_fin_alpha, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)c.partials, nb, c.cg_d);
-    prof_before(c, PK_CG_UPDATE, (double)nsys * c.V * 6 * 64);
-    hipLaunchKernelGGL(k_cg_c, site_grid(c, nsys), dim3(kNT), 0, c.stream, c.V, (const CgState *)c.cg_d, c.x, c.r,
+    prof_before(c, PK_CG_UPDATE, (double)nsys * c.V * 6 * NC * 16);
+    hipLaunchKernelGGL(k_cg_c<NC>, site_grid(c, nsys), dim3(kNT), 0, c.stream, c.V, (const CgState *)c.cg_d, c.x, c.r,
                        (const double2 *)c.pv[parity ^ 1], (const double2 *)c.Ap, c.partials);
     prof_after(c, PK_CG_UPDATE);
     hipLaunchKernelGGL(k_fin_beta<false>, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)c.partials,
@@ -848,26 +876,10 @@ void launch_fin_beta(Ctx &c, int nsys, int nb, bool mixed, bool even) {
 int launch_cg_update(Ctx &c, int nsys, int n, const double2 *p) {
     const dim3 g((n + kNT - 1) / kNT, nsys);
     prof_before(c, PK_CG_UPDATE, (double)nsys * n * 6 * 64);
-    hipLaunchKernelGGL(k_cg_c, g, dim3(kNT), 0, c.stream, n, (const CgState *)c.cg_d, c.x, c.r, p,
+    hipLaunchKernelGGL(k_cg_c<4>, g, dim3(kNT), 0, c.stream, n, (const CgState *)c.cg_d, c.x, c.r, p,
                        (const double2 *)c.Ap, c.partials);
     prof_after(c, PK_CG_UPDATE);
     return (int)g.x;
-}
-
-int launch_mp_update(Ctx &c, int nsys, int n, const float2 *p) {
-    const dim3 g((n + kNT - 1) / kNT, nsys);
-    prof_before(c, PK_CG_UPDATE, (double)nsys * n * 6 * 32);
-    hipLaunchKernelGGL(k_mp_update, g, dim3(kNT), 0, c.stream, n, (const CgState *)c.cg_d, c.xs, c.rs, p,
-                       (const float2 *)c.Aps, c.partials);
-    prof_after(c, PK_CG_UPDATE);
-    return (int)g.x;
-}
-
-int launch_mp_accum(Ctx &c, int nsys, int n) {
-    hipLaunchKernelGGL(k_mp_accum, dim3((n + kNT - 1) / kNT, nsys), dim3(kNT), 0, c.stream, n,
-                       (const CgState *)c.cg_d, c.x, c.xs);
-    YCN_HIP(hipGetLastError());
-    return YCN_OK;
 }
 
 int to_f32_n(Ctx &c, const double *a, float *b, int64_t n, const int *halt, double *copy) {
@@ -947,10 +959,10 @@ int cg_autotune(Ctx &c) {
         us.clear();
         for (int tile : cands)
             us.push_back(time_it(
-                [&](int par) { (void)launch_normal_op(c, L, c.phi[c.cur], c.nSys, YCN_DAGGER, par, tile); }));
+                [&](int par) { (void)launch_normal_op<2>(c, L, c.phi[c.cur], c.nSys, YCN_DAGGER, par, tile); }));
         for (int i : cands32)
             us.push_back(time_it([&](int par) {
-                launch_fused<float>(c, i, c.nSys, false, c.phis, c.cg_d, (const float2 *)c.rs, c.ps[par],
+                launch_fused<float, 2>(c, i, c.nSys, false, c.phis, c.cg_d, (const float2 *)c.rs, c.ps[par],
                                     c.ps[par ^ 1], c.Aps, c.partials);
             }));
         tune_store(0, c, us);
@@ -1027,14 +1039,23 @@ int stats_from_mirror(Ctx &c, int nsys, SolveStats *st) {
     return YCN_OK;
 }
 
-int cg_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, uint32_t streamBase, uint64_t step,
-             SolveStats *st) {
+int cg_solve(Ctx &c, const double *phi, int nsys, int mtype, SpinorForm form, bool gen, uint32_t streamBase,
+             uint64_t step, SolveStats *st) {
     if (c.p.precond == YCN_PRECOND_CNN && mtype == YCN_DAGGER)
         return fcg_solve(c, phi, nsys, mtype, gen, streamBase, step, st);
     // mixed precision where the FP32 tiles fit the lattice (with even-odd preconditioning
     // the fermion force may run mixed on shapes the plain FP32 tiles do not cover)
-    if ((c.p.cgPrecision == YCN_CG_MIXED && c.rs) || c.p.precond == YCN_PRECOND_CNN)
-        return mp_solve(c, phi, nsys, mtype, gen, streamBase, step, st);
+    const bool mixed = (c.p.cgPrecision == YCN_CG_MIXED && c.rs) || c.p.precond == YCN_PRECOND_CNN;
+    if (form == kPacked)
+        return mixed ? mp_solve<2>(c, phi, nsys, mtype, gen, streamBase, step, st)
+                     : fp64_solve<2>(c, phi, nsys, mtype, gen, streamBase, step, st);
+    return mixed ? mp_solve<4>(c, phi, nsys, mtype, gen, streamBase, step, st)
+                 : fp64_solve<4>(c, phi, nsys, mtype, gen, streamBase, step, st);
+}
+
+template <int NC>
+static int fp64_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, uint32_t streamBase, uint64_t step,
+                      SolveStats *st) {
     const LatticeArgs L = largs(c);
     const dim3 g = site_grid(c, nsys);
     const int nb = site_blocks(c);
@@ -1042,10 +1063,10 @@ int cg_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, uint32_t 
     if (rc) return rc;
     const int maxIter = c.p.cgMaxIter, maxRestarts = 4;
     if (gen)
-        hipLaunchKernelGGL(k_cg_setup<true>, g, dim3(kNT), 0, c.stream, L, (const uint64_t *)c.seed_d, streamBase,
+        hipLaunchKernelGGL((k_cg_setup<NC, true>), g, dim3(kNT), 0, c.stream, L, (const uint64_t *)c.seed_d, streamBase,
                            step, c.eta, c.x, c.r, c.pv[0], c.pv[1], c.partials);
     else
-        hipLaunchKernelGGL(k_cg_setup<false>, g, dim3(kNT), 0, c.stream, L, (const uint64_t *)c.seed_d, streamBase,
+        hipLaunchKernelGGL((k_cg_setup<NC, false>), g, dim3(kNT), 0, c.stream, L, (const uint64_t *)c.seed_d, streamBase,
                            step, c.eta, c.x, c.r, c.pv[0], c.pv[1], c.partials);
     hipLaunchKernelGGL(k_fin_setup, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)c.partials, nb, c.cg_d,
                        c.active, c.p.cgTol, c.p.cgTolMode, maxIter, maxRestarts);
@@ -1059,8 +1080,8 @@ int cg_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, uint32_t 
             // about `chunk` iterations as captured graphs of kGraphIters, then poll
             const int n = std::min(chunk, hardCap - launched);
             for (int k = 0; k < n; k += kGraphIters) {
-                rc = run_chunk(c, phi, nsys, mtype, kGraphIters, YCN_CG_FP64, c.tile64,
-                               [&](int i) { launch_iteration(c, L, phi, nsys, mtype, i & 1); });
+                rc = run_chunk(c, phi, nsys, mtype, kGraphIters, YCN_CG_FP64, NC, c.tile64,
+                               [&](int i) { launch_iteration<NC>(c, L, phi, nsys, mtype, i & 1); });
                 if (rc) return rc;
             }
             launched += ((n + kGraphIters - 1) / kGraphIters) * kGraphIters;
@@ -1070,12 +1091,12 @@ int cg_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, uint32_t 
         }
         // FP64 true residual (restarts systems in YCN_TOL_REL_TRUE mode while above tol)
         if (mtype == YCN_DAGGER) {
-            hipLaunchKernelGGL(k_true_a<false>, g, dim3(kNT), 0, c.stream, L, phi, (const double2 *)c.x, c.t);
-            hipLaunchKernelGGL((k_true_b<true, false>), g, dim3(kNT), 0, c.stream, L, phi, (const CgState *)c.cg_d,
+            hipLaunchKernelGGL((k_true_a<NC, false>), g, dim3(kNT), 0, c.stream, L, phi, (const double2 *)c.x, c.t);
+            hipLaunchKernelGGL((k_true_b<NC, true, false>), g, dim3(kNT), 0, c.stream, L, phi, (const CgState *)c.cg_d,
                                (const double2 *)c.eta, (const double2 *)c.t, c.r, (float2 *)nullptr, c.partials);
         } else {
-            hipLaunchKernelGGL(k_true_a<true>, g, dim3(kNT), 0, c.stream, L, phi, (const double2 *)c.x, c.t);
-            hipLaunchKernelGGL((k_true_b<false, false>), g, dim3(kNT), 0, c.stream, L, phi, (const CgState *)c.cg_d,
+            hipLaunchKernelGGL((k_true_a<NC, true>), g, dim3(kNT), 0, c.stream, L, phi, (const double2 *)c.x, c.t);
+            hipLaunchKernelGGL((k_true_b<NC, false, false>), g, dim3(kNT), 0, c.stream, L, phi, (const CgState *)c.cg_d,
                                (const double2 *)c.eta, (const double2 *)c.t, c.r, (float2 *)nullptr, c.partials);
         }
         hipLaunchKernelGGL(k_fin_true, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)c.partials, nb, c.cg_d,
@@ -1136,13 +1157,14 @@ void mp_free(Ctx &c) {
         if (slot) { (void)hipFree(slot); slot = nullptr; }
 }
 
+template <int NC>
 static void launch_mp_iteration(Ctx &c, int nsys, int mtype, int parity) {
     const float2 *pold = c.ps[parity];
     float2 *pnew = c.ps[parity ^ 1];
     int nbF;
     if (c.tile32 >= 0) {
-        prof_before(c, PK_NORMAL_OP, (double)nsys * c.V * (4 * 32 + 4));
-        launch_fused<float>(c, c.tile32, nsys, mtype != YCN_DAGGER, c.phis, c.cg_d, (const float2 *)c.rs, pold, pnew,
+        prof_before(c, PK_NORMAL_OP, (double)nsys * c.V * (4 * NC * 8 + 4));
+        launch_fused<float, NC>(c, c.tile32, nsys, mtype != YCN_DAGGER, c.phis, c.cg_d, (const float2 *)c.rs, pold, pnew,
                             c.Aps, c.partials);
         prof_after(c, PK_NORMAL_OP);
         nbF = fused_args(c, kTiles32[c.tile32].TT, kTiles32[c.tile32].TX).tilesPerSys;
@@ -1153,32 +1175,33 @@ static void launch_mp_iteration(Ctx &c, int nsys, int mtype, int parity) {
         const dim3 g = site_grid(c, nsys);
         float2 *t = reinterpret_cast<float2 *>(c.t);
         // read r, p_old, phi, write p', t; read t, p', phi, write Ap  (7S + 2P, FP32)
-        prof_before(c, PK_NORMAL_OP, (double)nsys * c.V * (7 * 32 + 8));
+        prof_before(c, PK_NORMAL_OP, (double)nsys * c.V * (7 * NC * 8 + 8));
         if (mtype == YCN_DAGGER) {
-            hipLaunchKernelGGL(k_cg_a32<false>, g, dim3(kNT), 0, c.stream, L, (const float *)c.phis,
+            hipLaunchKernelGGL((k_cg_a32<NC, false>), g, dim3(kNT), 0, c.stream, L, (const float *)c.phis,
                                (const CgState *)c.cg_d, (const float2 *)c.rs, pold, pnew, t);
-            hipLaunchKernelGGL(k_cg_b32<true>, g, dim3(kNT), 0, c.stream, L, (const float *)c.phis,
+            hipLaunchKernelGGL((k_cg_b32<NC, true>), g, dim3(kNT), 0, c.stream, L, (const float *)c.phis,
                                (const CgState *)c.cg_d, (const float2 *)t, (const float2 *)pnew, c.Aps, c.partials);
         } else {
-            hipLaunchKernelGGL(k_cg_a32<true>, g, dim3(kNT), 0, c.stream, L, (const float *)c.phis,
+            hipLaunchKernelGGL((k_cg_a32<NC, true>), g, dim3(kNT), 0, c.stream, L, (const float *)c.phis,
                                (const CgState *)c.cg_d, (const float2 *)c.rs, pold, pnew, t);
-            hipLaunchKernelGGL(k_cg_b32<false>, g, dim3(kNT), 0, c.stream, L, (const float *)c.phis,
+            hipLaunchKernelGGL((k_cg_b32<NC, false>), g, dim3(kNT), 0, c.stream, L, (const float *)c.phis,
                                (const CgState *)c.cg_d, (const float2 *)t, (const float2 *)pnew, c.Aps, c.partials);
         }
         prof_after(c, PK_NORMAL_OP);
         nbF = site_blocks(c);
     }
     hipLaunchKernelGGL(k_fin_alpha, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)c.partials, nbF, c.cg_d);
-    prof_before(c, PK_CG_UPDATE, (double)nsys * c.V * 6 * 32);
-    hipLaunchKernelGGL(k_mp_update, site_grid(c, nsys), dim3(kNT), 0, c.stream, c.V, (const CgState *)c.cg_d, c.xs,
+    prof_before(c, PK_CG_UPDATE, (double)nsys * c.V * 6 * NC * 8);
+    hipLaunchKernelGGL(k_mp_update<NC>, site_grid(c, nsys), dim3(kNT), 0, c.stream, c.V, (const CgState *)c.cg_d, c.xs,
                        c.rs, (const float2 *)pnew, (const float2 *)c.Aps, c.partials);
     prof_after(c, PK_CG_UPDATE);
     hipLaunchKernelGGL(k_fin_beta<true>, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)c.partials,
                        site_blocks(c), c.cg_d, c.active);
 }
 
-int mp_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, uint32_t streamBase, uint64_t step,
-             SolveStats *st) {
+template <int NC>
+static int mp_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, uint32_t streamBase, uint64_t step,
+                    SolveStats *st) {
     if (!c.rs) {
         c.err = "mixed-precision CG: the context has no FP32 buffers";
         return YCN_ERR_UNSUPPORTED;
@@ -1195,10 +1218,10 @@ int mp_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, uint32_t 
     if (rc) return rc;
     const int maxIter = c.p.cgMaxIter;
     if (gen)
-        hipLaunchKernelGGL(k_mp_setup<true>, g, dim3(kNT), 0, c.stream, L, (const uint64_t *)c.seed_d, streamBase,
+        hipLaunchKernelGGL((k_mp_setup<NC, true>), g, dim3(kNT), 0, c.stream, L, (const uint64_t *)c.seed_d, streamBase,
                            step, c.eta, c.x, c.xs, c.rs, c.ps[0], c.ps[1], c.partials);
     else
-        hipLaunchKernelGGL(k_mp_setup<false>, g, dim3(kNT), 0, c.stream, L, (const uint64_t *)c.seed_d, streamBase,
+        hipLaunchKernelGGL((k_mp_setup<NC, false>), g, dim3(kNT), 0, c.stream, L, (const uint64_t *)c.seed_d, streamBase,
                            step, c.eta, c.x, c.xs, c.rs, c.ps[0], c.ps[1], c.partials);
     hipLaunchKernelGGL(k_fin_setup, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)c.partials, nb, c.cg_d,
                        c.active, c.p.cgTol, c.p.cgTolMode, maxIter, 0);
@@ -1210,19 +1233,19 @@ int mp_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, uint32_t 
     rc = poll_active(c, active);
     if (rc) return rc;
     while (active > 0 && launched < hardCap) {
-        rc = run_chunk(c, nullptr, nsys, mtype, nIt, YCN_CG_MIXED, c.tile32,
-                       [&](int i) { launch_mp_iteration(c, nsys, mtype, i & 1); });
+        rc = run_chunk(c, nullptr, nsys, mtype, nIt, YCN_CG_MIXED, NC, c.tile32,
+                       [&](int i) { launch_mp_iteration<NC>(c, nsys, mtype, i & 1); });
         if (rc) return rc;
         launched += nIt;
         // reliable update: x += xs; rs = b - A x in FP64
-        hipLaunchKernelGGL(k_mp_accum, g, dim3(kNT), 0, c.stream, c.V, (const CgState *)c.cg_d, c.x, c.xs);
+        hipLaunchKernelGGL(k_mp_accum<NC>, g, dim3(kNT), 0, c.stream, c.V, (const CgState *)c.cg_d, c.x, c.xs);
         if (mtype == YCN_DAGGER) {
-            hipLaunchKernelGGL(k_true_a<false>, g, dim3(kNT), 0, c.stream, L, phi, (const double2 *)c.x, c.t);
-            hipLaunchKernelGGL((k_true_b<true, true>), g, dim3(kNT), 0, c.stream, L, phi, (const CgState *)c.cg_d,
+            hipLaunchKernelGGL((k_true_a<NC, false>), g, dim3(kNT), 0, c.stream, L, phi, (const double2 *)c.x, c.t);
+            hipLaunchKernelGGL((k_true_b<NC, true, true>), g, dim3(kNT), 0, c.stream, L, phi, (const CgState *)c.cg_d,
                                (const double2 *)c.eta, (const double2 *)c.t, c.r, c.rs, c.partials);
         } else {
-            hipLaunchKernelGGL(k_true_a<true>, g, dim3(kNT), 0, c.stream, L, phi, (const double2 *)c.x, c.t);
-            hipLaunchKernelGGL((k_true_b<false, true>), g, dim3(kNT), 0, c.stream, L, phi, (const CgState *)c.cg_d,
+            hipLaunchKernelGGL((k_true_a<NC, true>), g, dim3(kNT), 0, c.stream, L, phi, (const double2 *)c.x, c.t);
+            hipLaunchKernelGGL((k_true_b<NC, false, true>), g, dim3(kNT), 0, c.stream, L, phi, (const CgState *)c.cg_d,
                                (const double2 *)c.eta, (const double2 *)c.t, c.r, c.rs, c.partials);
         }
         hipLaunchKernelGGL(k_fin_mp_true<false>, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)c.partials,
@@ -1234,17 +1257,35 @@ int mp_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, uint32_t 
     return read_stats(c, nsys, st);
 }
 
-int fermion_drift(Ctx &c, const double *phi, double *drift) {
+int fermion_drift(Ctx &c, const double *phi, SpinorForm form, double *drift) {
     const LatticeArgs L = largs(c);
     const double fac = -c.p.g * (c.p.driftMode == 1 ? c.p.cutFraction * c.p.cutFraction : 1.0);
-    hipLaunchKernelGGL(k_drift, site_grid(c, c.nRep), dim3(kNT), 0, c.stream, L, phi, (const double2 *)c.x,
+    hipLaunchKernelGGL(form == kPacked ? &k_drift<2> : &k_drift<4>, site_grid(c, c.nRep), dim3(kNT), 0, c.stream, L, phi, (const double2 *)c.x,
                        (const double2 *)c.eta, drift, fac);
     YCN_HIP(hipGetLastError());
     return YCN_OK;
 }
 
-int spinor_slices(Ctx &c, const double2 *psi, double *out_dev) {
-    hipLaunchKernelGGL(k_spinor_slices, dim3(c.p.Nt), dim3(kNT), 0, c.stream, psi, c.p.Nt, c.p.Nx, out_dev);
+// D^-1 src for the packed real source in c.eta (main.cu:441-469: CG on D D^dag, then
+// D^dag), left in out
+int plain_propagator(Ctx &c, const double *phi, double2 *out, SolveStats *st) {
+    int rc = cg_solve(c, phi, 1, YCN_NORMAL, kPacked, false, 0, 0, st);
+    if (rc) return rc;
+    const LatticeArgs L = largs(c);
+    hipLaunchKernelGGL((k_dirac<2, true>), site_grid(c, 1), dim3(kNT), 0, c.stream, L, phi, (const double2 *)c.x, out);
+    YCN_HIP(hipGetLastError());
+    return YCN_OK;
+}
+
+// the measurement's source (1, 1, 0, 0) at site 0, in c.eta
+int point_source(Ctx &c, SpinorForm form) {
+    hipLaunchKernelGGL(k_point_source, site_grid(c, 1), dim3(kNT), 0, c.stream, c.V, (int)form, c.eta);
+    YCN_HIP(hipGetLastError());
+    return YCN_OK;
+}
+
+int spinor_slices(Ctx &c, const double2 *psi, SpinorForm form, double *out_dev) {
+    hipLaunchKernelGGL(form == kPacked ? &k_spinor_slices<2> : &k_spinor_slices<4>, dim3(c.p.Nt), dim3(kNT), 0, c.stream, psi, c.p.Nt, c.p.Nx, out_dev);
     YCN_HIP(hipGetLastError());
     return YCN_OK;
 }
@@ -1257,16 +1298,17 @@ int spinor_slices(Ctx &c, const double2 *psi, double *out_dev) {
 // The FP64 true residual with the plain operator decides convergence.
 // ===========================================================================
 static void launch_fcg_iteration(Ctx &c, int nsys, int mtype, int parity) {
+    constexpr int NC = kComplex;   // the network mixes real and imaginary channels
     const float2 *pold = c.ps[parity];
     float2 *pnew = c.ps[parity ^ 1];
-    prof_before(c, PK_NORMAL_OP, (double)nsys * c.V * (4 * 32 + 4));
-    launch_fused<float>(c, c.tile32, nsys, mtype != YCN_DAGGER, c.phis, c.cg_d, (const float2 *)c.zs, pold, pnew,
+    prof_before(c, PK_NORMAL_OP, (double)nsys * c.V * (4 * NC * 8 + 4));
+    launch_fused<float, NC>(c, c.tile32, nsys, mtype != YCN_DAGGER, c.phis, c.cg_d, (const float2 *)c.zs, pold, pnew,
                         c.Aps, c.partials);
     prof_after(c, PK_NORMAL_OP);
     const int nbF = fused_args(c, kTiles32[c.tile32].TT, kTiles32[c.tile32].TX).tilesPerSys;
     hipLaunchKernelGGL(k_fin_alpha_fcg, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)c.partials, nbF, c.cg_d);
-    prof_before(c, PK_CG_UPDATE, (double)nsys * c.V * 6 * 32);
-    hipLaunchKernelGGL(k_mp_update, site_grid(c, nsys), dim3(kNT), 0, c.stream, c.V, (const CgState *)c.cg_d, c.xs,
+    prof_before(c, PK_CG_UPDATE, (double)nsys * c.V * 6 * NC * 8);
+    hipLaunchKernelGGL(k_mp_update<NC>, site_grid(c, nsys), dim3(kNT), 0, c.stream, c.V, (const CgState *)c.cg_d, c.xs,
                        c.rs, (const float2 *)pnew, (const float2 *)c.Aps, c.partials);
     prof_after(c, PK_CG_UPDATE);
     hipLaunchKernelGGL(k_fin_beta<true>, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)c.partials,
@@ -1277,6 +1319,7 @@ static void launch_fcg_iteration(Ctx &c, int nsys, int mtype, int parity) {
 
 int fcg_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, uint32_t streamBase, uint64_t step,
               SolveStats *st) {
+    constexpr int NC = kComplex;
     if (c.tile32 < 0 || !c.zs) {
         c.err = "the learned preconditioner needs Nt % 16 == 0 and Nx % 16 == 0";
         return YCN_ERR_UNSUPPORTED;
@@ -1294,10 +1337,10 @@ int fcg_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, uint32_t
     if (rc) return rc;
     const int maxIter = c.p.cgMaxIter;
     if (gen)
-        hipLaunchKernelGGL(k_mp_setup<true>, g, dim3(kNT), 0, c.stream, L, (const uint64_t *)c.seed_d, streamBase,
+        hipLaunchKernelGGL((k_mp_setup<NC, true>), g, dim3(kNT), 0, c.stream, L, (const uint64_t *)c.seed_d, streamBase,
                            step, c.eta, c.x, c.xs, c.rs, c.ps[0], c.ps[1], c.partials);
     else
-        hipLaunchKernelGGL(k_mp_setup<false>, g, dim3(kNT), 0, c.stream, L, (const uint64_t *)c.seed_d, streamBase,
+        hipLaunchKernelGGL((k_mp_setup<NC, false>), g, dim3(kNT), 0, c.stream, L, (const uint64_t *)c.seed_d, streamBase,
                            step, c.eta, c.x, c.xs, c.rs, c.ps[0], c.ps[1], c.partials);
     hipLaunchKernelGGL(k_fin_setup, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)c.partials, nb, c.cg_d,
                        c.active, c.p.cgTol, c.p.cgTolMode, maxIter, 0);
@@ -1313,13 +1356,13 @@ int fcg_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, uint32_t
     rc = poll_active(c, active);
     if (rc) return rc;
     while (active > 0 && launched < hardCap) {
-        rc = run_chunk(c, nullptr, nsys, mtype, nIt, 2 /* flexible */, c.tile32,
+        rc = run_chunk(c, nullptr, nsys, mtype, nIt, 2 /* flexible */, NC, c.tile32,
                        [&](int i) { launch_fcg_iteration(c, nsys, mtype, i & 1); });
         if (rc) return rc;
         launched += nIt;
-        hipLaunchKernelGGL(k_mp_accum, g, dim3(kNT), 0, c.stream, c.V, (const CgState *)c.cg_d, c.x, c.xs);
-        hipLaunchKernelGGL(k_true_a<false>, g, dim3(kNT), 0, c.stream, L, phi, (const double2 *)c.x, c.t);
-        hipLaunchKernelGGL((k_true_b<true, true>), g, dim3(kNT), 0, c.stream, L, phi, (const CgState *)c.cg_d,
+        hipLaunchKernelGGL(k_mp_accum<NC>, g, dim3(kNT), 0, c.stream, c.V, (const CgState *)c.cg_d, c.x, c.xs);
+        hipLaunchKernelGGL((k_true_a<NC, false>), g, dim3(kNT), 0, c.stream, L, phi, (const double2 *)c.x, c.t);
+        hipLaunchKernelGGL((k_true_b<NC, true, true>), g, dim3(kNT), 0, c.stream, L, phi, (const CgState *)c.cg_d,
                            (const double2 *)c.eta, (const double2 *)c.t, c.r, c.rs, c.partials);
         const double refRate = (c.plainIters > 0 && c.p.cgTol > 0.0) ? std::log10(c.p.cgTol) / c.plainIters : 0.0;
         hipLaunchKernelGGL(k_fin_mp_true<true>, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)c.partials, nb,
@@ -1346,6 +1389,7 @@ __global__ void __launch_bounds__(kNT) k_sub(const double2 *__restrict__ a, doub
 // evenly spaced iterations; once a solve has converged each pair (r_k, e_k = x* - x_k)
 // drives one Adam step of the network.  The chain itself advances as usual.
 int train_preconditioner(Ctx &c, uint64_t step0, int nsteps, int pairsPerSolve, float lr, int *pairsUsed) {
+    constexpr int NC = kComplex;
     if (c.nSys != 1) { c.err = "training runs on a single system (nReplicas = nNoise = 1)"; return YCN_ERR_UNSUPPORTED; }
     if (!c.cnnW || c.tile32 < 0) { c.err = "the learned preconditioner is not available on this lattice"; return YCN_ERR_UNSUPPORTED; }
     const size_t sp = (size_t)4 * c.V;
@@ -1371,15 +1415,15 @@ int train_preconditioner(Ctx &c, uint64_t step0, int nsteps, int pairsPerSolve, 
         // FP64 CG (the reference recurrence) with snapshots
         rc = set_int(c, c.active, 1);
         if (rc) return rc;
-        hipLaunchKernelGGL(k_cg_setup<true>, g, dim3(kNT), 0, c.stream, L, (const uint64_t *)c.seed_d, 1u, step, c.eta,
+        hipLaunchKernelGGL((k_cg_setup<NC, true>), g, dim3(kNT), 0, c.stream, L, (const uint64_t *)c.seed_d, 1u, step, c.eta,
                            c.x, c.r, c.pv[0], c.pv[1], c.partials);
         hipLaunchKernelGGL(k_fin_setup, dim3(1), dim3(kNT), 0, c.stream, (const double2 *)c.partials, nb, c.cg_d,
                            c.active, c.p.cgTol, c.p.cgTolMode, c.p.cgMaxIter, 4);
         const int pred = std::max(kGraphIters * (pairsPerSolve + 1), c.lastIters);
         int launched = 0, active = 1, taken = 0;
         while (active > 0 && launched < c.p.cgMaxIter) {
-            rc = run_chunk(c, phi, 1, YCN_DAGGER, kGraphIters, YCN_CG_FP64, c.tile64,
-                           [&](int i) { launch_iteration(c, L, phi, 1, YCN_DAGGER, i & 1); });
+            rc = run_chunk(c, phi, 1, YCN_DAGGER, kGraphIters, YCN_CG_FP64, NC, c.tile64,
+                           [&](int i) { launch_iteration<NC>(c, L, phi, 1, YCN_DAGGER, i & 1); });
             if (rc) return rc;
             launched += kGraphIters;
             if (taken < pairsPerSolve && launched >= (taken + 1) * pred / (pairsPerSolve + 1)) {
@@ -1397,7 +1441,7 @@ int train_preconditioner(Ctx &c, uint64_t step0, int nsteps, int pairsPerSolve, 
         if (rc) return rc;
         if (st.iters_max > 0) c.plainIters = st.iters_max;   // the flexible solver's yardstick
         // fermion drift and update: the chain advances exactly as a plain step
-        rc = fermion_drift(c, phi, c.drift);
+        rc = fermion_drift(c, phi, kComplex, c.drift);
         if (rc) return rc;
         rc = bosonic_update(c, c.p.adaptive ? 0 : 1);
         if (rc) return rc;

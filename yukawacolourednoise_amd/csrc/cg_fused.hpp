@@ -12,6 +12,8 @@
 // against 7S + 2P for the two-stencil dataflow.  Tiles are handed to the 8 XCDs in
 // contiguous bands so halo re-reads stay in one XCD's L2.
 #pragma once
+#include <type_traits>
+
 #include "ycn_device.hpp"
 #include "ycn_internal.hpp"
 
@@ -89,7 +91,7 @@ struct FusedArgs {
 
 __device__ __forceinline__ int wrapi(int a, int n) { return a < 0 ? a + n : (a >= n ? a - n : a); }
 
-template <typename R, int TT, int TX, bool DAG1>
+template <typename R, int TT, int TX, int NC, bool DAG1>
 __global__ void __launch_bounds__(TT *TX)
 k_cg_normal_fused(FusedArgs A, const R *__restrict__ phi, CgState *st,
                   const typename Vec2<R>::T *__restrict__ r, const typename Vec2<R>::T *__restrict__ pold,
@@ -99,8 +101,8 @@ k_cg_normal_fused(FusedArgs A, const R *__restrict__ phi, CgState *st,
     constexpr int NT = TT * TX;
     constexpr int W2 = TX + 4, H2 = TT + 4, N2 = W2 * H2;
     constexpr int W1 = TX + 2, H1 = TT + 2, N1 = W1 * H1;
-    __shared__ V2 P[4][N2];
-    __shared__ V2 Q[4][N1];
+    __shared__ V2 P[NC][N2];
+    __shared__ V2 Q[NC][N1];
     __shared__ R F[N1];
     __shared__ double2 red[NT / kWave > 0 ? NT / kWave : 1];
 
@@ -112,7 +114,7 @@ k_cg_normal_fused(FusedArgs A, const R *__restrict__ phi, CgState *st,
     const int ty = tile / A.tilesX, tx = tile - ty * A.tilesX;
     const int t0 = ty * TT, x0 = tx * TX;
     const int Nt = A.Nt, Nx = A.Nx;
-    const size_t V = A.V, off = (size_t)sys * 4 * V;
+    const size_t V = A.V, off = (size_t)sys * NC * V;
     const R beta = (R)st[sys].beta;
     const R *ph = phi + (size_t)(sys / A.nNoise) * V;
 
@@ -121,7 +123,7 @@ k_cg_normal_fused(FusedArgs A, const R *__restrict__ phi, CgState *st,
         const int gt = wrapi(t0 - 2 + row, Nt), gx = wrapi(x0 - 2 + col, Nx);
         const size_t gs = (size_t)gt * Nx + gx;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
+        for (int c = 0; c < NC; ++c) {
             const V2 a = r[off + c * V + gs], b = pold[off + c * V + gs];
             P[c][w] = mk2<R>(a.x + beta * b.x, a.y + beta * b.y);
         }
@@ -143,7 +145,7 @@ k_cg_normal_fused(FusedArgs A, const R *__restrict__ phi, CgState *st,
         const R sf = (gt == Nt - 1) ? (R)-1 : (R)1, sb = (gt == 0) ? (R)-1 : (R)1;
         const R d = d0 + g * F[w];
 #pragma unroll
-        for (int f = 0; f < 4; f += 2) {
+        for (int f = 0; f < NC; f += 2) {
             V2 o0, o1;
             wilson_flavour_r<DAG1, R, V2>(hp, hm, hr, h, d, P[f][i2], P[f + 1][i2], P[f][i2 + W2], P[f + 1][i2 + W2],
                                           sf, P[f][i2 - W2], P[f + 1][i2 - W2], sb, P[f][i2 + 1], P[f + 1][i2 + 1],
@@ -164,7 +166,7 @@ k_cg_normal_fused(FusedArgs A, const R *__restrict__ phi, CgState *st,
     const R d = d0 + g * F[i1];
     double2 acc = make_double2(0.0, 0.0);
 #pragma unroll
-    for (int f = 0; f < 4; f += 2) {
+    for (int f = 0; f < NC; f += 2) {
         V2 o0, o1;
         wilson_flavour_r<!DAG1, R, V2>(hp, hm, hr, h, d, Q[f][i1], Q[f + 1][i1], Q[f][i1 + W1], Q[f + 1][i1 + W1], sf,
                                        Q[f][i1 - W1], Q[f + 1][i1 - W1], sb, Q[f][i1 + 1], Q[f + 1][i1 + 1],
@@ -176,7 +178,7 @@ k_cg_normal_fused(FusedArgs A, const R *__restrict__ phi, CgState *st,
         Ap[off + (f + 1) * V + gs] = o1;
         // conj(p) * Ap accumulated in double
         acc.x += (double)(p0.x * o0.x + p0.y * o0.y) + (double)(p1.x * o1.x + p1.y * o1.y);
-        acc.y += (double)(p0.x * o0.y - p0.y * o0.x) + (double)(p1.x * o1.y - p1.y * o1.x);
+        if (NC == 4) acc.y += (double)(p0.x * o0.y - p0.y * o0.x) + (double)(p1.x * o1.y - p1.y * o1.x);
     }
     acc = block_sum2<NT>(acc, red);
     if (threadIdx.x == 0) part[(size_t)sys * nb + blockIdx.x] = acc;
@@ -196,16 +198,16 @@ constexpr TileShape kTiles32[] = {{8, 32}, {4, 64}, {16, 16}, {8, 64}, {16, 32},
 constexpr int kNumTiles64 = sizeof(kTiles64) / sizeof(kTiles64[0]);
 constexpr int kNumTiles32 = sizeof(kTiles32) / sizeof(kTiles32[0]);
 
-template <typename R, int TT, int TX>
+template <typename R, int TT, int TX, int NC>
 inline void launch_fused_tt(hipStream_t s, int nsys, bool dag1, const FusedArgs &A, const R *phi, CgState *st,
                             const typename Vec2<R>::T *r, const typename Vec2<R>::T *pold, typename Vec2<R>::T *pnew,
                             typename Vec2<R>::T *Ap, double2 *part) {
     dim3 grid(A.tilesPerSys, nsys), block(TT * TX);
     if (dag1)
-        hipLaunchKernelGGL((k_cg_normal_fused<R, TT, TX, true>), grid, block, 0, s, A, phi, st, r, pold, pnew, Ap,
+        hipLaunchKernelGGL((k_cg_normal_fused<R, TT, TX, NC, true>), grid, block, 0, s, A, phi, st, r, pold, pnew, Ap,
                            part);
     else
-        hipLaunchKernelGGL((k_cg_normal_fused<R, TT, TX, false>), grid, block, 0, s, A, phi, st, r, pold, pnew, Ap,
+        hipLaunchKernelGGL((k_cg_normal_fused<R, TT, TX, NC, false>), grid, block, 0, s, A, phi, st, r, pold, pnew, Ap,
                            part);
 }
 
@@ -227,37 +229,37 @@ inline FusedArgs fused_args(const Ctx &c, int TT, int TX) {
 inline bool tile_fits(const Ctx &c, TileShape t) { return c.p.Nt % t.TT == 0 && c.p.Nx % t.TX == 0; }
 
 // launch the fused normal operator with tile index `ti` of the table for R
-template <typename R>
+template <typename R, int NC>
 inline void launch_fused(const Ctx &c, int ti, int nsys, bool dag1, const R *phi, CgState *st,
                          const typename Vec2<R>::T *r, const typename Vec2<R>::T *pold, typename Vec2<R>::T *pnew,
-                         typename Vec2<R>::T *Ap, double2 *part);
-
-template <>
-inline void launch_fused<double>(const Ctx &c, int ti, int nsys, bool dag1, const double *phi, CgState *st,
-                                 const double2 *r, const double2 *pold, double2 *pnew, double2 *Ap, double2 *part) {
-    const TileShape t = kTiles64[ti];
+                         typename Vec2<R>::T *Ap, double2 *part) {
+    constexpr bool f64 = sizeof(R) == 8;
+    const TileShape t = f64 ? kTiles64[ti] : kTiles32[ti];
     const FusedArgs A = fused_args(c, t.TT, t.TX);
-    switch (ti) {
-    case 0: launch_fused_tt<double, 8, 32>(c.stream, nsys, dag1, A, phi, st, r, pold, pnew, Ap, part); break;
-    case 1: launch_fused_tt<double, 4, 64>(c.stream, nsys, dag1, A, phi, st, r, pold, pnew, Ap, part); break;
-    case 2: launch_fused_tt<double, 16, 16>(c.stream, nsys, dag1, A, phi, st, r, pold, pnew, Ap, part); break;
-    default: launch_fused_tt<double, 4, 32>(c.stream, nsys, dag1, A, phi, st, r, pold, pnew, Ap, part); break;
+    auto go = [&](auto tt, auto tx) {
+        launch_fused_tt<R, decltype(tt)::value, decltype(tx)::value, NC>(c.stream, nsys, dag1, A, phi, st, r, pold,
+                                                                         pnew, Ap, part);
+    };
+#define YCN_TILE_CASE(T, X) \
+    case T * 1000 + X: go(std::integral_constant<int, T>(), std::integral_constant<int, X>()); break
+    if constexpr (f64) {
+        switch (t.TT * 1000 + t.TX) {
+            YCN_TILE_CASE(8, 32);
+            YCN_TILE_CASE(4, 64);
+            YCN_TILE_CASE(16, 16);
+            YCN_TILE_CASE(4, 32);
+        }
+    } else {
+        switch (t.TT * 1000 + t.TX) {
+            YCN_TILE_CASE(8, 32);
+            YCN_TILE_CASE(4, 64);
+            YCN_TILE_CASE(16, 16);
+            YCN_TILE_CASE(8, 64);
+            YCN_TILE_CASE(16, 32);
+            YCN_TILE_CASE(4, 16);
+        }
     }
-}
-
-template <>
-inline void launch_fused<float>(const Ctx &c, int ti, int nsys, bool dag1, const float *phi, CgState *st,
-                                const float2 *r, const float2 *pold, float2 *pnew, float2 *Ap, double2 *part) {
-    const TileShape t = kTiles32[ti];
-    const FusedArgs A = fused_args(c, t.TT, t.TX);
-    switch (ti) {
-    case 0: launch_fused_tt<float, 8, 32>(c.stream, nsys, dag1, A, phi, st, r, pold, pnew, Ap, part); break;
-    case 1: launch_fused_tt<float, 4, 64>(c.stream, nsys, dag1, A, phi, st, r, pold, pnew, Ap, part); break;
-    case 2: launch_fused_tt<float, 16, 16>(c.stream, nsys, dag1, A, phi, st, r, pold, pnew, Ap, part); break;
-    case 3: launch_fused_tt<float, 8, 64>(c.stream, nsys, dag1, A, phi, st, r, pold, pnew, Ap, part); break;
-    case 4: launch_fused_tt<float, 16, 32>(c.stream, nsys, dag1, A, phi, st, r, pold, pnew, Ap, part); break;
-    default: launch_fused_tt<float, 4, 16>(c.stream, nsys, dag1, A, phi, st, r, pold, pnew, Ap, part); break;
-    }
+#undef YCN_TILE_CASE
 }
 
 }  // namespace ycn

@@ -651,9 +651,9 @@ int cnn_train_step(Ctx &c, const double2 *r, const double2 *e, const float *phis
     S0.beta = 0.0;
     S0.done = 0;
     YCN_HIP(hipMemcpyAsync(c.cg_d, &S0, sizeof(CgState), hipMemcpyHostToDevice, c.stream));
-    launch_fused<float>(c, c.tile32, 1, false, phis, c.cg_d, (const float2 *)c.rs, c.ps[0], c.ps[1], c.Aps,
+    launch_fused<float, kComplex>(c, c.tile32, 1, false, phis, c.cg_d, (const float2 *)c.rs, c.ps[0], c.ps[1], c.Aps,
                         c.partials);
-    launch_fused<float>(c, c.tile32, 1, false, phis, c.cg_d, (const float2 *)c.Aps, c.ps[0], c.ps[1], c.zs,
+    launch_fused<float, kComplex>(c, c.tile32, 1, false, phis, c.cg_d, (const float2 *)c.Aps, c.ps[0], c.ps[1], c.zs,
                         c.partials);
     hipLaunchKernelGGL(k_dot_f2, dim3(nred), dim3(kCT), 0, c.stream, (const float2 *)c.Aps, (const float2 *)c.Aps,
                        4 * V, red);

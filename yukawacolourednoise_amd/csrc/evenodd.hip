@@ -1557,7 +1557,7 @@ static int eo_mixed_chunk(Ctx &c, const double *phi, int nsys, int n, bool graph
     if (graphed) {   // already inside a capture: the launches themselves
         for (int i = 0; i < n; ++i) launch_eo_pf_iteration(c, nsys, i);
     } else {
-        const int rc = run_chunk(c, nullptr, nsys, YCN_DAGGER, n, 4, c.tileEo32,
+        const int rc = run_chunk(c, nullptr, nsys, YCN_DAGGER, n, 4, kComplex, c.tileEo32,
                                  [&](int i) { launch_eo_pf_iteration(c, nsys, i); });
         if (rc) return rc;
     }
@@ -1671,7 +1671,7 @@ int eo_solve(Ctx &c, const double *phi, int nsys, bool gen, uint32_t streamBase,
         while (active > 0 && launched < hardCap) {
             const int n = std::min(chunk, hardCap - launched);
             for (int k = 0; k < n; k += kGraphIters) {
-                rc = run_chunk(c, phi, nsys, YCN_DAGGER, kGraphIters, 3, c.tileEo64,
+                rc = run_chunk(c, phi, nsys, YCN_DAGGER, kGraphIters, 3, kComplex, c.tileEo64,
                                [&](int i) { launch_eo_iteration(c, nsys, phi, i & 1); });
                 if (rc) return rc;
             }

@@ -410,7 +410,7 @@ int ycn_cg_solve(ycn_ctx *ctx, const double *phi, const double *b, double *x, in
     const int save = c.nNoise;
     c.nNoise = 1;
     SolveStats st;
-    rc = cg_solve(c, phi_dev, 1, mtype, false, 0, 0, &st);
+    rc = cg_solve(c, phi_dev, 1, mtype, kComplex, false, 0, 0, &st);
     c.nNoise = save;
     if (rc) return rc;
     if ((rc = soa_to_aos(c, c.x, (double *)aos.p, 1))) return rc;
@@ -426,9 +426,12 @@ static int force_impl(Ctx &c, uint64_t step, uint32_t streamBase, SolveStats *st
         if (rc) return rc;
         return eo_drift(c, c.phi[c.cur], c.drift);
     }
-    int rc = cg_solve(c, c.phi[c.cur], c.nSys, YCN_DAGGER, true, streamBase, step, st);
+    // eta and D are real: packed real vectors, except where the network mixes in imaginary
+    // channels
+    const SpinorForm form = c.p.precond == YCN_PRECOND_CNN ? kComplex : kPacked;
+    int rc = cg_solve(c, c.phi[c.cur], c.nSys, YCN_DAGGER, form, true, streamBase, step, st);
     if (rc) return rc;
-    return fermion_drift(c, c.phi[c.cur], c.drift);
+    return fermion_drift(c, c.phi[c.cur], form, c.drift);
 }
 
 int ycn_fermion_force(ycn_ctx *ctx, uint64_t step, double *drift, ycn_cg_stats *stats) {
@@ -566,28 +569,17 @@ int ycn_measure(ycn_ctx *ctx, int replica, uint64_t step, ycn_observables *obs, 
     o.clamp_events = S[replica].clamps;
     const double *phi_rep = c.phi[c.cur] + (size_t)replica * c.V;
     if (corr) {
-        // point source (main.cu:441-469): delta_{x,0} (1,1,0,0); CG on D D^dag, then D^dag,
-        // i.e. D^-1 src (with even-odd preconditioning: the Schur-complement solve)
-        std::vector<double> src(8 * (size_t)c.V, 0.0);
-        src[0] = 1.0;
-        src[2] = 1.0;
-        DevTmp aos;
-        const size_t nb = sizeof(double) * src.size();
-        YCN_HIP(hipMalloc(&aos.p, nb));
-        YCN_HIP(hipMemcpyAsync(aos.p, src.data(), nb, hipMemcpyHostToDevice, c.stream));
-        if ((rc = aos_to_soa(c, (const double *)aos.p, c.eta, 1))) return rc;
+        // D^-1 of the point source delta_{x,0} (1,1,0,0) (main.cu:441-469; with even-odd
+        // preconditioning by the Schur-complement solve)
         const int save = c.nNoise;
         c.nNoise = 1;
         SolveStats st;
-        if (c.p.evenOdd && eo_available(c)) {
-            rc = eo_propagator(c, phi_rep, c.t, &st);
-        } else {
-            rc = cg_solve(c, phi_rep, 1, YCN_NORMAL, false, 0, 0, &st);
-            if (!rc) rc = dirac_apply(c, phi_rep, c.x, c.t, 1, 1);
-        }
+        const bool eo = c.p.evenOdd && eo_available(c);
+        rc = point_source(c, eo ? kComplex : kPacked);
+        if (!rc) rc = eo ? eo_propagator(c, phi_rep, c.t, &st) : plain_propagator(c, phi_rep, c.t, &st);
         c.nNoise = save;
         if (rc) return rc;
-        if ((rc = spinor_slices(c, c.t, cr))) return rc;
+        if ((rc = spinor_slices(c, c.t, eo ? kComplex : kPacked, cr))) return rc;
         YCN_HIP(hipMemcpyAsync(corr, cr, sizeof(double) * Nt, hipMemcpyDeviceToHost, c.stream));
         YCN_HIP(hipStreamSynchronize(c.stream));
     }

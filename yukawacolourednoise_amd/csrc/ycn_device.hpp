@@ -188,4 +188,39 @@ __device__ __forceinline__ void eta_site(const uint64_t *seeds, uint32_t streamB
     b[3] = make_double2(g1.y, 0.0);
 }
 
+// ---------------------------------------------------------------------------
+// Packed real spinors.  D is a real matrix, the same for both flavours, and eta is real
+// (FermionicDrift.cu:102-110), so every vector of a fermion-force solve is real: the
+// imaginary halves of the complex form are exactly zero throughout.  The packed form keeps
+// two planes per system, plane s = (flavour 0, flavour 1) of spin s as the two members of a
+// V2, so the complex form's kernels run on it with NC = 2 planes instead of 4: half the
+// bytes, LDS and arithmetic, and the same products and sums.  The complex form (NC = 4)
+// stays for complex right-hand sides and the learned preconditioner.
+// ---------------------------------------------------------------------------
+template <int NC>
+__device__ __forceinline__ void eta_planes(const uint64_t *seeds, uint32_t streamBase, uint64_t step, int sys,
+                                           int nNoise, int s, double2 b[NC]) {
+    double2 e[4];
+    eta_site(seeds, streamBase, step, sys, nNoise, s, e);
+    if constexpr (NC == 4) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) b[c] = e[c];
+    } else {
+        b[0] = make_double2(e[0].x, e[2].x);
+        b[1] = make_double2(e[1].x, e[3].x);
+    }
+}
+// conj(a) b of one plane; the packed members are two reals, whose product sum is real
+template <int NC>
+__device__ __forceinline__ double2 pdot(double2 a, double2 b) {
+    if constexpr (NC == 4) return cdotc(a, b);
+    return make_double2(a.x * b.x + a.y * b.y, 0.0);
+}
+// alpha v of one plane (alpha is real in the packed form)
+template <int NC>
+__device__ __forceinline__ double2 pscale(double2 al, double2 v) {
+    if constexpr (NC == 4) return cmul(al, v);
+    return cscl(al.x, v);
+}
+
 }  // namespace ycn

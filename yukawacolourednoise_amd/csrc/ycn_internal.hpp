@@ -189,7 +189,7 @@ struct Ctx {
     // captured CG iteration chunks: key -> executable graph
     struct GraphEntry {
         const void *phi;
-        int nsys, mtype, n, precision, tile;
+        int nsys, mtype, n, precision, planes, tile;
         hipGraphExec_t exec;
     };
     std::vector<GraphEntry> graphs;
@@ -243,21 +243,26 @@ struct SolveStats {
     int iters_max = 0, restarts = 0, converged = 1, systems = 0;
     double rr_max = 0, true_rel_max = 0, iters_mean = 0;
 };
+// planes of two reals per site of a solve's vectors (ycn_device.hpp): complex components, or
+// the packed real form of the fermion force
+enum SpinorForm { kComplex = 4, kPacked = 2 };
 int cg_alloc(Ctx &c);
 void cg_free(Ctx &c);
 int cg_autotune(Ctx &c);
 // mixed precision (cg_mixed.hip)
 int mp_alloc(Ctx &c);
 void mp_free(Ctx &c);
-int mp_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, uint32_t streamBase, uint64_t step,
-             SolveStats *st);
 int dirac_apply(Ctx &c, const double *phi_dev, const double2 *in, double2 *out, int nsys, int dagger);
 // b: if gen, eta is generated from (seeds, streamBase + j, step); else eta must hold b.
-int cg_solve(Ctx &c, const double *phi_dev, int nsys, int mtype, bool gen, uint32_t streamBase,
+int cg_solve(Ctx &c, const double *phi_dev, int nsys, int mtype, SpinorForm form, bool gen, uint32_t streamBase,
              uint64_t step, SolveStats *st);
-int fermion_drift(Ctx &c, const double *phi_dev, double *drift_dev);
+// the solver's vectors of the last fermion-force solve (form) -> drift
+int fermion_drift(Ctx &c, const double *phi_dev, SpinorForm form, double *drift_dev);
+// measurement: the point source in c.eta, and D^-1 of it in out (packed)
+int point_source(Ctx &c, SpinorForm form);
+int plain_propagator(Ctx &c, const double *phi, double2 *out, SolveStats *st);
 // correlator / trace helpers
-int spinor_slices(Ctx &c, const double2 *psi, double *out_dev);
+int spinor_slices(Ctx &c, const double2 *psi, SpinorForm form, double *out_dev);
 
 // cnn.hip
 int cnn_alloc(Ctx &c);
@@ -293,13 +298,11 @@ int stats_from_mirror(Ctx &c, int nsys, SolveStats *st);
 int read_stats(Ctx &c, int nsys, SolveStats *st);
 // CG building blocks shared with the even-odd solver (cg.hip): finalize alpha / beta from
 // the partials in c.partials, the BLAS-1 updates x += alpha p, r -= alpha Ap on
-// [nsys][4][n] vectors (c.x, c.r, c.Ap; mixed: c.xs, c.rs, c.Aps), returning their block
-// count, the reliable-update accumulation x += x_s, and an FP64 -> FP32 copy.
+// [nsys][4][n] vectors (c.x, c.r, c.Ap), returning their block count, and an FP64 -> FP32
+// copy.
 void launch_fin_alpha(Ctx &c, int nsys, int nb);
 void launch_fin_beta(Ctx &c, int nsys, int nb, bool mixed, bool even);
 int launch_cg_update(Ctx &c, int nsys, int n, const double2 *p);
-int launch_mp_update(Ctx &c, int nsys, int n, const float2 *p);
-int launch_mp_accum(Ctx &c, int nsys, int n);
 // b = (float)a over n entries; halt: return at once while *halt is set; copy: also
 // copy a there (FP64)
 int to_f32_n(Ctx &c, const double *a, float *b, int64_t n, const int *halt = nullptr, double *copy = nullptr);
