@@ -22,7 +22,7 @@ def test_packed_force(gpu, Nt, Nx, r, vectors):
         c.set_field(phi)
         d, st = c.fermion_force(3)
     dr, sr = O.fermion_drift(orc, phi, 3)
-    assert st["iters"] == sr["iters"]
+    assert vectors * st["iters"] == sr["iters"]   # the oracle adds up its solves
     assert rel(d, dr) < RTOL
 
 
@@ -38,5 +38,5 @@ def test_complex_solve_after_packed_force(gpu):
         c.set_field(phi)
         c.fermion_force(0)
         x, _ = c.cg_solve(b)
-    xr, _ = O.cg_solve(orc, phi, b)
+    xr, _ = O.cg(orc, phi, b, Y.YCN_DAGGER)
     assert rel(x, xr) < RTOL

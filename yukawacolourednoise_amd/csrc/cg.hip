@@ -1269,7 +1269,12 @@ int fermion_drift(Ctx &c, const double *phi, SpinorForm form, double *drift) {
 // D^-1 src for the packed real source in c.eta (main.cu:441-469: CG on D D^dag, then
 // D^dag), left in out
 int plain_propagator(Ctx &c, const double *phi, double2 *out, SolveStats *st) {
-    int rc = cg_solve(c, phi, 1, YCN_NORMAL, kPacked, false, 0, 0, st);
+    int rc;
+    if (onchip_plain(c)) {
+        rc = onchip_propagator(c, phi, out);
+        return rc ? rc : read_stats(c, 1, st);
+    }
+    rc = cg_solve(c, phi, 1, YCN_NORMAL, kPacked, false, 0, 0, st);
     if (rc) return rc;
     const LatticeArgs L = largs(c);
     hipLaunchKernelGGL((k_dirac<2, true>), site_grid(c, 1), dim3(kNT), 0, c.stream, L, phi, (const double2 *)c.x, out);

@@ -259,6 +259,7 @@ int ycn_create(const ycn_params *p, ycn_ctx **out) {
     // YCN_STEP_GRAPHS=0 keeps ycn_langevin_run on single eagerly launched steps (with
     // captured CG chunks) where it would replay whole captured steps; results are identical
     if (const char *sg = std::getenv("YCN_STEP_GRAPHS")) c.stepGraphsOn = std::atoi(sg) != 0;
+    if ((rc = onchip_init(c))) return bail(rc);
     if ((rc = cg_autotune(c))) return bail(rc);
     if (c.p.evenOdd) {
         if (c.p.precond == YCN_PRECOND_CNN) {
@@ -425,6 +426,10 @@ static int force_impl(Ctx &c, uint64_t step, uint32_t streamBase, SolveStats *st
         int rc = eo_solve(c, c.phi[c.cur], c.nSys, true, streamBase, step, st);
         if (rc) return rc;
         return eo_drift(c, c.phi[c.cur], c.drift);
+    }
+    if (onchip_plain(c)) {   // the whole solve and its drift in one launch
+        const int rc = onchip_force(c, c.phi[c.cur], streamBase, step);
+        return rc ? rc : read_stats(c, c.nSys, st);
     }
     // eta and D are real: packed real vectors, except where the network mixes in imaginary
     // channels

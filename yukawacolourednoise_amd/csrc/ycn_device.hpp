@@ -62,12 +62,36 @@ __device__ __forceinline__ double2 normal_pair(uint64_t seed, uint32_t stream, u
 }
 
 // ---------------------------------------------------------------------------
-// deterministic reductions: wave64 butterfly, then LDS across waves
+// deterministic reductions: DPP within a wave, then LDS across waves
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
+// a DPP lane permutation of a double (its two 32-bit halves)
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xF, 0xF, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+// v of one lane in every lane
+__device__ __forceinline__ double lane_f64(double v, int lane) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane((int)b, lane), hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+// sum over each row of 16 lanes, in every lane of the row: the partner at distance 1 and 2
+// (quad permutations), then the mirrored half row and row
+__device__ __forceinline__ double row_sum(double v) {
+    v += dpp_f64<0xB1>(v);    // quad_perm [1, 0, 3, 2]
+    v += dpp_f64<0x4E>(v);    // quad_perm [2, 3, 0, 1]
+    v += dpp_f64<0x141>(v);   // row_half_mirror
+    v += dpp_f64<0x140>(v);   // row_mirror
     return v;
+}
+// sum over the wave, in every lane.  DPP moves cost a few cycles where the LDS permute of
+// __shfl_xor costs a round trip of about 100 for each of its six steps.
+__device__ __forceinline__ double wave_sum(double v) {
+    v = row_sum(v);
+    return (lane_f64(v, 0) + lane_f64(v, 16)) + (lane_f64(v, 32) + lane_f64(v, 48));
 }
 __device__ __forceinline__ double wave_max(double v) {
 #pragma unroll

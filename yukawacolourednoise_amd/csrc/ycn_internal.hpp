@@ -194,6 +194,7 @@ struct Ctx {
     };
     std::vector<GraphEntry> graphs;
     bool useGraphs = true;
+    bool onchip = false;                  // solves that fit one workgroup run in one launch (YCN_ONCHIP=0: never)
 
     // profiling
     int profTarget = PK_NONE;
@@ -306,6 +307,13 @@ int launch_cg_update(Ctx &c, int nsys, int n, const double2 *p);
 // b = (float)a over n entries; halt: return at once while *halt is set; copy: also
 // copy a there (FP64)
 int to_f32_n(Ctx &c, const double *a, float *b, int64_t n, const int *halt = nullptr, double *copy = nullptr);
+
+// fermion-force solves of one workgroup per system (onchip.hip): whether the plain solvers'
+// packed solves take it, the force into c.drift, and D^-1 of the source in c.eta
+int onchip_init(Ctx &c);
+bool onchip_plain(const Ctx &c);
+int onchip_force(Ctx &c, const double *phi, uint32_t streamBase, uint64_t step);
+int onchip_propagator(Ctx &c, const double *phi, double2 *out);
 
 // even-odd preconditioned fermion force (evenodd.hip)
 bool eo_available(const Ctx &c);
