@@ -1,18 +1,27 @@
 // noise.hip -- coloured noise on gfx950 (replaces ColouredNoise,
 // code/src/colouredNoise.cpp:16-29,40-67,138-178, and its cuFFT D2Z/Z2D calls).
 //
-// Three LDS passes, all mixed-radix Stockham FFTs (radix 4/2 specialised, any other
-// prime factor by a direct DFT):
+// Mixed-radix Stockham FFTs in LDS (radix 16, 8, 4, 2, 3, 5 and 7 butterflies in registers,
+// any other prime by a direct DFT), in three passes:
 //   rows_fwd : Philox N(0,1) field generated in registers, rows t and t+1 packed as
 //              z = xi_t + i xi_{t+1}, forward FFT along x, untangled into the two
-//              half spectra (kx = 0..Nx/2) -> spec[rep][t][kx]
+//              half spectra -> spec[rep][t][kx]
 //   cols     : each kx column: forward FFT along t, mask (kx <= kmax[kt] ? 1/V : 0),
 //              inverse FFT along t, in place
 //   rows_inv : rows t, t+1 re-packed with the Hermitian extension (C2R convention:
 //              imaginary parts of the kx = 0 and kx = Nx/2 bins are ignored), inverse
 //              FFT along x, real/imag parts -> noise rows t, t+1
+// Columns beyond the cutoff, kx > kmaxAll, are neither written, transformed nor read: with
+// cutoff s about a share s sqrt(2) of them is kept.  A lattice whose half spectrum fits LDS
+// takes one block per replica and one launch for everything.
 // Algorithmic HBM traffic ~ 8 (rows_fwd write) + 16 (cols r/w) + 8 + 8 (rows_inv)
 // = 40 bytes per site.
+//
+// What bounds it is latency: at 1024 x 1024 a pass holds 512 lines of 1024 points, four
+// waves per CU at 8 points per thread, and each FFT pass is an LDS round trip, a barrier and
+// a twiddle load.  So the passes are few (1024 = 16 x 8 x 8), index divisions are
+// multiplications, LDS rows are padded against the power-of-two strides of the first pass,
+// and a launch has as many blocks as lines allow.
 #include <math.h>
 
 #include <algorithm>
@@ -25,67 +34,193 @@
 namespace ycn {
 
 constexpr int kFftThreads = 256;
-constexpr int kFftLdsBytes = 65536;  // two ping-pong buffers per block
+constexpr int kFftLdsBytes = 73760;  // two padded ping-pong buffers per block (one line of 2048)
 
 // ---------------------------------------------------------------------------
-// LDS Stockham FFT over `lines` lines of length n stored at a[line*n + e].
-// Returns the buffer holding the result (a or b).  sign -1 forward, +1 inverse.
+// DFTs of one butterfly in registers, natural order in and out
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ double2 tw_get(const double2 *tw, int e, int sign) {
-    const double2 w = tw[e];
-    return sign < 0 ? w : make_double2(w.x, -w.y);
+// v times -i (forward) or +i (inverse)
+template <bool INV>
+__device__ __forceinline__ double2 rot(double2 v) {
+    return INV ? make_double2(-v.y, v.x) : make_double2(v.y, -v.x);
+}
+// v times exp(-+ i phi), given (cos phi, sin phi)
+template <bool INV>
+__device__ __forceinline__ double2 twid(double2 v, double2 w) {   // w = exp(-i phi) from the table
+    return INV ? make_double2(v.x * w.x + v.y * w.y, v.y * w.x - v.x * w.y) : cmul(v, w);
+}
+template <bool INV>
+__device__ __forceinline__ void dft4(double2 &a, double2 &b, double2 &c, double2 &d) {
+    const double2 t0 = cadd(a, c), t1 = csub(a, c), t2 = cadd(b, d), t3 = rot<INV>(csub(b, d));
+    a = cadd(t0, t2);
+    b = cadd(t1, t3);
+    c = csub(t0, t2);
+    d = csub(t1, t3);
+}
+// cos(2 pi k / R), sin(2 pi k / R) of the odd radices
+template <int R> struct OddRoots;
+template <> struct OddRoots<3> {
+    static constexpr double c[3] = {1.0, -0.5, -0.5};
+    static constexpr double s[3] = {0.0, 0.86602540378443864676, -0.86602540378443864676};
+};
+template <> struct OddRoots<5> {
+    static constexpr double c[5] = {1.0, 0.30901699437494742410, -0.80901699437494742410, -0.80901699437494742410,
+                                    0.30901699437494742410};
+    static constexpr double s[5] = {0.0, 0.95105651629515357212, 0.58778525229247312917, -0.58778525229247312917,
+                                    -0.95105651629515357212};
+};
+template <> struct OddRoots<7> {
+    static constexpr double c[7] = {1.0, 0.62348980185873353053, -0.22252093395631440429, -0.90096886790241912624,
+                                    -0.90096886790241912624, -0.22252093395631440429, 0.62348980185873353053};
+    static constexpr double s[7] = {0.0, 0.78183148246802980871, 0.97492791218182360702, 0.43388373911755812048,
+                                    -0.43388373911755812048, -0.97492791218182360702, -0.78183148246802980871};
+};
+template <int R, bool INV>
+__device__ __forceinline__ void dft(double2 (&v)[R]) {
+    if constexpr (R == 2) {
+        const double2 a = v[0];
+        v[0] = cadd(a, v[1]);
+        v[1] = csub(a, v[1]);
+    } else if constexpr (R == 4) {
+        dft4<INV>(v[0], v[1], v[2], v[3]);
+    } else if constexpr (R == 8) {
+        constexpr double h = 0.70710678118654752440;
+        dft4<INV>(v[0], v[2], v[4], v[6]);
+        dft4<INV>(v[1], v[3], v[5], v[7]);
+        v[3] = twid<INV>(v[3], make_double2(h, -h));
+        v[5] = rot<INV>(v[5]);
+        v[7] = twid<INV>(v[7], make_double2(-h, -h));
+        double2 o[8];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            o[k] = cadd(v[2 * k], v[2 * k + 1]);
+            o[k + 4] = csub(v[2 * k], v[2 * k + 1]);
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = o[k];
+    } else if constexpr (R == 16) {
+        // 4 x 4: columns, twiddles exp(-2 pi i n k / 16), rows
+        constexpr double h = 0.70710678118654752440, c = 0.92387953251128675613, d = 0.38268343236508977173;
+#pragma unroll
+        for (int n = 0; n < 4; ++n) dft4<INV>(v[n], v[n + 4], v[n + 8], v[n + 12]);
+        v[5] = twid<INV>(v[5], make_double2(c, -d));
+        v[9] = twid<INV>(v[9], make_double2(h, -h));
+        v[13] = twid<INV>(v[13], make_double2(d, -c));
+        v[6] = twid<INV>(v[6], make_double2(h, -h));
+        v[10] = rot<INV>(v[10]);
+        v[14] = twid<INV>(v[14], make_double2(-h, -h));
+        v[7] = twid<INV>(v[7], make_double2(d, -c));
+        v[11] = twid<INV>(v[11], make_double2(-h, -h));
+        v[15] = twid<INV>(v[15], make_double2(-c, d));
+#pragma unroll
+        for (int k = 0; k < 4; ++k) dft4<INV>(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
+        // X[k1 + 4 k2] sits at v[4 k1 + k2]: transpose
+        double2 o[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) o[k] = v[4 * (k & 3) + (k >> 2)];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) v[k] = o[k];
+    } else {
+        // odd prime: pairs q, R - q
+        constexpr int M = (R - 1) / 2;
+        double2 sm[M], df[M], o[R];
+        o[0] = v[0];
+#pragma unroll
+        for (int q = 0; q < M; ++q) {
+            sm[q] = cadd(v[q + 1], v[R - 1 - q]);
+            df[q] = csub(v[q + 1], v[R - 1 - q]);
+            o[0] = cadd(o[0], sm[q]);
+        }
+#pragma unroll
+        for (int k = 1; k <= M; ++k) {
+            double2 e = v[0], f = make_double2(0.0, 0.0);
+#pragma unroll
+            for (int q = 0; q < M; ++q) {
+                e = cadd(e, cscl(OddRoots<R>::c[((q + 1) * k) % R], sm[q]));
+                f = cadd(f, cscl(OddRoots<R>::s[((q + 1) * k) % R], df[q]));
+            }
+            f = rot<INV>(f);
+            o[k] = cadd(e, f);
+            o[R - k] = csub(e, f);
+        }
+#pragma unroll
+        for (int k = 0; k < R; ++k) v[k] = o[k];
+    }
 }
 
-__device__ double2 *lds_fft(double2 *a, double2 *b, int lines, const FftPlan &P, int sign) {
-    const int n = P.n;
+// ---------------------------------------------------------------------------
+// LDS Stockham FFT over `lines` lines of length n, element e of a line at fft_at(e) of its
+// row of fft_row(n) entries: one entry of padding in eight, so that the first pass's stores
+// at strides of the radix spread over the banks.
+// ---------------------------------------------------------------------------
+__host__ __device__ __forceinline__ int fft_at(int e) { return e + (e >> 3); }
+__host__ __device__ __forceinline__ int fft_row(int n) { return n + (n >> 3) + 1; }
+// a / n for 0 <= a < 2^22 with inv = 1 / n in single precision: (a + 1/2) / n lies at least
+// 1 / (2n) from an integer and the roundings move it by less
+__device__ __forceinline__ int fast_div(int a, float inv) { return (int)(((float)a + 0.5f) * inv); }
+
+template <int R, bool INV>
+__device__ __forceinline__ void fft_pass(const double2 *a, double2 *b, int lines, int n, int Ns,
+                                         const double2 *__restrict__ tw) {
+    const int nb = n / R, tstride = nb / Ns, row = fft_row(n);
+    const float invNb = 1.0f / (float)nb, invNs = 1.0f / (float)Ns;
+    for (int w = threadIdx.x; w < nb * lines; w += blockDim.x) {
+        const int line = fast_div(w, invNb), j = w - line * nb;
+        const int jd = fast_div(j, invNs), jm = j - jd * Ns;
+        const double2 *in = a + line * row;
+        double2 *out = b + line * row;
+        double2 v[R];
+#pragma unroll
+        for (int q = 0; q < R; ++q) v[q] = in[fft_at(j + q * nb)];
+        if (jm) {
+            const int ts = jm * tstride;
+#pragma unroll
+            for (int q = 1; q < R; ++q) v[q] = twid<INV>(v[q], tw[q * ts]);
+        }
+        dft<R, INV>(v);
+        const int o = jd * Ns * R + jm;
+#pragma unroll
+        for (int k = 0; k < R; ++k) out[fft_at(o + k * Ns)] = v[k];
+    }
+}
+
+// any other prime factor: one thread per output, a direct sum of R terms
+template <bool INV>
+__device__ void fft_pass_prime(const double2 *a, double2 *b, int lines, const FftPlan &P, int R, int Ns) {
+    const int n = P.n, nb = n / R, tstride = nb / Ns, row = fft_row(n);
+    for (int w = threadIdx.x; w < n * lines; w += blockDim.x) {
+        const int line = w / n, o = w - line * n;
+        const int jd = o / (Ns * R), rem = o - jd * Ns * R, k = rem / Ns, jm = rem - k * Ns;
+        const int j = jd * Ns + jm;
+        const double2 *in = a + line * row;
+        // exponent per input: the Stockham twiddle and the DFT kernel w_R^{qk}, modulo n
+        const int step = (jm * tstride + k * nb) % n;
+        double2 acc = in[fft_at(j)];
+        int e = 0;
+        for (int q = 1; q < R; ++q) {
+            e += step;
+            if (e >= n) e -= n;
+            acc = cadd(acc, twid<INV>(in[fft_at(j + q * nb)], P.tw[e]));
+        }
+        b[line * row + fft_at(o)] = acc;
+    }
+}
+
+// transforms a (barrier before and after); returns the buffer holding the result (a or b)
+template <bool INV>
+__device__ double2 *lds_fft(double2 *a, double2 *b, int lines, const FftPlan &P) {
     int Ns = 1;
     for (int f = 0; f < P.nf; ++f) {
         const int R = P.radix[f];
-        const int nb = n / R;
-        const int tstride = n / (Ns * R);
-        for (int w = threadIdx.x; w < nb * lines; w += blockDim.x) {
-            const int line = w / nb, j = w - line * nb;
-            const double2 *xin = a + line * n;
-            double2 *yout = b + line * n;
-            const int jm = j % Ns;
-            const int tstep = jm * tstride;
-            const int idx = (j / Ns) * Ns * R + jm;
-            if (R == 4) {
-                double2 v0 = xin[j], v1 = xin[j + nb], v2 = xin[j + 2 * nb], v3 = xin[j + 3 * nb];
-                if (tstep) {
-                    v1 = cmul(v1, tw_get(P.tw, tstep, sign));
-                    v2 = cmul(v2, tw_get(P.tw, 2 * tstep, sign));
-                    v3 = cmul(v3, tw_get(P.tw, 3 * tstep, sign));
-                }
-                const double2 t0 = cadd(v0, v2), t1 = csub(v0, v2), t2 = cadd(v1, v3);
-                const double2 d = csub(v1, v3);
-                // (v1 - v3) * (-i) forward, * (+i) inverse
-                const double2 t3 = sign < 0 ? make_double2(d.y, -d.x) : make_double2(-d.y, d.x);
-                yout[idx] = cadd(t0, t2);
-                yout[idx + Ns] = cadd(t1, t3);
-                yout[idx + 2 * Ns] = csub(t0, t2);
-                yout[idx + 3 * Ns] = csub(t1, t3);
-            } else if (R == 2) {
-                double2 v0 = xin[j], v1 = xin[j + nb];
-                if (tstep) v1 = cmul(v1, tw_get(P.tw, tstep, sign));
-                yout[idx] = cadd(v0, v1);
-                yout[idx + Ns] = csub(v0, v1);
-            } else {
-                // direct DFT of size R read straight from LDS
-                const int nR = n / R;
-                for (int k = 0; k < R; ++k) {
-                    double2 acc = make_double2(0.0, 0.0);
-                    for (int q = 0; q < R; ++q) {
-                        double2 v = xin[j + q * nb];
-                        const int e1 = q * tstep;                  // Stockham twiddle
-                        const int e2 = ((q * k) % R) * nR;         // DFT kernel w_R^{qk}
-                        const int e = (e1 + e2) % n;
-                        v = cmul(v, tw_get(P.tw, e, sign));
-                        acc = cadd(acc, v);
-                    }
-                    yout[idx + k * Ns] = acc;
-                }
-            }
+        switch (R) {
+        case 16: fft_pass<16, INV>(a, b, lines, P.n, Ns, P.tw); break;
+        case 8: fft_pass<8, INV>(a, b, lines, P.n, Ns, P.tw); break;
+        case 4: fft_pass<4, INV>(a, b, lines, P.n, Ns, P.tw); break;
+        case 2: fft_pass<2, INV>(a, b, lines, P.n, Ns, P.tw); break;
+        case 3: fft_pass<3, INV>(a, b, lines, P.n, Ns, P.tw); break;
+        case 5: fft_pass<5, INV>(a, b, lines, P.n, Ns, P.tw); break;
+        case 7: fft_pass<7, INV>(a, b, lines, P.n, Ns, P.tw); break;
+        default: fft_pass_prime<INV>(a, b, lines, P, R, Ns); break;
         }
         __syncthreads();
         double2 *tmp = a;
@@ -96,101 +231,131 @@ __device__ double2 *lds_fft(double2 *a, double2 *b, int lines, const FftPlan &P,
     return a;
 }
 
+// Row pairs pair0 .. pair0 + np - 1 of the white field into the LDS lines a: from xi, or
+// generated.  A Philox call gives the normals of two sites, which lie in one row when Nx is
+// even: a thread then takes both.
+__device__ __forceinline__ void load_rows(double2 *a, const double *__restrict__ xi, uint64_t seed, uint64_t step,
+                                          int pair0, int np, int Nt, int Nx) {
+    const int row = fft_row(Nx);
+    if (!xi && Nx % 2 == 0) {
+        const int Nh = Nx / 2;
+        const float inv = 1.0f / (float)Nh;
+        for (int w = threadIdx.x; w < np * Nh; w += blockDim.x) {
+            const int l = fast_div(w, inv), x = 2 * (w - l * Nh);
+            const int t0 = 2 * (pair0 + l);
+            double2 g0 = make_double2(0.0, 0.0), g1 = g0;
+            if (t0 < Nt) g0 = normal_pair(seed, 0u, step, ((uint64_t)t0 * Nx + x) >> 1);
+            if (t0 + 1 < Nt) g1 = normal_pair(seed, 0u, step, ((uint64_t)(t0 + 1) * Nx + x) >> 1);
+            a[l * row + fft_at(x)] = make_double2(g0.x, g1.x);
+            a[l * row + fft_at(x + 1)] = make_double2(g0.y, g1.y);
+        }
+        return;
+    }
+    for (int w = threadIdx.x; w < np * Nx; w += blockDim.x) {
+        const int l = w / Nx, x = w - l * Nx;
+        double v[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int t = 2 * (pair0 + l) + u;
+            const int64_t i = (int64_t)t * Nx + x;
+            v[u] = 0.0;
+            if (t < Nt) {
+                if (xi) {
+                    v[u] = xi[i];
+                } else {
+                    const double2 g = normal_pair(seed, 0u, step, (uint64_t)(i >> 1));
+                    v[u] = (i & 1) ? g.y : g.x;
+                }
+            }
+        }
+        a[l * row + fft_at(x)] = make_double2(v[0], v[1]);
+    }
+}
+
+// the half spectra of rows t0, t0 + 1 at column k from their packed transform (a line)
+__device__ __forceinline__ void untangle(const double2 *line, int k, int Nx, double2 &A, double2 &B) {
+    // A = (Z_k + conj Z_-k)/2 ; B = (Z_k - conj Z_-k)/(2i)
+    const double2 zk = line[fft_at(k)], zm = line[fft_at(k == 0 ? 0 : Nx - k)];
+    A = make_double2(0.5 * (zk.x + zm.x), 0.5 * (zk.y - zm.y));
+    B = make_double2(0.5 * (zk.y + zm.y), -0.5 * (zk.x - zm.x));
+}
+
+// the packed line's entries k and Nx - k from the half spectra A, B of rows t0, t0 + 1
+__device__ __forceinline__ void retangle(double2 *line, int k, int Nx, double2 A, double2 B) {
+    if (k == 0 || 2 * k == Nx) A.y = B.y = 0.0;
+    line[fft_at(k)] = make_double2(A.x - B.y, A.y + B.x);
+    if (k > 0 && 2 * k != Nx) line[fft_at(Nx - k)] = make_double2(A.x + B.y, B.x - A.y);
+}
+
 // ---------------------------------------------------------------------------
 // pass 1: Philox field + forward row FFTs (two rows per complex transform)
 // grid: (ceil(Nt / (2*lpb)), nRep)
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(kFftThreads)
 k_noise_rows_fwd(const double *__restrict__ xi, const uint64_t *__restrict__ seeds, uint64_t step,
-                 double2 *__restrict__ spec, int Nt, int Nx, int H, int lpb, FftPlan P, const StepCtl *ctl) {
+                 double2 *__restrict__ spec, int Nt, int Nx, int H, int nk, int lpb, FftPlan P, const StepCtl *ctl) {
     extern __shared__ double2 lds[];
     if (ctl) {   // a graph-captured step: counter from the control block, nothing while halted
         if (ctl->halt) return;
         step = ctl->step;
     }
-    double2 *a = lds, *b = lds + lpb * Nx;
+    const int row = fft_row(Nx);
+    double2 *a = lds, *b = lds + lpb * row;
     const int rep = blockIdx.y;
-    const int V = Nt * Nx;
-    const uint64_t seed = seeds[rep];
     const int pair0 = blockIdx.x * lpb;
-    for (int w = threadIdx.x; w < lpb * Nx; w += blockDim.x) {
-        const int l = w / Nx, x = w - l * Nx;
-        const int t0 = 2 * (pair0 + l), t1 = t0 + 1;
-        double v0 = 0.0, v1 = 0.0;
-        if (t0 < Nt) {
-            const int64_t i0 = (int64_t)t0 * Nx + x;
-            if (xi) {
-                v0 = xi[(size_t)rep * V + i0];
-                if (t1 < Nt) v1 = xi[(size_t)rep * V + i0 + Nx];
-            } else {
-                const double2 g0 = normal_pair(seed, 0u, step, (uint64_t)(i0 >> 1));
-                v0 = (i0 & 1) ? g0.y : g0.x;
-                if (t1 < Nt) {
-                    const int64_t i1 = i0 + Nx;
-                    const double2 g1 = normal_pair(seed, 0u, step, (uint64_t)(i1 >> 1));
-                    v1 = (i1 & 1) ? g1.y : g1.x;
-                }
-            }
-        }
-        a[w] = make_double2(v0, v1);
-    }
+    load_rows(a, xi ? xi + (size_t)rep * Nt * Nx : nullptr, seeds[rep], step, pair0, lpb, Nt, Nx);
     __syncthreads();
-    double2 *res = lds_fft(a, b, lpb, P, -1);
+    const double2 *res = lds_fft<false>(a, b, lpb, P);
     double2 *out = spec + (size_t)rep * Nt * H;
-    for (int w = threadIdx.x; w < lpb * H; w += blockDim.x) {
-        const int l = w / H, k = w - l * H;
-        const int t0 = 2 * (pair0 + l), t1 = t0 + 1;
+    const float inv = 1.0f / (float)nk;
+    for (int w = threadIdx.x; w < lpb * nk; w += blockDim.x) {
+        const int l = fast_div(w, inv), k = w - l * nk;
+        const int t0 = 2 * (pair0 + l);
         if (t0 >= Nt) continue;
-        const double2 zk = res[l * Nx + k];
-        const double2 zm = res[l * Nx + (k == 0 ? 0 : Nx - k)];
-        // A = (Z_k + conj Z_-k)/2 ; B = (Z_k - conj Z_-k)/(2i)
-        const double2 A = make_double2(0.5 * (zk.x + zm.x), 0.5 * (zk.y - zm.y));
-        const double2 dd = make_double2(zk.x - zm.x, zk.y + zm.y);
-        const double2 B = make_double2(0.5 * dd.y, -0.5 * dd.x);
+        double2 A, B;
+        untangle(res + l * row, k, Nx, A, B);
         out[(size_t)t0 * H + k] = A;
-        if (t1 < Nt) out[(size_t)t1 * H + k] = B;
+        if (t0 + 1 < Nt) out[(size_t)(t0 + 1) * H + k] = B;
     }
 }
 
 // ---------------------------------------------------------------------------
 // pass 2: column FFT along t, mask, inverse FFT along t (in place)
-// grid: (ceil(H / lpb), nRep)
+// grid: (ceil(nk / lpb), nRep).  Neighbouring column groups share the cache lines of their
+// rows, so blocks are handed to the 8 XCDs in contiguous bands of groups.
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(kFftThreads)
-k_noise_cols(double2 *__restrict__ spec, const int *__restrict__ kmax, int kmaxAll, double invV, int Nt, int H,
-             int lpb, FftPlan P, const StepCtl *ctl) {
+k_noise_cols(double2 *__restrict__ spec, const int *__restrict__ kmax, int nk, double invV, int Nt, int H, int lpb,
+             FftPlan P, const StepCtl *ctl) {
     extern __shared__ double2 lds[];
     if (ctl && ctl->halt) return;
-    double2 *a = lds, *b = lds + lpb * Nt;
-    const int rep = blockIdx.y;
-    const int k0 = blockIdx.x * lpb;
-    const int nl = min(lpb, H - k0);
+    const int row = fft_row(Nt);
+    double2 *a = lds, *b = lds + lpb * row;
+    const int rep = blockIdx.y, nb = gridDim.x;
+    const int band = (nb + 7) / 8, full = nb % 8 == 0 ? 8 : nb % 8;   // XCDs 0 .. full - 1 hold `band` groups
+    const int xcd = blockIdx.x % 8;
+    const int g = xcd * band - max(0, xcd - full) + (int)blockIdx.x / 8;
+    const int k0 = g * lpb;
+    const int nl = min(lpb, nk - k0);
     double2 *s = spec + (size_t)rep * Nt * H;
-    if (k0 > kmaxAll) {
-        // every mode of these columns is cut
-        for (int w = threadIdx.x; w < nl * Nt; w += blockDim.x) {
-            const int t = w / nl, l = w - t * nl;
-            s[(size_t)t * H + k0 + l] = make_double2(0.0, 0.0);
-        }
-        return;
-    }
+    const float inv = 1.0f / (float)lpb;
     for (int w = threadIdx.x; w < lpb * Nt; w += blockDim.x) {
-        const int t = w / lpb, l = w - t * lpb;
-        a[l * Nt + t] = (l < nl) ? s[(size_t)t * H + k0 + l] : make_double2(0.0, 0.0);
+        const int t = fast_div(w, inv), l = w - t * lpb;
+        a[l * row + fft_at(t)] = (l < nl) ? s[(size_t)t * H + k0 + l] : make_double2(0.0, 0.0);
     }
     __syncthreads();
-    double2 *res = lds_fft(a, b, lpb, P, -1);
+    double2 *res = lds_fft<false>(a, b, lpb, P);
     double2 *oth = (res == a) ? b : a;
     for (int w = threadIdx.x; w < lpb * Nt; w += blockDim.x) {
-        const int l = w / Nt, kt = w - l * Nt;
-        const double m = (k0 + l <= kmax[kt]) ? invV : 0.0;
-        res[w] = cscl(m, res[w]);
+        const int kt = fast_div(w, inv), l = w - kt * lpb;
+        const int at = l * row + fft_at(kt);
+        res[at] = cscl((k0 + l <= kmax[kt]) ? invV : 0.0, res[at]);
     }
     __syncthreads();
-    double2 *fin = lds_fft(res, oth, lpb, P, +1);
+    const double2 *fin = lds_fft<true>(res, oth, lpb, P);
     for (int w = threadIdx.x; w < lpb * Nt; w += blockDim.x) {
-        const int t = w / lpb, l = w - t * lpb;
-        if (l < nl) s[(size_t)t * H + k0 + l] = fin[l * Nt + t];
+        const int t = fast_div(w, inv), l = w - t * lpb;
+        if (l < nl) s[(size_t)t * H + k0 + l] = fin[l * row + fft_at(t)];
     }
 }
 
@@ -198,66 +363,150 @@ k_noise_cols(double2 *__restrict__ spec, const int *__restrict__ kmax, int kmaxA
 // pass 3: inverse row FFTs (C2R), two rows per complex transform
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(kFftThreads)
-k_noise_rows_inv(const double2 *__restrict__ spec, double *__restrict__ noise, int Nt, int Nx, int H, int lpb,
+k_noise_rows_inv(const double2 *__restrict__ spec, double *__restrict__ noise, int Nt, int Nx, int H, int nk, int lpb,
                  FftPlan P, const StepCtl *ctl) {
     extern __shared__ double2 lds[];
     if (ctl && ctl->halt) return;
-    double2 *a = lds, *b = lds + lpb * Nx;
+    const int row = fft_row(Nx);
+    double2 *a = lds, *b = lds + lpb * row;
     const int rep = blockIdx.y;
     const int pair0 = blockIdx.x * lpb;
     const double2 *s = spec + (size_t)rep * Nt * H;
-    const bool evenNx = (Nx % 2) == 0;
-    for (int w = threadIdx.x; w < lpb * Nx; w += blockDim.x) {
-        const int l = w / Nx, k = w - l * Nx;
-        const int t0 = 2 * (pair0 + l), t1 = t0 + 1;
-        double2 A = make_double2(0.0, 0.0), B = make_double2(0.0, 0.0);
-        if (t0 < Nt) {
-            const bool lower = k < H;
-            const int kk = lower ? k : Nx - k;
-            A = s[(size_t)t0 * H + kk];
-            if (t1 < Nt) B = s[(size_t)t1 * H + kk];
-            if (!lower) { A.y = -A.y; B.y = -B.y; }
-            if (k == 0 || (evenNx && k == Nx / 2)) { A.y = 0.0; B.y = 0.0; }
+    const float inv = 1.0f / (float)H;
+    for (int w = threadIdx.x; w < lpb * H; w += blockDim.x) {
+        const int l = fast_div(w, inv), k = w - l * H;
+        const int t0 = 2 * (pair0 + l);
+        double2 A = make_double2(0.0, 0.0), B = A;
+        if (t0 < Nt && k < nk) {
+            A = s[(size_t)t0 * H + k];
+            if (t0 + 1 < Nt) B = s[(size_t)(t0 + 1) * H + k];
         }
-        a[w] = make_double2(A.x - B.y, A.y + B.x);
+        retangle(a + l * row, k, Nx, A, B);
     }
     __syncthreads();
-    double2 *res = lds_fft(a, b, lpb, P, +1);
+    const double2 *res = lds_fft<true>(a, b, lpb, P);
     double *o = noise + (size_t)rep * Nt * Nx;
+    const float invX = 1.0f / (float)Nx;
     for (int w = threadIdx.x; w < lpb * Nx; w += blockDim.x) {
-        const int l = w / Nx, x = w - l * Nx;
-        const int t0 = 2 * (pair0 + l), t1 = t0 + 1;
+        const int l = fast_div(w, invX), x = w - l * Nx;
+        const int t0 = 2 * (pair0 + l);
         if (t0 >= Nt) continue;
-        const double2 z = res[w];
+        const double2 z = res[l * row + fft_at(x)];
         o[(size_t)t0 * Nx + x] = z.x;
-        if (t1 < Nt) o[(size_t)t1 * Nx + x] = z.y;
+        if (t0 + 1 < Nt) o[(size_t)(t0 + 1) * Nx + x] = z.y;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// the three passes of a small lattice by one block per replica, the spectrum in LDS
+// (buffers of `cap` entries): the same arithmetic in one launch
+// ---------------------------------------------------------------------------
+constexpr int kOneThreads = 512;
+constexpr int kOneLdsBytes = 81920;
+__global__ void __launch_bounds__(kOneThreads)
+k_noise_one(const double *__restrict__ xi, const uint64_t *__restrict__ seeds, uint64_t step,
+            const int *__restrict__ kmax, int nk, double invV, double *__restrict__ noise, int Nt, int Nx, int cap,
+            FftPlan PX, FftPlan PT, const StepCtl *ctl) {
+    extern __shared__ double2 lds[];
+    if (ctl) {
+        if (ctl->halt) return;
+        step = ctl->step;
+    }
+    const int rep = blockIdx.x, np = (Nt + 1) / 2, H = Nx / 2 + 1, rowX = fft_row(Nx), rowT = fft_row(Nt);
+    double2 *a = lds, *b = lds + cap;
+    load_rows(a, xi ? xi + (size_t)rep * Nt * Nx : nullptr, seeds[rep], step, 0, np, Nt, Nx);
+    __syncthreads();
+    double2 *res = lds_fft<false>(a, b, np, PX);
+    double2 *oth = (res == a) ? b : a;
+    for (int w = threadIdx.x; w < np * nk; w += blockDim.x) {
+        const int l = w / nk, k = w - l * nk;
+        double2 A, B;
+        untangle(res + l * rowX, k, Nx, A, B);
+        oth[k * rowT + fft_at(2 * l)] = A;
+        if (2 * l + 1 < Nt) oth[k * rowT + fft_at(2 * l + 1)] = B;
+    }
+    __syncthreads();
+    double2 *col = lds_fft<false>(oth, res, nk, PT);
+    oth = (col == oth) ? res : oth;
+    for (int w = threadIdx.x; w < nk * Nt; w += blockDim.x) {
+        const int k = w / Nt, kt = w - k * Nt;
+        const int at = k * rowT + fft_at(kt);
+        col[at] = cscl((k <= kmax[kt]) ? invV : 0.0, col[at]);
+    }
+    __syncthreads();
+    double2 *fin = lds_fft<true>(col, oth, nk, PT);
+    oth = (fin == a) ? b : a;
+    for (int w = threadIdx.x; w < np * H; w += blockDim.x) {
+        const int l = w / H, k = w - l * H;
+        double2 A = make_double2(0.0, 0.0), B = A;
+        if (k < nk) {
+            A = fin[k * rowT + fft_at(2 * l)];
+            if (2 * l + 1 < Nt) B = fin[k * rowT + fft_at(2 * l + 1)];
+        }
+        retangle(oth + l * rowX, k, Nx, A, B);
+    }
+    __syncthreads();
+    const double2 *out = lds_fft<true>(oth, fin, np, PX);
+    double *o = noise + (size_t)rep * Nt * Nx;
+    for (int w = threadIdx.x; w < np * Nx; w += blockDim.x) {
+        const int l = w / Nx, x = w - l * Nx;
+        const double2 z = out[l * rowX + fft_at(x)];
+        o[(size_t)(2 * l) * Nx + x] = z.x;
+        if (2 * l + 1 < Nt) o[(size_t)(2 * l + 1) * Nx + x] = z.y;
     }
 }
 
 // twiddle table tw[e] = exp(-2 pi i e / n), e < n (both entry points build it this way,
 // so their transforms agree bit for bit)
-__global__ void __launch_bounds__(kFftThreads) k_twiddles(double2 *__restrict__ tw, int n) {
-    const int e = blockIdx.x * kFftThreads + threadIdx.x;
-    if (e >= n) return;
+__device__ __forceinline__ double2 twiddle(int e, int n) {
     double s, c;
     sincospi(-2.0 * (double)e / (double)n, &s, &c);
-    tw[e] = make_double2(c, s);
+    return make_double2(c, s);
+}
+__global__ void __launch_bounds__(kFftThreads) k_twiddles(double2 *__restrict__ tw, int n) {
+    const int e = blockIdx.x * kFftThreads + threadIdx.x;
+    if (e < n) tw[e] = twiddle(e, n);
 }
 
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
-// radix factors of n: 4s, then 2s, then odd primes (direct DFTs); false if more than
+// radix factors of n: for its power of two as few passes as radix 16 and 8 give (1024 =
+// 16 x 8 x 8), then 3, 5, 7 and the other odd primes (direct DFTs); false if more than
 // kMaxFactors are needed
 static bool factor_plan(int n, FftPlan &P) {
     P.n = n;
     P.nf = 0;
-    int m = n;
-    while (m % 4 == 0 && P.nf < kMaxFactors) { P.radix[P.nf++] = 4; m /= 4; }
-    while (m % 2 == 0 && P.nf < kMaxFactors) { P.radix[P.nf++] = 2; m /= 2; }
-    for (int q = 3; m > 1 && P.nf < kMaxFactors; q += 2)
-        while (m % q == 0 && P.nf < kMaxFactors) { P.radix[P.nf++] = q; m /= q; }
-    return m == 1;
+    int m = n, e = 0;
+    while (m % 2 == 0) {
+        m /= 2;
+        ++e;
+    }
+    auto put = [&](int r) {
+        if (P.nf < kMaxFactors) P.radix[P.nf] = r;
+        ++P.nf;
+    };
+    if (e == 1) {
+        put(2);
+    } else if (e == 2) {
+        put(4);
+    } else if (e > 2) {
+        // passes of 3 and 4 bits: p = ceil(e / 4) passes, the first e - 3 p of them radix 16
+        // (e = 5: 8 x 4)
+        if (e == 5) {
+            put(8);
+            put(4);
+        } else {
+            const int p = (e + 3) / 4, wide = e - 3 * p;
+            for (int k = 0; k < p; ++k) put(k < wide ? 16 : 8);
+        }
+    }
+    for (int q = 3; m > 1; q += 2)
+        while (m % q == 0) {
+            put(q);
+            m /= q;
+        }
+    return P.nf <= kMaxFactors;
 }
 
 static int make_plan(Ctx &c, int n, FftPlan &P) {
@@ -313,11 +562,25 @@ static int build_mask(Ctx &c, std::vector<int> &kmax) {
 }
 #pragma clang fp contract(on)
 
-static int lines_per_block(int n) { return std::max(1, std::min(64, kFftLdsBytes / (2 * (int)sizeof(double2) * n))); }
+// Lines per block of a pass over `lines` lines of length n (all replicas): as few as give
+// 512 blocks (two per CU), within the LDS of a block, and at least `least` where the lattice
+// has them (columns: two neighbouring ones, 32 bytes of each row).
+static int lines_per_block(int n, int lines, int least) {
+    const int most = std::max(1, kFftLdsBytes / (2 * (int)sizeof(double2) * fft_row(n)));
+    return std::min(most, std::max(least, lines / 512));
+}
+// threads of such a block: eight points each, the register butterflies' usual share
+static int fft_threads(int points) {
+    return std::min(kFftThreads, std::max(kWave, (points / 8 + kWave - 1) / kWave * kWave));
+}
+// entries of one LDS buffer of the one-block form
+static int one_block_entries(int Nt, int Nx, int nk) {
+    return std::max((Nt + 1) / 2 * fft_row(Nx), nk * fft_row(Nt));
+}
 
 int noise_init(Ctx &c) {
     const int Nt = c.p.Nt, Nx = c.p.Nx;
-    if ((size_t)2 * sizeof(double2) * std::max(Nt, Nx) > (size_t)kFftLdsBytes) {
+    if ((size_t)2 * sizeof(double2) * fft_row(std::max(Nt, Nx)) > (size_t)kFftLdsBytes) {
         c.err = "lattice extent too large for the LDS FFT (max 2048)";
         return YCN_ERR_UNSUPPORTED;
     }
@@ -356,19 +619,33 @@ int noise_generate(Ctx &c, uint64_t step, const double *xi_dev, double *out_dev)
 static int launch_noise(hipStream_t s, int Nt, int Nx, int nRep, const double *xi_dev, const uint64_t *seeds,
                         uint64_t step, double2 *spec, const int *kmax, int kmaxAll, const FftPlan &planX,
                         const FftPlan &planT, double *out_dev, Ctx *prof, const StepCtl *ctl = nullptr) {
-    const int H = Nx / 2 + 1;
-    const int lx = lines_per_block(Nx), lt = lines_per_block(Nt);
+    const int H = Nx / 2 + 1, nk = kmaxAll + 1;   // columns up to the cutoff
+    const double invV = 1.0 / ((double)Nt * (double)Nx);
     const int npairs = (Nt + 1) / 2;
-    dim3 g1((npairs + lx - 1) / lx, nRep), g2((H + lt - 1) / lt, nRep);
-    const size_t sh1 = (size_t)2 * lx * Nx * sizeof(double2), sh2 = (size_t)2 * lt * Nt * sizeof(double2);
-    hipLaunchKernelGGL(k_noise_rows_fwd, g1, dim3(kFftThreads), sh1, s, xi_dev, seeds, step, spec, Nt, Nx, H, lx,
-                       planX, ctl);
-    if (prof) prof_before(*prof, PK_NOISE_COLS, 32.0 * (double)nRep * Nt * H);
-    hipLaunchKernelGGL(k_noise_cols, g2, dim3(kFftThreads), sh2, s, spec, kmax, kmaxAll,
-                       1.0 / ((double)Nt * (double)Nx), Nt, H, lt, planT, ctl);
-    if (prof) prof_after(*prof, PK_NOISE_COLS);
-    hipLaunchKernelGGL(k_noise_rows_inv, g1, dim3(kFftThreads), sh1, s, (const double2 *)spec, out_dev, Nt, Nx, H,
-                       lx, planX, ctl);
+    // One block per replica where the half spectrum fits it.  Three launches take about 5 us
+    // each on a small lattice, one block about 8 us for all of a 64 x 64 one; its time grows
+    // with the lattice while theirs does not.
+    const int cap = one_block_entries(Nt, Nx, std::max(nk, 1));
+    const size_t shOne = (size_t)2 * cap * sizeof(double2);
+    if (shOne <= (size_t)kOneLdsBytes) {
+        if (prof) prof_before(*prof, PK_NOISE_COLS, 40.0 * (double)nRep * Nt * Nx);
+        hipLaunchKernelGGL(k_noise_one, dim3(nRep), dim3(kOneThreads), shOne, s, xi_dev, seeds, step, kmax, nk, invV,
+                           out_dev, Nt, Nx, cap, planX, planT, ctl);
+        if (prof) prof_after(*prof, PK_NOISE_COLS);
+        return hipGetLastError() == hipSuccess ? YCN_OK : YCN_ERR_HIP;
+    }
+    const int lx = lines_per_block(Nx, npairs * nRep, 1), lt = lines_per_block(Nt, nk * nRep, 2);
+    dim3 g1((npairs + lx - 1) / lx, nRep), g2((nk + lt - 1) / lt, nRep);
+    const dim3 b1(fft_threads(lx * Nx)), b2(fft_threads(lt * Nt));
+    const size_t sh1 = (size_t)2 * lx * fft_row(Nx) * sizeof(double2);
+    const size_t sh2 = (size_t)2 * lt * fft_row(Nt) * sizeof(double2);
+    hipLaunchKernelGGL(k_noise_rows_fwd, g1, b1, sh1, s, xi_dev, seeds, step, spec, Nt, Nx, H, nk, lx, planX, ctl);
+    if (nk > 0) {
+        if (prof) prof_before(*prof, PK_NOISE_COLS, 32.0 * (double)nRep * Nt * nk);
+        hipLaunchKernelGGL(k_noise_cols, g2, b2, sh2, s, spec, kmax, nk, invV, Nt, H, lt, planT, ctl);
+        if (prof) prof_after(*prof, PK_NOISE_COLS);
+    }
+    hipLaunchKernelGGL(k_noise_rows_inv, g1, b1, sh1, s, (const double2 *)spec, out_dev, Nt, Nx, H, nk, lx, planX, ctl);
     return hipGetLastError() == hipSuccess ? YCN_OK : YCN_ERR_HIP;
 }
 
@@ -435,9 +712,6 @@ const char *noise_noalloc_error() { return g_naErr; }
 struct NaSeeds {
     uint64_t v[kNaMaxRep];
 };
-__global__ void k_na_seeds(NaSeeds s, uint64_t *__restrict__ dst, int n) {
-    if ((int)threadIdx.x < n) dst[threadIdx.x] = s.v[threadIdx.x];
-}
 
 // kmax[kt] of the mask on the device, in the host's IEEE order (momentum_squared, no
 // contraction; correctly rounded double multiply, divide and add), so both entry points
@@ -448,19 +722,39 @@ __device__ double na_coord_sq(int c, int n) {
     const double t = __ddiv_rn(__dmul_rn(__dmul_rn(k, 2.0), M_PI), (double)n);
     return __dmul_rn(t, t);
 }
-__global__ void __launch_bounds__(kFftThreads) k_na_mask(int *__restrict__ kmax, int Nt, int Nx, int H, double cutSq) {
-    const int kt = blockIdx.x * kFftThreads + threadIdx.x;
-    if (kt >= Nt) return;
+// rows keep a prefix of their columns (the rounded momentum grows with k): its end by
+// bisection
+__device__ int na_kmax(int kt, int Nt, int Nx, int H, double cutSq) {
     const double mt = __dadd_rn(0.0, na_coord_sq(kt, Nt));
-    int km = -1;
-    for (int k = 0; k < H; ++k) {
+    int lo = -1, hi = H;   // kept up to lo, cut from hi on
+    while (hi - lo > 1) {
+        const int k = (lo + hi) / 2;
         const double m = __dadd_rn(mt, na_coord_sq(k, Nx));
-        if (!(m >= 0.0 && m <= cutSq)) break;
-        km = k;
+        if (m >= 0.0 && m <= cutSq)
+            lo = k;
+        else
+            hi = k;
     }
-    kmax[kt] = km;
+    return lo;
 }
 #pragma clang fp contract(on)
+
+// everything a call reads besides its arguments, in one launch: block row 0 fills the x
+// twiddles, row 1 the t twiddles, row 2 the mask rows and the seeds (one launch of about 5 us
+// for the 56 us that a serial search per mask row and four launches took at 1024 x 1024)
+__global__ void __launch_bounds__(kFftThreads)
+k_na_setup(NaSeeds s, int nRep, uint64_t *__restrict__ seeds, double2 *__restrict__ twX, double2 *__restrict__ twT,
+           int *__restrict__ kmax, int Nt, int Nx, int H, double cutSq) {
+    const int e = blockIdx.x * kFftThreads + threadIdx.x;
+    if (blockIdx.y == 0) {
+        if (e < Nx) twX[e] = twiddle(e, Nx);
+    } else if (blockIdx.y == 1) {
+        if (e < Nt) twT[e] = twiddle(e, Nt);
+    } else {
+        if (e < Nt) kmax[e] = na_kmax(e, Nt, Nx, H, cutSq);
+        if (e < nRep) seeds[e] = s.v[e];
+    }
+}
 
 // largest kept kx over all rows: row kt = 0 (p_t = 0) keeps the most, since adding
 // p_t^2 >= 0 and rounding cannot lower the momentum
@@ -492,11 +786,9 @@ static int na_run(const ycn_params *p, const uint64_t *seeds, uint64_t step, dou
     NaSeeds sd{};
     for (int i = 0; i < nRep; ++i) sd.v[i] = seeds ? seeds[i] : p->seed;
     const double cutSq = cut_squared(p->cutFraction);
-    hipLaunchKernelGGL(k_na_seeds, dim3(1), dim3(kNaMaxRep), 0, s, sd, seed_d, nRep);
-    hipLaunchKernelGGL(k_twiddles, dim3((Nx + kFftThreads - 1) / kFftThreads), dim3(kFftThreads), 0, s, twX, Nx);
-    hipLaunchKernelGGL(k_twiddles, dim3((Nt + kFftThreads - 1) / kFftThreads), dim3(kFftThreads), 0, s, twT, Nt);
-    hipLaunchKernelGGL(k_na_mask, dim3((Nt + kFftThreads - 1) / kFftThreads), dim3(kFftThreads), 0, s, kmax, Nt, Nx,
-                       H, cutSq);
+    const int blocks = (std::max({Nx, Nt, nRep}) + kFftThreads - 1) / kFftThreads;
+    hipLaunchKernelGGL(k_na_setup, dim3(blocks, 3), dim3(kFftThreads), 0, s, sd, nRep, seed_d, twX, twT, kmax, Nt, Nx, H,
+                       cutSq);
     pX.tw = twX;
     pT.tw = twT;
     if (launch_noise(s, Nt, Nx, nRep, nullptr, seed_d, step, spec, kmax, na_kmax_all(Nt, Nx, cutSq), pX, pT, noise,

@@ -276,7 +276,6 @@ static int launch_plain(Ctx &c, const OnchipArgs &A, int nsys, int threads, cons
                         uint64_t step, double2 *wout, double *drift) {
     auto *k = A.r == 1.0 ? &k_onchip_plain<K, true, DAG1, GEN> : &k_onchip_plain<K, false, DAG1, GEN>;
     const size_t lds = sizeof(double2) * 4 * (size_t)A.V;
-    YCN_HIP(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL(k, dim3(nsys), dim3(threads), lds, c.stream, A, phi, (const uint64_t *)c.seed_d, streamBase,
                        step, c.eta, wout, drift, c.cg_d);
     YCN_HIP(hipGetLastError());

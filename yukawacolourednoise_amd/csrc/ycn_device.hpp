@@ -57,8 +57,9 @@ __device__ __forceinline__ double2 normal_pair(uint64_t seed, uint32_t stream, u
     const double u1 = (double)(a + 1) * 0x1p-53;
     const double u2 = (double)b * 0x1p-53;
     const double rho = sqrt(-2.0 * log(u1));
-    const double th = (2.0 * M_PI) * u2;
-    return make_double2(rho * cos(th), rho * sin(th));
+    double sn, cs;
+    sincospi(2.0 * u2, &sn, &cs);   // no reduction of the argument by pi, one call for both
+    return make_double2(rho * cs, rho * sn);
 }
 
 // ---------------------------------------------------------------------------
