@@ -160,10 +160,10 @@ __host__ __device__ __forceinline__ int fft_row(int n) { return n + (n >> 3) + 1
 __device__ __forceinline__ int fast_div(int a, float inv) { return (int)(((float)a + 0.5f) * inv); }
 
 template <int R, bool INV>
-__device__ __forceinline__ void fft_pass(const double2 *a, double2 *b, int lines, int n, int Ns,
+__device__ __forceinline__ void fft_pass(const double2 *a, double2 *b, int lines, int row, const FftPass &F,
                                          const double2 *__restrict__ tw) {
-    const int nb = n / R, tstride = nb / Ns, row = fft_row(n);
-    const float invNb = 1.0f / (float)nb, invNs = 1.0f / (float)Ns;
+    const int nb = F.nb, Ns = F.Ns, tstride = F.tstride;
+    const float invNb = F.invNb, invNs = F.invNs;
     for (int w = threadIdx.x; w < nb * lines; w += blockDim.x) {
         const int line = fast_div(w, invNb), j = w - line * nb;
         const int jd = fast_div(j, invNs), jm = j - jd * Ns;
@@ -186,8 +186,8 @@ __device__ __forceinline__ void fft_pass(const double2 *a, double2 *b, int lines
 
 // any other prime factor: one thread per output, a direct sum of R terms
 template <bool INV>
-__device__ void fft_pass_prime(const double2 *a, double2 *b, int lines, const FftPlan &P, int R, int Ns) {
-    const int n = P.n, nb = n / R, tstride = nb / Ns, row = fft_row(n);
+__device__ void fft_pass_prime(const double2 *a, double2 *b, int lines, const FftPlan &P, const FftPass &F) {
+    const int n = P.n, R = F.R, Ns = F.Ns, nb = F.nb, tstride = F.tstride, row = fft_row(n);
     for (int w = threadIdx.x; w < n * lines; w += blockDim.x) {
         const int line = w / n, o = w - line * n;
         const int jd = o / (Ns * R), rem = o - jd * Ns * R, k = rem / Ns, jm = rem - k * Ns;
@@ -209,24 +209,23 @@ __device__ void fft_pass_prime(const double2 *a, double2 *b, int lines, const Ff
 // transforms a (barrier before and after); returns the buffer holding the result (a or b)
 template <bool INV>
 __device__ double2 *lds_fft(double2 *a, double2 *b, int lines, const FftPlan &P) {
-    int Ns = 1;
+    const int row = fft_row(P.n);
     for (int f = 0; f < P.nf; ++f) {
-        const int R = P.radix[f];
-        switch (R) {
-        case 16: fft_pass<16, INV>(a, b, lines, P.n, Ns, P.tw); break;
-        case 8: fft_pass<8, INV>(a, b, lines, P.n, Ns, P.tw); break;
-        case 4: fft_pass<4, INV>(a, b, lines, P.n, Ns, P.tw); break;
-        case 2: fft_pass<2, INV>(a, b, lines, P.n, Ns, P.tw); break;
-        case 3: fft_pass<3, INV>(a, b, lines, P.n, Ns, P.tw); break;
-        case 5: fft_pass<5, INV>(a, b, lines, P.n, Ns, P.tw); break;
-        case 7: fft_pass<7, INV>(a, b, lines, P.n, Ns, P.tw); break;
-        default: fft_pass_prime<INV>(a, b, lines, P, R, Ns); break;
+        const FftPass &F = P.pass[f];
+        switch (F.R) {
+        case 16: fft_pass<16, INV>(a, b, lines, row, F, P.tw); break;
+        case 8: fft_pass<8, INV>(a, b, lines, row, F, P.tw); break;
+        case 4: fft_pass<4, INV>(a, b, lines, row, F, P.tw); break;
+        case 2: fft_pass<2, INV>(a, b, lines, row, F, P.tw); break;
+        case 3: fft_pass<3, INV>(a, b, lines, row, F, P.tw); break;
+        case 5: fft_pass<5, INV>(a, b, lines, row, F, P.tw); break;
+        case 7: fft_pass<7, INV>(a, b, lines, row, F, P.tw); break;
+        default: fft_pass_prime<INV>(a, b, lines, P, F); break;
         }
         __syncthreads();
         double2 *tmp = a;
         a = b;
         b = tmp;
-        Ns *= R;
     }
     return a;
 }
@@ -471,35 +470,42 @@ __global__ void __launch_bounds__(kFftThreads) k_twiddles(double2 *__restrict__ 
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
-// radix factors of n: for its power of two as few passes as radix 16 and 8 give (1024 =
-// 16 x 8 x 8), then 3, 5, 7 and the other odd primes (direct DFTs); false if more than
-// kMaxFactors are needed
+// Passes of a transform of length n, its power of two first.  Long lines: as few passes as
+// radix 16 and 8 give (1024 = 16 x 8 x 8).  Lines of up to 32: radix 4, since a short line's
+// radix-16 butterfly is 660 instructions of one thread while the block's others idle (16 x 16:
+// 13.5 -> 10.0 us a field; 64 x 64 prefers 8 x 8, 22.5 us against 23.3).  Then 3, 5, 7 and the other odd primes (direct DFTs).  false if more
+// than kMaxFactors are needed.
 static bool factor_plan(int n, FftPlan &P) {
     P.n = n;
     P.nf = 0;
-    int m = n, e = 0;
+    int m = n, e = 0, Ns = 1;
     while (m % 2 == 0) {
         m /= 2;
         ++e;
     }
     auto put = [&](int r) {
-        if (P.nf < kMaxFactors) P.radix[P.nf] = r;
-        ++P.nf;
-    };
-    if (e == 1) {
-        put(2);
-    } else if (e == 2) {
-        put(4);
-    } else if (e > 2) {
-        // passes of 3 and 4 bits: p = ceil(e / 4) passes, the first e - 3 p of them radix 16
-        // (e = 5: 8 x 4)
-        if (e == 5) {
-            put(8);
-            put(4);
-        } else {
-            const int p = (e + 3) / 4, wide = e - 3 * p;
-            for (int k = 0; k < p; ++k) put(k < wide ? 16 : 8);
+        if (P.nf < kMaxFactors) {
+            FftPass &F = P.pass[P.nf];
+            F.R = r;
+            F.nb = n / r;
+            F.Ns = Ns;
+            F.tstride = F.nb / Ns;
+            F.invNb = 1.0f / (float)F.nb;
+            F.invNs = 1.0f / (float)Ns;
         }
+        ++P.nf;
+        Ns *= r;
+    };
+    if (n <= 32 || e <= 2) {
+        for (; e >= 2; e -= 2) put(4);
+        if (e) put(2);
+    } else if (e == 5) {
+        put(8);
+        put(4);
+    } else {
+        // passes of 3 and 4 bits: p = ceil(e / 4) passes, the first e - 3 p of them radix 16
+        const int p = (e + 3) / 4, wide = e - 3 * p;
+        for (int k = 0; k < p; ++k) put(k < wide ? 16 : 8);
     }
     for (int q = 3; m > 1; q += 2)
         while (m % q == 0) {

@@ -14,11 +14,15 @@ namespace ycn {
 // ---------------------------------------------------------------------------
 // FFT plan for one transform length (mixed radix, Stockham in LDS).
 // ---------------------------------------------------------------------------
-constexpr int kMaxFactors = 24;
+constexpr int kMaxFactors = 12;   // an extent of up to 2048 takes at most 8
+struct FftPass {                  // one Stockham pass and what its index arithmetic divides by
+    int R, nb, Ns, tstride;       // radix, n / R, product of the earlier radices, nb / Ns
+    float invNb, invNs;
+};
 struct FftPlan {
     int n;
     int nf;
-    int radix[kMaxFactors];
+    FftPass pass[kMaxFactors];
     const double2 *tw;  // device: tw[e] = exp(-2 pi i e / n), e < n
 };
 
