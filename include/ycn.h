@@ -255,7 +255,10 @@ int ycn_precond_train(ycn_ctx *ctx, uint64_t step0, int nsteps, int pairsPerSolv
  * end returns the summed duration and count of the launches that did work (launches
  * shorter than a quarter of the 90th percentile exited at once for converged systems and
  * are left out) and the algorithmic bytes moved per launch (averaged over the launches: the
- * pipelined iteration's launches alternate between two traffic figures).  The pipelined even-odd FP32
+ * pipelined iteration's launches alternate between two traffic figures).  The fermion-force
+ * solvers run on packed real spinors, half the bytes of this interface's complex ones: the
+ * figures count the packed vectors, except the pipelined even-odd FP32 iteration's, which
+ * count complex ones (100 B per site and launch; packed 52 B).  The pipelined even-odd FP32
  * iteration with the finalize in the next launch's prologue is the exception: its
  * chunks hold nothing but back-to-back launches of that kernel, so one event pair
  * brackets each chunk and the count is the iterations done in it.  Kernel names:

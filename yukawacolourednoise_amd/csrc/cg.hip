@@ -89,15 +89,15 @@ k_dirac(LatticeArgs L, const double *__restrict__ phi, const double2 *__restrict
     for (int c = 0; c < NC; ++c) q[c * V + s] = o[c];
 }
 
-// (1, 1, 0, 0) at site 0: in both forms the first members of planes 0 and 1
-__global__ void __launch_bounds__(kNT) k_point_source(int V, int planes, double2 *__restrict__ eta) {
-    const int s = blockIdx.x * kNT + threadIdx.x;
-    if (s >= V) return;
-    for (int c = 0; c < planes; ++c) eta[(size_t)c * V + s] = make_double2(s == 0 && c < 2 ? 1.0 : 0.0, 0.0);
-}
-
 __global__ void k_set_int(int *p, int v) {
     if (threadIdx.x == 0 && blockIdx.x == 0) *p = v;
+}
+
+// (1, 1, 0, 0) at site 0: both spins of flavour 0
+__global__ void __launch_bounds__(kNT) k_point_source(int V, double2 *__restrict__ eta) {
+    const int s = blockIdx.x * kNT + threadIdx.x;
+    if (s >= V) return;
+    eta[s] = eta[(size_t)V + s] = make_double2(s == 0 ? 1.0 : 0.0, 0.0);
 }
 
 // ---------------------------------------------------------------------------
@@ -586,8 +586,7 @@ k_drift(LatticeArgs L, const double *__restrict__ phi, const double2 *__restrict
 }
 
 // corr[t] = sum_x sum_k Re psi (gpuTimeSlices_spinors, reductions.cu:176-191);
-// one block per time slice, fixed-order block reduction.
-template <int NC>
+// one block per time slice of a packed spinor, fixed-order block reduction.
 __global__ void __launch_bounds__(kNT)
 k_spinor_slices(const double2 *__restrict__ psi, int Nt, int Nx, double *__restrict__ out) {
     __shared__ double2 lds[kNT / kWave];
@@ -596,10 +595,7 @@ k_spinor_slices(const double2 *__restrict__ psi, int Nt, int Nx, double *__restr
     double2 acc = make_double2(0.0, 0.0);
     for (int x = threadIdx.x; x < Nx; x += kNT) {
         const size_t s = (size_t)t * Nx + x;
-        if (NC == 4)
-            acc.x += psi[s].x + psi[V + s].x + psi[2 * V + s].x + psi[3 * V + s].x;
-        else
-            acc.x += psi[s].x + psi[V + s].x + psi[s].y + psi[V + s].y;
+        acc.x += psi[s].x + psi[V + s].x + psi[s].y + psi[V + s].y;
     }
     acc = block_sum2<kNT>(acc, lds);
     if (threadIdx.x == 0) out[t] = acc.x;
@@ -875,8 +871,8 @@ void launch_fin_beta(Ctx &c, int nsys, int nb, bool mixed, bool even) {
 
 int launch_cg_update(Ctx &c, int nsys, int n, const double2 *p) {
     const dim3 g((n + kNT - 1) / kNT, nsys);
-    prof_before(c, PK_CG_UPDATE, (double)nsys * n * 6 * 64);
-    hipLaunchKernelGGL(k_cg_c<4>, g, dim3(kNT), 0, c.stream, n, (const CgState *)c.cg_d, c.x, c.r, p,
+    prof_before(c, PK_CG_UPDATE, (double)nsys * n * 6 * 32);
+    hipLaunchKernelGGL(k_cg_c<kPacked>, g, dim3(kNT), 0, c.stream, n, (const CgState *)c.cg_d, c.x, c.r, p,
                        (const double2 *)c.Ap, c.partials);
     prof_after(c, PK_CG_UPDATE);
     return (int)g.x;
@@ -1136,7 +1132,7 @@ int mp_alloc(Ctx &c) {
     YCN_HIP(hipMalloc(&c.phis, sizeof(float) * (size_t)c.nRep * c.V));
     YCN_HIP(hipMemset(c.phis, 0, sizeof(float) * (size_t)c.nRep * c.V));
     if (c.p.evenOdd) {   // second Ap buffer and third direction buffer of the pipelined even-odd iteration (half lattice)
-        const size_t h = (size_t)c.nSys * 4 * (c.V / 2);
+        const size_t h = (size_t)c.nSys * kPacked * (c.V / 2);
         float2 **pf[] = {&c.pfA1, &c.pfP2};
         for (float2 **b : pf) {
             YCN_HIP(hipMalloc(b, sizeof(float2) * h));
@@ -1282,15 +1278,15 @@ int plain_propagator(Ctx &c, const double *phi, double2 *out, SolveStats *st) {
     return YCN_OK;
 }
 
-// the measurement's source (1, 1, 0, 0) at site 0, in c.eta
-int point_source(Ctx &c, SpinorForm form) {
-    hipLaunchKernelGGL(k_point_source, site_grid(c, 1), dim3(kNT), 0, c.stream, c.V, (int)form, c.eta);
+// the measurement's source (1, 1, 0, 0) at site 0, packed, in c.eta
+int point_source(Ctx &c) {
+    hipLaunchKernelGGL(k_point_source, site_grid(c, 1), dim3(kNT), 0, c.stream, c.V, c.eta);
     YCN_HIP(hipGetLastError());
     return YCN_OK;
 }
 
-int spinor_slices(Ctx &c, const double2 *psi, SpinorForm form, double *out_dev) {
-    hipLaunchKernelGGL(form == kPacked ? &k_spinor_slices<2> : &k_spinor_slices<4>, dim3(c.p.Nt), dim3(kNT), 0, c.stream, psi, c.p.Nt, c.p.Nx, out_dev);
+int spinor_slices(Ctx &c, const double2 *psi, double *out_dev) {
+    hipLaunchKernelGGL(k_spinor_slices, dim3(c.p.Nt), dim3(kNT), 0, c.stream, psi, c.p.Nt, c.p.Nx, out_dev);
     YCN_HIP(hipGetLastError());
     return YCN_OK;
 }

@@ -12,12 +12,13 @@
 //
 // Half-lattice vectors use the compact checkerboard order of the reference's even-odd
 // blocks (commented out in Dirac.cu:256-379): site (t, x) of a parity at t * Nx/2 +
-// (x >> 1), SoA planes [sys][c][Vh].  Needs even Nt and Nx.
+// (x >> 1).  Needs even Nt and Nx.  All vectors are packed real spinors (ycn_device.hpp):
+// planes [sys][c][Vh], c the spin, each entry (flavour 0, flavour 1).
 //
 // FP64: one CG iteration = k_eo_normal_fused (p' = r + beta p, v = S p', Ap = S^T v,
 // |v|^2: four half-lattice hops through LDS) + the BLAS-1 update on Vh sites: 5S + P
 // bytes per site of the full lattice, against 10S + P for the unpreconditioned
-// iteration.  Mixed precision: one launch per pipelined FP32 iteration (132 B per site),
+// iteration.  Mixed precision: one launch per pipelined FP32 iteration (52 B per site),
 // its finalize in the next launch's prologue or a separate kernel, and FP64 reliable
 // updates whose residual b - S x and S^T of it take one fused launch.
 #include <algorithm>
@@ -76,13 +77,13 @@ __device__ __forceinline__ T &at(T *base, unsigned idx) {
 // Hopping (K for DAG, H otherwise) at site (t, x); ld(t', x', c) returns component c of
 // the input at neighbour (t', x') of the other parity.
 template <bool DAG, typename R, typename V2, typename Ld>
-__device__ __forceinline__ void eo_hop(const EoArgs &A, int t, int x, Ld ld, V2 o[4]) {
+__device__ __forceinline__ void eo_hop(const EoArgs &A, int t, int x, Ld ld, V2 o[2]) {
     const int tp = (t == A.Nt - 1) ? 0 : t + 1, tm = (t == 0) ? A.Nt - 1 : t - 1;
     const int xp = (x == A.Nx - 1) ? 0 : x + 1, xm = (x == 0) ? A.Nx - 1 : x - 1;
     const R sf = (t == A.Nt - 1) ? (R)-1 : (R)1, sb = (t == 0) ? (R)-1 : (R)1;
     const R hp = (R)(0.5 * (A.r + 1.0)), hm = (R)(0.5 * (A.r - 1.0)), hr = (R)(0.5 * A.r), h = (R)0.5;
 #pragma unroll
-    for (int f = 0; f < 4; f += 2)
+    for (int f = 0; f < 2; f += 2)
         hop_flavour_r<DAG, R, V2>(hp, hm, hr, h, ld(tp, x, f), ld(tp, x, f + 1), sf, ld(tm, x, f), ld(tm, x, f + 1),
                                   sb, ld(t, xp, f), ld(t, xp, f + 1), ld(t, xm, f), ld(t, xm, f + 1), o[f], o[f + 1]);
 }
@@ -101,26 +102,26 @@ k_eo_eta(EoArgs A, const uint64_t *__restrict__ seeds, uint32_t streamBase, uint
     if (eo_halted(A)) return;
     if (A.stepPtr) step = *A.stepPtr;
     const int sys = blockIdx.y, s = blockIdx.x * kNT + threadIdx.x;
-    const size_t V = A.V, off = (size_t)sys * 4 * V;
+    const size_t V = A.V, off = (size_t)sys * 2 * V;
     double2 acc = make_double2(0.0, 0.0);
     if (s < A.V) {
-        double2 b[4];
+        double2 b[2];
         if (GEN) {
-            eta_site(seeds, streamBase, step, sys, A.nNoise, s, b);
+            eta_planes<2>(seeds, streamBase, step, sys, A.nNoise, s, b);
 #pragma unroll
-            for (int c = 0; c < 4; ++c) eta[off + c * V + s] = b[c];
+            for (int c = 0; c < 2; ++c) eta[off + c * V + s] = b[c];
         } else {
 #pragma unroll
-            for (int c = 0; c < 4; ++c) b[c] = eta[off + c * V + s];
+            for (int c = 0; c < 2; ++c) b[c] = eta[off + c * V + s];
         }
 #pragma unroll
-        for (int c = 0; c < 4; ++c) acc.x += b[c].x * b[c].x + b[c].y * b[c].y;
+        for (int c = 0; c < 2; ++c) acc.x += b[c].x * b[c].x + b[c].y * b[c].y;
         const int t = s / A.Nx, x = s - t * A.Nx;
         if ((t + x) & 1) {
             const double inv = 1.0 / (2.0 * A.r + A.M + A.g * phi[(size_t)(sys / A.nNoise) * V + s]);
-            const size_t j = (size_t)sys * 4 * A.Vh + eo_j(A, t, x);
+            const size_t j = (size_t)sys * 2 * A.Vh + eo_j(A, t, x);
 #pragma unroll
-            for (int c = 0; c < 4; ++c) u[j + (size_t)c * A.Vh] = make_double2(b[c].x * inv, b[c].y * inv);
+            for (int c = 0; c < 2; ++c) u[j + (size_t)c * A.Vh] = make_double2(b[c].x * inv, b[c].y * inv);
         }
     }
     acc = block_sum2<kNT>(acc, lds);
@@ -136,14 +137,14 @@ k_eo_rhs(EoArgs A, const double2 *__restrict__ eta, const double2 *__restrict__ 
     int t, x;
     eo_site(A, 0, j, t, x);
     const size_t V = A.V, Vh = A.Vh;
-    const double2 *e = eta + (size_t)sys * 4 * V;
-    const double2 *uo = u + (size_t)sys * 4 * Vh;
-    double2 k[4];
+    const double2 *e = eta + (size_t)sys * 2 * V;
+    const double2 *uo = u + (size_t)sys * 2 * Vh;
+    double2 k[2];
     eo_hop<true, double, double2>(A, t, x, [&](int tn, int xn, int c) { return uo[c * Vh + eo_j(A, tn, xn)]; }, k);
     const size_t fs = (size_t)t * A.Nx + x;
-    double2 *bo = b + (size_t)sys * 4 * Vh;
+    double2 *bo = b + (size_t)sys * 2 * Vh;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) bo[c * Vh + j] = csub(e[c * V + fs], k[c]);
+    for (int c = 0; c < 2; ++c) bo[c * Vh + j] = csub(e[c * V + fs], k[c]);
 }
 
 // U_o = A_o^-1 K_oe in_e (DAG) or A_o^-1 H_oe in_e
@@ -155,14 +156,14 @@ k_eo_hop_oe(EoArgs A, const double *__restrict__ phi, const double2 *__restrict_
     if (j >= A.Vh) return;
     int t, x;
     eo_site(A, 1, j, t, x);
-    const size_t Vh = A.Vh, off = (size_t)sys * 4 * Vh;
+    const size_t Vh = A.Vh, off = (size_t)sys * 2 * Vh;
     const double *ph = phi + (size_t)(sys / A.nNoise) * A.V;
-    double2 k[4];
+    double2 k[2];
     eo_hop<DAG, double, double2>(A, t, x, [&](int tn, int xn, int c) { return in[off + c * Vh + eo_j(A, tn, xn)]; },
                                  k);
     const double inv = 1.0 / (2.0 * A.r + A.M + A.g * ph[(size_t)t * A.Nx + x]);
 #pragma unroll
-    for (int c = 0; c < 4; ++c) U[off + c * Vh + j] = make_double2(k[c].x * inv, k[c].y * inv);
+    for (int c = 0; c < 2; ++c) U[off + c * Vh + j] = make_double2(k[c].x * inv, k[c].y * inv);
 }
 
 // half-lattice vectors a setup launch also clears at its sites (any may be null)
@@ -183,18 +184,18 @@ k_eo_hop_eo(EoArgs A, const double *__restrict__ phi, const double2 *__restrict_
     __shared__ double2 lds[kNT / kWave];
     if (eo_halted(A)) return;
     const int sys = blockIdx.y, j = blockIdx.x * kNT + threadIdx.x;
-    const size_t Vh = A.Vh, off = (size_t)sys * 4 * Vh;
+    const size_t Vh = A.Vh, off = (size_t)sys * 2 * Vh;
     double2 acc = make_double2(0.0, 0.0);
     if (j < A.Vh) {
         int t, x;
         eo_site(A, 0, j, t, x);
         const double *ph = phi + (size_t)(sys / A.nNoise) * A.V;
-        double2 k[4];
+        double2 k[2];
         eo_hop<DAG, double, double2>(A, t, x, [&](int tn, int xn, int c) { return U[off + c * Vh + eo_j(A, tn, xn)]; },
                                      k);
         const double d = 2.0 * A.r + A.M + A.g * ph[(size_t)t * A.Nx + x];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
+        for (int c = 0; c < 2; ++c) {
             const double2 iv = in[off + c * Vh + j];
             double2 v = make_double2(d * iv.x - k[c].x, d * iv.y - k[c].y);
             if (MODE == 1) v = csub(b[off + c * Vh + j], v);
@@ -234,55 +235,46 @@ k_eo_drift(EoArgs A, const double *__restrict__ phi, const double2 *__restrict__
     double acc = 0.0;
     for (int jn = 0; jn < A.nNoise; ++jn) {
         const size_t sys = (size_t)rep * A.nNoise + jn;
-        const double2 *ce = chi_e + sys * 4 * Vh;
-        const double2 *e = eta + sys * 4 * V;
-        double2 ch[4];
+        const double2 *ce = chi_e + sys * 2 * Vh;
+        const double2 *e = eta + sys * 2 * V;
+        double2 ch[2];
         if (odd) {
-            double2 k[4];
+            double2 k[2];
             eo_hop<true, double, double2>(A, t, x, [&](int tn, int xn, int c) { return ce[c * Vh + eo_j(A, tn, xn)]; },
                                           k);
             const double inv = 1.0 / d;
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
+            for (int c = 0; c < 2; ++c) {
                 const double2 ev = e[c * V + s];
                 ch[c] = make_double2((ev.x - k[c].x) * inv, (ev.y - k[c].y) * inv);
             }
         } else {
 #pragma unroll
-            for (int c = 0; c < 4; ++c) ch[c] = ce[c * Vh + eo_j(A, t, x)];
+            for (int c = 0; c < 2; ++c) ch[c] = ce[c * Vh + eo_j(A, t, x)];
         }
-        double2 sm = cdotc(ch[0], e[s]);
-        sm = cadd(sm, cdotc(ch[1], e[V + s]));
-        sm = cadd(sm, cdotc(ch[2], e[2 * V + s]));
-        sm = cadd(sm, cdotc(ch[3], e[3 * V + s]));
-        acc += sm.x;
+        const double2 e0 = e[s], e1 = e[V + s];
+        acc += (ch[0].x * e0.x + ch[0].y * e0.y) + (ch[1].x * e1.x + ch[1].y * e1.y);
     }
     drift[(size_t)rep * V + s] = (A.nNoise == 1) ? fac * acc : fac * acc / (double)A.nNoise;
 }
 
 // gamma_5 = sigma_2 on each flavour's spin pair, (c0, c1) -> (-i c1, i c0); with it
-// gamma_5 D gamma_5 = D^dag for the Wilson-Yukawa operator (Dirac.cu:144-190)
-__device__ __forceinline__ void g5_pair(double2 a0, double2 a1, double2 &o0, double2 &o1) {
-    o0 = make_double2(a1.y, -a1.x);
-    o1 = make_double2(-a0.y, a0.x);
-}
+// gamma_5 D gamma_5 = D^dag for the Wilson-Yukawa operator (Dirac.cu:144-190).  For a real
+// source gamma_5 src = i (-c1, c0): the solve runs on the real spinor (-c1, c0), and since
+// gamma_5 i (a0, a1) = (a1, -a0) the result is real too.
 
-// v = gamma_5 v in place (system 0)
+// v = -i gamma_5 v in place (system 0): (c0, c1) -> (-c1, c0)
 __global__ void __launch_bounds__(kNT) k_g5(int V, double2 *__restrict__ v) {
     const int s = blockIdx.x * kNT + threadIdx.x;
     if (s >= V) return;
-#pragma unroll
-    for (int f = 0; f < 4; f += 2) {
-        double2 o0, o1;
-        g5_pair(v[f * V + s], v[(f + 1) * V + s], o0, o1);
-        v[f * V + s] = o0;
-        v[(f + 1) * V + s] = o1;
-    }
+    const double2 a = v[s], b = v[V + s];
+    v[s] = make_double2(-b.x, -b.y);
+    v[V + s] = a;
 }
 
 // The measurement's propagator from the even-odd solve of D^dag chi = eta with
-// eta = gamma_5 src (system 0): chi on both parities (the odd sites rebuilt as in
-// k_eo_drift) and out = gamma_5 chi = D^-1 src, full lattice, SoA.
+// eta = -i gamma_5 src (system 0): chi on both parities (the odd sites rebuilt as in
+// k_eo_drift) and out = gamma_5 i chi = D^-1 src, full lattice, packed.
 __global__ void __launch_bounds__(kNT)
 k_eo_propagator(EoArgs A, const double *__restrict__ phi, const double2 *__restrict__ chi_e,
                 const double2 *__restrict__ eta, double2 *__restrict__ out) {
@@ -290,28 +282,23 @@ k_eo_propagator(EoArgs A, const double *__restrict__ phi, const double2 *__restr
     if (s >= A.V) return;
     const size_t V = A.V, Vh = A.Vh;
     const int t = s / A.Nx, x = s - t * A.Nx;
-    double2 ch[4];
+    double2 ch[2];
     if ((t + x) & 1) {
-        double2 k[4];
+        double2 k[2];
         eo_hop<true, double, double2>(A, t, x, [&](int tn, int xn, int c) { return chi_e[c * Vh + eo_j(A, tn, xn)]; },
                                       k);
         const double inv = 1.0 / (2.0 * A.r + A.M + A.g * phi[s]);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
+        for (int c = 0; c < 2; ++c) {
             const double2 ev = eta[c * V + s];
             ch[c] = make_double2((ev.x - k[c].x) * inv, (ev.y - k[c].y) * inv);
         }
     } else {
 #pragma unroll
-        for (int c = 0; c < 4; ++c) ch[c] = chi_e[c * Vh + eo_j(A, t, x)];
+        for (int c = 0; c < 2; ++c) ch[c] = chi_e[c * Vh + eo_j(A, t, x)];
     }
-#pragma unroll
-    for (int f = 0; f < 4; f += 2) {
-        double2 o0, o1;
-        g5_pair(ch[f], ch[f + 1], o0, o1);
-        out[f * V + s] = o0;
-        out[(f + 1) * V + s] = o1;
-    }
+    out[s] = ch[1];
+    out[V + s] = make_double2(-ch[0].x, -ch[0].y);
 }
 
 // ---------------------------------------------------------------------------
@@ -539,7 +526,7 @@ k_fin_pf_chunk(const double2 *__restrict__ slotLast, const double2 *__restrict__
 // tile's TT*TX/2 even sites.  LDS holds the tile plus a 4-site halo, (TT+8) x (TX+8)
 // sites in full-lattice coordinates, split by lattice parity: E[c][row][k] and
 // O[c][row][k] hold the site of that parity in array row `row`, column 2k or 2k+1
-// (k = column >> 1), four SoA planes each.  Lanes of a wave take consecutive k, so every
+// (k = column >> 1), two planes (spins) each.  Lanes of a wave take consecutive k, so every
 // neighbour read (rows row +- 1 at the same k, the same row at k or k +- 1) is a
 // contiguous run: no bank conflicts.  Each stage fills the parity it produces on a halo
 // one site smaller than the stage before:
@@ -550,7 +537,7 @@ k_fin_pf_chunk(const double2 *__restrict__ slotLast, const double2 *__restrict__
 //   4: Ap = d v - H W on the tile's even sites          (= S^T S p')
 // The diagonal d = 2r + M + g phi is staged per parity for the whole array.  |v|^2 over
 // the tile (= <p', Ap>) is the block's partial.  HBM traffic per launch: read r, p_old
-// (Vh sites each) and phi, write p', Ap: 4 S/2 + P per site of the full lattice.
+// (Vh sites each) and phi, write p', Ap: 4 S/2 + P per site of the full lattice (S = 32 B in FP64).
 constexpr int eo_threads(int tt, int tx) { return (tt * tx / 2 < kWave) ? kWave : tt * tx / 2; }
 
 // PF = false: the operator alone, p' = r + beta p_old, partial <p', Ap> = |v|^2.
@@ -602,7 +589,7 @@ constexpr int eo_threads(int tt, int tx) { return (tt * tx / 2 < kWave) ? kWave 
 // Pairs never straddle a chunk (chunks have an even number of launches), and a system
 // pauses only after an odd launch (after whole pairs), except at the iteration cap; the
 // reliable update's k_pf_reliable then adds the deferred term.  Per even site and launch:
-// 168 B (even) and 232 B (odd).  XM and RM do not apply to the FP64 forms (PF = false).
+// 88 B (even) and 120 B (odd).  XM and RM do not apply to the FP64 forms (PF = false).
 template <typename R, int TT, int TX, bool PF, bool PERSIST = false, bool RU = false, bool WR1 = false, int XM = 1,
           int RM = 0>
 __global__ void __launch_bounds__(eo_threads(TT, TX))
@@ -621,8 +608,8 @@ k_eo_normal_fused(EoArgs A, const R *__restrict__ phi, CgState *st, const typena
     // O and FO hold only array rows 1 .. H - 2 (odd sites are needed on the 3-site halo at
     // most): odd-site entry (row, k) sits at (row - 1) K + k, 7-8 % less LDS per block
     constexpr int HO = H - 2;
-    __shared__ V2 E[4][H * K];
-    __shared__ V2 O[4][HO * K];
+    __shared__ V2 E[2][H * K];
+    __shared__ V2 O[2][HO * K];
     __shared__ R FE[H * K], FO[HO * K];
     __shared__ double2 red[NT / kWave > 0 ? NT / kWave : 1];
     __shared__ double2 red2[NT / kWave > 0 ? NT / kWave : 1];
@@ -632,7 +619,7 @@ k_eo_normal_fused(EoArgs A, const R *__restrict__ phi, CgState *st, const typena
     const int nTiles = A.tilesPerSys;
     const int Nt = A.Nt, Nx = A.Nx, Nh = A.Nh;
     const unsigned Vh = (unsigned)A.Vh;
-    const size_t off = (size_t)sys * 4 * A.Vh;   // this system's vectors
+    const size_t off = (size_t)sys * 2 * A.Vh;   // this system's vectors
     r += off;
     if (!RU) {
         pold += off;
@@ -664,7 +651,7 @@ k_eo_normal_fused(EoArgs A, const R *__restrict__ phi, CgState *st, const typena
     // array's even sites.  Array (row, col) is lattice site (t0 - 4 + row, x0 - 4 + col);
     // its parity is (row + col) & 1 because t0 + x0 is even.
     struct Regs {
-        V2 ra[M0][4], pa[M0][4], aa[M0][4], xa[M0][4];
+        V2 ra[M0][2], pa[M0][2], aa[M0][2], xa[M0][2];
         R fe[M0], fo[M0];
         unsigned jj[M0];
     };
@@ -680,7 +667,7 @@ k_eo_normal_fused(EoArgs A, const R *__restrict__ phi, CgState *st, const typena
                 G.jj[u] = (unsigned)(gt * Nh + (gxE >> 1));
                 const bool inner = row >= 4 && row < 4 + TT && colE >= 4 && colE < 4 + TX;
 #pragma unroll
-                for (int c = 0; c < 4; ++c) {
+                for (int c = 0; c < 2; ++c) {
                     const unsigned i = c * Vh + G.jj[u];
                     G.ra[u][c] = at(r, i);
                     if (!RU) G.pa[u][c] = at(pold, i);
@@ -705,7 +692,7 @@ k_eo_normal_fused(EoArgs A, const R *__restrict__ phi, CgState *st, const typena
                 const bool inner = row >= 4 && row < 4 + TT && colE >= 4 && colE < 4 + TX;
                 R rs = 0;   // |r'|^2 of the site (4 terms in R, then accumulated in FP64)
 #pragma unroll
-                for (int c = 0; c < 4; ++c) {
+                for (int c = 0; c < 2; ++c) {
                     const unsigned i = c * Vh + G.jj[u];
                     V2 a = G.ra[u][c];   // r_{idx-1}, or p_{idx-2} (RM = 2)
                     const V2 b = RU ? a : G.pa[u][c];
@@ -756,14 +743,14 @@ k_eo_normal_fused(EoArgs A, const R *__restrict__ phi, CgState *st, const typena
     auto stages = [&](int t0, int x0) {
         // hopping at site q from the other-parity array N (component stride NS, entries
         // shifted down by SH: 0 for E, K for O)
-        auto hop_at = [&](auto dag, auto ns, auto sh, const Site &q, const V2 *N, V2 o[4]) {
+        auto hop_at = [&](auto dag, auto ns, auto sh, const Site &q, const V2 *N, V2 o[2]) {
             constexpr bool DAG = decltype(dag)::value;
             constexpr int NS = decltype(ns)::value, SH = decltype(sh)::value;
             const int gt = wrapf(t0 - 4 + q.row, Nt, A.invNt);
             const R sf = (gt == Nt - 1) ? (R)-1 : (R)1, sb = (gt == 0) ? (R)-1 : (R)1;
             const int itf = q.itf - SH, itb = q.itb - SH, ixf = q.ixf - SH, ixb = q.ixb - SH;
 #pragma unroll
-            for (int f = 0; f < 4; f += 2) {
+            for (int f = 0; f < 2; f += 2) {
                 const V2 *N0 = N + f * NS, *N1 = N + (f + 1) * NS;
                 if constexpr (WR1)
                     hop_flavour_r1<DAG, R, V2>(N0[itf], N1[itf], sf, N0[itb], N1[itb], sb, N0[ixf], N1[ixf], N0[ixb],
@@ -780,17 +767,17 @@ k_eo_normal_fused(EoArgs A, const R *__restrict__ phi, CgState *st, const typena
         // stage 1: U = K p' / d on odd sites, 3-site halo
         for (int w = threadIdx.x; w < (TT + 6) * ((TX + 6) / 2); w += NT) {
             const Site q = site_of(w, 3, 1);
-            V2 o[4];
+            V2 o[2];
             hop_at(std::true_type(), FromE(), Sh0(), q, &E[0][0], o);
             const R inv = (R)1 / FO[q.i - K];
 #pragma unroll
-            for (int c = 0; c < 4; ++c) O[c][q.i - K] = mk2<R>(o[c].x * inv, o[c].y * inv);
+            for (int c = 0; c < 2; ++c) O[c][q.i - K] = mk2<R>(o[c].x * inv, o[c].y * inv);
         }
         __syncthreads();
         // stage 2: v = d p' - K U on even sites, 2-site halo; |v|^2 over the tile
         for (int w = threadIdx.x; w < (TT + 4) * ((TX + 4) / 2); w += NT) {
             const Site q = site_of(w, 2, 0);
-            V2 o[4];
+            V2 o[2];
             hop_at(std::true_type(), FromO(), ShK(), q, &O[0][0], o);
             const R d = FE[q.i];
             const bool inner = q.row >= 4 && q.row < 4 + TT && q.col >= 4 && q.col < 4 + TX;
@@ -799,7 +786,7 @@ k_eo_normal_fused(EoArgs A, const R *__restrict__ phi, CgState *st, const typena
                 jb = (unsigned)(wrapf(t0 - 4 + q.row, Nt, A.invNt) * Nh + (wrapf(x0 - 4 + q.col, Nx, A.invNx) >> 1));
             R vs = 0;
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
+            for (int c = 0; c < 2; ++c) {
                 const V2 pv = E[c][q.i];
                 V2 v = mk2<R>(d * pv.x - o[c].x, d * pv.y - o[c].y);
                 if (RU) {
@@ -815,24 +802,24 @@ k_eo_normal_fused(EoArgs A, const R *__restrict__ phi, CgState *st, const typena
         // stage 3: W = H v / d on odd sites, 1-site halo
         for (int w = threadIdx.x; w < (TT + 2) * ((TX + 2) / 2); w += NT) {
             const Site q = site_of(w, 1, 1);
-            V2 o[4];
+            V2 o[2];
             hop_at(std::false_type(), FromE(), Sh0(), q, &E[0][0], o);
             const R inv = (R)1 / FO[q.i - K];
 #pragma unroll
-            for (int c = 0; c < 4; ++c) O[c][q.i - K] = mk2<R>(o[c].x * inv, o[c].y * inv);
+            for (int c = 0; c < 2; ++c) O[c][q.i - K] = mk2<R>(o[c].x * inv, o[c].y * inv);
         }
         __syncthreads();
         // stage 4: Ap = d v - H W on the tile's even sites (PF: and |Ap|^2)
         for (int w = threadIdx.x; w < TT * (TX / 2); w += NT) {
             const Site q = site_of(w, 0, 0);
-            V2 o[4];
+            V2 o[2];
             hop_at(std::false_type(), FromO(), ShK(), q, &O[0][0], o);
             const R d = FE[q.i];
             // stage-4 sites are the tile's own: no wrap
             const unsigned j = (unsigned)((t0 - 4 + q.row) * Nh + ((x0 - 4 + q.col) >> 1));
             R as = 0;
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
+            for (int c = 0; c < 2; ++c) {
                 const V2 v = E[c][q.i];
                 const V2 a = mk2<R>(d * v.x - o[c].x, d * v.y - o[c].y);
                 at(Ap, c * Vh + j) = a;
@@ -971,9 +958,9 @@ k_pf_reliable(int n, const CgState *__restrict__ st, double2 *__restrict__ x, fl
     const int m = st[sys].iter - st[sys].iter0, slot = m >= 1 ? (m - 1) % 3 : 0;
     const float2 *src = slot == 1 ? p1 : slot == 2 ? p2 : p0;
     const double a = (m & 1) ? st[sys].ab[(m - 1) & 1].x : 0.0;
-    const size_t off = (size_t)sys * 4 * n;
+    const size_t off = (size_t)sys * 2 * n;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
+    for (int c = 0; c < 2; ++c) {
         const size_t i = off + (size_t)c * n + s;
         const float2 d = xs[i];
         const double2 xv = x[i];
@@ -1133,11 +1120,11 @@ int eo_pf_alloc(Ctx &c) {
     return YCN_OK;
 }
 
-// even extents; the fused kernels address one system's four FP64 half-lattice
-// components and phi through 32-bit byte offsets and wrap halo coordinates with wrapf
+// even extents; the fused kernels address one system's FP64 half-lattice planes and
+// phi through 32-bit byte offsets and wrap halo coordinates with wrapf
 // (|a| < 2^22)
 static bool eo_shape_ok(const Ctx &c) {
-    return c.p.Nt % 2 == 0 && c.p.Nx % 2 == 0 && (size_t)4 * (c.V / 2) * sizeof(double2) < ((size_t)1 << 32) &&
+    return c.p.Nt % 2 == 0 && c.p.Nx % 2 == 0 && c.V < (1 << 27) &&
            c.p.Nt < (1 << 21) && c.p.Nx < (1 << 21);
 }
 
@@ -1237,7 +1224,7 @@ static int launch_eo_fused(Ctx &c, int ti, int nsys, const double *phi, const do
     b.pold = pold;
     b.pnew = pnew;
     b.Ap = Ap;
-    prof_before(c, PK_NORMAL_OP, (double)nsys * c.V * (2 * 64 + 8));
+    prof_before(c, PK_NORMAL_OP, (double)nsys * c.V * (4 * 16 + 8));
     switch (ti) {
     case 0: (void)launch_eo_tt<double, 8, 32>(c, nsys, A, phi, false, false, b); break;
     case 1: (void)launch_eo_tt<double, 16, 16>(c, nsys, A, phi, false, false, b); break;
@@ -1300,8 +1287,10 @@ static int launch_eo_pf(Ctx &c, int ti, int nsys, int idx, int finMode) {
     b.r = idx == 0 ? c.rs : eo_pdir(c, idx - 2);
     b.pold = eo_pdir(c, idx - 1);
     b.pnew = eo_pdir(c, idx);
-    // half-lattice FP32 vectors (16 B per site of the full lattice): read p_{idx-2} (or r),
-    // Ap, p and write p, Ap, and x_s read and written in odd launches; and read phi
+    // half-lattice FP32 vectors: read p_{idx-2} (or r), Ap, p and write p, Ap, and x_s read and
+    // written in odd launches; and read phi.  The figure counts the vectors as the complex
+    // spinors of the interface (16 B per site of the full lattice), as ycn_profile_end
+    // documents; packed they are half that.
     const int vecs = (idx & 1) ? 7 : 5;
     prof_before(c, PK_NORMAL_OP, (double)nsys * c.V * (vecs * 16 + 4));
     const bool ps = t.persist;
@@ -1435,7 +1424,7 @@ struct EoBufs {
     double2 *b, *U, *res;
 };
 static EoBufs eo_bufs(Ctx &c, int nsys) {
-    const size_t h = (size_t)nsys * 4 * (c.V / 2);
+    const size_t h = (size_t)nsys * 2 * (c.V / 2);
     return {c.t, c.t + h, c.Ap};
 }
 
@@ -1557,7 +1546,7 @@ static int eo_mixed_chunk(Ctx &c, const double *phi, int nsys, int n, bool graph
     if (graphed) {   // already inside a capture: the launches themselves
         for (int i = 0; i < n; ++i) launch_eo_pf_iteration(c, nsys, i);
     } else {
-        const int rc = run_chunk(c, nullptr, nsys, YCN_DAGGER, n, 4, kComplex, c.tileEo32,
+        const int rc = run_chunk(c, nullptr, nsys, YCN_DAGGER, n, 4, kPacked, c.tileEo32,
                                  [&](int i) { launch_eo_pf_iteration(c, nsys, i); });
         if (rc) return rc;
     }
@@ -1671,7 +1660,7 @@ int eo_solve(Ctx &c, const double *phi, int nsys, bool gen, uint32_t streamBase,
         while (active > 0 && launched < hardCap) {
             const int n = std::min(chunk, hardCap - launched);
             for (int k = 0; k < n; k += kGraphIters) {
-                rc = run_chunk(c, phi, nsys, YCN_DAGGER, kGraphIters, 3, kComplex, c.tileEo64,
+                rc = run_chunk(c, phi, nsys, YCN_DAGGER, kGraphIters, 3, kPacked, c.tileEo64,
                                [&](int i) { launch_eo_iteration(c, nsys, phi, i & 1); });
                 if (rc) return rc;
             }

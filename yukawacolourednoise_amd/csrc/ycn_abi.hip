@@ -580,11 +580,11 @@ int ycn_measure(ycn_ctx *ctx, int replica, uint64_t step, ycn_observables *obs, 
         c.nNoise = 1;
         SolveStats st;
         const bool eo = c.p.evenOdd && eo_available(c);
-        rc = point_source(c, eo ? kComplex : kPacked);
+        rc = point_source(c);
         if (!rc) rc = eo ? eo_propagator(c, phi_rep, c.t, &st) : plain_propagator(c, phi_rep, c.t, &st);
         c.nNoise = save;
         if (rc) return rc;
-        if ((rc = spinor_slices(c, c.t, eo ? kComplex : kPacked, cr))) return rc;
+        if ((rc = spinor_slices(c, c.t, cr))) return rc;
         YCN_HIP(hipMemcpyAsync(corr, cr, sizeof(double) * Nt, hipMemcpyDeviceToHost, c.stream));
         YCN_HIP(hipStreamSynchronize(c.stream));
     }

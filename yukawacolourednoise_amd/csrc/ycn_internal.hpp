@@ -263,11 +263,11 @@ int cg_solve(Ctx &c, const double *phi_dev, int nsys, int mtype, SpinorForm form
              uint64_t step, SolveStats *st);
 // the solver's vectors of the last fermion-force solve (form) -> drift
 int fermion_drift(Ctx &c, const double *phi_dev, SpinorForm form, double *drift_dev);
-// measurement: the point source in c.eta, and D^-1 of it in out (packed)
-int point_source(Ctx &c, SpinorForm form);
+// measurement: the packed point source in c.eta, and D^-1 of it in out (packed)
+int point_source(Ctx &c);
 int plain_propagator(Ctx &c, const double *phi, double2 *out, SolveStats *st);
 // correlator / trace helpers
-int spinor_slices(Ctx &c, const double2 *psi, SpinorForm form, double *out_dev);
+int spinor_slices(Ctx &c, const double2 *psi, double *out_dev);
 
 // cnn.hip
 int cnn_alloc(Ctx &c);
@@ -303,8 +303,8 @@ int stats_from_mirror(Ctx &c, int nsys, SolveStats *st);
 int read_stats(Ctx &c, int nsys, SolveStats *st);
 // CG building blocks shared with the even-odd solver (cg.hip): finalize alpha / beta from
 // the partials in c.partials, the BLAS-1 updates x += alpha p, r -= alpha Ap on
-// [nsys][4][n] vectors (c.x, c.r, c.Ap), returning their block count, and an FP64 -> FP32
-// copy.
+// packed [nsys][2][n] vectors (c.x, c.r, c.Ap), returning their block count, and an FP64 ->
+// FP32 copy.
 void launch_fin_alpha(Ctx &c, int nsys, int nb);
 void launch_fin_beta(Ctx &c, int nsys, int nb, bool mixed, bool even);
 int launch_cg_update(Ctx &c, int nsys, int n, const double2 *p);
