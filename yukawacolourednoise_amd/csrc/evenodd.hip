@@ -1456,7 +1456,7 @@ static void launch_fin_pf_chunk(Ctx &c, int nsys, int n) {
 // starts from 0.9 times the largest ratio need / stop0 the systems of this one reported
 // (the first solve starts from tol |r_0|).  A threshold that proves too loose is
 // tightened by the true-residual check as before; one too tight costs a few iterations.
-static void eo_learn_stop_scale(Ctx &c, int nsys) {
+void eo_learn_stop_scale(Ctx &c, int nsys) {
     if (c.p.cgTolMode != YCN_TOL_REL_TRUE) return;
     double r = 0.0;
     for (int k = 0; k < nsys; ++k)
@@ -1697,6 +1697,10 @@ int eo_propagator(Ctx &c, const double *phi, double2 *out, SolveStats *st) {
     hipLaunchKernelGGL(k_g5, dim3(nbV), dim3(kNT), 0, c.stream, c.V, c.eta);
     const int pred = c.eoPredIters, last = c.lastIters;
     const double scale = c.eoStopScale;
+    if (onchip_eo(c)) {
+        const int rc = onchip_eo_propagator(c, phi, out);
+        return rc ? rc : read_stats(c, 1, st);
+    }
     int rc = eo_solve(c, phi, 1, false, 0, 0, st);
     c.eoPredIters = pred;
     c.lastIters = last;

@@ -17,8 +17,7 @@
 #include <cstdlib>
 
 #include "cg_fused.hpp"
-#include "ycn_device.hpp"
-#include "ycn_internal.hpp"
+#include "onchip.hpp"
 
 namespace ycn {
 
@@ -34,19 +33,6 @@ struct OnchipArgs {
     int mode, maxIter, maxRestarts;
     double fac;          // drift factor
 };
-
-// The sum of v over the block in every thread.  red holds two rows of 16 slots, used in
-// turn: between two uses of a row every thread passes the barrier of the other.
-__device__ __forceinline__ double onchip_sum(double v, double (*red)[16], int &turn) {
-    v = wave_sum(v);
-    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave, nw = blockDim.x / kWave;
-    if (lane == 0) red[turn][wave] = v;
-    __syncthreads();
-    const int k = lane & 15;
-    v = row_sum(k < nw ? red[turn][k] : 0.0);
-    turn ^= 1;
-    return v;
-}
 
 // A site's four neighbours, two registers: their sites (below kOnchipSites) in 15 bits
 // each, (t+1, t-1) and (x+1, x-1), and the antiperiodic signs of the time hops in the two
@@ -68,6 +54,7 @@ template <bool DAG, bool WR1>
 __device__ __forceinline__ void onchip_dirac(const OnchipArgs &A, const double2 *B, OnchipNbr n, double d, double2 a0,
                                              double2 a1, double2 &o0, double2 &o1) {
     const double2 *B1 = B + A.V;
+    n = {fresh(n.t), fresh(n.x)};
     const unsigned tf = n.t & 0x7FFF, tb = (n.t >> 15) & 0x7FFF, xf = n.x & 0x7FFF, xb = n.x >> 15;
     const double sf = onchip_sign(n.t), sb = onchip_sign(n.t << 1);
     if constexpr (WR1) {
@@ -303,17 +290,23 @@ static int onchip_launch(Ctx &c, const double *phi, int nsys, uint32_t streamBas
                                  : launch_plain<2, DAG1, GEN>(c, A, nsys, threads, phi, streamBase, step, wout, drift);
 }
 
-// the fermion force of every system into c.drift; the states stay on the device
-int onchip_force(Ctx &c, const double *phi, uint32_t streamBase, uint64_t step) {
-    const bool one = c.nNoise == 1;
-    double *share = one ? c.drift : reinterpret_cast<double *>(c.Ap);
-    int rc = onchip_launch<false, true>(c, phi, c.nSys, streamBase, step, nullptr, share);
-    if (rc || one) return rc;
+// where a solve leaves its systems' drifts: the drift itself, or with several noise vectors
+// their shares in scratch, which onchip_mean averages
+double *onchip_share(Ctx &c) { return c.nNoise == 1 ? c.drift : reinterpret_cast<double *>(c.Ap); }
+
+int onchip_mean(Ctx &c) {
+    if (c.nNoise == 1) return YCN_OK;
     const double fac = -c.p.g * (c.p.driftMode == 1 ? c.p.cutFraction * c.p.cutFraction : 1.0);
-    hipLaunchKernelGGL(k_onchip_mean, dim3((c.V + 255) / 256, c.nRep), dim3(256), 0, c.stream, (const double *)share,
-                       c.drift, c.V, c.nNoise, fac);
+    hipLaunchKernelGGL(k_onchip_mean, dim3((c.V + 255) / 256, c.nRep), dim3(256), 0, c.stream,
+                       (const double *)onchip_share(c), c.drift, c.V, c.nNoise, fac);
     YCN_HIP(hipGetLastError());
     return YCN_OK;
+}
+
+// the fermion force of every system into c.drift; the states stay on the device
+int onchip_force(Ctx &c, const double *phi, uint32_t streamBase, uint64_t step) {
+    const int rc = onchip_launch<false, true>(c, phi, c.nSys, streamBase, step, nullptr, onchip_share(c));
+    return rc ? rc : onchip_mean(c);
 }
 
 // D^-1 of the packed source in c.eta (system 0, c.nNoise = 1) into out

@@ -422,6 +422,12 @@ int ycn_cg_solve(ycn_ctx *ctx, const double *phi, const double *b, double *x, in
 }
 
 static int force_impl(Ctx &c, uint64_t step, uint32_t streamBase, SolveStats *st) {
+    if (onchip_eo(c)) {
+        int rc = onchip_eo_force(c, c.phi[c.cur], streamBase, step, nullptr);
+        if (!rc) rc = read_stats(c, c.nSys, st);
+        if (!rc) eo_learn_stop_scale(c, c.nSys);
+        return rc;
+    }
     if (c.p.evenOdd) {   // chi = (D^dag)^-1 eta through the Schur complement on the even sites
         int rc = eo_solve(c, c.phi[c.cur], c.nSys, true, streamBase, step, st);
         if (rc) return rc;

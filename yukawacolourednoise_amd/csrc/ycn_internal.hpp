@@ -318,6 +318,13 @@ int onchip_init(Ctx &c);
 bool onchip_plain(const Ctx &c);
 int onchip_force(Ctx &c, const double *phi, uint32_t streamBase, uint64_t step);
 int onchip_propagator(Ctx &c, const double *phi, double2 *out);
+double *onchip_share(Ctx &c);
+int onchip_mean(Ctx &c);
+// the same for the even-odd solvers (onchip_eo.hip); ctl (or null): the starting threshold
+// from the control block of a run
+bool onchip_eo(const Ctx &c);
+int onchip_eo_force(Ctx &c, const double *phi, uint32_t streamBase, uint64_t step, const StepCtl *ctl);
+int onchip_eo_propagator(Ctx &c, const double *phi, double2 *out);
 
 // even-odd preconditioned fermion force (evenodd.hip)
 bool eo_available(const Ctx &c);
@@ -334,6 +341,8 @@ int eo_drift(Ctx &c, const double *phi, double *drift, const StepCtl *ctl = null
 bool eo_graph_eligible(const Ctx &c);
 int eo_graph_run(Ctx &c, uint64_t step0, int nsteps, SolveStats *tot);
 int eo_propagator(Ctx &c, const double *phi, double2 *out, SolveStats *st);
+// the next solve's starting threshold from the states in the pinned mirror
+void eo_learn_stop_scale(Ctx &c, int nsys);
 
 // precision conversion
 int spinor_to_f32(Ctx &c, const double2 *a, float2 *b, int nsys);
