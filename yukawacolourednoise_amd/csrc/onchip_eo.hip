@@ -125,7 +125,7 @@ template <int K, bool WR1, bool GEN, bool PROP>
 __global__ void __launch_bounds__(kOnchipEoThreads)
 k_onchip_eo(OnchipEoArgs A, const double *__restrict__ phi, const uint64_t *__restrict__ seeds, uint32_t streamBase,
             uint64_t step, double2 *eta, double2 *bg, double *__restrict__ drift, double2 *__restrict__ out,
-            CgState *__restrict__ st, const StepCtl *__restrict__ ctl) {
+            CgState *__restrict__ st, const double *__restrict__ ratioIn, double *__restrict__ ratioOut, int nsys) {
     using L = EoLds<K>;
     extern __shared__ double2 sh[];
     __shared__ double red[2][16];
@@ -229,7 +229,15 @@ k_onchip_eo(OnchipEoArgs A, const double *__restrict__ phi, const uint64_t *__re
     const double enorm2 = onchip_sum(acc, red, turn);
     double rr = onchip_sum(rn, red, turn);
     double beta = 0.0, need = 0.0, trueRel = 0.0;
-    const double scale = ctl ? ctl->stopScale : A.stopScale;
+    // the starting threshold: the context's, or learned from the solve before as
+    // eo_learn_stop_scale does (ratioIn: that solve's ratios, and the scale it started from)
+    double scale = A.stopScale;
+    if (ratioIn) {
+        double m = 0.0;
+        for (int k = threadIdx.x; k < nsys; k += blockDim.x) m = fmax(m, ratioIn[k]);
+        m = onchip_max(m, red, turn);
+        scale = m > 0.0 ? fmin(1.0, fmax(1e-3, 0.9 * m)) : ratioIn[nsys];
+    }
     const double stop0 = A.mode == YCN_TOL_ABS_RECURSIVE ? A.tol : A.tol * sqrt(rr);
     double stop = A.mode == YCN_TOL_REL_TRUE ? stop0 * scale : stop0;
     int iter = 0, restarts = 0;
@@ -333,6 +341,10 @@ k_onchip_eo(OnchipEoArgs A, const double *__restrict__ phi, const uint64_t *__re
         s.true_rel = trueRel;
         s.need = need;
         s.stop0 = stop0;
+        if (ratioOut) {
+            ratioOut[sys] = need > 0.0 && stop0 > 0.0 ? need / stop0 : 0.0;
+            if (sys == 0) ratioOut[nsys] = scale;
+        }
     }
 }
 
@@ -344,7 +356,7 @@ bool onchip_eo(const Ctx &c) {
 
 template <bool GEN, bool PROP>
 static int launch_eo(Ctx &c, const double *phi, int nsys, uint32_t streamBase, uint64_t step, double *drift,
-                     double2 *out, const StepCtl *ctl) {
+                     double2 *out, const double *ratioIn, double *ratioOut) {
     OnchipEoArgs A;
     A.Nt = c.p.Nt;
     A.Nx = c.p.Nx;
@@ -368,7 +380,7 @@ static int launch_eo(Ctx &c, const double *phi, int nsys, uint32_t streamBase, u
         constexpr int KK = decltype(kTag)::value;
         auto *k = A.r == 1.0 ? &k_onchip_eo<KK, true, GEN, PROP> : &k_onchip_eo<KK, false, GEN, PROP>;
         hipLaunchKernelGGL(k, dim3(nsys), dim3(threads), 2 * EoLds<KK>::bytes, c.stream, A, phi,
-                           (const uint64_t *)c.seed_d, streamBase, step, c.eta, c.t, drift, out, c.cg_d, ctl);
+                           (const uint64_t *)c.seed_d, streamBase, step, c.eta, c.t, drift, out, c.cg_d, ratioIn, ratioOut, nsys);
     };
     if (K == 1)
         go(std::integral_constant<int, 1>());
@@ -378,13 +390,21 @@ static int launch_eo(Ctx &c, const double *phi, int nsys, uint32_t streamBase, u
     return YCN_OK;
 }
 
-int onchip_eo_force(Ctx &c, const double *phi, uint32_t streamBase, uint64_t step, const StepCtl *ctl) {
-    const int rc = launch_eo<true, false>(c, phi, c.nSys, streamBase, step, onchip_share(c), nullptr, ctl);
+int onchip_eo_force(Ctx &c, const double *phi, uint32_t streamBase, uint64_t step, bool chained) {
+    const bool learn = c.p.cgTolMode == YCN_TOL_REL_TRUE && c.ratio;
+    const size_t row = (size_t)c.nSys + 1;
+    const double *in = learn && chained ? c.ratio + row * c.ratioTurn : nullptr;
+    double *out = nullptr;
+    if (learn) {
+        c.ratioTurn ^= 1;
+        out = c.ratio + row * c.ratioTurn;
+    }
+    const int rc = launch_eo<true, false>(c, phi, c.nSys, streamBase, step, onchip_share(c), nullptr, in, out);
     return rc ? rc : onchip_mean(c);
 }
 
 int onchip_eo_propagator(Ctx &c, const double *phi, double2 *out) {
-    return launch_eo<false, true>(c, phi, 1, 0, 0, nullptr, out, nullptr);
+    return launch_eo<false, true>(c, phi, 1, 0, 0, nullptr, out, nullptr, nullptr);
 }
 
 }  // namespace ycn

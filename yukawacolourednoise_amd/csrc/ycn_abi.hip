@@ -163,6 +163,7 @@ void ycn_destroy(ycn_ctx *ctx) {
     cg_free(c);
     mp_free(c);
     cnn_free(c);
+    onchip_free(c);
     if (c.pairR) (void)hipFree(c.pairR);
     if (c.pairX) (void)hipFree(c.pairX);
     double **bufs[] = {&c.phi[0], &c.phi[1], &c.noise, &c.drift, &c.m2_d, &c.phiStage};
@@ -423,7 +424,7 @@ int ycn_cg_solve(ycn_ctx *ctx, const double *phi, const double *b, double *x, in
 
 static int force_impl(Ctx &c, uint64_t step, uint32_t streamBase, SolveStats *st) {
     if (onchip_eo(c)) {
-        int rc = onchip_eo_force(c, c.phi[c.cur], streamBase, step, nullptr);
+        int rc = onchip_eo_force(c, c.phi[c.cur], streamBase, step, false);
         if (!rc) rc = read_stats(c, c.nSys, st);
         if (!rc) eo_learn_stop_scale(c, c.nSys);
         return rc;
@@ -504,6 +505,14 @@ int ycn_langevin_step(ycn_ctx *ctx, uint64_t step, double *eps, ycn_cg_stats *st
     CHECK_CTX(ctx);
     Ctx &c = *ctx;
     SolveStats st;
+    st.systems = c.nSys;
+    if (onchip_steps(c)) {
+        st.iters_mean = 0;
+        const int rc = onchip_run(c, step, 1, &st, eps);
+        if (rc) return rc;
+        fill_stats(st, stats);
+        return st.converged ? YCN_OK : YCN_ERR_NOT_CONVERGED;
+    }
     int rc = step_impl(c, step, &st);
     if (rc) return rc;
     if (eps) {
@@ -527,6 +536,13 @@ int ycn_langevin_run(ycn_ctx *ctx, uint64_t step0, int nsteps, ycn_cg_stats *sta
     SolveStats tot;
     tot.systems = c.nSys;
     tot.iters_mean = 0;   // summed over the steps, divided at the end
+    if (onchip_steps(c)) {
+        const int rc = onchip_run(c, step0, nsteps, &tot, nullptr);
+        if (rc) return rc;
+        tot.iters_mean = nsteps ? tot.iters_mean / nsteps : 0;
+        fill_stats(tot, stats);
+        return tot.converged ? YCN_OK : YCN_ERR_NOT_CONVERGED;
+    }
     int i = 0;
     for (; i < nsteps && !eo_graph_eligible(c); ++i) {
         SolveStats st;

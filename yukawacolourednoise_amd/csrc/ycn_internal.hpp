@@ -99,6 +99,15 @@ struct StepCtl {
     int rounds[7];        // and the iteration count at each
 };
 
+// What one replica's update reports of a Langevin step, in pinned host memory: the step size
+// and the figures of its solves.  seq is written last, with the number the host waits for.
+struct StepReport {
+    double eps, iterSum, rrMax, trueRelMax;
+    double ratio;         // even-odd: largest need / stop0 of the solves (0: none)
+    int iterMax, restarts, converged;
+    uint32_t seq;
+};
+
 enum ProfKernel { PK_NONE = -1, PK_NORMAL_OP = 0, PK_CG_UPDATE, PK_DIRAC, PK_NOISE_COLS, PK_BOSONIC, PK_CNN, PK_COUNT };
 
 struct Ctx {
@@ -198,6 +207,11 @@ struct Ctx {
     };
     std::vector<GraphEntry> graphs;
     bool useGraphs = true;
+    StepReport *report = nullptr;         // [kRunSlots][nRep], pinned: steps whose solves are held on chip
+    uint32_t reportSeq = 0;               // number of the last step enqueued
+    double *ratio = nullptr;              // [2][nSys + 1]: need / stop0 of the last two on-chip even-odd solves, and
+                                          // the threshold scale each started from
+    int ratioTurn = 0;
     bool onchip = false;                  // solves that fit one workgroup run in one launch (YCN_ONCHIP=0: never)
 
     // profiling
@@ -320,11 +334,16 @@ int onchip_force(Ctx &c, const double *phi, uint32_t streamBase, uint64_t step);
 int onchip_propagator(Ctx &c, const double *phi, double2 *out);
 double *onchip_share(Ctx &c);
 int onchip_mean(Ctx &c);
-// the same for the even-odd solvers (onchip_eo.hip); ctl (or null): the starting threshold
-// from the control block of a run
+// the same for the even-odd solvers (onchip_eo.hip); chained: the starting threshold learned on
+// the device from the solve before (a run's later steps), else c.eoStopScale
 bool onchip_eo(const Ctx &c);
-int onchip_eo_force(Ctx &c, const double *phi, uint32_t streamBase, uint64_t step, const StepCtl *ctl);
+int onchip_eo_force(Ctx &c, const double *phi, uint32_t streamBase, uint64_t step, bool chained);
 int onchip_eo_propagator(Ctx &c, const double *phi, double2 *out);
+// Langevin steps of such a context: enqueued one after the other, the host waits once for
+// their reports; eps (nRep, or null): the last step's sizes
+bool onchip_steps(const Ctx &c);
+int onchip_run(Ctx &c, uint64_t step0, int nsteps, SolveStats *tot, double *eps);
+void onchip_free(Ctx &c);
 
 // even-odd preconditioned fermion force (evenodd.hip)
 bool eo_available(const Ctx &c);
