@@ -1,0 +1,67 @@
+"""The plain mixed solver's pipelined iteration: every tile with either finalize, on several
+systems at once and on the smallest lattice each tile takes, and an odd iteration cap, which
+ends after an even launch whose x update the reliable update has to add."""
+import numpy as np
+import pytest
+
+import oracle as O
+from test_gpu_parity import mk, rel
+
+pytestmark = pytest.mark.gpu
+
+TILES = [(4, 16), (8, 32), (16, 16), (16, 32), (32, 32), (8, 64), (16, 64)]
+
+
+@pytest.mark.parametrize("fin", ["fused", "separate"])
+@pytest.mark.parametrize("tile", range(len(TILES)))
+@pytest.mark.parametrize("scale,r", [(1, 1.0), (4, 0.7)])
+def test_every_tile(gpu, monkeypatch, tile, fin, scale, r):
+    """One tile (its halo is the tile itself) and 4 x 4 of them: converged drifts of two noise
+    vectors against the oracle's FP64 drift, to what the tolerance leaves (1e-8, as for the
+    other mixed solvers)."""
+    monkeypatch.setenv("YCN_TILE_PL", str(tile))
+    monkeypatch.setenv("YCN_PL_FIN", fin)
+    monkeypatch.setenv("YCN_ONCHIP", "0")
+    Y = gpu
+    Nt, Nx = scale * TILES[tile][0], scale * TILES[tile][1]
+    p, orc = mk(Y, Nt=Nt, Nx=Nx, r=r, nNoise=2, cgTol=1e-10, cgTolMode=1, cgMaxIter=20000)
+    p.cgPrecision = Y.YCN_CG_MIXED
+    phi = 1.0 + O.hot_start(Nt + Nx, Nt, Nx)
+    with Y.Context(p) as c:
+        c.set_field(phi)
+        d, st = c.fermion_force(3)
+    dr, _ = O.fermion_drift(orc, phi, 3)
+    assert st["converged"] == 1 and st["true_rel_resid"] <= 1e-10
+    assert rel(d, dr) < 1e-8
+
+
+@pytest.mark.parametrize("cap", [61, 62])
+def test_odd_cap(gpu, monkeypatch, cap):
+    Y = gpu
+    res = {}
+    phi = O.hot_start(11, 32, 64)
+    monkeypatch.setenv("YCN_ONCHIP", "0")
+    for n in (cap - 1, cap, cap + 1):
+        p, _ = mk(Y, Nt=32, Nx=64, M=0.3, g=0.5, cgTol=1e-30, cgTolMode=1, cgMaxIter=n)
+        p.cgPrecision = Y.YCN_CG_MIXED
+        with Y.Context(p) as c:
+            c.set_field(phi)
+            d, st = c.fermion_force(5)
+        assert st["converged"] == 0 and st["iters"] == n
+        res[n] = d
+    # the drifts converge: a dropped update would leave the odd cap where the one before it is
+    step = np.linalg.norm(res[cap] - res[cap - 1])
+    assert step > 0.2 * np.linalg.norm(res[cap + 1] - res[cap - 1]) > 0
+
+
+def test_measured_correlator(gpu, monkeypatch):
+    """D D^dag, the operator of the measurement's propagator, through the same iteration."""
+    monkeypatch.setenv("YCN_ONCHIP", "0")
+    Y = gpu
+    p, orc = mk(Y, Nt=32, Nx=48, cgTol=1e-11, cgTolMode=1, cgMaxIter=20000)
+    p.cgPrecision = Y.YCN_CG_MIXED
+    phi = 1.0 + O.hot_start(5, 32, 48)
+    with Y.Context(p) as c:
+        c.set_field(phi)
+        _, _, corr = c.measure(0, 3)
+    assert rel(corr, O.correlator(orc, phi)[0]) < 1e-9

@@ -29,6 +29,7 @@
 
 #include "cg_fused.hpp"
 #include "cg_host.hpp"
+#include "pipelined.hpp"
 #include "ycn_device.hpp"
 #include "ycn_internal.hpp"
 
@@ -135,11 +136,16 @@ k_fin_setup(const double2 *__restrict__ part, int nb, CgState *__restrict__ st, 
     S.rr_prev = tot.x;
     S.rrRel = tot.x;
     S.bnorm2 = tot.x;
+    S.enorm2 = tot.x;
+    S.iter0 = 0;
+    S.nRu = 0;
+    S.need = 0.0;
     S.tol = tol;
     S.mode = mode;
     S.maxIter = maxIter;
     S.maxRestarts = maxRestarts;
     S.stop = (mode == YCN_TOL_ABS_RECURSIVE) ? tol : tol * sqrt(tot.x);
+    S.stop0 = S.stop;
     S.beta = 0.0;
     S.alpha = make_double2(0.0, 0.0);
     S.iter = 0;
@@ -619,7 +625,7 @@ template <int NC, bool GEN>
 __global__ void __launch_bounds__(kNT)
 k_mp_setup(LatticeArgs L, const uint64_t *__restrict__ seeds, uint32_t streamBase, uint64_t step,
            double2 *__restrict__ eta, double2 *__restrict__ x, float2 *__restrict__ xs, float2 *__restrict__ rs,
-           float2 *__restrict__ p0, float2 *__restrict__ p1, double2 *__restrict__ part) {
+           float2 *__restrict__ p0, float2 *__restrict__ p1, float2 *__restrict__ ap, double2 *__restrict__ part) {
     __shared__ double2 lds[kNT / kWave];
     const int sys = blockIdx.y;
     const size_t V = L.V;
@@ -644,7 +650,10 @@ k_mp_setup(LatticeArgs L, const uint64_t *__restrict__ seeds, uint32_t streamBas
             xs[i] = make_float2(0.f, 0.f);
             rs[i] = bs;
             p0[i] = bs;
-            p1[i] = bs;
+            if (ap)   // pipelined: the first launch reads p0 and Ap with zero coefficients
+                ap[i] = make_float2(0.f, 0.f);
+            else
+                p1[i] = bs;
             acc.x += b[c].x * b[c].x + b[c].y * b[c].y;
         }
     }
@@ -1140,6 +1149,8 @@ int mp_alloc(Ctx &c) {
         }
         int rc = eo_pf_alloc(c);
         if (rc) return rc;
+    } else if (c.p.cgPrecision == YCN_CG_MIXED && c.p.precond == YCN_PRECOND_NONE) {
+        return pl_alloc(c);
     }
     return YCN_OK;
 }
@@ -1195,6 +1206,21 @@ static void launch_mp_iteration(Ctx &c, int nsys, int mtype, int parity) {
                        site_blocks(c), c.cg_d, c.active);
 }
 
+// the reliable update's residual r_s = b - A x in FP64, |r|^2 in c.partials
+template <int NC>
+static void launch_true_residual(Ctx &c, const LatticeArgs &L, const double *phi, int nsys, int mtype) {
+    const dim3 g = site_grid(c, nsys);
+    if (mtype == YCN_DAGGER) {
+        hipLaunchKernelGGL((k_true_a<NC, false>), g, dim3(kNT), 0, c.stream, L, phi, (const double2 *)c.x, c.t);
+        hipLaunchKernelGGL((k_true_b<NC, true, true>), g, dim3(kNT), 0, c.stream, L, phi, (const CgState *)c.cg_d,
+                           (const double2 *)c.eta, (const double2 *)c.t, c.r, c.rs, c.partials);
+    } else {
+        hipLaunchKernelGGL((k_true_a<NC, true>), g, dim3(kNT), 0, c.stream, L, phi, (const double2 *)c.x, c.t);
+        hipLaunchKernelGGL((k_true_b<NC, false, true>), g, dim3(kNT), 0, c.stream, L, phi, (const CgState *)c.cg_d,
+                           (const double2 *)c.eta, (const double2 *)c.t, c.r, c.rs, c.partials);
+    }
+}
+
 template <int NC>
 static int mp_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, uint32_t streamBase, uint64_t step,
                     SolveStats *st) {
@@ -1205,6 +1231,8 @@ static int mp_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, ui
     const LatticeArgs L = largs(c);
     const dim3 g = site_grid(c, nsys);
     const int nb = site_blocks(c);
+    const bool pipelined = NC == kPacked && pl_available(c);
+    float2 *ap0 = pipelined ? c.Aps : nullptr;
     // FP32 copy of the field(s) these systems use
     const int nrepUsed = (nsys + c.nNoise - 1) / c.nNoise;
     const int64_t nconv = std::min<int64_t>((int64_t)c.nRep * c.V, (int64_t)nrepUsed * c.V);
@@ -1215,13 +1243,25 @@ static int mp_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, ui
     const int maxIter = c.p.cgMaxIter;
     if (gen)
         hipLaunchKernelGGL((k_mp_setup<NC, true>), g, dim3(kNT), 0, c.stream, L, (const uint64_t *)c.seed_d, streamBase,
-                           step, c.eta, c.x, c.xs, c.rs, c.ps[0], c.ps[1], c.partials);
+                           step, c.eta, c.x, c.xs, c.rs, c.ps[0], c.ps[1], ap0, c.partials);
     else
         hipLaunchKernelGGL((k_mp_setup<NC, false>), g, dim3(kNT), 0, c.stream, L, (const uint64_t *)c.seed_d, streamBase,
-                           step, c.eta, c.x, c.xs, c.rs, c.ps[0], c.ps[1], c.partials);
+                           step, c.eta, c.x, c.xs, c.rs, c.ps[0], c.ps[1], ap0, c.partials);
     hipLaunchKernelGGL(k_fin_setup, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)c.partials, nb, c.cg_d,
                        c.active, c.p.cgTol, c.p.cgTolMode, maxIter, 0);
     YCN_HIP(hipGetLastError());
+    if (pipelined)   // chunks of the pipelined iteration, each closed by x += x_s, r = b - A x
+        return pf_loop(c, nsys, 0, st, [&](int n) -> int {
+            const int rcc = pl_iterations(c, nsys, mtype, n);
+            if (rcc) return rcc;
+            hipLaunchKernelGGL(k_pf_reliable, g, dim3(kNT), 0, c.stream, c.V, (const CgState *)c.cg_d, c.x, c.xs,
+                               (const float2 *)c.ps[1], (const float2 *)c.pfP2, c.ps[0]);
+            launch_true_residual<NC>(c, L, phi, nsys, mtype);
+            hipLaunchKernelGGL(k_fin_pf_true, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)c.partials,
+                               (const double2 *)c.partials, nb, c.cg_d, c.active);
+            YCN_HIP(hipGetLastError());
+            return YCN_OK;
+        });
     const int every = std::max(1, c.p.reliableEvery);
     const int nIt = every + (every & 1);   // even: keeps the p parity
     const int hardCap = maxIter + nIt + 8;
@@ -1235,15 +1275,7 @@ static int mp_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, ui
         launched += nIt;
         // reliable update: x += xs; rs = b - A x in FP64
         hipLaunchKernelGGL(k_mp_accum<NC>, g, dim3(kNT), 0, c.stream, c.V, (const CgState *)c.cg_d, c.x, c.xs);
-        if (mtype == YCN_DAGGER) {
-            hipLaunchKernelGGL((k_true_a<NC, false>), g, dim3(kNT), 0, c.stream, L, phi, (const double2 *)c.x, c.t);
-            hipLaunchKernelGGL((k_true_b<NC, true, true>), g, dim3(kNT), 0, c.stream, L, phi, (const CgState *)c.cg_d,
-                               (const double2 *)c.eta, (const double2 *)c.t, c.r, c.rs, c.partials);
-        } else {
-            hipLaunchKernelGGL((k_true_a<NC, true>), g, dim3(kNT), 0, c.stream, L, phi, (const double2 *)c.x, c.t);
-            hipLaunchKernelGGL((k_true_b<NC, false, true>), g, dim3(kNT), 0, c.stream, L, phi, (const CgState *)c.cg_d,
-                               (const double2 *)c.eta, (const double2 *)c.t, c.r, c.rs, c.partials);
-        }
+        launch_true_residual<NC>(c, L, phi, nsys, mtype);
         hipLaunchKernelGGL(k_fin_mp_true<false>, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)c.partials,
                            nb, c.cg_d, c.active, 0.0);
         YCN_HIP(hipGetLastError());
@@ -1270,7 +1302,13 @@ int plain_propagator(Ctx &c, const double *phi, double2 *out, SolveStats *st) {
         rc = onchip_propagator(c, phi, out);
         return rc ? rc : read_stats(c, 1, st);
     }
+    // its iteration count does not size the force solves' chunks
+    const int pred = c.eoPredIters, last = c.lastIters;
+    const std::vector<int> rounds = c.eoRounds;
     rc = cg_solve(c, phi, 1, YCN_NORMAL, kPacked, false, 0, 0, st);
+    c.eoPredIters = pred;
+    c.lastIters = last;
+    c.eoRounds = rounds;
     if (rc) return rc;
     const LatticeArgs L = largs(c);
     hipLaunchKernelGGL((k_dirac<2, true>), site_grid(c, 1), dim3(kNT), 0, c.stream, L, phi, (const double2 *)c.x, out);
@@ -1339,10 +1377,10 @@ int fcg_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, uint32_t
     const int maxIter = c.p.cgMaxIter;
     if (gen)
         hipLaunchKernelGGL((k_mp_setup<NC, true>), g, dim3(kNT), 0, c.stream, L, (const uint64_t *)c.seed_d, streamBase,
-                           step, c.eta, c.x, c.xs, c.rs, c.ps[0], c.ps[1], c.partials);
+                           step, c.eta, c.x, c.xs, c.rs, c.ps[0], c.ps[1], (float2 *)nullptr, c.partials);
     else
         hipLaunchKernelGGL((k_mp_setup<NC, false>), g, dim3(kNT), 0, c.stream, L, (const uint64_t *)c.seed_d, streamBase,
-                           step, c.eta, c.x, c.xs, c.rs, c.ps[0], c.ps[1], c.partials);
+                           step, c.eta, c.x, c.xs, c.rs, c.ps[0], c.ps[1], (float2 *)nullptr, c.partials);
     hipLaunchKernelGGL(k_fin_setup, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)c.partials, nb, c.cg_d,
                        c.active, c.p.cgTol, c.p.cgTolMode, maxIter, 0);
     // z = CNN(b), rz = <b, z>, p' = z on the first iteration

@@ -30,13 +30,14 @@
 
 #include "cg_fused.hpp"
 #include "cg_host.hpp"
+#include "pipelined.hpp"
 #include "ycn_device.hpp"
 #include "ycn_internal.hpp"
 
 namespace ycn {
 
 namespace {
-constexpr int kNT = 256;
+constexpr int kNT = kPfNT;
 }
 
 struct EoArgs {
@@ -66,14 +67,6 @@ __device__ __forceinline__ int eo_j(const EoArgs &A, int t, int x) { return t * 
 __device__ __forceinline__ int wrapf(int a, int n, float inv) {
     return a - n * (int)floorf(((float)a + 0.5f) * inv);
 }
-// element idx of a buffer through a 32-bit byte offset (the buffers of one system are
-// below 4 GiB), so that the load or store takes a scalar base and a vector offset
-template <typename T>
-__device__ __forceinline__ T &at(T *base, unsigned idx) {
-    using C = typename std::conditional<std::is_const<T>::value, const char, char>::type;
-    return *reinterpret_cast<T *>(reinterpret_cast<C *>(base) + (unsigned)(idx * (unsigned)sizeof(T)));
-}
-
 // Hopping (K for DAG, H otherwise) at site (t, x); ld(t', x', c) returns component c of
 // the input at neighbour (t', x') of the other parity.
 template <bool DAG, typename R, typename V2, typename Ld>
@@ -304,20 +297,6 @@ k_eo_propagator(EoArgs A, const double *__restrict__ phi, const double2 *__restr
 // ---------------------------------------------------------------------------
 // finalize kernels (one block per system, fixed-order sums)
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ double2 eo_fin_sum(const double2 *part, int nb, double2 *lds) {
-    double2 acc = make_double2(0.0, 0.0);
-    int i = threadIdx.x;
-    for (; i + 7 * kNT < nb; i += 8 * kNT) {
-        double2 v[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = part[i + u * kNT];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) acc = cadd(acc, v[u]);
-    }
-    for (; i < nb; i += kNT) acc = cadd(acc, part[i]);
-    return block_sum2<kNT>(acc, lds);
-}
-
 // |eta|^2 and |c|^2 = |S^T b|^2: rr, thresholds and run flags of a new solve
 __global__ void __launch_bounds__(kNT)
 k_fin_eo_setup(const double2 *__restrict__ partE, int nbE, const double2 *__restrict__ partC, int nbC,
@@ -329,8 +308,8 @@ k_fin_eo_setup(const double2 *__restrict__ partE, int nbE, const double2 *__rest
         stopScale = ctl->stopScale;
     }
     const int sys = blockIdx.x;
-    const double2 e = eo_fin_sum(partE + (size_t)sys * nbE, nbE, lds0);
-    const double2 cc = eo_fin_sum(partC + (size_t)sys * nbC, nbC, lds1);
+    const double2 e = pf_fin_sum(partE + (size_t)sys * nbE, nbE, lds0);
+    const double2 cc = pf_fin_sum(partC + (size_t)sys * nbC, nbC, lds1);
     if (threadIdx.x) return;
     CgState &S = st[sys];
     S.enorm2 = e.x;
@@ -370,7 +349,7 @@ __global__ void __launch_bounds__(kNT)
 k_fin_eo_true(const double2 *__restrict__ part, int nb, CgState *__restrict__ st, int *__restrict__ active) {
     __shared__ double2 lds[kNT / kWave];
     const int sys = blockIdx.x;
-    const double2 tot = eo_fin_sum(part + (size_t)sys * nb, nb, lds);
+    const double2 tot = pf_fin_sum(part + (size_t)sys * nb, nb, lds);
     if (threadIdx.x) return;
     CgState &S = st[sys];
     S.true_rel = S.enorm2 > 0.0 ? sqrt(tot.x / S.enorm2) : sqrt(tot.x);
@@ -386,136 +365,6 @@ k_fin_eo_true(const double2 *__restrict__ part, int nb, CgState *__restrict__ st
         }
     } else {
         S.converged = S.true_rel <= S.tol ? 1 : 0;
-    }
-}
-
-// ---------------------------------------------------------------------------
-// finalize of the pipelined FP32 iteration
-// ---------------------------------------------------------------------------
-// Sums of one system's nb block partials of the pipelined iteration (pp[2 b] = (mu, nu),
-// pp[2 b + 1] = (rho, 0)) by one block in a fixed order: thread t adds entries t, t + NT,
-// ..., each round issuing its U loads before adding; valid in thread 0.
-template <int NT>
-__device__ void sum_pf_partials(const double2 *pp, int nb, double2 *lds0, double2 *lds1, double2 &mn, double2 &rh) {
-    constexpr int U = 4;
-    double2 a0 = make_double2(0.0, 0.0), a1 = make_double2(0.0, 0.0);
-    for (int base = threadIdx.x; base < nb; base += U * NT) {
-        double2 v[2 * U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int k = base + u * NT;
-            v[2 * u] = k < nb ? pp[2 * k] : make_double2(0.0, 0.0);
-            v[2 * u + 1] = k < nb ? pp[2 * k + 1] : make_double2(0.0, 0.0);
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            a0 = cadd(a0, v[2 * u]);
-            a1 = cadd(a1, v[2 * u + 1]);
-        }
-    }
-    mn = block_sum2<NT>(a0, lds0);
-    rh = block_sum2<NT>(a1, lds1);
-}
-
-// The decision after iteration number `iter` of the pipelined iteration, from (mu, nu)
-// and the exact rho of that iteration: alpha = rho / mu and beta = (alpha^2 nu - rho) /
-// rho for the next one (a negative prediction, from cancellation, restarts the
-// direction).  Pause at the stop after an even number of iterations (the last direction
-// applied is then in p[1]), at the cap, or on a non-positive <p, Ap>; a reliable update
-// follows a pause.
-struct PfStep {
-    double alpha, beta;
-    bool stop;
-};
-__device__ __forceinline__ PfStep pf_decide(double mu, double nu, double rho, int iter, const CgState &S) {
-    PfStep d;
-    d.stop = (iter >= S.maxIter) || (sqrt(rho) <= S.stop && !(iter & 1)) || (!(mu > 0.0) && !(iter & 1)) ||
-             (rho < kReliableDrop * kReliableDrop * S.rrRel && !(iter & 1)) || !isfinite(mu) || !isfinite(rho);
-    d.alpha = (mu > 0.0) ? rho / mu : 0.0;
-    double rhoNext = d.alpha * d.alpha * nu - rho;
-    if (!(rhoNext > 0.0)) rhoNext = 0.0;
-    d.beta = (rho > 0.0) ? rhoNext / rho : 0.0;
-    return d;
-}
-
-// the finalize of one iteration from its sums (thread 0): iteration count, rho, pause or
-// the next alpha, beta; commit = false only keeps the sums (timing launches)
-__device__ __forceinline__ void pf_commit(CgState &S, double2 mn, double2 rh, int *active, int commit) {
-    if (!commit) {
-        S.rz = mn.x + mn.y + rh.x;   // a field the even-odd iteration never reads
-        return;
-    }
-    S.iter += 1;
-    const PfStep d = pf_decide(mn.x, mn.y, rh.x, S.iter, S);
-    S.rr_prev = S.rr;
-    S.rr = rh.x;
-    if (d.stop) {
-        S.done = 1;
-        atomicSub(active, 1);
-        return;
-    }
-    S.alpha = make_double2(d.alpha, 0.0);
-    S.beta = d.beta;
-}
-
-// the separate finalize of one iteration (one block per system, after a finMode 0
-// launch); commit = false only reduces (timing)
-template <int NT>
-__global__ void __launch_bounds__(NT)
-k_fin_pf(const double2 *__restrict__ part, int nb, CgState *__restrict__ st, int *__restrict__ active, int commit) {
-    __shared__ double2 lds0[NT / kWave], lds1[NT / kWave];
-    CgState &S = st[blockIdx.x];
-    const int skip = S.done;
-    double2 mn, rh;
-    sum_pf_partials<NT>(part + 2 * (size_t)blockIdx.x * nb, nb, lds0, lds1, mn, rh);
-    if (skip || threadIdx.x) return;
-    pf_commit(S, mn, rh, active, commit);
-}
-
-// the same with one wave per system (systems with at most kNT block partials: one or a
-// few loads per lane and a shuffle reduction, no LDS or barriers)
-__global__ void __launch_bounds__(kNT)
-k_fin_pf_wave(const double2 *__restrict__ part, int nb, int nsys, CgState *__restrict__ st, int *__restrict__ active,
-              int commit) {
-    const int sys = blockIdx.x * (kNT / kWave) + (int)threadIdx.x / kWave;
-    const int lane = threadIdx.x & (kWave - 1);
-    if (sys >= nsys) return;
-    CgState &S = st[sys];
-    const int skip = S.done;
-    const double2 *pp = part + 2 * (size_t)sys * nb;
-    double2 a0 = make_double2(0.0, 0.0), a1 = make_double2(0.0, 0.0);
-    for (int k = lane; k < nb; k += kWave) {
-        a0 = cadd(a0, pp[2 * k]);
-        a1 = cadd(a1, pp[2 * k + 1]);
-    }
-    const double2 mn = make_double2(wave_sum(a0.x), wave_sum(a0.y));
-    const double2 rh = make_double2(wave_sum(a1.x), wave_sum(a1.y));
-    if (skip || lane) return;
-    pf_commit(S, mn, rh, active, commit);
-}
-
-// Finalize at the end of a chunk of n launches that finalized each other in their
-// prologues (finMode 1): launch n - 1's partials in slotLast, launch n - 2's in slotPrev.
-// Systems that paused inside the chunk already hold their state.
-template <int NT>
-__global__ void __launch_bounds__(NT)
-k_fin_pf_chunk(const double2 *__restrict__ slotLast, const double2 *__restrict__ slotPrev, int nb, int n,
-               CgState *__restrict__ st, int *__restrict__ active) {
-    __shared__ double2 lds0[NT / kWave], lds1[NT / kWave];
-    CgState &S = st[blockIdx.x];
-    if (S.done) return;
-    double2 mn, rh, mp, rp;
-    sum_pf_partials<NT>(slotLast + 2 * (size_t)blockIdx.x * nb, nb, lds0, lds1, mn, rh);
-    __syncthreads();
-    sum_pf_partials<NT>(slotPrev + 2 * (size_t)blockIdx.x * nb, nb, lds0, lds1, mp, rp);
-    if (threadIdx.x) return;
-    S.iter = S.iter0 + n;
-    const PfStep d = pf_decide(mn.x, mn.y, rh.x, S.iter, S);
-    S.rr_prev = rp.x;
-    S.rr = rh.x;
-    if (d.stop) {
-        S.done = 1;
-        atomicSub(active, 1);
     }
 }
 
@@ -928,93 +777,6 @@ k_eo_normal_fused(EoArgs A, const R *__restrict__ phi, CgState *st, const typena
     }
 }
 
-// one wave per system for few partials, 1024 threads once a system has more partials
-// than four rounds of 256 threads cover
-static void launch_fin_pf(Ctx &c, int nsys, int nb, int commit) {
-    if (nb <= kNT)
-        hipLaunchKernelGGL(k_fin_pf_wave, dim3((nsys + kNT / kWave - 1) / (kNT / kWave)), dim3(kNT), 0, c.stream,
-                           (const double2 *)c.partials, nb, nsys, c.cg_d, c.active, commit);
-    else if (nb > 4 * kNT)
-        hipLaunchKernelGGL(k_fin_pf<1024>, dim3(nsys), dim3(1024), 0, c.stream, (const double2 *)c.partials, nb,
-                           c.cg_d, c.active, commit);
-    else
-        hipLaunchKernelGGL(k_fin_pf<kNT>, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)c.partials, nb,
-                           c.cg_d, c.active, commit);
-}
-
-// reliable update of the pipelined iteration: x += x_s (FP64), x_s = 0, and the last
-// direction applied copied to p[0], where the next chunk's launch 0 reads it.  After m
-// launches (m counted from the state per system) that is p_{m-2}, in rotation slot
-// (m - 1) mod 3 of p[0], p[1], p2.  For odd m (a stop at the iteration cap after an even
-// launch) the even launch's deferred term alpha_{m-1} p_{m-2} is added too, with the alpha
-// it recorded in ab.
-__global__ void __launch_bounds__(kNT)
-k_pf_reliable(int n, const CgState *__restrict__ st, double2 *__restrict__ x, float2 *__restrict__ xs,
-              const float2 *__restrict__ p1, const float2 *__restrict__ p2, float2 *__restrict__ p0) {
-    const int sys = blockIdx.y;
-    if (st[sys].final_) return;
-    const int s = blockIdx.x * kNT + threadIdx.x;
-    if (s >= n) return;
-    const int m = st[sys].iter - st[sys].iter0, slot = m >= 1 ? (m - 1) % 3 : 0;
-    const float2 *src = slot == 1 ? p1 : slot == 2 ? p2 : p0;
-    const double a = (m & 1) ? st[sys].ab[(m - 1) & 1].x : 0.0;
-    const size_t off = (size_t)sys * 2 * n;
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-        const size_t i = off + (size_t)c * n + s;
-        const float2 d = xs[i];
-        const double2 xv = x[i];
-        double2 xn = make_double2(xv.x + (double)d.x, xv.y + (double)d.y);
-        const float2 pk = (slot != 0 || (m & 1)) ? src[i] : make_float2(0.f, 0.f);
-        if (m & 1) xn = make_double2(xn.x + a * (double)pk.x, xn.y + a * (double)pk.y);
-        x[i] = xn;
-        xs[i] = make_float2(0.f, 0.f);
-        if (slot != 0) p0[i] = pk;
-    }
-}
-
-// after the reliable update of the pipelined iteration: partRes = |b_e - S x_e|^2 and
-// partN = |S^T (b_e - S x_e)|^2 (the new normal residual).  Converged on the system residual, or resume with alpha = 0 (r already is the true
-// residual) and beta = |r_true|^2 / |r_prev|^2 (the direction is kept)
-__global__ void __launch_bounds__(kNT)
-k_fin_eo_pf_true(const double2 *__restrict__ partRes, const double2 *__restrict__ partN, int nb,
-                 CgState *__restrict__ st, int *__restrict__ active) {
-    __shared__ double2 lds0[kNT / kWave], lds1[kNT / kWave];
-    const int sys = blockIdx.x;
-    const int skip = st[sys].final_;
-    const double2 res = eo_fin_sum(partRes + (size_t)sys * nb, nb, lds0);
-    const double2 rn = eo_fin_sum(partN + (size_t)sys * nb, nb, lds1);
-    if (skip || threadIdx.x) return;
-    CgState &S = st[sys];
-    S.true_rel = S.enorm2 > 0.0 ? sqrt(res.x / S.enorm2) : sqrt(res.x);
-    S.restarts += 1;
-    if (S.nRu < kMaxRounds) S.ruIter[S.nRu] = S.iter;
-    S.nRu += 1;
-    // paused at the stop (not for the drop since the last anchor): the normal-equation
-    // threshold the true residual asks for
-    if (S.done && sqrt(S.rr) <= S.stop && S.true_rel > 0.0) S.need = sqrt(rn.x) * S.tol / S.true_rel;
-    const bool conv = (S.mode == YCN_TOL_REL_TRUE) ? (S.true_rel <= S.tol) : (sqrt(rn.x) <= S.stop);
-    if (conv || S.iter >= S.maxIter) {
-        S.converged = conv ? 1 : 0;
-        S.final_ = 1;
-        if (!S.done) {
-            S.done = 1;
-            atomicSub(active, 1);
-        }
-        return;
-    }
-    S.alpha = make_double2(0.0, 0.0);
-    S.beta = (S.rr_prev > 0.0) ? rn.x / S.rr_prev : 0.0;
-    S.rr = rn.x;
-    S.rrRel = rn.x;
-    S.iter0 = S.iter;   // the next chunk's launches count from here
-    if (S.mode == YCN_TOL_REL_TRUE && sqrt(rn.x) <= S.stop) S.stop = sqrt(rn.x) * 0.5 * S.tol / S.true_rel;
-    if (S.done) {
-        S.done = 0;
-        atomicAdd(active, 1);
-    }
-}
-
 // graph-captured Langevin steps: start of a step.  The count of active systems of its
 // solve, and the halt flag and counter the step's coloured noise reads, copied into a
 // second block (noise): the noise runs on a branch of the graph beside the solve, whose
@@ -1262,13 +1024,6 @@ static int launch_eo_ru(Ctx &c, int nsys, const double *phi, const double2 *x, c
     }
 }
 
-// direction p_k (k >= -1) of a chunk of pipelined launches: the three buffers in rotation,
-// p_{-1} (the direction kept across the reliable update) in ps[0]
-static float2 *eo_pdir(const Ctx &c, int k) {
-    float2 *const rot[3] = {c.ps[0], c.ps[1], c.pfP2};
-    return rot[(k + 1) % 3];
-}
-
 // the pipelined FP32 iteration's fused kernel (finMode as in k_eo_normal_fused) with
 // tile `ti` as launch idx of a chunk (idx & 1: the Ap and partial-slot parity, the
 // directions in rotation); returns the block partials per system
@@ -1283,10 +1038,10 @@ static int launch_eo_pf(Ctx &c, int ti, int nsys, int idx, int finMode) {
     b.Ap_in = par ? c.pfA1 : c.Aps;
     b.Ap = par ? c.Aps : c.pfA1;
     b.xs = c.xs;
-    // direction p_k in eo_pdir(c, k); launch 0 reads r, the others p_{idx-2}
-    b.r = idx == 0 ? c.rs : eo_pdir(c, idx - 2);
-    b.pold = eo_pdir(c, idx - 1);
-    b.pnew = eo_pdir(c, idx);
+    // direction p_k in pf_dir(c, k); launch 0 reads r, the others p_{idx-2}
+    b.r = idx == 0 ? c.rs : pf_dir(c, idx - 2);
+    b.pold = pf_dir(c, idx - 1);
+    b.pnew = pf_dir(c, idx);
     // half-lattice FP32 vectors: read p_{idx-2} (or r), Ap, p and write p, Ap, and x_s read and
     // written in odd launches; and read phi.  The figure counts the vectors as the complex
     // spinors of the interface (16 B per site of the full lattice), as ycn_profile_end
@@ -1445,12 +1200,6 @@ static void launch_eo_pf_iteration(Ctx &c, int nsys, int i) {
     }
     launch_fin_pf(c, nsys, launch_eo_pf(c, c.tileEo32, nsys, i, 0), 1);
 }
-// after a chunk of n prologue-finalized launches (n even: launch n - 1 wrote slot 1)
-static void launch_fin_pf_chunk(Ctx &c, int nsys, int n) {
-    hipLaunchKernelGGL(k_fin_pf_chunk<kNT>, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)c.pfSlot[(n - 1) & 1],
-                       (const double2 *)c.pfSlot[n & 1], c.eoPfBlocks, n, c.cg_d, c.active);
-}
-
 // Relative mode: the recursive (normal-equation) residual at which the FP64 true
 // residual reaches tol varies little between consecutive solves, so the next solve
 // starts from 0.9 times the largest ratio need / stop0 the systems of this one reported
@@ -1554,84 +1303,18 @@ static int eo_mixed_chunk(Ctx &c, const double *phi, int nsys, int n, bool graph
     hipLaunchKernelGGL(k_pf_reliable, gH, dim3(kNT), 0, c.stream, Vh, (const CgState *)c.cg_d, c.x, c.xs,
                        (const float2 *)c.ps[1], (const float2 *)c.pfP2, c.ps[0]);
     const int nbR = launch_eo_ru(c, nsys, phi, c.x, B.b, c.r, c.rs, partRu, partRu2);
-    hipLaunchKernelGGL(k_fin_eo_pf_true, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)partRu,
+    hipLaunchKernelGGL(k_fin_pf_true, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)partRu,
                        (const double2 *)partRu2, nbR, c.cg_d, c.active);
     YCN_HIP(hipGetLastError());
     return YCN_OK;
 }
 
-// Length of the next chunk: the reliable-update interval until the predicted iteration
-// count is near, then just past it (a multiple of 8), so that few launches run after the
-// systems have paused.
-static int eo_chunk_len(const Ctx &c, int pred, int itDone) {
-    const int every = std::max(1, c.p.reliableEvery);
-    const int nIt = every + (every & 1);
-    const int rem = pred - itDone + 4;
-    if (pred > 0 && rem < nIt) return std::max(8, (rem + 7) / 8 * 8);
-    return nIt;
-}
-
-// the eager loop polls once it is within this many iterations of the prediction
-static int eo_poll_margin(int pred) { return std::max(8, pred / 8); }
-
-// The pipelined FP32 solve from the state the setup (or an unfinished captured solve)
-// left, until every system is final, polling the systems only where they may have
-// converged; itDone: iterations already done (the chunk lengths count from there).
-// The summary goes to *st, the iteration count and the starting threshold of the next
-// solve are learned from it.
+// The pipelined FP32 solve from the state the setup (or an unfinished captured solve) left,
+// until every system is final; itDone: iterations already done.
 static int eo_mixed_loop(Ctx &c, const double *phi, int nsys, int itDone, SolveStats *st) {
-    const int every = std::max(1, c.p.reliableEvery);
-    const int nIt = every + (every & 1);
-    const int hardCap = c.p.cgMaxIter + nIt + 8;
-    int launched = 0, active = nsys, rc;
-    // profiling the iteration with the prologue finalize: a chunk is nothing but
-    // back-to-back iteration launches, so one event pair brackets it and its working
-    // launches are the iterations the systems did in it (the most of any system)
-    const bool chunkProf = c.profTarget == PK_NORMAL_OP && c.eoFinFused;
-    std::vector<int> itPrev(chunkProf ? nsys : 0, 0);
-    bool polled = true;
-    while (active > 0 && launched < hardCap) {
-        const int n = eo_chunk_len(c, c.eoPredIters, itDone);
-        const int slot = chunkProf ? prof_chunk_begin(c, PK_NORMAL_OP) : -1;
-        rc = eo_mixed_chunk(c, phi, nsys, n, false);
-        prof_chunk_end(c, slot);
-        if (rc) return rc;
-        launched += n;
-        // poll only where the systems may have converged: well short of the previous
-        // solve's iteration count they cannot have, so the next chunk is enqueued at
-        // once (its kernels exit at once for systems that are final after all)
-        if (c.eoPredIters > 0 && itDone + n + eo_poll_margin(c.eoPredIters) < c.eoPredIters && !chunkProf) {
-            itDone += n;
-            polled = false;
-            continue;
-        }
-        rc = poll_iters(c, nsys, active, itDone);
-        if (rc) return rc;
-        polled = true;
-        if (chunkProf) {
-            int work = 0;
-            for (int k = 0; k < nsys; ++k) {
-                work = std::max(work, c.cg_h[k].iter - itPrev[k]);
-                itPrev[k] = c.cg_h[k].iter;
-            }
-            if (slot >= 0) c.evWork[slot] = work;
-        }
-    }
-    if (!polled) {   // the launch cap ended the loop after a skipped poll
-        rc = poll_iters(c, nsys, active, itDone);
-        if (rc) return rc;
-    }
-    SolveStats out;   // the last poll left the final states in the mirror
-    rc = stats_from_mirror(c, nsys, &out);
-    if (rc) return rc;
-    c.eoPredIters = out.iters_max;
-    int kMax = 0;
-    for (int k = 1; k < nsys; ++k)
-        if (c.cg_h[k].iter > c.cg_h[kMax].iter) kMax = k;
-    c.eoRounds.assign(c.cg_h[kMax].ruIter, c.cg_h[kMax].ruIter + std::min(c.cg_h[kMax].nRu, kMaxRounds));
-    eo_learn_stop_scale(c, nsys);
-    if (st) *st = out;
-    return YCN_OK;
+    const int rc = pf_loop(c, nsys, itDone, st, [&](int n) { return eo_mixed_chunk(c, phi, nsys, n, false); });
+    if (!rc) eo_learn_stop_scale(c, nsys);
+    return rc;
 }
 
 // Solve S chi_e = b_e for every system (eta from the Philox streams when gen); chi_e is
@@ -1757,9 +1440,9 @@ static std::vector<int> eo_main_chunks(const Ctx &c, int pred) {
     std::vector<int> v;
     int itDone = 0;
     do {
-        v.push_back(eo_chunk_len(c, pred, itDone));
+        v.push_back(pf_chunk_len(c, pred, itDone));
         itDone += v.back();
-    } while (itDone + eo_poll_margin(pred) < pred && itDone < cap);
+    } while (itDone + pf_poll_margin(pred) < pred && itDone < cap);
     return v;
 }
 

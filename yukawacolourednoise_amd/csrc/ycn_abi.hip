@@ -262,6 +262,7 @@ int ycn_create(const ycn_params *p, ycn_ctx **out) {
     if (const char *sg = std::getenv("YCN_STEP_GRAPHS")) c.stepGraphsOn = std::atoi(sg) != 0;
     if ((rc = onchip_init(c))) return bail(rc);
     if ((rc = cg_autotune(c))) return bail(rc);
+    if ((rc = pl_autotune(c))) return bail(rc);
     if (c.p.evenOdd) {
         if (c.p.precond == YCN_PRECOND_CNN) {
             c.err = "even-odd preconditioning and the learned preconditioner are exclusive";

@@ -166,6 +166,7 @@ struct Ctx {
     // direction buffer (the directions rotate through ps[0], ps[1], pfP2)
     float2 *pfA1 = nullptr, *pfP2 = nullptr;
     double2 *pfSlot[2] = {nullptr, nullptr};   // block partials of prologue-finalized launches
+    int tilePl = -1;                      // tile of the plain pipelined FP32 iteration (-1: not available)
     bool eoFinFused = false;              // pipelined iteration finalizes in the next launch's prologue
     int eoPfBlocks = 0;                   // blocks per system of those launches (same tile throughout)
     float *phis = nullptr;
@@ -282,6 +283,12 @@ int point_source(Ctx &c);
 int plain_propagator(Ctx &c, const double *phi, double2 *out, SolveStats *st);
 // correlator / trace helpers
 int spinor_slices(Ctx &c, const double2 *psi, double *out_dev);
+
+// pipelined FP32 iteration of the plain mixed solver (plain.hip)
+int pl_alloc(Ctx &c);
+int pl_autotune(Ctx &c);
+bool pl_available(const Ctx &c);
+int pl_iterations(Ctx &c, int nsys, int mtype, int n);
 
 // cnn.hip
 int cnn_alloc(Ctx &c);
