@@ -1,29 +1,36 @@
-"""The plain mixed solver's pipelined iteration: every tile with either finalize, on several
-systems at once and on the smallest lattice each tile takes, and an odd iteration cap, which
-ends after an even launch whose x update the reliable update has to add."""
+"""The plain solvers' pipelined iterations, FP32 (mixed precision) and FP64: every tile with either
+finalize, on several systems at once, on the smallest lattice each tile takes and on lattices that
+it does not divide; odd iteration caps, which end after an even launch whose x update is still to
+be added; caps on both sides of a captured chunk's end; restarts from the true residual."""
 import numpy as np
 import pytest
 
 import oracle as O
-from test_gpu_parity import mk, rel
+from test_gpu_parity import RTOL, mk, rel
 
 pytestmark = pytest.mark.gpu
 
 TILES = [(4, 16), (8, 32), (16, 16), (16, 32), (32, 32), (8, 64), (16, 64)]
 
 
+def extents(tile, scale):
+    """scale tiles each way; scale 0: two tiles and a part in time, one and a part in space."""
+    TT, TX = TILES[tile]
+    return (scale * TT, scale * TX) if scale else (2 * TT + 3, TX + 1)
+
+
 @pytest.mark.parametrize("fin", ["fused", "separate"])
 @pytest.mark.parametrize("tile", range(len(TILES)))
-@pytest.mark.parametrize("scale,r", [(1, 1.0), (4, 0.7)])
+@pytest.mark.parametrize("scale,r", [(1, 1.0), (4, 0.7), (0, 1.0)])
 def test_every_tile(gpu, monkeypatch, tile, fin, scale, r):
-    """One tile (its halo is the tile itself) and 4 x 4 of them: converged drifts of two noise
-    vectors against the oracle's FP64 drift, to what the tolerance leaves (1e-8, as for the
-    other mixed solvers)."""
+    """One tile (its halo is the tile itself), 4 x 4 of them and cut-off ones: converged drifts of
+    two noise vectors against the oracle's FP64 drift, to what the tolerance leaves (1e-8, as for
+    the other mixed solvers)."""
     monkeypatch.setenv("YCN_TILE_PL", str(tile))
     monkeypatch.setenv("YCN_PL_FIN", fin)
     monkeypatch.setenv("YCN_ONCHIP", "0")
     Y = gpu
-    Nt, Nx = scale * TILES[tile][0], scale * TILES[tile][1]
+    Nt, Nx = extents(tile, scale)
     p, orc = mk(Y, Nt=Nt, Nx=Nx, r=r, nNoise=2, cgTol=1e-10, cgTolMode=1, cgMaxIter=20000)
     p.cgPrecision = Y.YCN_CG_MIXED
     phi = 1.0 + O.hot_start(Nt + Nx, Nt, Nx)
@@ -65,3 +72,42 @@ def test_measured_correlator(gpu, monkeypatch):
         c.set_field(phi)
         _, _, corr = c.measure(0, 3)
     assert rel(corr, O.correlator(orc, phi)[0]) < 1e-9
+
+
+@pytest.mark.parametrize("fin", ["fused", "separate"])
+@pytest.mark.parametrize("tile", range(len(TILES)))
+@pytest.mark.parametrize("scale,r,cap", [(1, 0.7, 13), (0, 1.0, 12), (0, 0.7, 1), (2, 1.0, 26)])
+def test_fp64_every_tile(gpu, monkeypatch, tile, fin, scale, r, cap):
+    """Fixed iteration counts: the oracle's count, and its iterate to rounding."""
+    monkeypatch.setenv("YCN_TILE_PL", str(tile))
+    monkeypatch.setenv("YCN_PL_FIN", fin)
+    monkeypatch.setenv("YCN_ONCHIP", "0")
+    Y = gpu
+    Nt, Nx = extents(tile, scale)
+    p, orc = mk(Y, Nt=Nt, Nx=Nx, r=r, nNoise=2, cgTol=0.0, cgTolMode=0, cgMaxIter=cap)
+    phi = 1.0 + O.hot_start(Nt + Nx, Nt, Nx)
+    with Y.Context(p) as c:
+        c.set_field(phi)
+        d, st = c.fermion_force(3)
+    dr, sr = O.fermion_drift(orc, phi, 3)
+    assert 2 * st["iters"] == sr["iters"]   # the oracle adds up its solves
+    assert rel(d, dr) < RTOL
+
+
+@pytest.mark.parametrize("mode,tol", [(0, 1e-9), (1, 1e-10), (1, 3e-15)])
+def test_fp64_stop(gpu, monkeypatch, mode, tol):
+    """Both tolerance modes; 3e-15 is near where rounding holds the true residual above the
+    recursive one, so that the solve restarts from it."""
+    monkeypatch.setenv("YCN_ONCHIP", "0")
+    Y = gpu
+    Nt, Nx = 45, 50
+    p, orc = mk(Y, Nt=Nt, Nx=Nx, cgTol=tol, cgTolMode=mode, cgMaxIter=20000)
+    phi = 1.0 + O.hot_start(8, Nt, Nx)
+    with Y.Context(p) as c:
+        c.set_field(phi)
+        d, st = c.fermion_force(3)
+    dr, sr = O.fermion_drift(orc, phi, 3)
+    print(f"# {tol}: {st} oracle {sr}", flush=True)
+    if tol > 1e-12:
+        assert st["converged"] == 1 and st["iters"] == sr["iters"]
+    assert rel(d, dr) < 1e-8

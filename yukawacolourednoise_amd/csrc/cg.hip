@@ -138,6 +138,8 @@ k_fin_setup(const double2 *__restrict__ part, int nb, CgState *__restrict__ st, 
     S.bnorm2 = tot.x;
     S.enorm2 = tot.x;
     S.iter0 = 0;
+    S.pfBase = 0;
+    S.pfLaunch = 0;
     S.nRu = 0;
     S.need = 0.0;
     S.tol = tol;
@@ -214,11 +216,14 @@ k_fin_true(const double2 *__restrict__ part, int nb, CgState *__restrict__ st, i
     CgState &S = st[sys];
     const double bn = sqrt(S.bnorm2);
     S.true_rel = bn > 0.0 ? sqrt(tot.x) / bn : sqrt(tot.x);
+    S.pfLaunch = 0;
     if (S.mode != YCN_TOL_REL_TRUE) return;
     if (S.true_rel > S.tol && S.iter < S.maxIter && S.restarts < S.maxRestarts) {
         S.restarts += 1;   // r already holds b - A x; p' = r on the next iteration
         S.rr = tot.x;
         S.beta = 0.0;
+        S.iter0 = S.iter;
+        S.pfBase = S.iter;
         S.done = 0;
         S.converged = 0;
         atomicAdd(active, 1);
@@ -1080,20 +1085,26 @@ static int fp64_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, 
     int launched = 0, active = nsys;
     int chunk = std::max(kGraphIters, std::min(c.lastIters, maxIter));
     const int hardCap = maxIter * (maxRestarts + 1) + 2 * kGraphIters;
+    const bool pipelined = NC == kPacked && p64_available(c);
     for (int guard = 0; guard < maxRestarts + 2; ++guard) {
+        bool first = true;
         while (active > 0 && launched < hardCap) {
-            // about `chunk` iterations as captured graphs of kGraphIters, then poll
+            // about `chunk` iterations as captured graphs, then poll
             const int n = std::min(chunk, hardCap - launched);
-            for (int k = 0; k < n; k += kGraphIters) {
-                rc = run_chunk(c, phi, nsys, mtype, kGraphIters, YCN_CG_FP64, NC, c.tile64,
-                               [&](int i) { launch_iteration<NC>(c, L, phi, nsys, mtype, i & 1); });
+            for (int k = 0, m = kGraphIters; k < n; k += m, launched += m) {
+                if (pipelined)
+                    rc = p64_iterations(c, phi, nsys, mtype, first, &m);
+                else
+                    rc = run_chunk(c, phi, nsys, mtype, kGraphIters, YCN_CG_FP64, NC, c.tile64,
+                                   [&](int i) { launch_iteration<NC>(c, L, phi, nsys, mtype, i & 1); });
                 if (rc) return rc;
+                first = false;
             }
-            launched += ((n + kGraphIters - 1) / kGraphIters) * kGraphIters;
             rc = poll_active(c, active);
             if (rc) return rc;
             chunk = std::max(kGraphIters, std::min(64, chunk / 2));
         }
+        if (pipelined) p64_close(c, nsys);
         // FP64 true residual (restarts systems in YCN_TOL_REL_TRUE mode while above tol)
         if (mtype == YCN_DAGGER) {
             hipLaunchKernelGGL((k_true_a<NC, false>), g, dim3(kNT), 0, c.stream, L, phi, (const double2 *)c.x, c.t);
@@ -1149,8 +1160,6 @@ int mp_alloc(Ctx &c) {
         }
         int rc = eo_pf_alloc(c);
         if (rc) return rc;
-    } else if (c.p.cgPrecision == YCN_CG_MIXED && c.p.precond == YCN_PRECOND_NONE) {
-        return pl_alloc(c);
     }
     return YCN_OK;
 }

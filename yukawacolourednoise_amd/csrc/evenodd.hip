@@ -1105,7 +1105,7 @@ int eo_autotune(Ctx &c) {
             for (int i = 0; i < kNumEo32; ++i) {
                 if (!eo_fits(c, kEoTiles32[i])) continue;
                 us[kNumEo64 + 2 * i] =
-                    time_it([&](int k) { launch_fin_pf(c, c.nSys, launch_eo_pf(c, i, c.nSys, k, 0), 0); });
+                    time_it([&](int k) { launch_fin_pf(c, c.nSys, launch_eo_pf(c, i, c.nSys, k, 0), 0, c.partials); });
                 us[kNumEo64 + 2 * i + 1] = time_it([&](int k) { (void)launch_eo_pf(c, i, c.nSys, k, 2); });
             }
         tune_store(1, c, us);
@@ -1198,7 +1198,7 @@ static void launch_eo_pf_iteration(Ctx &c, int nsys, int i) {
         c.eoPfBlocks = launch_eo_pf(c, c.tileEo32, nsys, i, 1);
         return;
     }
-    launch_fin_pf(c, nsys, launch_eo_pf(c, c.tileEo32, nsys, i, 0), 1);
+    launch_fin_pf(c, nsys, launch_eo_pf(c, c.tileEo32, nsys, i, 0), 1, c.partials);
 }
 // Relative mode: the recursive (normal-equation) residual at which the FP64 true
 // residual reaches tol varies little between consecutive solves, so the next solve

@@ -152,6 +152,71 @@ __device__ __forceinline__ bool pf_prologue(CgState *st, int sys, int idx, int f
     return false;
 }
 
+// ---------------------------------------------------------------------------
+// finalize of the pipelined FP64 iterations
+// ---------------------------------------------------------------------------
+// The decision after a launch that would complete iteration number `iter` of the textbook
+// recurrence (its r update included): alpha, and |r|^2 after it from the recurrence.  That
+// prediction is off by a few eps rho, so it is not taken below 1e-13 rho; and where rho itself,
+// summed exactly, has reached the stop, the step is not taken.  Stop as the unpipelined
+// iteration does (k_fin_beta): at the stop, at the cap, or on a NaN.
+struct P64Step {
+    double alpha, beta, rr;
+    int iter;
+    bool stop, conv;
+};
+__device__ __forceinline__ P64Step p64_decide(double mu, double nu, double rho, int iter, const CgState &S) {
+    P64Step d;
+    if (sqrt(rho) <= S.stop) return {0.0, 0.0, rho, iter - 1, true, true};
+    d.iter = iter;
+    d.alpha = rho / mu;
+    d.rr = d.alpha * d.alpha * nu - rho;
+    if (d.rr <= 1e-13 * rho) d.rr = 1e-13 * rho;
+    d.beta = d.rr / rho;
+    d.conv = sqrt(d.rr) <= S.stop;
+    d.stop = !(sqrt(d.rr) > S.stop) || iter >= S.maxIter;
+    return d;
+}
+// a system stops after the launch that iteration `it` names, its last x updates left to the close
+__device__ __forceinline__ void p64_stop(CgState &S, int it, const P64Step &d, int *active) {
+    S.done = 1;
+    S.converged = d.conv ? 1 : 0;
+    S.pfLaunch = it - S.pfBase;
+    atomicSub(active, 1);
+}
+
+// pf_prologue for FP64
+template <int NT>
+__device__ __forceinline__ bool p64_prologue(CgState *st, int sys, int idx, int finMode, const double2 *prevPart,
+                                             int *active, double2 *red, double2 *red2, double *bc, int *pause,
+                                             double &alpha, double &beta) {
+    alpha = st[sys].alpha.x;
+    beta = st[sys].beta;
+    if (finMode == 0 || idx == 0) return true;
+    const int nb = (int)gridDim.x;
+    double2 mn, rh;
+    sum_pf_partials<NT>(prevPart + 2 * (size_t)sys * nb, nb, red, red2, mn, rh);
+    if (threadIdx.x == 0) {
+        CgState &S = st[sys];
+        const int it = S.iter0 + idx;
+        const P64Step d = p64_decide(mn.x, mn.y, rh.x, it, S);
+        bc[0] = d.alpha;
+        bc[1] = d.beta;
+        *pause = finMode == 1 && d.stop;
+        if (finMode == 1 && d.stop && blockIdx.x == 0) {
+            S.alpha = make_double2(d.alpha, 0.0);
+            S.iter = d.iter;
+            S.rr_prev = rh.x;
+            S.rr = d.rr;
+            p64_stop(S, it, d, active);
+        }
+    }
+    __syncthreads();
+    alpha = bc[0];
+    beta = bc[1];
+    return !*pause;
+}
+
 // the separate finalize of one iteration (one block per system, after a finMode 0
 // launch); commit = false only reduces (timing)
 template <int NT>
@@ -215,15 +280,15 @@ k_fin_pf_chunk(const double2 *__restrict__ slotLast, const double2 *__restrict__
 
 // one wave per system for few partials, 1024 threads once a system has more partials
 // than four rounds of 256 threads cover
-inline void launch_fin_pf(Ctx &c, int nsys, int nb, int commit) {
+inline void launch_fin_pf(Ctx &c, int nsys, int nb, int commit, const double2 *part) {
     if (nb <= kPfNT)
         hipLaunchKernelGGL(k_fin_pf_wave, dim3((nsys + kPfNT / kWave - 1) / (kPfNT / kWave)), dim3(kPfNT), 0, c.stream,
-                           (const double2 *)c.partials, nb, nsys, c.cg_d, c.active, commit);
+                           part, nb, nsys, c.cg_d, c.active, commit);
     else if (nb > 4 * kPfNT)
-        hipLaunchKernelGGL(k_fin_pf<1024>, dim3(nsys), dim3(1024), 0, c.stream, (const double2 *)c.partials, nb,
+        hipLaunchKernelGGL(k_fin_pf<1024>, dim3(nsys), dim3(1024), 0, c.stream, part, nb,
                            c.cg_d, c.active, commit);
     else
-        hipLaunchKernelGGL(k_fin_pf<kPfNT>, dim3(nsys), dim3(kPfNT), 0, c.stream, (const double2 *)c.partials, nb,
+        hipLaunchKernelGGL(k_fin_pf<kPfNT>, dim3(nsys), dim3(kPfNT), 0, c.stream, part, nb,
                            c.cg_d, c.active, commit);
 }
 

@@ -1,17 +1,19 @@
-// plain.hip -- the pipelined FP32 iteration of the plain mixed-precision solver on D^dag D or
-// D D^dag (packed real spinors): one launch per CG iteration.
+// plain.hip -- the pipelined iterations of the plain solvers on D^dag D or D D^dag (packed real
+// spinors), FP32 for mixed precision and FP64: one launch per CG iteration.
 //
 // The iteration is the even-odd one's (k_eo_normal_fused in evenodd.hip): CG with the residual
 // norm recurrence of D'Azevedo, Eijkhout and Romine (LAPACK Working Note 56, 1993), so that one
 // reduction per iteration suffices and the x and r updates move into the next application of
-// the operator; r rebuilt from the directions after launch 0 of a chunk, x_s updated by every
+// the operator; r rebuilt from the directions after launch 0 of a chunk, x (x_s) updated by every
 // other launch for both; the finalize in the next launch's prologue or a launch of its own.
-// Per site and launch it reads p_{k-2} (or r), Ap, p and phi and writes p and Ap, and every other
-// launch updates x_s: 84 and 116 B, against 4 x 16 + 4 and 6 x 16 B in four launches (operator,
-// alpha, update, beta) before.
+// In FP32, per site and launch it reads p_{k-2} (or r), Ap, p and phi and writes p and Ap, and
+// every other launch updates x_s: 84 and 116 B, against 4 x 16 + 4 and 6 x 16 B in four launches
+// (operator, alpha, update, beta) before.  FP64: twice that, against 328 B in four launches.
 //
-// What bounds it: at 512 x 512 the vectors stay in the caches and a launch is latency, its chain
-// of partial sums, loads, two stencil stages and a reduction.
+// What bounds it: at 512 x 512 in FP32 the vectors stay in the caches and a launch is latency,
+// its chain of partial sums, loads, two stencil stages and a reduction.  At 1024 x 1024 in FP64
+// it moves 210 MB per launch out of the 256 MB last-level cache; an iteration takes 40 us there
+// against 68 us for the four launches.
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -23,51 +25,104 @@ namespace ycn {
 
 struct PlArgs {
     int Nt, Nx, V, nNoise;
-    float hp, hm, hr, d0, g;
+    double r, d0, g;
     int tilesX, tilesPerSys, xcdRemap;
 };
 
-// v times d minus the hop of D (DAG = false) or D^dag at array entry i of N (rows of W)
-template <bool DAG, bool WR1>
-__device__ __forceinline__ float4 pl_dirac(const PlArgs &A, const float4 *N, int i, int W, float sf, float sb, float d,
-                                           float4 v) {
-    const float2 *const N2 = reinterpret_cast<const float2 *>(N);
-    const float sTb = DAG ? sf : sb, sTf = DAG ? sb : sf;
-    const int iTb = DAG ? i + W : i - W, iTf = DAG ? i - W : i + W;
-    const float4 xf = DAG ? N[i - 1] : N[i + 1], xb = DAG ? N[i + 1] : N[i - 1];
-    const float2 tb0 = N2[2 * iTb], tf1 = N2[2 * iTf + 1];
-    float4 o;
-    if constexpr (WR1) {
-        o.x = sTb * tb0.x + 0.5f * ((xf.x + xb.x) + (xb.z - xf.z));
-        o.y = sTb * tb0.y + 0.5f * ((xf.y + xb.y) + (xb.w - xf.w));
-        o.z = sTf * tf1.x + 0.5f * ((xf.z + xb.z) + (xb.x - xf.x));
-        o.w = sTf * tf1.y + 0.5f * ((xf.w + xb.w) + (xb.y - xf.y));
-    } else {
-        const float2 tb1 = N2[2 * iTb + 1], tf0 = N2[2 * iTf];
-        const float ap = A.hp * sTb, am = A.hm * sTf, bm = A.hm * sTb, bp = A.hp * sTf;
-        o.x = ap * tb0.x + am * tf0.x + A.hr * (xf.x + xb.x) + 0.5f * (xb.z - xf.z);
-        o.y = ap * tb0.y + am * tf0.y + A.hr * (xf.y + xb.y) + 0.5f * (xb.w - xf.w);
-        o.z = bm * tb1.x + bp * tf1.x + A.hr * (xf.z + xb.z) + 0.5f * (xb.x - xf.x);
-        o.w = bm * tb1.y + bp * tf1.y + A.hr * (xf.w + xb.w) + 0.5f * (xb.y - xf.y);
+// a site's packed spinor: spins 0 and 1, each (flavour 0, flavour 1)
+template <typename R>
+struct Sp {
+    typename Vec2<R>::T a, b;
+};
+// n of them in LDS, read and written without bank conflicts: whole 16-byte entries in FP32, a
+// plane per spin in FP64
+template <typename R, int N>
+struct SpLds;
+template <int N>
+struct SpLds<float, N> {
+    float4 e[N];
+    __device__ __forceinline__ Sp<float> get(int i) const {
+        const float4 v = e[i];
+        return {make_float2(v.x, v.y), make_float2(v.z, v.w)};
     }
-    return make_float4(d * v.x - o.x, d * v.y - o.y, d * v.z - o.z, d * v.w - o.w);
+    __device__ __forceinline__ float2 s0(int i) const { return reinterpret_cast<const float2 *>(e)[2 * i]; }
+    __device__ __forceinline__ float2 s1(int i) const { return reinterpret_cast<const float2 *>(e)[2 * i + 1]; }
+    __device__ __forceinline__ void set(int i, Sp<float> v) { e[i] = make_float4(v.a.x, v.a.y, v.b.x, v.b.y); }
+};
+template <int N>
+struct SpLds<double, N> {
+    double2 e[2][N];
+    __device__ __forceinline__ Sp<double> get(int i) const { return {e[0][i], e[1][i]}; }
+    __device__ __forceinline__ double2 s0(int i) const { return e[0][i]; }
+    __device__ __forceinline__ double2 s1(int i) const { return e[1][i]; }
+    __device__ __forceinline__ void set(int i, Sp<double> v) {
+        e[0][i] = v.a;
+        e[1][i] = v.b;
+    }
+};
+
+template <typename R>
+__device__ __forceinline__ double sq(Sp<R> v) {
+    return (double)((v.a.x * v.a.x + v.a.y * v.a.y) + (v.b.x * v.b.x + v.b.y * v.b.y));
 }
-__device__ __forceinline__ float sq4(float4 v) { return (v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w); }
-__device__ __forceinline__ float4 axpy4(float4 u, float s, float4 v) {
-    return make_float4(u.x + s * v.x, u.y + s * v.y, u.z + s * v.z, u.w + s * v.w);
+template <typename R>
+__device__ __forceinline__ Sp<R> axpy(Sp<R> u, R s, Sp<R> v) {
+    return {mk2<R>(u.a.x + s * v.a.x, u.a.y + s * v.a.y), mk2<R>(u.b.x + s * v.b.x, u.b.y + s * v.b.y)};
+}
+// a spinor of two planes of V entries
+template <typename R, typename P>
+__device__ __forceinline__ Sp<R> load_sp(P *v, unsigned V, unsigned i) {
+    return {at(v, i), at(v, V + i)};
+}
+template <typename R, typename P>
+__device__ __forceinline__ void store_sp(P *v, unsigned V, unsigned i, Sp<R> s) {
+    at(v, i) = s.a;
+    at(v, V + i) = s.b;
 }
 
-// One launch of the iteration; XM, RM, idx and finMode as in k_eo_normal_fused.  A block owns a
-// TT x TX tile; a thread keeps the same M0 entries of the tile with its 2-site halo through all
-// stages, so that an entry's own values stay in registers.
-template <int TT, int TX, int NT, bool DAG1, bool WR1, int XM, int RM>
+// v times d minus the hop of D (DAG = false) or D^dag at array entry i of N (rows of W)
+template <typename R, bool DAG, bool WR1, typename Lds>
+__device__ __forceinline__ Sp<R> pl_dirac(R r, const Lds &N, int i, int W, R sf, R sb, R d, Sp<R> v) {
+    using V2 = typename Vec2<R>::T;
+    const R h = (R)0.5, sTb = DAG ? sf : sb, sTf = DAG ? sb : sf;
+    const int iTb = DAG ? i + W : i - W, iTf = DAG ? i - W : i + W;
+    const Sp<R> xf = N.get(DAG ? i - 1 : i + 1), xb = N.get(DAG ? i + 1 : i - 1);
+    const V2 tb0 = N.s0(iTb), tf1 = N.s1(iTf);
+    Sp<R> o;
+    if constexpr (WR1) {
+        o.a.x = sTb * tb0.x + h * ((xf.a.x + xb.a.x) + (xb.b.x - xf.b.x));
+        o.a.y = sTb * tb0.y + h * ((xf.a.y + xb.a.y) + (xb.b.y - xf.b.y));
+        o.b.x = sTf * tf1.x + h * ((xf.b.x + xb.b.x) + (xb.a.x - xf.a.x));
+        o.b.y = sTf * tf1.y + h * ((xf.b.y + xb.b.y) + (xb.a.y - xf.a.y));
+    } else {
+        const V2 tb1 = N.s1(iTb), tf0 = N.s0(iTf);
+        const R hp = h * (r + (R)1), hm = h * (r - (R)1), hr = h * r;
+        const R ap = hp * sTb, am = hm * sTf, bm = hm * sTb, bp = hp * sTf;
+        o.a.x = ap * tb0.x + am * tf0.x + hr * (xf.a.x + xb.a.x) + h * (xb.b.x - xf.b.x);
+        o.a.y = ap * tb0.y + am * tf0.y + hr * (xf.a.y + xb.a.y) + h * (xb.b.y - xf.b.y);
+        o.b.x = bm * tb1.x + bp * tf1.x + hr * (xf.b.x + xb.b.x) + h * (xb.a.x - xf.a.x);
+        o.b.y = bm * tb1.y + bp * tf1.y + hr * (xf.b.y + xb.b.y) + h * (xb.a.y - xf.a.y);
+    }
+    return {mk2<R>(d * v.a.x - o.a.x, d * v.a.y - o.a.y), mk2<R>(d * v.b.x - o.b.x, d * v.b.y - o.b.y)};
+}
+
+// One launch of the iteration.  XM, RM, idx and finMode as in k_eo_normal_fused; FIRST forms
+// (XM 0, RM 1) read r and skip its update, alpha being 0.  A block owns a TT x TX tile (cut
+// off at the lattice's edges); a thread keeps the same M0 entries of the tile with its 2-site
+// halo through all stages, so that an entry's own values stay in registers.  FP64 keeps one
+// array in LDS, for p and then for D p, with a barrier more, so that three blocks of 32 x 32
+// sites fit a compute unit instead of one.
+template <typename R, int TT, int TX, int NT, bool DAG1, bool WR1, int XM, int RM>
 __global__ void __launch_bounds__(NT)
-k_pl_pf(PlArgs A, const float *__restrict__ phi, CgState *st, const float2 *__restrict__ r,
-        const float2 *__restrict__ Ap_in, const float2 *__restrict__ pold, float2 *__restrict__ pnew,
-        float2 *__restrict__ Ap, float2 *__restrict__ xs, double2 *__restrict__ part, int finMode, int idx,
+k_pl_pf(PlArgs A, const R *__restrict__ phi, CgState *st, const typename Vec2<R>::T *__restrict__ r,
+        const typename Vec2<R>::T *__restrict__ Ap_in, const typename Vec2<R>::T *__restrict__ pold,
+        typename Vec2<R>::T *__restrict__ pnew, typename Vec2<R>::T *__restrict__ Ap,
+        typename Vec2<R>::T *__restrict__ xs, double2 *__restrict__ part, int finMode, int idx,
         const double2 *__restrict__ prevPart, int *active) {
     constexpr int H = TT + 4, W = TX + 4, N = H * W, M0 = (N + NT - 1) / NT;
-    __shared__ float4 P[N], Q[N];
+    constexpr bool FP64 = sizeof(R) == 8;
+    __shared__ SpLds<R, N> P;
+    __shared__ SpLds<R, FP64 ? 1 : N> Q32;
     __shared__ double2 red[NT / kWave], red2[NT / kWave];
     __shared__ double bc[3];
     __shared__ int pause;
@@ -81,15 +136,16 @@ k_pl_pf(PlArgs A, const float *__restrict__ phi, CgState *st, const float2 *__re
     pnew += off;
     Ap += off;
     xs += off;
-    const float *ph = phi + (size_t)(sys / A.nNoise) * V;
+    const R *ph = phi + (size_t)(sys / A.nNoise) * V;
     int tile = blockIdx.x;   // contiguous bands of tiles per XCD
     if (A.xcdRemap) tile = (tile % 8) * (A.tilesPerSys / 8) + tile / 8;
     const int ty = tile / A.tilesX, t0 = ty * TT, x0 = (tile - ty * A.tilesX) * TX;
+    const int rowEnd = min(TT, A.Nt - t0) + 2, colEnd = min(TX, A.Nx - x0) + 2;
 
     // an entry's place: 1 = within the 1-site halo, 2 = the tile's own; 4, 8: the hops across
     // the time boundary, forward and backward
-    float4 a[M0], p[M0], q[M0], xv[M0];
-    float d[M0];
+    Sp<R> a[M0], p[M0], q[M0], xv[M0];
+    R d[M0];
     unsigned gs[M0];
     int at_[M0];
 #pragma unroll
@@ -101,49 +157,42 @@ k_pl_pf(PlArgs A, const float *__restrict__ phi, CgState *st, const float2 *__re
             const int gt = wrapi(t0 - 2 + row, A.Nt), gx = wrapi(x0 - 2 + col, A.Nx);
             gs[u] = (unsigned)(gt * A.Nx + gx);
             const bool in1 = row >= 1 && row < H - 1 && col >= 1 && col < W - 1;
-            const bool in2 = row >= 2 && row < H - 2 && col >= 2 && col < W - 2;
+            const bool in2 = row >= 2 && row < rowEnd && col >= 2 && col < colEnd;
             at_[u] = (in1 ? 1 : 0) | (in2 ? 2 : 0) | (gt == A.Nt - 1 ? 4 : 0) | (gt == 0 ? 8 : 0);
-            const float2 r0 = at(r, gs[u]), r1 = at(r, V + gs[u]), p0 = at(pold, gs[u]), p1 = at(pold, V + gs[u]),
-                         q0 = at(Ap_in, gs[u]), q1 = at(Ap_in, V + gs[u]);
-            a[u] = make_float4(r0.x, r0.y, r1.x, r1.y);
-            p[u] = make_float4(p0.x, p0.y, p1.x, p1.y);
-            q[u] = make_float4(q0.x, q0.y, q1.x, q1.y);
-            if (XM != 0 && in2) {
-                const float2 x0_ = at(xs, gs[u]), x1_ = at(xs, V + gs[u]);
-                xv[u] = make_float4(x0_.x, x0_.y, x1_.x, x1_.y);
-            }
+            a[u] = load_sp<R>(r, V, gs[u]);
+            p[u] = load_sp<R>(pold, V, gs[u]);
+            if (RM == 2) q[u] = load_sp<R>(Ap_in, V, gs[u]);
+            if (XM != 0 && in2) xv[u] = load_sp<R>(xs, V, gs[u]);
             d[u] = at(ph, gs[u]);
         }
     }
     const double2 prev = RM == 2 ? st[sys].ab[(idx - 1) & 1] : make_double2(0.0, 0.0);
     double alphaD, betaD;
-    if (!pf_prologue<NT>(st, sys, idx, finMode, prevPart, part, active, red, red2, bc, &pause, alphaD, betaD)) return;
+    if constexpr (FP64) {
+        if (!p64_prologue<NT>(st, sys, idx, finMode, prevPart, active, red, red2, bc, &pause, alphaD, betaD)) return;
+    } else {
+        if (!pf_prologue<NT>(st, sys, idx, finMode, prevPart, part, active, red, red2, bc, &pause, alphaD, betaD))
+            return;
+    }
     if (blockIdx.x == 0 && threadIdx.x == 0) st[sys].ab[idx & 1] = make_double2(alphaD, betaD);
-    const float alpha = (float)alphaD, beta = (float)betaD, alphaPrev = (float)prev.x, betaPrev = (float)prev.y;
+    const R alpha = (R)alphaD, beta = (R)betaD, alphaPrev = (R)prev.x, betaPrev = (R)prev.y;
+    const R wr = (R)A.r;
 
     double rho = 0.0, mu = 0.0, nu = 0.0;
 #pragma unroll
     for (int u = 0; u < M0; ++u) {
         const int i = threadIdx.x + u * NT;
         if (i < N) {
-            d[u] = A.d0 + A.g * d[u];
-            const float4 p2 = a[u];
-            if (RM == 2) a[u] = axpy4(p[u], -betaPrev, a[u]);
-            a[u] = axpy4(a[u], -alpha, q[u]);
+            d[u] = (R)A.d0 + (R)A.g * d[u];
+            const Sp<R> p2 = a[u];
+            if (RM == 2) a[u] = axpy<R>(axpy<R>(p[u], -betaPrev, a[u]), -alpha, q[u]);
             if (at_[u] & 2) {
-                rho += (double)sq4(a[u]);
-                if (XM == 2) {
-                    xv[u] = axpy4(axpy4(xv[u], alphaPrev, p2), alpha, p[u]);
-                    at(xs, gs[u]) = make_float2(xv[u].x, xv[u].y);
-                    at(xs, V + gs[u]) = make_float2(xv[u].z, xv[u].w);
-                }
+                rho += sq(a[u]);
+                if (XM == 2) store_sp<R>(xs, V, gs[u], axpy<R>(axpy<R>(xv[u], alphaPrev, p2), alpha, p[u]));
             }
-            p[u] = axpy4(a[u], beta, p[u]);
-            P[i] = p[u];
-            if (at_[u] & 2) {
-                at(pnew, gs[u]) = make_float2(p[u].x, p[u].y);
-                at(pnew, V + gs[u]) = make_float2(p[u].z, p[u].w);
-            }
+            p[u] = axpy<R>(a[u], beta, p[u]);
+            P.set(i, p[u]);
+            if (at_[u] & 2) store_sp<R>(pnew, V, gs[u], p[u]);
         }
     }
     __syncthreads();
@@ -151,27 +200,88 @@ k_pl_pf(PlArgs A, const float *__restrict__ phi, CgState *st, const float2 *__re
     for (int u = 0; u < M0; ++u)
         if (at_[u] & 1) {
             const int i = threadIdx.x + u * NT;
-            q[u] = pl_dirac<DAG1, WR1>(A, P, i, W, at_[u] & 4 ? -1.f : 1.f, at_[u] & 8 ? -1.f : 1.f, d[u], p[u]);
-            Q[i] = q[u];
-            if (at_[u] & 2) mu += (double)sq4(q[u]);
+            q[u] = pl_dirac<R, DAG1, WR1>(wr, P, i, W, at_[u] & 4 ? (R)-1 : (R)1, at_[u] & 8 ? (R)-1 : (R)1, d[u],
+                                          p[u]);
+            if constexpr (!FP64) Q32.set(i, q[u]);
+            if (at_[u] & 2) mu += sq(q[u]);
         }
-    __syncthreads();
+    if constexpr (FP64) {
+        __syncthreads();
 #pragma unroll
-    for (int u = 0; u < M0; ++u)
-        if (at_[u] & 2) {
-            const int i = threadIdx.x + u * NT;
-            const float4 o = pl_dirac<!DAG1, WR1>(A, Q, i, W, at_[u] & 4 ? -1.f : 1.f, at_[u] & 8 ? -1.f : 1.f, d[u],
-                                                  q[u]);
-            at(Ap, gs[u]) = make_float2(o.x, o.y);
-            at(Ap, V + gs[u]) = make_float2(o.z, o.w);
-            nu += (double)sq4(o);
-        }
+        for (int u = 0; u < M0; ++u)
+            if (at_[u] & 1) P.set(threadIdx.x + u * NT, q[u]);
+    }
+    __syncthreads();
+    auto second = [&](const auto &Q) {
+#pragma unroll
+        for (int u = 0; u < M0; ++u)
+            if (at_[u] & 2) {
+                const int i = threadIdx.x + u * NT;
+                const Sp<R> o = pl_dirac<R, !DAG1, WR1>(wr, Q, i, W, at_[u] & 4 ? (R)-1 : (R)1,
+                                                        at_[u] & 8 ? (R)-1 : (R)1, d[u], q[u]);
+                store_sp<R>(Ap, V, gs[u], o);
+                nu += sq(o);
+            }
+    };
+    if constexpr (FP64)
+        second(P);
+    else
+        second(Q32);
     const size_t pidx = (size_t)sys * gridDim.x + blockIdx.x;
     const double2 t1 = block_sum2<NT>(make_double2(mu, nu), red);
     const double2 t2 = block_sum2<NT>(make_double2(rho, 0.0), red2);
     if (threadIdx.x == 0) {
         part[2 * pidx] = t1;
         part[2 * pidx + 1] = t2;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// FP64: end of a phase of launches
+// ---------------------------------------------------------------------------
+// Finalize after the launches of a chunk that finalized each other (n of them), or after one
+// launch (n = 1); commit = 0 only reduces (timing).
+template <int NT>
+__global__ void __launch_bounds__(NT)
+k_fin_p64(const double2 *__restrict__ part, int nb, int n, CgState *__restrict__ st, int *__restrict__ active,
+          int commit) {
+    __shared__ double2 lds0[NT / kWave], lds1[NT / kWave];
+    CgState &S = st[blockIdx.x];
+    const int skip = S.done;
+    double2 mn, rh;
+    sum_pf_partials<NT>(part + 2 * (size_t)blockIdx.x * nb, nb, lds0, lds1, mn, rh);
+    if (skip || threadIdx.x) return;
+    if (!commit) {
+        S.rz = mn.x + mn.y + rh.x;   // a field the plain iteration never reads
+        return;
+    }
+    const P64Step d = p64_decide(mn.x, mn.y, rh.x, S.iter0 + n, S);
+    S.alpha = make_double2(d.alpha, 0.0);
+    S.beta = d.beta;
+    S.iter = d.iter;
+    S.rr_prev = rh.x;
+    S.rr = d.rr;
+    S.iter0 += n;
+    if (d.stop) p64_stop(S, S.iter0, d, active);
+}
+
+// The x updates that the launches of a phase have left to later ones, added to x of the systems
+// that stopped after m = pfLaunch launches: alpha_{m-1} p_{m-1}, and after an odd number of
+// launches alpha_{m-2} p_{m-2} before it.
+__global__ void __launch_bounds__(kPfNT)
+k_p64_close(int n, const CgState *__restrict__ st, double2 *__restrict__ x, const double2 *__restrict__ d0,
+            const double2 *__restrict__ d1, const double2 *__restrict__ d2) {
+    const int sys = blockIdx.y, m = st[sys].pfLaunch, i = blockIdx.x * kPfNT + threadIdx.x;
+    if (m == 0 || i >= n) return;
+    const double2 *const rot[3] = {d0, d1, d2};
+    const double2 *p = rot[m % 3], *pp = rot[(m + 2) % 3];
+    const double al = st[sys].alpha.x, alPrev = (m & 1) && m > 1 ? st[sys].ab[0].x : 0.0;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+        const size_t k = ((size_t)sys * 2 + s) * n + i;
+        double2 v = x[k];
+        if (alPrev != 0.0) v = make_double2(v.x + alPrev * pp[k].x, v.y + alPrev * pp[k].y);
+        x[k] = make_double2(v.x + al * p[k].x, v.y + al * p[k].y);
     }
 }
 
@@ -185,38 +295,48 @@ struct PlTile {
 constexpr PlTile kPlTiles[] = {{4, 16, 192}, {8, 32, 448}, {16, 16, 448}, {16, 32, 384}, {32, 32, 448}, {8, 64, 448},
                                {16, 64, 704}};
 constexpr int kNumPl = sizeof(kPlTiles) / sizeof(kPlTiles[0]);
+constexpr int kP64Launches = 12;   // per captured FP64 chunk: keeps both buffer rotations
 
-static bool pl_fits(const Ctx &c, PlTile t) { return c.p.Nt % t.TT == 0 && c.p.Nx % t.TX == 0; }
+// a tile need not divide the lattice, but its halo may wrap around only once
+static bool pl_fits(const Ctx &c, PlTile t) {
+    auto ok = [](int n, int T) { return n >= 2 && (n % T == 0 || n > T); };
+    return ok(c.p.Nt, t.TT) && ok(c.p.Nx, t.TX);
+}
+static int pl_blocks(const Ctx &c, PlTile t) {
+    return ((c.p.Nt + t.TT - 1) / t.TT) * ((c.p.Nx + t.TX - 1) / t.TX);
+}
 
-// launch idx of a chunk (buffers as in the even-odd iteration's launch_eo_pf, on the full
-// lattice); returns the block partials per system
-template <int TT, int TX, int NT>
-static int launch_pl_tt(const Ctx &c, int nsys, bool dag1, int idx, int finMode) {
+template <typename R>
+struct PlPtrs {
+    using V2 = typename Vec2<R>::T;
+    const R *phi;
+    const V2 *r, *Ap_in, *pold;
+    V2 *pnew, *Ap, *x;
+};
+
+// launch idx of a chunk; form 0: launch 0 of a phase (r read), 1: odd launches, 2: even ones;
+// returns the block partials per system
+template <typename R, int TT, int TX, int NT>
+static int launch_pl_tt(const Ctx &c, int nsys, bool dag1, int idx, int form, int finMode, const PlPtrs<R> &b) {
     PlArgs A;
     A.Nt = c.p.Nt;
     A.Nx = c.p.Nx;
     A.V = c.V;
     A.nNoise = c.nNoise;
-    A.hp = (float)(0.5 * (c.p.r + 1.0));
-    A.hm = (float)(0.5 * (c.p.r - 1.0));
-    A.hr = (float)(0.5 * c.p.r);
-    A.d0 = (float)(2.0 * c.p.r + c.p.M);
-    A.g = (float)c.p.g;
-    A.tilesX = c.p.Nx / TX;
-    A.tilesPerSys = (c.p.Nt / TT) * A.tilesX;
+    A.r = c.p.r;
+    A.d0 = 2.0 * c.p.r + c.p.M;
+    A.g = c.p.g;
+    A.tilesX = (c.p.Nx + TX - 1) / TX;
+    A.tilesPerSys = pl_blocks(c, {TT, TX, NT});
     A.xcdRemap = A.tilesPerSys % 8 == 0 ? 1 : 0;
-    const int par = idx & 1, form = idx == 0 ? 0 : par ? 1 : 2;
-    const float2 *r = idx == 0 ? c.rs : pf_dir(c, idx - 2);
-    double2 *part = finMode ? c.pfSlot[par] : c.partials;
     auto go = [&](auto dagTag, auto wrTag) {
         constexpr bool D = decltype(dagTag)::value, W1 = decltype(wrTag)::value;
-        using K = decltype(&k_pl_pf<TT, TX, NT, D, W1, 0, 1>);
-        const K ks[3] = {&k_pl_pf<TT, TX, NT, D, W1, 0, 1>, &k_pl_pf<TT, TX, NT, D, W1, 2, 2>,
-                         &k_pl_pf<TT, TX, NT, D, W1, 0, 2>};
-        hipLaunchKernelGGL(ks[form], dim3(A.tilesPerSys, nsys), dim3(NT), 0, c.stream, A, (const float *)c.phis, c.cg_d,
-                           r, (const float2 *)(par ? c.pfA1 : c.Aps), (const float2 *)pf_dir(c, idx - 1),
-                           pf_dir(c, idx), par ? c.Aps : c.pfA1, c.xs, part, finMode, idx,
-                           (const double2 *)c.pfSlot[par ^ 1], c.active);
+        using K = decltype(&k_pl_pf<R, TT, TX, NT, D, W1, 0, 1>);
+        const K ks[3] = {&k_pl_pf<R, TT, TX, NT, D, W1, 0, 1>, &k_pl_pf<R, TT, TX, NT, D, W1, 2, 2>,
+                         &k_pl_pf<R, TT, TX, NT, D, W1, 0, 2>};
+        hipLaunchKernelGGL(ks[form], dim3(A.tilesPerSys, nsys), dim3(NT), 0, c.stream, A, b.phi, c.cg_d, b.r, b.Ap_in,
+                           b.pold, b.pnew, b.Ap, b.x, c.pfSlot[idx & 1], finMode, idx,
+                           (const double2 *)c.pfSlot[~idx & 1], c.active);
     };
     const bool w1 = c.p.r == 1.0;
     if (dag1)
@@ -226,45 +346,101 @@ static int launch_pl_tt(const Ctx &c, int nsys, bool dag1, int idx, int finMode)
     return A.tilesPerSys;
 }
 
-static int launch_pl(Ctx &c, int ti, int nsys, bool dag1, int idx, int finMode) {
+template <typename R>
+static int launch_pl_any(Ctx &c, int ti, int nsys, bool dag1, int idx, int form, int finMode, const PlPtrs<R> &b) {
     const PlTile t = kPlTiles[ti];
-    prof_before(c, PK_NORMAL_OP, (double)nsys * c.V * ((idx & 1 ? 7 : 5) * 16 + 4));
+    prof_before(c, PK_NORMAL_OP, (double)nsys * c.V * ((idx & 1 ? 7 : 5) * 4 + 1) * sizeof(R));
     int nb = 0;
     switch (t.TT * 1000 + t.TX) {
-    case 4016: nb = launch_pl_tt<4, 16, 192>(c, nsys, dag1, idx, finMode); break;
-    case 8032: nb = launch_pl_tt<8, 32, 448>(c, nsys, dag1, idx, finMode); break;
-    case 16016: nb = launch_pl_tt<16, 16, 448>(c, nsys, dag1, idx, finMode); break;
-    case 16032: nb = launch_pl_tt<16, 32, 384>(c, nsys, dag1, idx, finMode); break;
-    case 32032: nb = launch_pl_tt<32, 32, 448>(c, nsys, dag1, idx, finMode); break;
-    case 8064: nb = launch_pl_tt<8, 64, 448>(c, nsys, dag1, idx, finMode); break;
-    default: nb = launch_pl_tt<16, 64, 704>(c, nsys, dag1, idx, finMode); break;
+    case 4016: nb = launch_pl_tt<R, 4, 16, 192>(c, nsys, dag1, idx, form, finMode, b); break;
+    case 8032: nb = launch_pl_tt<R, 8, 32, 448>(c, nsys, dag1, idx, form, finMode, b); break;
+    case 16016: nb = launch_pl_tt<R, 16, 16, 448>(c, nsys, dag1, idx, form, finMode, b); break;
+    case 16032: nb = launch_pl_tt<R, 16, 32, 384>(c, nsys, dag1, idx, form, finMode, b); break;
+    case 32032: nb = launch_pl_tt<R, 32, 32, 448>(c, nsys, dag1, idx, form, finMode, b); break;
+    case 8064: nb = launch_pl_tt<R, 8, 64, 448>(c, nsys, dag1, idx, form, finMode, b); break;
+    default: nb = launch_pl_tt<R, 16, 64, 704>(c, nsys, dag1, idx, form, finMode, b); break;
     }
     prof_after(c, PK_NORMAL_OP);
     return nb;
 }
 
-// the buffers beyond the mixed solver's: second Ap, third direction, the partial slots of
-// prologue-finalized launches (64-site tiles at the smallest)
-int pl_alloc(Ctx &c) {
-    bool any = false;
-    for (const PlTile &t : kPlTiles) any = any || pl_fits(c, t);
-    if (!any || c.V >= (1 << 27)) return YCN_OK;   // 32-bit byte offsets into a system's two planes
+// FP32 launch idx of a chunk (buffers as in the even-odd iteration's launch_eo_pf, on the full
+// lattice)
+static int launch_pl(Ctx &c, int ti, int nsys, bool dag1, int idx, int finMode) {
+    const int par = idx & 1;
+    PlPtrs<float> b;
+    b.phi = c.phis;
+    b.r = idx == 0 ? c.rs : pf_dir(c, idx - 2);
+    b.Ap_in = par ? c.pfA1 : c.Aps;
+    b.pold = pf_dir(c, idx - 1);
+    b.pnew = pf_dir(c, idx);
+    b.Ap = par ? c.Aps : c.pfA1;
+    b.x = c.xs;
+    return launch_pl_any<float>(c, ti, nsys, dag1, idx, idx == 0 ? 0 : par ? 1 : 2, finMode, b);
+}
+
+// FP64 direction p_k of a phase: p[0] (p_{-1}, multiplied by 0), p[1], and r, which nothing reads
+// after launch 0
+static double2 *p64_dir(const Ctx &c, int k) {
+    double2 *const rot[3] = {c.pv[0], c.pv[1], c.r};
+    return rot[(k + 1) % 3];
+}
+// FP64 launch idx of a chunk (first: the phase's first), A p alternating between t and Ap
+static int launch_p64(Ctx &c, int ti, int nsys, const double *phi, bool dag1, int idx, bool first, int finMode) {
+    const int par = idx & 1;
+    PlPtrs<double> b;
+    b.phi = phi;
+    b.r = first && idx == 0 ? c.r : p64_dir(c, idx + 1);   // p_{idx-2}
+    b.Ap_in = par ? c.t : c.Ap;
+    b.pold = p64_dir(c, idx + 2);
+    b.pnew = p64_dir(c, idx);
+    b.Ap = par ? c.Ap : c.t;
+    b.x = c.x;
+    return launch_pl_any<double>(c, ti, nsys, dag1, idx, first && idx == 0 ? 0 : par ? 1 : 2, finMode, b);
+}
+static void launch_fin_p64(Ctx &c, int nsys, int nb, int n, const double2 *part, int commit) {
+    if (nb > 4 * kPfNT)
+        hipLaunchKernelGGL(k_fin_p64<1024>, dim3(nsys), dim3(1024), 0, c.stream, part, nb, n, c.cg_d, c.active, commit);
+    else
+        hipLaunchKernelGGL(k_fin_p64<kPfNT>, dim3(nsys), dim3(kPfNT), 0, c.stream, part, nb, n, c.cg_d, c.active,
+                           commit);
+}
+
+// the partial slots, and for mixed precision the buffers beyond the mixed solver's: second Ap,
+// third direction
+static int pl_alloc(Ctx &c, bool mixed) {
+    size_t nb = 0;
+    for (const PlTile &t : kPlTiles)
+        if (pl_fits(c, t)) nb = std::max(nb, (size_t)pl_blocks(c, t));
+    if (!nb || c.V >= (1 << 27)) return YCN_OK;   // 32-bit byte offsets into a system's two planes
     const size_t n = (size_t)c.nSys * kPacked * c.V;
-    for (float2 **b : {&c.pfA1, &c.pfP2}) {
-        YCN_HIP(hipMalloc(b, sizeof(float2) * n));
-        YCN_HIP(hipMemset(*b, 0, sizeof(float2) * n));
+    if (mixed)
+        for (float2 **b : {&c.pfA1, &c.pfP2}) {
+            YCN_HIP(hipMalloc(b, sizeof(float2) * n));
+            YCN_HIP(hipMemset(*b, 0, sizeof(float2) * n));
+        }
+    for (double2 *&slot : c.pfSlot) {
+        YCN_HIP(hipMalloc(&slot, sizeof(double2) * c.nSys * nb * 2));
+        YCN_HIP(hipMemset(slot, 0, sizeof(double2) * c.nSys * nb * 2));
     }
-    return eo_pf_alloc(c);
+    return YCN_OK;
 }
 
 bool pl_available(const Ctx &c) { return c.tilePl >= 0; }
+bool p64_available(const Ctx &c) { return c.tileP64 >= 0 && c.profTarget != PK_CG_UPDATE; }
 
-// times every tile that fits, with either finalize, and keeps the fastest pair
+// The pipelined iteration of the context's precision: times every tile that fits, with either
+// finalize, and keeps the fastest pair.
 int pl_autotune(Ctx &c) {
-    c.tilePl = -1;
-    if (c.p.evenOdd || !c.rs || !c.pfA1 || !c.pfP2 || !c.pfSlot[1]) return YCN_OK;
+    c.tilePl = c.tileP64 = -1;
+    if (c.p.evenOdd || c.p.precond != YCN_PRECOND_NONE || onchip_plain(c)) return YCN_OK;
+    const bool mixed = c.p.cgPrecision == YCN_CG_MIXED;
+    if (!mixed && std::getenv("YCN_TILE")) return YCN_OK;   // a forced tile of the unpipelined iteration
+    const int rc = pl_alloc(c, mixed);
+    if (rc || !c.pfSlot[1]) return rc;
     std::vector<double> us;
-    const bool memo = tune_lookup(2, c, us) && us.size() == 2 * (size_t)kNumPl;
+    const int memoKey = mixed ? 2 : 3;
+    const bool memo = tune_lookup(memoKey, c, us) && us.size() == 2 * (size_t)kNumPl;
     if (!memo) {
         us.assign(2 * kNumPl, 1e30);
         hipEvent_t e0, e1;
@@ -276,8 +452,10 @@ int pl_autotune(Ctx &c) {
             if (!pl_fits(c, kPlTiles[i])) continue;
             for (int m = 0; m < 2; ++m) {
                 auto launch = [&](int k) {
-                    const int nb = launch_pl(c, i, c.nSys, false, k, m ? 2 : 0);
-                    if (!m) launch_fin_pf(c, c.nSys, nb, 0);
+                    const int nb = mixed ? launch_pl(c, i, c.nSys, false, k, m ? 2 : 0)
+                                         : launch_p64(c, i, c.nSys, c.phi[c.cur], false, k, true, m ? 2 : 0);
+                    if (!m && mixed) launch_fin_pf(c, c.nSys, nb, 0, c.pfSlot[k & 1]);
+                    if (!m && !mixed) launch_fin_p64(c, c.nSys, nb, 1, c.pfSlot[k & 1], 0);
                 };
                 launch(0);
                 launch(1);
@@ -295,13 +473,15 @@ int pl_autotune(Ctx &c) {
         YCN_HIP(hipGetLastError());
         YCN_HIP(hipMemsetAsync(c.cg_d, 0, sizeof(CgState) * c.nSys, c.stream));
         YCN_HIP(hipStreamSynchronize(c.stream));
-        tune_store(2, c, us);
+        tune_store(memoKey, c, us);
     }
     const char *force = std::getenv("YCN_TILE_PL");   // forces a tile of the table (tests cover every one)
     const int f = force ? std::atoi(force) : -1;
     char line[96];
     double best = 1e30;
-    c.tuneReport += " | fp32 pipelined tiles (us/iteration, separate | prologue finalize):";
+    int &tile = mixed ? c.tilePl : c.tileP64;
+    c.tuneReport += mixed ? " | fp32 pipelined tiles (us/iteration, separate | prologue finalize):"
+                          : " | fp64 pipelined tiles (us/iteration, separate | prologue finalize):";
     for (int i = 0; i < kNumPl; ++i) {
         if (!pl_fits(c, kPlTiles[i])) continue;
         std::snprintf(line, sizeof line, " %dx%d %.1f|%.1f;", kPlTiles[i].TT, kPlTiles[i].TX, us[2 * i], us[2 * i + 1]);
@@ -309,7 +489,7 @@ int pl_autotune(Ctx &c) {
         for (int m = 0; m < 2; ++m)
             if ((f < 0 || f == i) && us[2 * i + m] < best) {
                 best = us[2 * i + m];
-                c.tilePl = i;
+                tile = i;
                 c.eoFinFused = m == 1;
             }
     }
@@ -317,18 +497,34 @@ int pl_autotune(Ctx &c) {
     return YCN_OK;
 }
 
-// n iterations of a chunk on the systems, from the context's residual and kept direction
+// n FP32 iterations of a chunk on the systems, from the context's residual and kept direction
 int pl_iterations(Ctx &c, int nsys, int mtype, int n) {
     const bool dag1 = mtype != YCN_DAGGER;
     const int rc = run_chunk(c, nullptr, nsys, mtype, n, 5, kPacked, c.tilePl, [&](int i) {
         const int nb = launch_pl(c, c.tilePl, nsys, dag1, i, c.eoFinFused ? 1 : 0);
-        c.eoPfBlocks = nb;
-        if (!c.eoFinFused) launch_fin_pf(c, nsys, nb, 1);
+        if (!c.eoFinFused) launch_fin_pf(c, nsys, nb, 1, c.pfSlot[i & 1]);
     });
     if (rc) return rc;
-    c.eoPfBlocks = (c.p.Nt / kPlTiles[c.tilePl].TT) * (c.p.Nx / kPlTiles[c.tilePl].TX);
+    c.eoPfBlocks = pl_blocks(c, kPlTiles[c.tilePl]);
     if (c.eoFinFused) launch_fin_pf_chunk(c, nsys, n);
     return YCN_OK;
+}
+
+// One captured chunk of FP64 iterations (first: of a phase, from the residual in r); returns the
+// launches in *n.  A phase is what runs until every system has stopped; p64_close ends it.
+int p64_iterations(Ctx &c, const double *phi, int nsys, int mtype, bool first, int *n) {
+    *n = kP64Launches;
+    const bool dag1 = mtype != YCN_DAGGER, fused = c.eoFinFused;
+    return run_chunk(c, phi, nsys, mtype, kP64Launches, first ? 6 : 7, kPacked, c.tileP64, [&](int i) {
+        const int nb = launch_p64(c, c.tileP64, nsys, phi, dag1, i, first, fused ? 1 : 0);
+        if (!fused || i == kP64Launches - 1)
+            launch_fin_p64(c, nsys, nb, fused ? kP64Launches : 1, c.pfSlot[i & 1], 1);
+    });
+}
+void p64_close(Ctx &c, int nsys) {
+    hipLaunchKernelGGL(k_p64_close, dim3((c.V + kPfNT - 1) / kPfNT, nsys), dim3(kPfNT), 0, c.stream, c.V,
+                       (const CgState *)c.cg_d, c.x, (const double2 *)p64_dir(c, 2), (const double2 *)p64_dir(c, 0),
+                       (const double2 *)p64_dir(c, 1));
 }
 
 }  // namespace ycn

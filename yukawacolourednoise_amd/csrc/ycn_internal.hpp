@@ -56,6 +56,8 @@ struct CgState {
     double rrRel;      // FP32 loops: recursive |r|^2 when the recursion was last anchored (start, reliable update)
     int nRu;           // pipelined even-odd solve: reliable updates so far
     int ruIter[7];     // pipelined even-odd solve: iteration count at each of the first seven
+    int pfBase;        // pipelined FP64 iteration: iterations done when the phase began
+    int pfLaunch;      // pipelined FP64 iteration: launches of the phase the system stopped in, until the next check
     double2 ab[2];     // pipelined even-odd solve (prologue finalize): alpha, beta of launch idx in ab[idx & 1]
 };
 constexpr int kMaxRounds = 7;
@@ -166,7 +168,7 @@ struct Ctx {
     // direction buffer (the directions rotate through ps[0], ps[1], pfP2)
     float2 *pfA1 = nullptr, *pfP2 = nullptr;
     double2 *pfSlot[2] = {nullptr, nullptr};   // block partials of prologue-finalized launches
-    int tilePl = -1;                      // tile of the plain pipelined FP32 iteration (-1: not available)
+    int tilePl = -1, tileP64 = -1;        // tiles of the plain pipelined FP32 and FP64 iterations (-1: not available)
     bool eoFinFused = false;              // pipelined iteration finalizes in the next launch's prologue
     int eoPfBlocks = 0;                   // blocks per system of those launches (same tile throughout)
     float *phis = nullptr;
@@ -285,10 +287,12 @@ int plain_propagator(Ctx &c, const double *phi, double2 *out, SolveStats *st);
 int spinor_slices(Ctx &c, const double2 *psi, double *out_dev);
 
 // pipelined FP32 iteration of the plain mixed solver (plain.hip)
-int pl_alloc(Ctx &c);
 int pl_autotune(Ctx &c);
 bool pl_available(const Ctx &c);
 int pl_iterations(Ctx &c, int nsys, int mtype, int n);
+bool p64_available(const Ctx &c);
+int p64_iterations(Ctx &c, const double *phi, int nsys, int mtype, bool first, int *n);
+void p64_close(Ctx &c, int nsys);
 
 // cnn.hip
 int cnn_alloc(Ctx &c);
