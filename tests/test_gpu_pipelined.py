@@ -111,3 +111,50 @@ def test_fp64_stop(gpu, monkeypatch, mode, tol):
     if tol > 1e-12:
         assert st["converged"] == 1 and st["iters"] == sr["iters"]
     assert rel(d, dr) < 1e-8
+
+
+EO_TILES = [(8, 32), (16, 32), (16, 16), (4, 32), (2, 32), (4, 16), (32, 32)]
+
+
+@pytest.mark.parametrize("fin", ["fused", "separate"])
+@pytest.mark.parametrize("tile", range(len(EO_TILES)))
+@pytest.mark.parametrize("scale,r,cap", [(1, 0.7, 12), (2, 1.0, 13), (3, 0.7, 1), (2, 1.0, 26)])
+def test_fp64_even_odd_every_tile(gpu, monkeypatch, tile, fin, scale, r, cap):
+    """The even-odd FP64 iteration at fixed iteration counts: the oracle's iterate to rounding."""
+    monkeypatch.setenv("YCN_TILE_PL", str(tile))
+    monkeypatch.setenv("YCN_EO_FIN", fin)
+    Y = gpu
+    Nt, Nx = scale * EO_TILES[tile][0], scale * EO_TILES[tile][1]
+    if Nx % 32 and Nt % 16:
+        Nx *= 2   # even-odd lattices need 32 | Nx or 16 | Nt, Nx
+    p, orc = mk(Y, Nt=Nt, Nx=Nx, r=r, nNoise=2, cgTol=0.0, cgTolMode=0, cgMaxIter=cap)
+    p.evenOdd = 1
+    orc.evenOdd = 1
+    phi = 1.0 + O.hot_start(Nt + Nx, Nt, Nx)
+    with Y.Context(p) as c:
+        c.set_field(phi)
+        d, st = c.fermion_force(3)
+    dr, _ = O.fermion_drift(orc, phi, 3)
+    assert st["iters"] == cap
+    assert rel(d, dr) < RTOL
+
+
+@pytest.mark.parametrize("mode,tol", [(0, 1e-9), (1, 1e-10), (1, 1e-13)])
+def test_fp64_even_odd_stop(gpu, monkeypatch, mode, tol):
+    """Both tolerance modes, one after the other solve: in the relative mode the second starts from
+    the first's learned threshold and may have to go on from where it stopped."""
+    monkeypatch.setenv("YCN_ONCHIP", "0")
+    Y = gpu
+    Nt, Nx = 48, 64
+    p, orc = mk(Y, Nt=Nt, Nx=Nx, M=0.1, cgTol=tol, cgTolMode=mode, cgMaxIter=20000)
+    p.evenOdd = 1
+    with Y.Context(p) as c:
+        for k in range(3):
+            phi = 0.3 * k + O.hot_start(8 + k, Nt, Nx)
+            c.set_field(phi)
+            d, st = c.fermion_force(3)
+            dr, sr = O.fermion_drift(orc, phi, 3)
+            print(f"# {tol}: {st}", flush=True)
+            assert st["converged"] == 1 and st["iters"] % 2 == 0
+            assert mode == 0 or st["true_rel_resid"] <= tol
+            assert rel(d, dr) < 1e-8

@@ -138,6 +138,7 @@ k_fin_setup(const double2 *__restrict__ part, int nb, CgState *__restrict__ st, 
     S.bnorm2 = tot.x;
     S.enorm2 = tot.x;
     S.iter0 = 0;
+    S.even = 0;
     S.pfBase = 0;
     S.pfLaunch = 0;
     S.nRu = 0;

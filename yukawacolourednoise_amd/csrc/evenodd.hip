@@ -60,13 +60,6 @@ __device__ __forceinline__ void eo_site(const EoArgs &A, int par, int j, int &t,
 }
 __device__ __forceinline__ int eo_j(const EoArgs &A, int t, int x) { return t * A.Nh + (x >> 1); }
 
-// a mod n in [0, n) without an integer division (the 4-site halo of a tile spans several
-// periods when an extent is smaller than 4, Nt = 2).  For |a| < 2^22 and inv = fl(1 / n),
-// (a + 1/2) / n lies at least 1 / (2n) from an integer and the two single-precision
-// roundings move it by less than |a + 1/2| / n * 2^-23, so the floor is exact.
-__device__ __forceinline__ int wrapf(int a, int n, float inv) {
-    return a - n * (int)floorf(((float)a + 0.5f) * inv);
-}
 // Hopping (K for DAG, H otherwise) at site (t, x); ld(t', x', c) returns component c of
 // the input at neighbour (t', x') of the other parity.
 template <bool DAG, typename R, typename V2, typename Ld>
@@ -329,6 +322,9 @@ k_fin_eo_setup(const double2 *__restrict__ partE, int nbE, const double2 *__rest
     S.alpha = make_double2(0.0, 0.0);
     S.iter = 0;
     S.iter0 = 0;
+    S.even = 1;
+    S.pfBase = 0;
+    S.pfLaunch = 0;
     S.restarts = 0;
     S.true_rel = 0.0;
     S.rz = 0.0;
@@ -353,12 +349,15 @@ k_fin_eo_true(const double2 *__restrict__ part, int nb, CgState *__restrict__ st
     if (threadIdx.x) return;
     CgState &S = st[sys];
     S.true_rel = S.enorm2 > 0.0 ? sqrt(tot.x / S.enorm2) : sqrt(tot.x);
+    S.pfLaunch = 0;
     if (S.mode != YCN_TOL_REL_TRUE) return;
     if (S.done && S.true_rel > 0.0) S.need = sqrt(S.rr) * S.tol / S.true_rel;   // paused at the stop
     if (S.true_rel > S.tol && S.iter < S.maxIter && S.restarts < S.maxRestarts) {
         S.restarts += 1;
         S.stop = sqrt(S.rr) * 0.5 * S.tol / S.true_rel;
         S.converged = 0;
+        S.iter0 = S.iter;
+        S.pfBase = S.iter;
         if (S.done) {
             S.done = 0;
             atomicAdd(active, 1);
@@ -389,69 +388,19 @@ k_fin_eo_true(const double2 *__restrict__ part, int nb, CgState *__restrict__ st
 // (Vh sites each) and phi, write p', Ap: 4 S/2 + P per site of the full lattice (S = 32 B in FP64).
 constexpr int eo_threads(int tt, int tx) { return (tt * tx / 2 < kWave) ? kWave : tt * tx / 2; }
 
-// PF = false: the operator alone, p' = r + beta p_old, partial <p', Ap> = |v|^2.
-// PF = true, the pipelined FP32 iteration with one reduction.  CG with the residual-norm
-// recurrence of D'Azevedo, Eijkhout and Romine (LAPACK Working Note 56, 1993): with
-// rho = |r|^2, mu = <p, Ap>, nu = |Ap|^2, alpha_k = rho_k / mu_k and <r_k, Ap_k> = mu_k,
-// rho_{k+1} = alpha_k^2 nu_k - rho_k, so beta_{k+1} is known before r_{k+1} exists and
-// the x, r updates move into the next operator application.  Stage 0 then forms, on its
-// even sites, r' = r - alpha Ap, p' = r' + beta p and (tile only) the x_s update; the block
-// partials are (mu, nu) and (rho', 0), rho' the exact |r'|^2 that re-anchors the
-// recurrence every iteration.  Ap ping-pongs between two buffers and the directions rotate
-// through three: blocks read the old ones on their halo while other blocks write the new
-// ones on their tiles.
-// PERSIST = true: the grid holds only as many blocks as are resident; each block walks
-// the tiles blockIdx.x, blockIdx.x + gridDim.x, ... and loads the next tile's stage-0
-// data into registers while it runs stages 1-4 of the current one, so global loads
-// overlap the LDS stages.  One partial per block (its tiles in order).
-// finMode (PF only): 0 = alpha and beta from the state, partials to part (k_fin_pf
-// follows).  1 = launch idx of a chunk finalizes launch idx - 1 in its prologue: every
-// block sums that launch's partials (prevPart) in the same fixed order and derives the
-// same alpha, beta and stop decision, so no finalize launch runs between iterations; a
-// stopping launch's block 0 records the pause and every block returns.  Launch 0 of a
-// chunk starts from the state, k_fin_pf_chunk closes the chunk, and the state is not
-// written otherwise during a chunk (blocks read iter0, not iter).  The per-block reads
-// of prevPart suit grids of resident blocks (PERSIST).  2 = the prologue's reductions
-// without pausing or writing the state (the autotuner's timing launches).
-// RU = true (FP64, PF = false): the reliable update's residual instead of an iteration.
-// Stage 0 stages x (r holds x, beta = 0), stage 2 forms res = b - S x with b (Ap_in) read
-// at its own sites, stage 4 writes r = S^T res (Ap) and its FP32 copy (out32); the
-// partials are |res|^2 (part) and |r|^2 (part2).  Systems already final are skipped.
-// WR1 = true: Wilson parameter r = 1 (hop_flavour_r1), chosen at launch when A.r == 1 (every
-// precision and mode).
-// The pipelined iteration keeps neither r nor x_s in every launch.  Block 0 of each launch
-// records the alpha, beta it used (from the prologue, or from the state that the separate
-// finalize wrote) in the state as ab[idx & 1] for the next launch, and the directions
-// rotate through three buffers.
-// RM (PF only), where r_{idx-1} comes from:
-//   1: read from r (launch 0 of a chunk, after the setup or a reliable update has put the
-//      residual there);
-//   2: rebuilt as r_{idx-1} = p_{idx-1} - beta_{idx-1} p_{idx-2}, the relation that formed
-//      p_{idx-1} (same FP32 beta); r then carries p_{idx-2}, read in place of the residual.
-//      The rebuild's rounding error is a few eps |p| against the eps |r| of a stored r
-//      (|p| is a few |r| in CG), and the FP64 reliable updates bound its drift as they do
-//      the recursion's.
-// XM (PF only), the x_s update:
-//   0: none (an even launch);
-//   2: the odd launch after it adds both terms, alpha_e p_{idx-2} + alpha p_{idx-1}, with
-//      p_{idx-2} the input RM = 2 reads anyway.
-// Pairs never straddle a chunk (chunks have an even number of launches), and a system
-// pauses only after an odd launch (after whole pairs), except at the iteration cap; the
-// reliable update's k_pf_reliable then adds the deferred term.  Per even site and launch:
-// 88 B (even) and 120 B (odd).  XM and RM do not apply to the FP64 forms (PF = false).
-template <typename R, int TT, int TX, bool PF, bool PERSIST = false, bool RU = false, bool WR1 = false, int XM = 1,
-          int RM = 0>
+// RU = true: the reliable update's residual instead of an iteration.  Stage 0 stages x (r holds
+// x, beta = 0), stage 2 forms res = b - S x with b (Ap_in) read at its own sites, stage 4 writes
+// r = S^T res (Ap) and its FP32 copy (out32); the partials are |res|^2 (part) and |r|^2 (part2).
+// Systems already final are skipped.
+// WR1 = true: Wilson parameter r = 1 (hop_flavour_r1), chosen at launch when A.r == 1.
+template <int TT, int TX, bool RU, bool WR1>
 __global__ void __launch_bounds__(eo_threads(TT, TX))
-k_eo_normal_fused(EoArgs A, const R *__restrict__ phi, CgState *st, const typename Vec2<R>::T *__restrict__ r,
-                  const typename Vec2<R>::T *__restrict__ Ap_in, const typename Vec2<R>::T *__restrict__ pold,
-                  typename Vec2<R>::T *__restrict__ pnew, typename Vec2<R>::T *__restrict__ Ap,
-                  typename Vec2<R>::T *__restrict__ xs, double2 *__restrict__ part, int finMode, int idx,
-                  const double2 *__restrict__ prevPart, int *active, float2 *__restrict__ out32,
+k_eo_normal_fused(EoArgs A, const double *__restrict__ phi, CgState *st, const double2 *__restrict__ r,
+                  const double2 *__restrict__ Ap_in, const double2 *__restrict__ pold, double2 *__restrict__ pnew,
+                  double2 *__restrict__ Ap, double2 *__restrict__ part, float2 *__restrict__ out32,
                   double2 *__restrict__ part2) {
-    static_assert(!(PF && RU), "the reliable-update residual runs in FP64 only");
-    static_assert(!PF || ((XM == 0 || XM == 2) && (RM == 1 || RM == 2)), "pipelined forms: XM 0, 2 and RM 1, 2");
-    static_assert(XM != 2 || RM == 2, "the pair's x_s update reads p_{idx-2}");
-    using V2 = typename Vec2<R>::T;
+    using R = double;
+    using V2 = double2;
     constexpr int H = TT + 8, K = (TX + 8) / 2, NT = eo_threads(TT, TX);
     constexpr int M0 = (H * K + NT - 1) / NT;
     // O and FO hold only array rows 1 .. H - 2 (odd sites are needed on the 3-site halo at
@@ -461,7 +410,6 @@ k_eo_normal_fused(EoArgs A, const R *__restrict__ phi, CgState *st, const typena
     __shared__ V2 O[2][HO * K];
     __shared__ R FE[H * K], FO[HO * K];
     __shared__ double2 red[NT / kWave > 0 ? NT / kWave : 1];
-    __shared__ double2 red2[NT / kWave > 0 ? NT / kWave : 1];
 
     const int sys = blockIdx.y;
     if (RU ? st[sys].final_ : st[sys].done) return;
@@ -475,15 +423,9 @@ k_eo_normal_fused(EoArgs A, const R *__restrict__ phi, CgState *st, const typena
         pnew += off;
     }
     Ap += off;
-    if (PF) xs += off;
-    if (PF || RU) Ap_in += off;
+    if (RU) Ap_in += off;
     if (RU) out32 += off;
-    R beta = RU ? (R)0 : (R)st[sys].beta;
-    R alpha = PF ? (R)st[sys].alpha.x : (R)0;
-    double alphaD = PF ? st[sys].alpha.x : 0.0, betaD = RU ? 0.0 : st[sys].beta;   // recorded in ab[idx & 1]
-    // RM = 2, XM = 2: the alpha, beta of launch idx - 1
-    const double2 prev = (PF && RM == 2) ? st[sys].ab[(idx - 1) & 1] : make_double2(0.0, 0.0);
-    const R betaPrev = (R)prev.y, alphaPrev = (R)prev.x;
+    const R beta = RU ? (R)0 : (R)st[sys].beta;
     const R *ph = phi + (size_t)(sys / A.nNoise) * A.V;
     const R hp = (R)(0.5 * (A.r + 1.0)), hm = (R)(0.5 * (A.r - 1.0)), hr = (R)(0.5 * A.r), h = (R)0.5;
     const R d0 = (R)(2.0 * A.r + A.M), g = (R)A.g;
@@ -500,7 +442,7 @@ k_eo_normal_fused(EoArgs A, const R *__restrict__ phi, CgState *st, const typena
     // array's even sites.  Array (row, col) is lattice site (t0 - 4 + row, x0 - 4 + col);
     // its parity is (row + col) & 1 because t0 + x0 is even.
     struct Regs {
-        V2 ra[M0][2], pa[M0][2], aa[M0][2], xa[M0][2];
+        V2 ra[M0][2], pa[M0][2];
         R fe[M0], fo[M0];
         unsigned jj[M0];
     };
@@ -514,23 +456,18 @@ k_eo_normal_fused(EoArgs A, const R *__restrict__ phi, CgState *st, const typena
                 const int colE = 2 * k + (row & 1), colO = 2 * k + 1 - (row & 1);
                 const int gxE = wrapf(x0 - 4 + colE, Nx, A.invNx), gxO = wrapf(x0 - 4 + colO, Nx, A.invNx);
                 G.jj[u] = (unsigned)(gt * Nh + (gxE >> 1));
-                const bool inner = row >= 4 && row < 4 + TT && colE >= 4 && colE < 4 + TX;
 #pragma unroll
                 for (int c = 0; c < 2; ++c) {
                     const unsigned i = c * Vh + G.jj[u];
                     G.ra[u][c] = at(r, i);
                     if (!RU) G.pa[u][c] = at(pold, i);
-                    if (PF) G.aa[u][c] = at(Ap_in, i);
-                    if (PF && XM != 0 && inner) G.xa[u][c] = at(xs, i);
                 }
                 G.fe[u] = at(ph, (unsigned)(gt * Nx + gxE));
                 G.fo[u] = at(ph, (unsigned)(gt * Nx + gxO));
             }
         }
     };
-    // stage 0 proper: p' (PF: r' = r - alpha Ap, x_s += alpha p) into LDS and, on the
-    // tile, to global memory; d on both parities
-    double rho = 0.0;
+    // stage 0 proper: p' into LDS and, on the tile, to global memory; d on both parities
     auto compute0 = [&](const Regs &G) {
 #pragma unroll
         for (int u = 0; u < M0; ++u) {
@@ -539,28 +476,13 @@ k_eo_normal_fused(EoArgs A, const R *__restrict__ phi, CgState *st, const typena
                 const int row = w / K, k = w - row * K;
                 const int colE = 2 * k + (row & 1);
                 const bool inner = row >= 4 && row < 4 + TT && colE >= 4 && colE < 4 + TX;
-                R rs = 0;   // |r'|^2 of the site (4 terms in R, then accumulated in FP64)
 #pragma unroll
                 for (int c = 0; c < 2; ++c) {
-                    const unsigned i = c * Vh + G.jj[u];
-                    V2 a = G.ra[u][c];   // r_{idx-1}, or p_{idx-2} (RM = 2)
-                    const V2 b = RU ? a : G.pa[u][c];
-                    if (PF && RM == 2) a = mk2<R>(b.x - betaPrev * a.x, b.y - betaPrev * a.y);
-                    if (PF) a = mk2<R>(a.x - alpha * G.aa[u][c].x, a.y - alpha * G.aa[u][c].y);
-                    const V2 pv = RU ? a : mk2<R>(a.x + beta * b.x, a.y + beta * b.y);
+                    const V2 a = G.ra[u][c];
+                    const V2 pv = RU ? a : mk2<R>(a.x + beta * G.pa[u][c].x, a.y + beta * G.pa[u][c].y);
                     E[c][w] = pv;
-                    if (inner && !RU) {
-                        at(pnew, i) = pv;
-                        if (PF) {
-                            const V2 xa = G.xa[u][c], p2 = G.ra[u][c];
-                            if (XM == 2)
-                                at(xs, i) = mk2<R>(xa.x + alphaPrev * p2.x + alpha * b.x,
-                                                   xa.y + alphaPrev * p2.y + alpha * b.y);
-                            rs += a.x * a.x + a.y * a.y;
-                        }
-                    }
+                    if (inner && !RU) at(pnew, c * Vh + G.jj[u]) = pv;
                 }
-                if (PF && inner) rho += (double)rs;
                 FE[w] = d0 + g * G.fe[u];
                 if (row >= 1 && row <= HO) FO[w - K] = d0 + g * G.fo[u];
             }
@@ -658,7 +580,7 @@ k_eo_normal_fused(EoArgs A, const R *__restrict__ phi, CgState *st, const typena
             for (int c = 0; c < 2; ++c) O[c][q.i - K] = mk2<R>(o[c].x * inv, o[c].y * inv);
         }
         __syncthreads();
-        // stage 4: Ap = d v - H W on the tile's even sites (PF: and |Ap|^2)
+        // stage 4: Ap = d v - H W on the tile's even sites (RU: and |r|^2)
         for (int w = threadIdx.x; w < TT * (TX / 2); w += NT) {
             const Site q = site_of(w, 0, 0);
             V2 o[2];
@@ -675,105 +597,22 @@ k_eo_normal_fused(EoArgs A, const R *__restrict__ phi, CgState *st, const typena
                 if (RU) at(out32, c * Vh + j) = make_float2((float)a.x, (float)a.y);
                 as += a.x * a.x + a.y * a.y;
             }
-            if (PF || RU) nu += (double)as;
+            if (RU) nu += (double)as;
         }
     };
 
-    // finMode 1, 2: finalize launch idx - 1 (its iteration is number iter0 + idx); false:
-    // the system pauses here
-    auto prologue = [&]() -> bool {
-        if (!PF || finMode == 0 || idx == 0) return true;
-        __shared__ double bc[3];   // alpha, beta, rho of launch idx - 1
-        __shared__ int pause;
-        const int nb = (int)gridDim.x;
-        double2 mn, rh;
-        sum_pf_partials<NT>(prevPart + 2 * (size_t)sys * nb, nb, red, red2, mn, rh);
-        if (threadIdx.x == 0) {
-            const PfStep d = pf_decide(mn.x, mn.y, rh.x, st[sys].iter0 + idx, st[sys]);
-            bc[0] = d.alpha;
-            bc[1] = d.beta;
-            bc[2] = rh.x;
-            pause = finMode == 1 && d.stop;
-        }
-        __syncthreads();
-        if (!pause) {
-            alpha = (R)bc[0];
-            beta = (R)bc[1];
-            alphaD = bc[0];
-            betaD = bc[1];
-            return true;
-        }
-        if (blockIdx.x == 0) {   // record the pause; rho of the iteration before it
-            double rprev = st[sys].rr;   // iteration iter0 (chunk start) when idx == 1
-            if (idx >= 2) {              // launch idx - 2's partials, in this launch's slot
-                double2 m2, r2;
-                sum_pf_partials<NT>(part + 2 * (size_t)sys * nb, nb, red, red2, m2, r2);
-                rprev = r2.x;
-            }
-            if (threadIdx.x == 0) {
-                CgState &S = st[sys];
-                S.iter = S.iter0 + idx;
-                S.rr_prev = rprev;
-                S.rr = bc[2];
-                S.done = 1;
-                atomicSub(active, 1);
-            }
-        }
-        return false;
-    };
-
-    // once alpha is fixed, a pipelined launch records its alpha, beta for the next one
-    auto record_ab = [&]() {
-        if constexpr (PF) {
-            if (blockIdx.x == 0 && threadIdx.x == 0) st[sys].ab[idx & 1] = make_double2(alphaD, betaD);
-        }
-    };
     Regs G;
     int t0, x0;
-    if (!PERSIST) {
-        origin(blockIdx.x, t0, x0);
-        load0(t0, x0, G);
-        if (!prologue()) return;
-        record_ab();
-        compute0(G);
-        __syncthreads();
-        stages(t0, x0);
-    } else {
-        int t = blockIdx.x;
-        origin(t, t0, x0);
-        load0(t0, x0, G);
-        if (!prologue()) return;
-        record_ab();
-        while (t < nTiles) {
-            compute0(G);
-            __syncthreads();
-            const int tn = t + (int)gridDim.x;
-            int n0 = 0, nx0 = 0;
-            if (tn < nTiles) {   // next tile's loads in flight during stages 1-4
-                origin(tn, n0, nx0);
-                load0(n0, nx0, G);
-            }
-            stages(t0, x0);
-            __syncthreads();     // stage 4 reads of E and O precede the next stage 0
-            t = tn;
-            t0 = n0;
-            x0 = nx0;
-        }
-    }
+    origin(blockIdx.x, t0, x0);
+    load0(t0, x0, G);
+    compute0(G);
+    __syncthreads();
+    stages(t0, x0);
     const size_t pidx = (size_t)sys * gridDim.x + blockIdx.x;
-    if (PF) {
-        const double2 t1 = block_sum2<NT>(make_double2(acc, nu), red);
-        const double2 t2 = block_sum2<NT>(make_double2(rho, 0.0), red2);
-        if (threadIdx.x == 0) {
-            part[2 * pidx] = t1;
-            part[2 * pidx + 1] = t2;
-        }
-    } else {
-        const double2 tot = block_sum2<NT>(make_double2(acc, RU ? nu : 0.0), red);
-        if (threadIdx.x == 0) {
-            part[pidx] = make_double2(tot.x, 0.0);
-            if (RU) part2[pidx] = make_double2(tot.y, 0.0);
-        }
+    const double2 tot = block_sum2<NT>(make_double2(acc, RU ? nu : 0.0), red);
+    if (threadIdx.x == 0) {
+        part[pidx] = make_double2(tot.x, 0.0);
+        if (RU) part2[pidx] = make_double2(tot.y, 0.0);
     }
 }
 
@@ -845,6 +684,12 @@ constexpr EoTileCfg kEoTiles64[] = {{8, 32, false}, {16, 16, false}, {4, 64, fal
 constexpr EoTileCfg kEoTiles32[] = {{8, 32, false},  {16, 32, false}, {8, 64, false},  {16, 16, false},
                                     {4, 64, false},  {2, 32, false},  {32, 32, false}, {16, 64, false},
                                     {8, 32, true},   {16, 32, true},  {16, 16, true},  {8, 64, true}};
+// tiles of the pipelined FP64 iteration
+struct EoTile {
+    int TT, TX;
+};
+constexpr EoTile kEoTilesP64[] = {{8, 32}, {16, 32}, {16, 16}, {4, 32}, {2, 32}, {4, 16}, {32, 32}};
+constexpr int kNumEoP64 = sizeof(kEoTilesP64) / sizeof(kEoTilesP64[0]);
 constexpr int kNumEo64 = sizeof(kEoTiles64) / sizeof(kEoTiles64[0]);
 constexpr int kNumEo32 = sizeof(kEoTiles32) / sizeof(kEoTiles32[0]);
 
@@ -869,7 +714,8 @@ static EoArgs eo_args(const Ctx &c, int TT, int TX) {
     return A;
 }
 
-static bool eo_fits(const Ctx &c, EoTileCfg t) { return c.p.Nt % t.TT == 0 && c.p.Nx % t.TX == 0; }
+template <typename Tile>
+static bool eo_fits(const Ctx &c, Tile t) { return c.p.Nt % t.TT == 0 && c.p.Nx % t.TX == 0; }
 
 // the two partial slots of prologue-finalized launches (launch idx writes slot idx & 1
 // and reads the other), sized for the smallest tile (64 sites: at most V / 64 blocks)
@@ -892,107 +738,25 @@ static bool eo_shape_ok(const Ctx &c) {
 
 bool eo_available(const Ctx &c) { return eo_shape_ok(c) && c.tileEo64 >= 0; }
 
-// buffers of one fused launch (PF: the pipelined iteration's Ap pair, directions and x_s)
-template <typename R>
-struct EoPtrs {
-    using V2 = typename Vec2<R>::T;
-    const V2 *r = nullptr;
-    const V2 *Ap_in = nullptr;
-    const V2 *pold = nullptr;
-    V2 *pnew = nullptr, *Ap = nullptr, *xs = nullptr;
-    double2 *part = nullptr;            // this launch's block partials
-    const double2 *prevPart = nullptr;  // finMode 1, 2: the previous launch's
-    int idx = 0;                        // launch index in the chunk
-};
-
-// resident blocks of a kernel on the whole device (persistent launches)
-static int resident_blocks(const void *kernel, int threads) {
-    int dev = 0, cus = 0, per = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) !=
-                                                 hipSuccess)
-        return 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, threads, 0) != hipSuccess) return 0;
-    return per * cus;
-}
-
-// returns the number of blocks per system (= partial slots per system)
-// the pipelined FP32 iteration's launch (persistent or one block per tile), WR1 as in
-// k_eo_normal_fused; returns the blocks per system
-// XM, RM as in k_eo_normal_fused: (0, 1) for launch 0 of a chunk, then (2, 2) and (0, 2)
-// alternating.  Persistent grids are sized by the form with the fewest resident blocks,
-// so that consecutive launches leave the same number of partials.
-template <int TT, int TX, bool WR1>
-static int launch_eo_pf_tt(const Ctx &c, int nsys, const EoArgs &A, const float *phi, bool persist,
-                           const EoPtrs<float> &b, int finMode) {
-    const dim3 block(eo_threads(TT, TX));
-    const int form = b.idx == 0 ? 0 : (b.idx & 1) ? 1 : 2;
-    auto pick = [&](auto persistTag) {
-        constexpr bool P = decltype(persistTag)::value;
-        using K = decltype(&k_eo_normal_fused<float, TT, TX, true, P, false, WR1, 0, 1>);
-        const K ks[3] = {&k_eo_normal_fused<float, TT, TX, true, P, false, WR1, 0, 1>,
-                         &k_eo_normal_fused<float, TT, TX, true, P, false, WR1, 2, 2>,
-                         &k_eo_normal_fused<float, TT, TX, true, P, false, WR1, 0, 2>};
-        return std::make_pair(ks[form], ks);
-    };
-    if (persist) {
-        const auto kk = pick(std::true_type());
-        static const int resident = [&] {
-            int m = 1 << 30;
-            for (int i = 0; i < 3; ++i)
-                m = std::min(m, resident_blocks(reinterpret_cast<const void *>(kk.second[i]), block.x));
-            return m;
-        }();
-        int g = std::min(A.tilesPerSys, std::max(resident, 8));
-        if (A.xcdRemap && g >= 8) g -= g % 8;   // keeps every block's tiles on one XCD's band
-        hipLaunchKernelGGL(kk.first, dim3(g, nsys), block, 0, c.stream, A, phi, c.cg_d, b.r, b.Ap_in, b.pold,
-                           b.pnew, b.Ap, b.xs, b.part, finMode, b.idx, b.prevPart, c.active, (float2 *)nullptr,
-                           (double2 *)nullptr);
-        return g;
-    }
-    hipLaunchKernelGGL(pick(std::false_type()).first, dim3(A.tilesPerSys, nsys), block, 0, c.stream, A, phi, c.cg_d,
-                       b.r, b.Ap_in, b.pold, b.pnew, b.Ap, b.xs, b.part, finMode, b.idx, b.prevPart, c.active,
-                       (float2 *)nullptr, (double2 *)nullptr);
-    return A.tilesPerSys;
-}
-
-template <typename R, int TT, int TX>
-static int launch_eo_tt(const Ctx &c, int nsys, const EoArgs &A, const R *phi, bool pf, bool persist,
-                        const EoPtrs<R> &b, int finMode = 0) {
-    const dim3 block(eo_threads(TT, TX));
-    if constexpr (std::is_same<R, float>::value) {
-        if (pf) {
-            return A.r == 1.0 ? launch_eo_pf_tt<TT, TX, true>(c, nsys, A, phi, persist, b, finMode)
-                              : launch_eo_pf_tt<TT, TX, false>(c, nsys, A, phi, persist, b, finMode);
-        }
-    }
-    if (A.r == 1.0)
-        hipLaunchKernelGGL((k_eo_normal_fused<R, TT, TX, false, false, false, true>), dim3(A.tilesPerSys, nsys), block,
-                           0, c.stream, A, phi, c.cg_d, b.r, b.Ap_in, b.pold, b.pnew, b.Ap, b.xs, c.partials, 0,
-                           0, (const double2 *)nullptr, (int *)nullptr, (float2 *)nullptr, (double2 *)nullptr);
-    else
-        hipLaunchKernelGGL((k_eo_normal_fused<R, TT, TX, false>), dim3(A.tilesPerSys, nsys), block, 0, c.stream, A,
-                           phi, c.cg_d, b.r, b.Ap_in, b.pold, b.pnew, b.Ap, b.xs, c.partials, 0, 0,
-                           (const double2 *)nullptr, (int *)nullptr, (float2 *)nullptr, (double2 *)nullptr);
-    return A.tilesPerSys;
-}
-
 // launch the fused Schur normal operator (FP64) with tile `ti`; returns the partial count
+template <int TT, int TX>
+static void launch_eo_tt(const Ctx &c, int nsys, const EoArgs &A, const double *phi, const double2 *r,
+                         const double2 *pold, double2 *pnew, double2 *Ap) {
+    auto *k = A.r == 1.0 ? &k_eo_normal_fused<TT, TX, false, true> : &k_eo_normal_fused<TT, TX, false, false>;
+    hipLaunchKernelGGL(k, dim3(A.tilesPerSys, nsys), dim3(eo_threads(TT, TX)), 0, c.stream, A, phi, c.cg_d, r,
+                       (const double2 *)nullptr, pold, pnew, Ap, c.partials, (float2 *)nullptr, (double2 *)nullptr);
+}
 static int launch_eo_fused(Ctx &c, int ti, int nsys, const double *phi, const double2 *r, const double2 *pold,
                            double2 *pnew, double2 *Ap) {
     const EoTileCfg t = kEoTiles64[ti];
     const EoArgs A = eo_args(c, t.TT, t.TX);
-    EoPtrs<double> b;
-    b.r = r;
-    b.pold = pold;
-    b.pnew = pnew;
-    b.Ap = Ap;
     prof_before(c, PK_NORMAL_OP, (double)nsys * c.V * (4 * 16 + 8));
     switch (ti) {
-    case 0: (void)launch_eo_tt<double, 8, 32>(c, nsys, A, phi, false, false, b); break;
-    case 1: (void)launch_eo_tt<double, 16, 16>(c, nsys, A, phi, false, false, b); break;
-    case 2: (void)launch_eo_tt<double, 4, 64>(c, nsys, A, phi, false, false, b); break;
-    case 3: (void)launch_eo_tt<double, 4, 32>(c, nsys, A, phi, false, false, b); break;
-    default: (void)launch_eo_tt<double, 2, 32>(c, nsys, A, phi, false, false, b); break;
+    case 0: launch_eo_tt<8, 32>(c, nsys, A, phi, r, pold, pnew, Ap); break;
+    case 1: launch_eo_tt<16, 16>(c, nsys, A, phi, r, pold, pnew, Ap); break;
+    case 2: launch_eo_tt<4, 64>(c, nsys, A, phi, r, pold, pnew, Ap); break;
+    case 3: launch_eo_tt<4, 32>(c, nsys, A, phi, r, pold, pnew, Ap); break;
+    default: launch_eo_tt<2, 32>(c, nsys, A, phi, r, pold, pnew, Ap); break;
     }
     prof_after(c, PK_NORMAL_OP);
     return A.tilesPerSys;
@@ -1004,11 +768,9 @@ static int launch_eo_fused(Ctx &c, int ti, int nsys, const double *phi, const do
 template <int TT, int TX>
 static int launch_eo_ru_tt(Ctx &c, int nsys, const EoArgs &A, const double *phi, const double2 *x, const double2 *b,
                            double2 *r, float2 *r32, double2 *partRes, double2 *partN) {
-    auto *k = A.r == 1.0 ? &k_eo_normal_fused<double, TT, TX, false, false, true, true>
-                         : &k_eo_normal_fused<double, TT, TX, false, false, true, false>;
+    auto *k = A.r == 1.0 ? &k_eo_normal_fused<TT, TX, true, true> : &k_eo_normal_fused<TT, TX, true, false>;
     hipLaunchKernelGGL(k, dim3(A.tilesPerSys, nsys), dim3(eo_threads(TT, TX)), 0, c.stream, A, phi, c.cg_d, x, b,
-                       (const double2 *)nullptr, (double2 *)nullptr, r, (double2 *)nullptr, partRes, 0, 0,
-                       (const double2 *)nullptr, (int *)nullptr, r32, partN);
+                       (const double2 *)nullptr, (double2 *)nullptr, r, partRes, r32, partN);
     return A.tilesPerSys;
 }
 static int launch_eo_ru(Ctx &c, int nsys, const double *phi, const double2 *x, const double2 *b, double2 *r,
@@ -1024,20 +786,31 @@ static int launch_eo_ru(Ctx &c, int nsys, const double *phi, const double2 *x, c
     }
 }
 
-// the pipelined FP32 iteration's fused kernel (finMode as in k_eo_normal_fused) with
-// tile `ti` as launch idx of a chunk (idx & 1: the Ap and partial-slot parity, the
-// directions in rotation); returns the block partials per system
+// scratch of a solve: b_e and U_o in c.t (first and second half), the residual in c.Ap
+struct EoBufs {
+    double2 *b, *U, *res;
+};
+static EoBufs eo_bufs(Ctx &c, int nsys) {
+    const size_t h = (size_t)nsys * 2 * (c.V / 2);
+    return {c.t, c.t + h, c.Ap};
+}
+
+// the pipelined FP32 iteration (k_eo_pf) with tile `ti` as launch idx of a chunk (idx & 1: the Ap
+// and partial-slot parity, the directions in rotation); returns the block partials per system
 static int launch_eo_pf(Ctx &c, int ti, int nsys, int idx, int finMode) {
     const EoTileCfg t = kEoTiles32[ti];
-    const EoArgs A = eo_args(c, t.TT, t.TX);
     const int par = idx & 1;
-    EoPtrs<float> b;
+    EoPfLaunch<float> b;
+    b.phi = c.phis;
     b.idx = idx;
+    b.form = idx == 0 ? 0 : par ? 1 : 2;
+    b.finMode = finMode;
+    b.persist = t.persist;
     b.part = finMode ? c.pfSlot[par] : c.partials;
     b.prevPart = c.pfSlot[par ^ 1];
     b.Ap_in = par ? c.pfA1 : c.Aps;
     b.Ap = par ? c.Aps : c.pfA1;
-    b.xs = c.xs;
+    b.x = c.xs;
     // direction p_k in pf_dir(c, k); launch 0 reads r, the others p_{idx-2}
     b.r = idx == 0 ? c.rs : pf_dir(c, idx - 2);
     b.pold = pf_dir(c, idx - 1);
@@ -1046,20 +819,39 @@ static int launch_eo_pf(Ctx &c, int ti, int nsys, int idx, int finMode) {
     // written in odd launches; and read phi.  The figure counts the vectors as the complex
     // spinors of the interface (16 B per site of the full lattice), as ycn_profile_end
     // documents; packed they are half that.
-    const int vecs = (idx & 1) ? 7 : 5;
-    prof_before(c, PK_NORMAL_OP, (double)nsys * c.V * (vecs * 16 + 4));
-    const bool ps = t.persist;
-    int nb = 0;
-    switch (t.TT * 1000 + t.TX) {
-    case 8032: nb = launch_eo_tt<float, 8, 32>(c, nsys, A, c.phis, true, ps, b, finMode); break;
-    case 16032: nb = launch_eo_tt<float, 16, 32>(c, nsys, A, c.phis, true, ps, b, finMode); break;
-    case 8064: nb = launch_eo_tt<float, 8, 64>(c, nsys, A, c.phis, true, ps, b, finMode); break;
-    case 16016: nb = launch_eo_tt<float, 16, 16>(c, nsys, A, c.phis, true, ps, b, finMode); break;
-    case 4064: nb = launch_eo_tt<float, 4, 64>(c, nsys, A, c.phis, true, ps, b, finMode); break;
-    case 2032: nb = launch_eo_tt<float, 2, 32>(c, nsys, A, c.phis, true, ps, b, finMode); break;
-    case 32032: nb = launch_eo_tt<float, 32, 32>(c, nsys, A, c.phis, true, ps, b, finMode); break;
-    default: nb = launch_eo_tt<float, 16, 64>(c, nsys, A, c.phis, true, ps, b, finMode); break;
-    }
+    prof_before(c, PK_NORMAL_OP, (double)nsys * c.V * ((par ? 7 : 5) * 16 + 4));
+    const int nb = launch_eo_pf32(c, t.TT, t.TX, nsys, b);
+    prof_after(c, PK_NORMAL_OP);
+    return nb;
+}
+
+// FP64 direction p_k of a phase: p[0] (p_{-1}), p[1], and r, which nothing reads after launch 0
+static double2 *eo_p64_dir(const Ctx &c, int k) {
+    double2 *const rot[3] = {c.pv[0], c.pv[1], c.r};
+    return rot[(k + 1) % 3];
+}
+// launch idx of a chunk of the pipelined FP64 iteration (first: of the phase's first chunk), A p
+// alternating between U_o's scratch and Ap
+static int launch_eo_p64(Ctx &c, int ti, int nsys, const double *phi, int idx, bool first, int finMode) {
+    const EoTile t = kEoTilesP64[ti];
+    const int par = idx & 1;
+    double2 *const U = eo_bufs(c, nsys).U;
+    EoPfLaunch<double> b;
+    b.phi = phi;
+    b.idx = idx;
+    b.form = first && idx == 0 ? 0 : par ? 1 : 2;
+    b.finMode = finMode;
+    b.persist = false;
+    b.part = c.pfSlot[par];
+    b.prevPart = c.pfSlot[par ^ 1];
+    b.Ap_in = par ? U : c.Ap;
+    b.Ap = par ? c.Ap : U;
+    b.x = c.x;
+    b.r = first && idx == 0 ? c.r : eo_p64_dir(c, idx + 1);   // p_{idx-2}
+    b.pold = eo_p64_dir(c, idx + 2);
+    b.pnew = eo_p64_dir(c, idx);
+    prof_before(c, PK_NORMAL_OP, (double)nsys * c.V * ((par ? 7 : 5) * 16 + 8));
+    const int nb = launch_eo_pf64(c, t.TT, t.TX, nsys, b);
     prof_after(c, PK_NORMAL_OP);
     return nb;
 }
@@ -1069,7 +861,7 @@ static dim3 half_grid(const Ctx &c, int nsys) { return dim3((c.V / 2 + kNT - 1) 
 // Times every even-odd tile that fits (FP64, and FP32 when the mixed buffers exist) on
 // the context's buffers and keeps the fastest.  The trial launches only touch CG scratch.
 int eo_autotune(Ctx &c) {
-    c.tileEo64 = c.tileEo32 = -1;
+    c.tileEo64 = c.tileEo32 = c.tileEoP64 = -1;
     if (!eo_shape_ok(c)) return YCN_OK;
     hipEvent_t e0, e1;
     YCN_HIP(hipEventCreate(&e0));
@@ -1160,6 +952,37 @@ int eo_autotune(Ctx &c) {
         }
         c.tuneReport += " (even-odd fp32 tile forced by YCN_TILE_EO32)";
     }
+    // FP64 contexts: the pipelined FP64 iteration's tiles, with either finalize
+    if (c.p.cgPrecision != YCN_CG_MIXED && c.tileEo64 >= 0 && c.pfSlot[1] && !onchip_eo(c) &&
+        !std::getenv("YCN_TILE_EO")) {
+        const bool memoP = tune_lookup(4, c, us) && us.size() == 2 * (size_t)kNumEoP64;
+        if (!memoP) {
+            us.assign(2 * kNumEoP64, 1e30);
+            for (int i = 0; i < kNumEoP64; ++i)
+                for (int m = 0; m < 2 && eo_fits(c, kEoTilesP64[i]); ++m)
+                    us[2 * i + m] = time_it([&](int k) {
+                        const int nb = launch_eo_p64(c, i, c.nSys, c.phi[c.cur], k, true, m ? 2 : 0);
+                        if (!m) launch_fin_p64(c, c.nSys, nb, 1, c.pfSlot[k & 1], 0);
+                    });
+            tune_store(4, c, us);
+        }
+        const char *force = std::getenv("YCN_TILE_PL");
+        const int f = force ? std::atoi(force) : -1;
+        best = 1e30;
+        c.tuneReport += " | even-odd fp64 pipelined tiles (us/iteration, separate | prologue finalize):";
+        for (int i = 0; i < kNumEoP64; ++i) {
+            if (!eo_fits(c, kEoTilesP64[i])) continue;
+            std::snprintf(line, sizeof line, " %dx%d %.1f|%.1f;", kEoTilesP64[i].TT, kEoTilesP64[i].TX, us[2 * i],
+                          us[2 * i + 1]);
+            c.tuneReport += line;
+            for (int m = 0; m < 2; ++m)
+                if ((f < 0 || f == i) && us[2 * i + m] < best && (m ? allowFused : allowSep)) {
+                    best = us[2 * i + m];
+                    c.tileEoP64 = i;
+                    c.eoFinFused = m == 1;
+                }
+        }
+    }
     if (c.tileEo32 >= 0) {
         const EoTileCfg t = kEoTiles32[c.tileEo32];
         std::snprintf(line, sizeof line, " | fp32 pipelined iteration: %dx%d%s, %s finalize", t.TT, t.TX,
@@ -1174,20 +997,22 @@ int eo_autotune(Ctx &c) {
     return YCN_OK;
 }
 
-// scratch of a solve: b_e and U_o in c.t (first and second half), the residual in c.Ap
-struct EoBufs {
-    double2 *b, *U, *res;
-};
-static EoBufs eo_bufs(Ctx &c, int nsys) {
-    const size_t h = (size_t)nsys * 2 * (c.V / 2);
-    return {c.t, c.t + h, c.Ap};
-}
-
 static void launch_eo_iteration(Ctx &c, int nsys, const double *phi, int parity) {
     const int nb = launch_eo_fused(c, c.tileEo64, nsys, phi, c.r, c.pv[parity], c.pv[parity ^ 1], c.Ap);
     launch_fin_alpha(c, nsys, nb);
     const int nbu = launch_cg_update(c, nsys, c.V / 2, c.pv[parity ^ 1]);
     launch_fin_beta(c, nsys, nbu, false, true);
+}
+
+// One captured chunk of pipelined FP64 iterations (first: of a phase, from the residual in r and the
+// direction in p[0]).  A phase is what runs until every system has stopped; the close ends it.
+static int eo_p64_iterations(Ctx &c, const double *phi, int nsys, bool first) {
+    const bool fused = c.eoFinFused;
+    return run_chunk(c, phi, nsys, YCN_DAGGER, kP64Launches, first ? 6 : 7, kPacked, c.tileEoP64, [&](int i) {
+        const int nb = launch_eo_p64(c, c.tileEoP64, nsys, phi, i, first, fused ? 1 : 0);
+        if (!fused || i == kP64Launches - 1)
+            launch_fin_p64(c, nsys, nb, fused ? kP64Launches : 1, c.pfSlot[i & 1], 1);
+    });
 }
 
 // launch i of a chunk of the pipelined FP32 iteration: one launch that finalizes its
@@ -1339,19 +1164,27 @@ int eo_solve(Ctx &c, const double *phi, int nsys, bool gen, uint32_t streamBase,
     int launched = 0, active = nsys;
     int chunk = std::max(kGraphIters, std::min(c.lastIters, maxIter));
     const int hardCap = maxIter * (maxRestarts + 1) + 2 * kGraphIters;
+    const bool pipelined = c.tileEoP64 >= 0 && c.profTarget != PK_CG_UPDATE;
     for (int guard = 0; guard < maxRestarts + 2; ++guard) {
+        bool first = true;
         while (active > 0 && launched < hardCap) {
             const int n = std::min(chunk, hardCap - launched);
-            for (int k = 0; k < n; k += kGraphIters) {
-                rc = run_chunk(c, phi, nsys, YCN_DAGGER, kGraphIters, 3, kPacked, c.tileEo64,
-                               [&](int i) { launch_eo_iteration(c, nsys, phi, i & 1); });
+            for (int k = 0, m = pipelined ? kP64Launches : kGraphIters; k < n; k += m, launched += m) {
+                if (pipelined)
+                    rc = eo_p64_iterations(c, phi, nsys, first);
+                else
+                    rc = run_chunk(c, phi, nsys, YCN_DAGGER, kGraphIters, 3, kPacked, c.tileEo64,
+                                   [&](int i) { launch_eo_iteration(c, nsys, phi, i & 1); });
                 if (rc) return rc;
+                first = false;
             }
-            launched += ((n + kGraphIters - 1) / kGraphIters) * kGraphIters;
             rc = poll_active(c, active);
             if (rc) return rc;
             chunk = std::max(kGraphIters, std::min(64, chunk / 2));
         }
+        if (pipelined)
+            hipLaunchKernelGGL(k_p64_close<true>, gH, dim3(kNT), 0, c.stream, c.V / 2, (const CgState *)c.cg_d, c.x,
+                               c.pv[0], (const double2 *)c.pv[1], c.r, (const double2 *)B.U, (const double2 *)c.Ap);
         // true residual of the unpreconditioned system, |b_e - S x_e| / |eta|
         hipLaunchKernelGGL(k_eo_hop_oe<true>, gH, dim3(kNT), 0, c.stream, A, phi, (const double2 *)c.x, B.U);
         hipLaunchKernelGGL((k_eo_hop_eo<true, 1>), gH, dim3(kNT), 0, c.stream, A, phi, (const double2 *)c.x,

@@ -6,6 +6,7 @@
 #include <type_traits>
 #include <vector>
 
+#include "cg_fused.hpp"
 #include "cg_host.hpp"
 #include "ycn_device.hpp"
 #include "ycn_internal.hpp"
@@ -22,6 +23,64 @@ __device__ __forceinline__ T &at(T *base, unsigned idx) {
     return *reinterpret_cast<T *>(reinterpret_cast<C *>(base) + (unsigned)(idx * (unsigned)sizeof(T)));
 }
 
+// a site's packed spinor: spins 0 and 1, each (flavour 0, flavour 1)
+template <typename R>
+struct Sp {
+    typename Vec2<R>::T a, b;
+};
+// n of them in LDS, read and written without bank conflicts: whole 16-byte entries in FP32, a
+// plane per spin in FP64
+template <typename R, int N>
+struct SpLds;
+template <int N>
+struct SpLds<float, N> {
+    float4 e[N];
+    __device__ __forceinline__ Sp<float> get(int i) const {
+        const float4 v = e[i];
+        return {make_float2(v.x, v.y), make_float2(v.z, v.w)};
+    }
+    __device__ __forceinline__ float2 s0(int i) const { return reinterpret_cast<const float2 *>(e)[2 * i]; }
+    __device__ __forceinline__ float2 s1(int i) const { return reinterpret_cast<const float2 *>(e)[2 * i + 1]; }
+    __device__ __forceinline__ void set(int i, Sp<float> v) { e[i] = make_float4(v.a.x, v.a.y, v.b.x, v.b.y); }
+};
+template <int N>
+struct SpLds<double, N> {
+    double2 e[2][N];
+    __device__ __forceinline__ Sp<double> get(int i) const { return {e[0][i], e[1][i]}; }
+    __device__ __forceinline__ double2 s0(int i) const { return e[0][i]; }
+    __device__ __forceinline__ double2 s1(int i) const { return e[1][i]; }
+    __device__ __forceinline__ void set(int i, Sp<double> v) {
+        e[0][i] = v.a;
+        e[1][i] = v.b;
+    }
+};
+
+template <typename R>
+__device__ __forceinline__ double sq(Sp<R> v) {
+    return (double)((v.a.x * v.a.x + v.a.y * v.a.y) + (v.b.x * v.b.x + v.b.y * v.b.y));
+}
+template <typename R>
+__device__ __forceinline__ Sp<R> axpy(Sp<R> u, R s, Sp<R> v) {
+    return {mk2<R>(u.a.x + s * v.a.x, u.a.y + s * v.a.y), mk2<R>(u.b.x + s * v.b.x, u.b.y + s * v.b.y)};
+}
+// a spinor of two planes of V entries
+template <typename R, typename P>
+__device__ __forceinline__ Sp<R> load_sp(P *v, unsigned V, unsigned i) {
+    return {at(v, i), at(v, V + i)};
+}
+template <typename R, typename P>
+__device__ __forceinline__ void store_sp(P *v, unsigned V, unsigned i, Sp<R> s) {
+    at(v, i) = s.a;
+    at(v, V + i) = s.b;
+}
+
+// a mod n in [0, n) without an integer division (the 4-site halo of a tile spans several
+// periods when an extent is smaller than 4, Nt = 2).  For |a| < 2^22 and inv = fl(1 / n),
+// (a + 1/2) / n lies at least 1 / (2n) from an integer and the two single-precision
+// roundings move it by less than |a + 1/2| / n * 2^-23, so the floor is exact.
+__device__ __forceinline__ int wrapf(int a, int n, float inv) {
+    return a - n * (int)floorf(((float)a + 0.5f) * inv);
+}
 __device__ __forceinline__ double2 pf_fin_sum(const double2 *part, int nb, double2 *lds) {
     double2 acc = make_double2(0.0, 0.0);
     int i = threadIdx.x;
@@ -159,7 +218,8 @@ __device__ __forceinline__ bool pf_prologue(CgState *st, int sys, int idx, int f
 // recurrence (its r update included): alpha, and |r|^2 after it from the recurrence.  That
 // prediction is off by a few eps rho, so it is not taken below 1e-13 rho; and where rho itself,
 // summed exactly, has reached the stop, the step is not taken.  Stop as the unpipelined
-// iteration does (k_fin_beta): at the stop, at the cap, or on a NaN.
+// iteration does (k_fin_beta): at the stop (after an even number of iterations where S.even), at
+// the cap, or on a NaN.
 struct P64Step {
     double alpha, beta, rr;
     int iter;
@@ -167,14 +227,14 @@ struct P64Step {
 };
 __device__ __forceinline__ P64Step p64_decide(double mu, double nu, double rho, int iter, const CgState &S) {
     P64Step d;
-    if (sqrt(rho) <= S.stop) return {0.0, 0.0, rho, iter - 1, true, true};
+    if (sqrt(rho) <= S.stop && !(S.even && !(iter & 1) && rho > 0.0)) return {0.0, 0.0, rho, iter - 1, true, true};
     d.iter = iter;
     d.alpha = rho / mu;
     d.rr = d.alpha * d.alpha * nu - rho;
     if (d.rr <= 1e-13 * rho) d.rr = 1e-13 * rho;
     d.beta = d.rr / rho;
     d.conv = sqrt(d.rr) <= S.stop;
-    d.stop = !(sqrt(d.rr) > S.stop) || iter >= S.maxIter;
+    d.stop = (!(sqrt(d.rr) > S.stop) && !(S.even && (iter & 1))) || iter >= S.maxIter;
     return d;
 }
 // a system stops after the launch that iteration `it` names, its last x updates left to the close
@@ -205,6 +265,7 @@ __device__ __forceinline__ bool p64_prologue(CgState *st, int sys, int idx, int 
         *pause = finMode == 1 && d.stop;
         if (finMode == 1 && d.stop && blockIdx.x == 0) {
             S.alpha = make_double2(d.alpha, 0.0);
+            S.beta = d.beta;
             S.iter = d.iter;
             S.rr_prev = rh.x;
             S.rr = d.rr;
@@ -215,6 +276,40 @@ __device__ __forceinline__ bool p64_prologue(CgState *st, int sys, int idx, int 
     alpha = bc[0];
     beta = bc[1];
     return !*pause;
+}
+
+// Finalize after the launches of a chunk that finalized each other (n of them), or after one
+// launch (n = 1); commit = 0 only reduces (timing).
+template <int NT>
+__global__ void __launch_bounds__(NT)
+k_fin_p64(const double2 *__restrict__ part, int nb, int n, CgState *__restrict__ st, int *__restrict__ active,
+          int commit) {
+    __shared__ double2 lds0[NT / kWave], lds1[NT / kWave];
+    CgState &S = st[blockIdx.x];
+    const int skip = S.done;
+    double2 mn, rh;
+    sum_pf_partials<NT>(part + 2 * (size_t)blockIdx.x * nb, nb, lds0, lds1, mn, rh);
+    if (skip || threadIdx.x) return;
+    if (!commit) {
+        S.rz = mn.x + mn.y + rh.x;   // a field the plain iteration never reads
+        return;
+    }
+    const P64Step d = p64_decide(mn.x, mn.y, rh.x, S.iter0 + n, S);
+    S.alpha = make_double2(d.alpha, 0.0);
+    S.beta = d.beta;
+    S.iter = d.iter;
+    S.rr_prev = rh.x;
+    S.rr = d.rr;
+    S.iter0 += n;
+    if (d.stop) p64_stop(S, S.iter0, d, active);
+}
+
+inline void launch_fin_p64(Ctx &c, int nsys, int nb, int n, const double2 *part, int commit) {
+    if (nb > 4 * kPfNT)
+        hipLaunchKernelGGL(k_fin_p64<1024>, dim3(nsys), dim3(1024), 0, c.stream, part, nb, n, c.cg_d, c.active, commit);
+    else
+        hipLaunchKernelGGL(k_fin_p64<kPfNT>, dim3(nsys), dim3(kPfNT), 0, c.stream, part, nb, n, c.cg_d, c.active,
+                           commit);
 }
 
 // the separate finalize of one iteration (one block per system, after a finMode 0
@@ -364,6 +459,54 @@ k_fin_pf_true(const double2 *__restrict__ partRes, const double2 *__restrict__ p
         atomicAdd(active, 1);
     }
 }
+
+constexpr int kP64Launches = 12;   // per captured FP64 chunk: keeps the rotations of both buffer sets
+
+// The x updates that the launches of an FP64 phase have left to later ones, added to x of the
+// systems that stopped after m = pfLaunch launches: alpha_{m-1} p_{m-1}, and after an odd number
+// of launches alpha_{m-2} p_{m-2} before it.  d0, d1, d2: the directions' rotation, p_{-1} in d0
+// and the phase's first r in d2.  KEEP: the next phase goes on from here, so r (into d2) and the
+// direction (into d0) are brought up too, from the A p of even (a0) and odd (a1) launches.
+template <bool KEEP>
+__global__ void __launch_bounds__(kPfNT)
+k_p64_close(int n, const CgState *__restrict__ st, double2 *__restrict__ x, double2 *__restrict__ d0,
+            const double2 *__restrict__ d1, double2 *__restrict__ d2, const double2 *__restrict__ a0,
+            const double2 *__restrict__ a1) {
+    const int sys = blockIdx.y, m = st[sys].pfLaunch, i = blockIdx.x * kPfNT + threadIdx.x;
+    if (m == 0 || i >= n) return;
+    const double al = st[sys].alpha.x;
+    const double2 ab = st[sys].ab[(m - 1) & 1];   // of launch m - 1: alpha_{m-2}, beta_{m-1}
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+        const size_t k = ((size_t)sys * 2 + s) * n + i;
+        const double2 v0 = d0[k], v1 = d1[k], v2 = d2[k];
+        const double2 p = m % 3 == 0 ? v0 : m % 3 == 1 ? v1 : v2, pp = m % 3 == 0 ? v2 : m % 3 == 1 ? v0 : v1;
+        double2 v = x[k];
+        if ((m & 1) && m > 1) v = make_double2(v.x + ab.x * pp.x, v.y + ab.x * pp.y);
+        x[k] = make_double2(v.x + al * p.x, v.y + al * p.y);
+        if (KEEP) {
+            const double2 q = (m & 1) ? a0[k] : a1[k];
+            const double2 rk = m == 1 ? v2 : make_double2(p.x - ab.y * pp.x, p.y - ab.y * pp.y);
+            d2[k] = make_double2(rk.x - al * q.x, rk.y - al * q.y);
+            d0[k] = p;
+        }
+    }
+}
+
+// a launch of the even-odd pipelined iteration (k_eo_pf)
+template <typename R>
+struct EoPfLaunch {
+    using V2 = typename Vec2<R>::T;
+    const R *phi;
+    const V2 *r, *Ap_in, *pold;
+    V2 *pnew, *Ap, *x;
+    double2 *part;
+    const double2 *prevPart;
+    int idx, form, finMode;
+    bool persist;
+};
+int launch_eo_pf32(const Ctx &c, int TT, int TX, int nsys, const EoPfLaunch<float> &b);
+int launch_eo_pf64(const Ctx &c, int TT, int TX, int nsys, const EoPfLaunch<double> &b);
 
 // direction p_k (k >= -1) of a chunk of pipelined launches: the three buffers in rotation,
 // p_{-1} (the direction kept across the reliable update) in ps[0]

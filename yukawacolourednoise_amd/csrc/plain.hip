@@ -1,7 +1,7 @@
 // plain.hip -- the pipelined iterations of the plain solvers on D^dag D or D D^dag (packed real
 // spinors), FP32 for mixed precision and FP64: one launch per CG iteration.
 //
-// The iteration is the even-odd one's (k_eo_normal_fused in evenodd.hip): CG with the residual
+// The iteration is the even-odd one's (k_eo_pf in eo_pipelined.hip): CG with the residual
 // norm recurrence of D'Azevedo, Eijkhout and Romine (LAPACK Working Note 56, 1993), so that one
 // reduction per iteration suffices and the x and r updates move into the next application of
 // the operator; r rebuilt from the directions after launch 0 of a chunk, x (x_s) updated by every
@@ -29,57 +29,6 @@ struct PlArgs {
     int tilesX, tilesPerSys, xcdRemap;
 };
 
-// a site's packed spinor: spins 0 and 1, each (flavour 0, flavour 1)
-template <typename R>
-struct Sp {
-    typename Vec2<R>::T a, b;
-};
-// n of them in LDS, read and written without bank conflicts: whole 16-byte entries in FP32, a
-// plane per spin in FP64
-template <typename R, int N>
-struct SpLds;
-template <int N>
-struct SpLds<float, N> {
-    float4 e[N];
-    __device__ __forceinline__ Sp<float> get(int i) const {
-        const float4 v = e[i];
-        return {make_float2(v.x, v.y), make_float2(v.z, v.w)};
-    }
-    __device__ __forceinline__ float2 s0(int i) const { return reinterpret_cast<const float2 *>(e)[2 * i]; }
-    __device__ __forceinline__ float2 s1(int i) const { return reinterpret_cast<const float2 *>(e)[2 * i + 1]; }
-    __device__ __forceinline__ void set(int i, Sp<float> v) { e[i] = make_float4(v.a.x, v.a.y, v.b.x, v.b.y); }
-};
-template <int N>
-struct SpLds<double, N> {
-    double2 e[2][N];
-    __device__ __forceinline__ Sp<double> get(int i) const { return {e[0][i], e[1][i]}; }
-    __device__ __forceinline__ double2 s0(int i) const { return e[0][i]; }
-    __device__ __forceinline__ double2 s1(int i) const { return e[1][i]; }
-    __device__ __forceinline__ void set(int i, Sp<double> v) {
-        e[0][i] = v.a;
-        e[1][i] = v.b;
-    }
-};
-
-template <typename R>
-__device__ __forceinline__ double sq(Sp<R> v) {
-    return (double)((v.a.x * v.a.x + v.a.y * v.a.y) + (v.b.x * v.b.x + v.b.y * v.b.y));
-}
-template <typename R>
-__device__ __forceinline__ Sp<R> axpy(Sp<R> u, R s, Sp<R> v) {
-    return {mk2<R>(u.a.x + s * v.a.x, u.a.y + s * v.a.y), mk2<R>(u.b.x + s * v.b.x, u.b.y + s * v.b.y)};
-}
-// a spinor of two planes of V entries
-template <typename R, typename P>
-__device__ __forceinline__ Sp<R> load_sp(P *v, unsigned V, unsigned i) {
-    return {at(v, i), at(v, V + i)};
-}
-template <typename R, typename P>
-__device__ __forceinline__ void store_sp(P *v, unsigned V, unsigned i, Sp<R> s) {
-    at(v, i) = s.a;
-    at(v, V + i) = s.b;
-}
-
 // v times d minus the hop of D (DAG = false) or D^dag at array entry i of N (rows of W)
 template <typename R, bool DAG, bool WR1, typename Lds>
 __device__ __forceinline__ Sp<R> pl_dirac(R r, const Lds &N, int i, int W, R sf, R sb, R d, Sp<R> v) {
@@ -106,7 +55,7 @@ __device__ __forceinline__ Sp<R> pl_dirac(R r, const Lds &N, int i, int W, R sf,
     return {mk2<R>(d * v.a.x - o.a.x, d * v.a.y - o.a.y), mk2<R>(d * v.b.x - o.b.x, d * v.b.y - o.b.y)};
 }
 
-// One launch of the iteration.  XM, RM, idx and finMode as in k_eo_normal_fused; FIRST forms
+// One launch of the iteration.  XM, RM, idx and finMode as in k_eo_pf; FIRST forms
 // (XM 0, RM 1) read r and skip its update, alpha being 0.  A block owns a TT x TX tile (cut
 // off at the lattice's edges); a thread keeps the same M0 entries of the tile with its 2-site
 // halo through all stages, so that an entry's own values stay in registers.  FP64 keeps one
@@ -174,7 +123,7 @@ k_pl_pf(PlArgs A, const R *__restrict__ phi, CgState *st, const typename Vec2<R>
         if (!pf_prologue<NT>(st, sys, idx, finMode, prevPart, part, active, red, red2, bc, &pause, alphaD, betaD))
             return;
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) st[sys].ab[idx & 1] = make_double2(alphaD, betaD);
+    if (blockIdx.x == 0 && threadIdx.x == 0) st[sys].ab[idx & 1] = make_double2(RM == 1 ? 0.0 : alphaD, betaD);
     const R alpha = (R)alphaD, beta = (R)betaD, alphaPrev = (R)prev.x, betaPrev = (R)prev.y;
     const R wr = (R)A.r;
 
@@ -237,55 +186,6 @@ k_pl_pf(PlArgs A, const R *__restrict__ phi, CgState *st, const typename Vec2<R>
 }
 
 // ---------------------------------------------------------------------------
-// FP64: end of a phase of launches
-// ---------------------------------------------------------------------------
-// Finalize after the launches of a chunk that finalized each other (n of them), or after one
-// launch (n = 1); commit = 0 only reduces (timing).
-template <int NT>
-__global__ void __launch_bounds__(NT)
-k_fin_p64(const double2 *__restrict__ part, int nb, int n, CgState *__restrict__ st, int *__restrict__ active,
-          int commit) {
-    __shared__ double2 lds0[NT / kWave], lds1[NT / kWave];
-    CgState &S = st[blockIdx.x];
-    const int skip = S.done;
-    double2 mn, rh;
-    sum_pf_partials<NT>(part + 2 * (size_t)blockIdx.x * nb, nb, lds0, lds1, mn, rh);
-    if (skip || threadIdx.x) return;
-    if (!commit) {
-        S.rz = mn.x + mn.y + rh.x;   // a field the plain iteration never reads
-        return;
-    }
-    const P64Step d = p64_decide(mn.x, mn.y, rh.x, S.iter0 + n, S);
-    S.alpha = make_double2(d.alpha, 0.0);
-    S.beta = d.beta;
-    S.iter = d.iter;
-    S.rr_prev = rh.x;
-    S.rr = d.rr;
-    S.iter0 += n;
-    if (d.stop) p64_stop(S, S.iter0, d, active);
-}
-
-// The x updates that the launches of a phase have left to later ones, added to x of the systems
-// that stopped after m = pfLaunch launches: alpha_{m-1} p_{m-1}, and after an odd number of
-// launches alpha_{m-2} p_{m-2} before it.
-__global__ void __launch_bounds__(kPfNT)
-k_p64_close(int n, const CgState *__restrict__ st, double2 *__restrict__ x, const double2 *__restrict__ d0,
-            const double2 *__restrict__ d1, const double2 *__restrict__ d2) {
-    const int sys = blockIdx.y, m = st[sys].pfLaunch, i = blockIdx.x * kPfNT + threadIdx.x;
-    if (m == 0 || i >= n) return;
-    const double2 *const rot[3] = {d0, d1, d2};
-    const double2 *p = rot[m % 3], *pp = rot[(m + 2) % 3];
-    const double al = st[sys].alpha.x, alPrev = (m & 1) && m > 1 ? st[sys].ab[0].x : 0.0;
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-        const size_t k = ((size_t)sys * 2 + s) * n + i;
-        double2 v = x[k];
-        if (alPrev != 0.0) v = make_double2(v.x + alPrev * pp[k].x, v.y + alPrev * pp[k].y);
-        x[k] = make_double2(v.x + al * p[k].x, v.y + al * p[k].y);
-    }
-}
-
-// ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
 // Tiles and the block sizes that their entries (with the halo) divide into with few idle threads.
@@ -295,7 +195,6 @@ struct PlTile {
 constexpr PlTile kPlTiles[] = {{4, 16, 192}, {8, 32, 448}, {16, 16, 448}, {16, 32, 384}, {32, 32, 448}, {8, 64, 448},
                                {16, 64, 704}};
 constexpr int kNumPl = sizeof(kPlTiles) / sizeof(kPlTiles[0]);
-constexpr int kP64Launches = 12;   // per captured FP64 chunk: keeps both buffer rotations
 
 // a tile need not divide the lattice, but its halo may wrap around only once
 static bool pl_fits(const Ctx &c, PlTile t) {
@@ -398,14 +297,6 @@ static int launch_p64(Ctx &c, int ti, int nsys, const double *phi, bool dag1, in
     b.x = c.x;
     return launch_pl_any<double>(c, ti, nsys, dag1, idx, first && idx == 0 ? 0 : par ? 1 : 2, finMode, b);
 }
-static void launch_fin_p64(Ctx &c, int nsys, int nb, int n, const double2 *part, int commit) {
-    if (nb > 4 * kPfNT)
-        hipLaunchKernelGGL(k_fin_p64<1024>, dim3(nsys), dim3(1024), 0, c.stream, part, nb, n, c.cg_d, c.active, commit);
-    else
-        hipLaunchKernelGGL(k_fin_p64<kPfNT>, dim3(nsys), dim3(kPfNT), 0, c.stream, part, nb, n, c.cg_d, c.active,
-                           commit);
-}
-
 // the partial slots, and for mixed precision the buffers beyond the mixed solver's: second Ap,
 // third direction
 static int pl_alloc(Ctx &c, bool mixed) {
@@ -522,9 +413,9 @@ int p64_iterations(Ctx &c, const double *phi, int nsys, int mtype, bool first, i
     });
 }
 void p64_close(Ctx &c, int nsys) {
-    hipLaunchKernelGGL(k_p64_close, dim3((c.V + kPfNT - 1) / kPfNT, nsys), dim3(kPfNT), 0, c.stream, c.V,
-                       (const CgState *)c.cg_d, c.x, (const double2 *)p64_dir(c, 2), (const double2 *)p64_dir(c, 0),
-                       (const double2 *)p64_dir(c, 1));
+    hipLaunchKernelGGL(k_p64_close<false>, dim3((c.V + kPfNT - 1) / kPfNT, nsys), dim3(kPfNT), 0, c.stream, c.V,
+                       (const CgState *)c.cg_d, c.x, c.pv[0], (const double2 *)c.pv[1], c.r, (const double2 *)nullptr,
+                       (const double2 *)nullptr);
 }
 
 }  // namespace ycn

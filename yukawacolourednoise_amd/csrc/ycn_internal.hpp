@@ -56,6 +56,7 @@ struct CgState {
     double rrRel;      // FP32 loops: recursive |r|^2 when the recursion was last anchored (start, reliable update)
     int nRu;           // pipelined even-odd solve: reliable updates so far
     int ruIter[7];     // pipelined even-odd solve: iteration count at each of the first seven
+    int even;          // pipelined FP64 iteration: stop after an even number of iterations
     int pfBase;        // pipelined FP64 iteration: iterations done when the phase began
     int pfLaunch;      // pipelined FP64 iteration: launches of the phase the system stopped in, until the next check
     double2 ab[2];     // pipelined even-odd solve (prologue finalize): alpha, beta of launch idx in ab[idx & 1]
@@ -160,6 +161,7 @@ struct Ctx {
     int tile64 = -1, tile32 = -1;
     // even-odd fused Schur normal operator tiles (-1: even-odd not available)
     int tileEo64 = -1, tileEo32 = -1;
+    int tileEoP64 = -1;   // tile of the pipelined FP64 iteration (-1: not available)
     std::string tuneReport;
 
     // mixed precision: [nSys][4][V] float2
