@@ -100,11 +100,14 @@ k_eo_pf(EoPfArgs A, const typename Vec2<R>::T *__restrict__ phi, CgState *st,
     constexpr bool FP64 = sizeof(R) == 8;
     __shared__ SpLds<R, N> E;
     __shared__ SpLds<R, N - 2 * K> O;   // rows 1 .. H - 2, shifted down by one row
-    __shared__ double2 red[NT / kWave], red2[NT / kWave];
-    __shared__ double bc[3];
+    __shared__ double red[3 * NT / kWave], bc[2];
     __shared__ int pause;
     const int sys = blockIdx.y;
-    if (st[sys].done) return;
+    const PfHead hd = pf_head(st[sys]);
+    const double2 prev = RM == 2 ? st[sys].ab[(idx - 1) & 1] : make_double2(0.0, 0.0);
+    PfParts<NT> parts;
+    if (finMode && idx) parts.load(prevPart + 2 * (size_t)sys * gridDim.x, (int)gridDim.x);
+    if (hd.done) return;
     const unsigned Vh = (unsigned)A.Vh;
     const size_t off = (size_t)sys * 2 * Vh;
     r += off;
@@ -157,12 +160,12 @@ k_eo_pf(EoPfArgs A, const typename Vec2<R>::T *__restrict__ phi, CgState *st,
     };
     int tile = blockIdx.x;
     load(tile);
-    const double2 prev = RM == 2 ? st[sys].ab[(idx - 1) & 1] : make_double2(0.0, 0.0);
     double alphaD, betaD;
     if constexpr (FP64) {
-        if (!p64_prologue<NT>(st, sys, idx, finMode, prevPart, active, red, red2, bc, &pause, alphaD, betaD)) return;
+        if (!p64_prologue<NT>(st, hd, sys, idx, finMode, parts, prevPart, active, red, bc, &pause, alphaD, betaD))
+            return;
     } else {
-        if (!pf_prologue<NT>(st, sys, idx, finMode, prevPart, part, active, red, red2, bc, &pause, alphaD, betaD))
+        if (!pf_prologue<NT>(st, hd, sys, idx, finMode, parts, prevPart, part, active, red, bc, &pause, alphaD, betaD))
             return;
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) st[sys].ab[idx & 1] = make_double2(RM == 1 ? 0.0 : alphaD, betaD);
@@ -173,6 +176,7 @@ k_eo_pf(EoPfArgs A, const typename Vec2<R>::T *__restrict__ phi, CgState *st,
     while (true) {
         Sp<R> e[M0], o[M0];   // the entry's even and odd site
         R de[M0], inv[M0];    // d of the even site, 1 / d of the odd one
+        R sg[M0], sf[M0], sb[M0];   // signs: row parity, hops across the time boundary
         unsigned j[M0];
         int place[M0];
 #pragma unroll
@@ -183,6 +187,9 @@ k_eo_pf(EoPfArgs A, const typename Vec2<R>::T *__restrict__ phi, CgState *st,
                 place[u] = at_[u] | G.edge[u];
                 j[u] = G.j[u];
                 const bool odd = place[u] & 64;
+                sg[u] = odd ? (R)-1 : (R)1;
+                sf[u] = place[u] & 16 ? (R)-1 : (R)1;
+                sb[u] = place[u] & 32 ? (R)-1 : (R)1;
                 de[u] = (R)A.d0 + (R)A.g * (odd ? G.f[u].y : G.f[u].x);
                 inv[u] = (R)1 / ((R)A.d0 + (R)A.g * (odd ? G.f[u].x : G.f[u].y));
                 Sp<R> a = G.a[u];
@@ -199,7 +206,6 @@ k_eo_pf(EoPfArgs A, const typename Vec2<R>::T *__restrict__ phi, CgState *st,
         }
         __syncthreads();
         if (PERSIST && tile + (int)gridDim.x < A.tilesPerSys) load(tile + (int)gridDim.x);
-        auto sgn = [](int p, int bit) { return p & bit ? (R)-1 : (R)1; };
         // odd sites: the entry's even site is the left neighbour in an even row
         auto odd_stage = [&](auto dag, int bit) {
 #pragma unroll
@@ -208,8 +214,7 @@ k_eo_pf(EoPfArgs A, const typename Vec2<R>::T *__restrict__ phi, CgState *st,
                     const int w = threadIdx.x + u * NT;
                     o[u] = scale<R>(-inv[u],
                                     eo_pf_hop<R, decltype(dag)::value, WR1>(wr, E, w, K, place[u] & 64 ? w - 1 : w + 1,
-                                                                            e[u], sgn(place[u], 64), sgn(place[u], 16),
-                                                                            sgn(place[u], 32)));
+                                                                            e[u], sg[u], sf[u], sb[u]));
                     O.set(w - K, o[u]);
                 }
         };
@@ -217,8 +222,7 @@ k_eo_pf(EoPfArgs A, const typename Vec2<R>::T *__restrict__ phi, CgState *st,
         auto even_site = [&](auto dag, int u) {
             const int w = threadIdx.x + u * NT - K;
             return axpy<R>(eo_pf_hop<R, decltype(dag)::value, WR1>(wr, O, w, K, place[u] & 64 ? w + 1 : w - 1, o[u],
-                                                                   -sgn(place[u], 64), sgn(place[u], 16),
-                                                                   sgn(place[u], 32)),
+                                                                   -sg[u], sf[u], sb[u]),
                            de[u], e[u]);
         };
         odd_stage(std::true_type(), 4);
@@ -244,13 +248,7 @@ k_eo_pf(EoPfArgs A, const typename Vec2<R>::T *__restrict__ phi, CgState *st,
         tile += (int)gridDim.x;
         if (tile >= A.tilesPerSys) break;   // (stage 0 writes E only, which stage 4 does not read)
     }
-    const size_t pidx = (size_t)sys * gridDim.x + blockIdx.x;
-    const double2 t1 = block_sum2<NT>(make_double2(mu, nu), red);
-    const double2 t2 = block_sum2<NT>(make_double2(rho, 0.0), red2);
-    if (threadIdx.x == 0) {
-        part[2 * pidx] = t1;
-        part[2 * pidx + 1] = t2;
-    }
+    store_pf_partials<NT>(part + 2 * ((size_t)sys * gridDim.x + blockIdx.x), mu, nu, rho, red);
 }
 
 // ---------------------------------------------------------------------------

@@ -98,29 +98,97 @@ __device__ __forceinline__ double2 pf_fin_sum(const double2 *part, int nb, doubl
 // ---------------------------------------------------------------------------
 // finalize of the pipelined FP32 iteration
 // ---------------------------------------------------------------------------
-// Sums of one system's nb block partials of the pipelined iteration (pp[2 b] = (mu, nu),
-// pp[2 b + 1] = (rho, 0)) by one block in a fixed order: thread t adds entries t, t + NT,
-// ..., each round issuing its U loads before adding; valid in thread 0.
+// the sums a launch leaves: mu = <p, Ap>, nu = |Ap|^2, rho = |r|^2
+struct Pf3 {
+    double mu, nu, rho;
+};
+// v of the lanes a permute swaps: lanes 32 .. 63 of a with lanes 0 .. 31 of b (HALF), or the odd
+// rows of 16 of a with the even rows of b; the sum of the two afterwards
+template <bool HALF>
+__device__ __forceinline__ double swap_add(double a, double b) {
+    const long long ia = __double_as_longlong(a), ib = __double_as_longlong(b);
+    auto sw = [](unsigned u, unsigned v) {
+        if constexpr (HALF)
+            return __builtin_amdgcn_permlane32_swap(u, v, false, false);
+        else
+            return __builtin_amdgcn_permlane16_swap(u, v, false, false);
+    };
+    const auto lo = sw((unsigned)ia, (unsigned)ib), hi = sw((unsigned)(ia >> 32), (unsigned)(ib >> 32));
+    return __longlong_as_double(((long long)hi[0] << 32) | lo[0]) +
+           __longlong_as_double(((long long)hi[1] << 32) | lo[1]);
+}
+// Sums over the block by one barrier, valid in wave 0: mu, nu, rho in every lane of its rows of 16
+// lanes 0, 1, 2.  The three sums share their steps: two swaps of lanes between registers leave each
+// in rows of its own, four steps within rows finish them (7 additions and 14 moves against 18 and
+// 52 for three separate sums).  red holds 3 NT / 64 numbers.
 template <int NT>
-__device__ void sum_pf_partials(const double2 *pp, int nb, double2 *lds0, double2 *lds1, double2 &mn, double2 &rh) {
-    constexpr int U = 4;
-    double2 a0 = make_double2(0.0, 0.0), a1 = make_double2(0.0, 0.0);
-    for (int base = threadIdx.x; base < nb; base += U * NT) {
-        double2 v[2 * U];
+__device__ __forceinline__ double block_sum3(double mu, double nu, double rho, double *red) {
+    constexpr int NW = NT / kWave;
+    static_assert(NW <= 16, "one row of lanes adds up the waves");
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave, row = lane >> 4, k = lane & 15;
+    const double v = row_sum(swap_add<false>(swap_add<true>(mu, nu), swap_add<true>(rho, rho)));   // mu, rho, nu, rho
+    if (k == 0 && row < 3) red[3 * wave + (row == 0 ? 0 : 3 - row)] = v;
+    __syncthreads();
+    return wave == 0 ? row_sum(row < 3 && k < NW ? red[3 * k + row] : 0.0) : 0.0;
+}
+// one system's nb block partials (pp[2 b] = (mu, nu), pp[2 b + 1].x = rho): the first loads, issued
+// ahead of other work, and the sums by one block in a fixed order (thread t adds entries t, t + NT,
+// ...; each round issues its U loads before adding); valid in wave 0
+template <int NT>
+struct PfParts {
+    static constexpr int U = 4;
+    double2 mn[U];
+    double rh[U];
+    __device__ __forceinline__ void load(const double2 *pp, int nb, int base) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int k = base + u * NT;
-            v[2 * u] = k < nb ? pp[2 * k] : make_double2(0.0, 0.0);
-            v[2 * u + 1] = k < nb ? pp[2 * k + 1] : make_double2(0.0, 0.0);
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            a0 = cadd(a0, v[2 * u]);
-            a1 = cadd(a1, v[2 * u + 1]);
+            mn[u] = make_double2(0.0, 0.0);
+            rh[u] = 0.0;
+            if (k < nb) {
+                mn[u] = pp[2 * k];
+                rh[u] = pp[2 * k + 1].x;
+            }
         }
     }
-    mn = block_sum2<NT>(a0, lds0);
-    rh = block_sum2<NT>(a1, lds1);
+    __device__ __forceinline__ void load(const double2 *pp, int nb) { load(pp, nb, threadIdx.x); }
+    __device__ __forceinline__ Pf3 sum(const double2 *pp, int nb, double *red) {
+        double mu = 0.0, nu = 0.0, rho = 0.0;
+        for (int base = threadIdx.x;;) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                mu += mn[u].x;
+                nu += mn[u].y;
+                rho += rh[u];
+            }
+            base += U * NT;
+            if (base - (int)threadIdx.x >= nb) break;
+            load(pp, nb, base);
+        }
+        const double s = block_sum3<NT>(mu, nu, rho, red);
+        return {lane_f64(s, 0), lane_f64(s, 16), lane_f64(s, 32)};
+    }
+};
+template <int NT>
+__device__ __forceinline__ Pf3 sum_pf_partials(const double2 *pp, int nb, double *red) {
+    PfParts<NT> q;
+    q.load(pp, nb);
+    return q.sum(pp, nb, red);
+}
+// a block's own partials
+template <int NT>
+__device__ __forceinline__ void store_pf_partials(double2 *pp, double mu, double nu, double rho, double *red) {
+    const double v = block_sum3<NT>(mu, nu, rho, red);
+    if (threadIdx.x < 48 && (threadIdx.x & 15) == 0) reinterpret_cast<double *>(pp)[threadIdx.x >> 4] = v;
+}
+
+// what a launch reads of the state, none of it written while the launch runs except done
+struct PfHead {
+    double alpha, beta, stop, rrRel, rr;
+    int iter0, maxIter, even, done;
+};
+__device__ __forceinline__ PfHead pf_head(const CgState &S) {
+    return {S.alpha.x, S.beta, S.stop, S.rrRel, S.rr, S.iter0, S.maxIter, S.even, S.done};
 }
 
 // The decision after iteration number `iter` of the pipelined iteration, from (mu, nu)
@@ -133,7 +201,8 @@ struct PfStep {
     double alpha, beta;
     bool stop;
 };
-__device__ __forceinline__ PfStep pf_decide(double mu, double nu, double rho, int iter, const CgState &S) {
+__device__ __forceinline__ PfStep pf_decide(const Pf3 &s, int iter, const PfHead &S) {
+    const double mu = s.mu, nu = s.nu, rho = s.rho;
     PfStep d;
     d.stop = (iter >= S.maxIter) || (sqrt(rho) <= S.stop && !(iter & 1)) || (!(mu > 0.0) && !(iter & 1)) ||
              (rho < kReliableDrop * kReliableDrop * S.rrRel && !(iter & 1)) || !isfinite(mu) || !isfinite(rho);
@@ -146,15 +215,15 @@ __device__ __forceinline__ PfStep pf_decide(double mu, double nu, double rho, in
 
 // the finalize of one iteration from its sums (thread 0): iteration count, rho, pause or
 // the next alpha, beta; commit = false only keeps the sums (timing launches)
-__device__ __forceinline__ void pf_commit(CgState &S, double2 mn, double2 rh, int *active, int commit) {
+__device__ __forceinline__ void pf_commit(CgState &S, const Pf3 &s, int *active, int commit) {
     if (!commit) {
-        S.rz = mn.x + mn.y + rh.x;   // a field the even-odd iteration never reads
+        S.rz = s.mu + s.nu + s.rho;   // a field these iterations never read
         return;
     }
     S.iter += 1;
-    const PfStep d = pf_decide(mn.x, mn.y, rh.x, S.iter, S);
+    const PfStep d = pf_decide(s, S.iter, pf_head(S));
     S.rr_prev = S.rr;
-    S.rr = rh.x;
+    S.rr = s.rho;
     if (d.stop) {
         S.done = 1;
         atomicSub(active, 1);
@@ -170,20 +239,19 @@ __device__ __forceinline__ void pf_commit(CgState &S, double2 mn, double2 rh, in
 // with rho of the iteration before it from launch idx - 2's partials, still in this launch's own
 // slot.  False: the system pauses here.  finMode 0 and launch 0 take alpha, beta from the state.
 template <int NT>
-__device__ __forceinline__ bool pf_prologue(CgState *st, int sys, int idx, int finMode, const double2 *prevPart,
-                                            const double2 *ownPart, int *active, double2 *red, double2 *red2,
-                                            double *bc, int *pause, double &alpha, double &beta) {
-    alpha = st[sys].alpha.x;
-    beta = st[sys].beta;
+__device__ __forceinline__ bool pf_prologue(CgState *st, const PfHead &hd, int sys, int idx, int finMode,
+                                            PfParts<NT> &parts, const double2 *prevPart, const double2 *ownPart,
+                                            int *active, double *red, double *bc, int *pause, double &alpha,
+                                            double &beta) {
+    alpha = hd.alpha;
+    beta = hd.beta;
     if (finMode == 0 || idx == 0) return true;
     const int nb = (int)gridDim.x;
-    double2 mn, rh;
-    sum_pf_partials<NT>(prevPart + 2 * (size_t)sys * nb, nb, red, red2, mn, rh);
+    const Pf3 s = parts.sum(prevPart + 2 * (size_t)sys * nb, nb, red);
     if (threadIdx.x == 0) {
-        const PfStep d = pf_decide(mn.x, mn.y, rh.x, st[sys].iter0 + idx, st[sys]);
+        const PfStep d = pf_decide(s, hd.iter0 + idx, hd);
         bc[0] = d.alpha;
         bc[1] = d.beta;
-        bc[2] = rh.x;
         *pause = finMode == 1 && d.stop;
     }
     __syncthreads();
@@ -193,17 +261,16 @@ __device__ __forceinline__ bool pf_prologue(CgState *st, int sys, int idx, int f
         return true;
     }
     if (blockIdx.x == 0) {
-        double rprev = st[sys].rr;   // iteration iter0 (chunk start) when idx == 1
+        double rprev = hd.rr;   // iteration iter0 (chunk start) when idx == 1
         if (idx >= 2) {
-            double2 m2, r2;
-            sum_pf_partials<NT>(ownPart + 2 * (size_t)sys * nb, nb, red, red2, m2, r2);
-            rprev = r2.x;
+            __syncthreads();
+            rprev = sum_pf_partials<NT>(ownPart + 2 * (size_t)sys * nb, nb, red).rho;
         }
         if (threadIdx.x == 0) {
             CgState &S = st[sys];
             S.iter = S.iter0 + idx;
             S.rr_prev = rprev;
-            S.rr = bc[2];
+            S.rr = s.rho;
             S.done = 1;
             atomicSub(active, 1);
         }
@@ -225,7 +292,8 @@ struct P64Step {
     int iter;
     bool stop, conv;
 };
-__device__ __forceinline__ P64Step p64_decide(double mu, double nu, double rho, int iter, const CgState &S) {
+__device__ __forceinline__ P64Step p64_decide(const Pf3 &s, int iter, const PfHead &S) {
+    const double mu = s.mu, nu = s.nu, rho = s.rho;
     P64Step d;
     if (sqrt(rho) <= S.stop && !(S.even && !(iter & 1) && rho > 0.0)) return {0.0, 0.0, rho, iter - 1, true, true};
     d.iter = iter;
@@ -247,27 +315,26 @@ __device__ __forceinline__ void p64_stop(CgState &S, int it, const P64Step &d, i
 
 // pf_prologue for FP64
 template <int NT>
-__device__ __forceinline__ bool p64_prologue(CgState *st, int sys, int idx, int finMode, const double2 *prevPart,
-                                             int *active, double2 *red, double2 *red2, double *bc, int *pause,
-                                             double &alpha, double &beta) {
-    alpha = st[sys].alpha.x;
-    beta = st[sys].beta;
+__device__ __forceinline__ bool p64_prologue(CgState *st, const PfHead &hd, int sys, int idx, int finMode,
+                                             PfParts<NT> &parts, const double2 *prevPart, int *active, double *red,
+                                             double *bc, int *pause, double &alpha, double &beta) {
+    alpha = hd.alpha;
+    beta = hd.beta;
     if (finMode == 0 || idx == 0) return true;
     const int nb = (int)gridDim.x;
-    double2 mn, rh;
-    sum_pf_partials<NT>(prevPart + 2 * (size_t)sys * nb, nb, red, red2, mn, rh);
+    const Pf3 s = parts.sum(prevPart + 2 * (size_t)sys * nb, nb, red);
     if (threadIdx.x == 0) {
-        CgState &S = st[sys];
-        const int it = S.iter0 + idx;
-        const P64Step d = p64_decide(mn.x, mn.y, rh.x, it, S);
+        const int it = hd.iter0 + idx;
+        const P64Step d = p64_decide(s, it, hd);
         bc[0] = d.alpha;
         bc[1] = d.beta;
         *pause = finMode == 1 && d.stop;
         if (finMode == 1 && d.stop && blockIdx.x == 0) {
+            CgState &S = st[sys];
             S.alpha = make_double2(d.alpha, 0.0);
             S.beta = d.beta;
             S.iter = d.iter;
-            S.rr_prev = rh.x;
+            S.rr_prev = s.rho;
             S.rr = d.rr;
             p64_stop(S, it, d, active);
         }
@@ -284,21 +351,20 @@ template <int NT>
 __global__ void __launch_bounds__(NT)
 k_fin_p64(const double2 *__restrict__ part, int nb, int n, CgState *__restrict__ st, int *__restrict__ active,
           int commit) {
-    __shared__ double2 lds0[NT / kWave], lds1[NT / kWave];
+    __shared__ double red[3 * NT / kWave];
     CgState &S = st[blockIdx.x];
-    const int skip = S.done;
-    double2 mn, rh;
-    sum_pf_partials<NT>(part + 2 * (size_t)blockIdx.x * nb, nb, lds0, lds1, mn, rh);
-    if (skip || threadIdx.x) return;
+    const PfHead hd = pf_head(S);
+    const Pf3 s = sum_pf_partials<NT>(part + 2 * (size_t)blockIdx.x * nb, nb, red);
+    if (hd.done || threadIdx.x) return;
     if (!commit) {
-        S.rz = mn.x + mn.y + rh.x;   // a field the plain iteration never reads
+        S.rz = s.mu + s.nu + s.rho;   // a field these iterations never read
         return;
     }
-    const P64Step d = p64_decide(mn.x, mn.y, rh.x, S.iter0 + n, S);
+    const P64Step d = p64_decide(s, hd.iter0 + n, hd);
     S.alpha = make_double2(d.alpha, 0.0);
     S.beta = d.beta;
     S.iter = d.iter;
-    S.rr_prev = rh.x;
+    S.rr_prev = s.rho;
     S.rr = d.rr;
     S.iter0 += n;
     if (d.stop) p64_stop(S, S.iter0, d, active);
@@ -317,13 +383,12 @@ inline void launch_fin_p64(Ctx &c, int nsys, int nb, int n, const double2 *part,
 template <int NT>
 __global__ void __launch_bounds__(NT)
 k_fin_pf(const double2 *__restrict__ part, int nb, CgState *__restrict__ st, int *__restrict__ active, int commit) {
-    __shared__ double2 lds0[NT / kWave], lds1[NT / kWave];
+    __shared__ double red[3 * NT / kWave];
     CgState &S = st[blockIdx.x];
     const int skip = S.done;
-    double2 mn, rh;
-    sum_pf_partials<NT>(part + 2 * (size_t)blockIdx.x * nb, nb, lds0, lds1, mn, rh);
+    const Pf3 s = sum_pf_partials<NT>(part + 2 * (size_t)blockIdx.x * nb, nb, red);
     if (skip || threadIdx.x) return;
-    pf_commit(S, mn, rh, active, commit);
+    pf_commit(S, s, active, commit);
 }
 
 // the same with one wave per system (systems with at most kPfNT block partials: one or a
@@ -337,15 +402,16 @@ k_fin_pf_wave(const double2 *__restrict__ part, int nb, int nsys, CgState *__res
     CgState &S = st[sys];
     const int skip = S.done;
     const double2 *pp = part + 2 * (size_t)sys * nb;
-    double2 a0 = make_double2(0.0, 0.0), a1 = make_double2(0.0, 0.0);
+    double mu = 0.0, nu = 0.0, rho = 0.0;
     for (int k = lane; k < nb; k += kWave) {
-        a0 = cadd(a0, pp[2 * k]);
-        a1 = cadd(a1, pp[2 * k + 1]);
+        const double2 mn = pp[2 * k];
+        mu += mn.x;
+        nu += mn.y;
+        rho += pp[2 * k + 1].x;
     }
-    const double2 mn = make_double2(wave_sum(a0.x), wave_sum(a0.y));
-    const double2 rh = make_double2(wave_sum(a1.x), wave_sum(a1.y));
+    const Pf3 s = {wave_sum(mu), wave_sum(nu), wave_sum(rho)};
     if (skip || lane) return;
-    pf_commit(S, mn, rh, active, commit);
+    pf_commit(S, s, active, commit);
 }
 
 // Finalize at the end of a chunk of n launches that finalized each other in their
@@ -355,18 +421,17 @@ template <int NT>
 __global__ void __launch_bounds__(NT)
 k_fin_pf_chunk(const double2 *__restrict__ slotLast, const double2 *__restrict__ slotPrev, int nb, int n,
                CgState *__restrict__ st, int *__restrict__ active) {
-    __shared__ double2 lds0[NT / kWave], lds1[NT / kWave];
+    __shared__ double red[3 * NT / kWave];
     CgState &S = st[blockIdx.x];
     if (S.done) return;
-    double2 mn, rh, mp, rp;
-    sum_pf_partials<NT>(slotLast + 2 * (size_t)blockIdx.x * nb, nb, lds0, lds1, mn, rh);
+    const Pf3 s = sum_pf_partials<NT>(slotLast + 2 * (size_t)blockIdx.x * nb, nb, red);
     __syncthreads();
-    sum_pf_partials<NT>(slotPrev + 2 * (size_t)blockIdx.x * nb, nb, lds0, lds1, mp, rp);
+    const Pf3 before = sum_pf_partials<NT>(slotPrev + 2 * (size_t)blockIdx.x * nb, nb, red);
     if (threadIdx.x) return;
     S.iter = S.iter0 + n;
-    const PfStep d = pf_decide(mn.x, mn.y, rh.x, S.iter, S);
-    S.rr_prev = rp.x;
-    S.rr = rh.x;
+    const PfStep d = pf_decide(s, S.iter, pf_head(S));
+    S.rr_prev = before.rho;
+    S.rr = s.rho;
     if (d.stop) {
         S.done = 1;
         atomicSub(active, 1);

@@ -72,11 +72,14 @@ k_pl_pf(PlArgs A, const R *__restrict__ phi, CgState *st, const typename Vec2<R>
     constexpr bool FP64 = sizeof(R) == 8;
     __shared__ SpLds<R, N> P;
     __shared__ SpLds<R, FP64 ? 1 : N> Q32;
-    __shared__ double2 red[NT / kWave], red2[NT / kWave];
-    __shared__ double bc[3];
+    __shared__ double red[3 * NT / kWave], bc[2];
     __shared__ int pause;
     const int sys = blockIdx.y;
-    if (st[sys].done) return;
+    const PfHead hd = pf_head(st[sys]);
+    const double2 prev = RM == 2 ? st[sys].ab[(idx - 1) & 1] : make_double2(0.0, 0.0);
+    PfParts<NT> parts;
+    if (finMode && idx) parts.load(prevPart + 2 * (size_t)sys * gridDim.x, (int)gridDim.x);
+    if (hd.done) return;
     const unsigned V = (unsigned)A.V;
     const size_t off = (size_t)sys * 2 * V;
     r += off;
@@ -115,12 +118,12 @@ k_pl_pf(PlArgs A, const R *__restrict__ phi, CgState *st, const typename Vec2<R>
             d[u] = at(ph, gs[u]);
         }
     }
-    const double2 prev = RM == 2 ? st[sys].ab[(idx - 1) & 1] : make_double2(0.0, 0.0);
     double alphaD, betaD;
     if constexpr (FP64) {
-        if (!p64_prologue<NT>(st, sys, idx, finMode, prevPart, active, red, red2, bc, &pause, alphaD, betaD)) return;
+        if (!p64_prologue<NT>(st, hd, sys, idx, finMode, parts, prevPart, active, red, bc, &pause, alphaD, betaD))
+            return;
     } else {
-        if (!pf_prologue<NT>(st, sys, idx, finMode, prevPart, part, active, red, red2, bc, &pause, alphaD, betaD))
+        if (!pf_prologue<NT>(st, hd, sys, idx, finMode, parts, prevPart, part, active, red, bc, &pause, alphaD, betaD))
             return;
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) st[sys].ab[idx & 1] = make_double2(RM == 1 ? 0.0 : alphaD, betaD);
@@ -176,13 +179,7 @@ k_pl_pf(PlArgs A, const R *__restrict__ phi, CgState *st, const typename Vec2<R>
         second(P);
     else
         second(Q32);
-    const size_t pidx = (size_t)sys * gridDim.x + blockIdx.x;
-    const double2 t1 = block_sum2<NT>(make_double2(mu, nu), red);
-    const double2 t2 = block_sum2<NT>(make_double2(rho, 0.0), red2);
-    if (threadIdx.x == 0) {
-        part[2 * pidx] = t1;
-        part[2 * pidx + 1] = t2;
-    }
+    store_pf_partials<NT>(part + 2 * ((size_t)sys * gridDim.x + blockIdx.x), mu, nu, rho, red);
 }
 
 // ---------------------------------------------------------------------------
