@@ -158,3 +158,23 @@ def test_fp64_even_odd_stop(gpu, monkeypatch, mode, tol):
             assert st["converged"] == 1 and st["iters"] % 2 == 0
             assert mode == 0 or st["true_rel_resid"] <= tol
             assert rel(d, dr) < 1e-8
+
+
+@pytest.mark.parametrize("fin", ["fused", "separate"])
+@pytest.mark.parametrize("tile,Nt,Nx,r", [(12, 64, 64, 1.0), (12, 128, 192, 0.7), (13, 32, 128, 0.7), (13, 96, 256, 1.0)])
+def test_large_even_odd_fp32_tiles(gpu, monkeypatch, tile, Nt, Nx, r, fin):
+    """The 64x64 and 32x128 tiles: one tile, whose halo is itself, and several; converged drifts of
+    two noise vectors as in test_every_tile."""
+    monkeypatch.setenv("YCN_TILE_EO32", str(tile))
+    monkeypatch.setenv("YCN_EO_FIN", fin)
+    Y = gpu
+    p, orc = mk(Y, Nt=Nt, Nx=Nx, r=r, nNoise=2, cgTol=1e-10, cgTolMode=1, cgMaxIter=20000)
+    p.evenOdd = 1
+    p.cgPrecision = Y.YCN_CG_MIXED
+    phi = 1.0 + O.hot_start(Nt + Nx, Nt, Nx)
+    with Y.Context(p) as c:
+        c.set_field(phi)
+        d, st = c.fermion_force(3)
+    dr, _ = O.fermion_drift(orc, phi, 3)
+    assert st["converged"] == 1 and st["true_rel_resid"] <= 1e-10
+    assert rel(d, dr) < 1e-8

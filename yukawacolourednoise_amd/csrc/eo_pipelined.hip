@@ -254,19 +254,8 @@ k_eo_pf(EoPfArgs A, const typename Vec2<R>::T *__restrict__ phi, CgState *st,
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
-// resident blocks of a kernel on the whole device (persistent launches)
-static int resident_blocks(const void *kernel, int threads) {
-    int dev = 0, cus = 0, per = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) !=
-                                                 hipSuccess)
-        return 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, threads, 0) != hipSuccess) return 0;
-    return per * cus;
-}
-
 // form 0: launch 0 of a phase (r read), 1: odd launches, 2: even ones; returns the block partials
-// per system.  Persistent grids are sized by the form with the fewest resident blocks, so that
-// consecutive launches leave the same number of partials.
+// per system
 template <typename R, int TT, int TX, int NT>
 static int launch_tt(const Ctx &c, int nsys, const EoPfLaunch<R> &b) {
     using V2 = typename Vec2<R>::T;
@@ -290,13 +279,8 @@ static int launch_tt(const Ctx &c, int nsys, const EoPfLaunch<R> &b) {
         static const K ks[3] = {&k_eo_pf<R, TT, TX, NT, P, W1, 0, 1>, &k_eo_pf<R, TT, TX, NT, P, W1, 2, 2>,
                                 &k_eo_pf<R, TT, TX, NT, P, W1, 0, 2>};
         if (P) {
-            static const int resident = [] {
-                int m = 1 << 30;
-                for (const K &k : ks) m = std::min(m, resident_blocks(reinterpret_cast<const void *>(k), NT));
-                return m;
-            }();
-            grid = std::min(A.tilesPerSys, std::max(resident, 8));
-            if (A.xcdRemap && grid >= 8) grid -= grid % 8;   // keeps every block's tiles on one XCD's band
+            static const int resident = resident_blocks(ks, NT);
+            grid = persistent_grid(resident, A.tilesPerSys);
         }
         hipLaunchKernelGGL(ks[b.form], dim3(grid, nsys), dim3(NT), 0, c.stream, A,
                            reinterpret_cast<const V2 *>(b.phi), c.cg_d, b.r, b.Ap_in, b.pold, b.pnew, b.Ap, b.x, b.part,
@@ -316,7 +300,16 @@ static int launch_tt(const Ctx &c, int nsys, const EoPfLaunch<R> &b) {
 }
 
 // Block sizes: the entries of the tile with its halo, TT + 8 rows of (TX + 8) / 2, spread over
-// threads with few idle ones.
+// threads with few idle ones.  What bounds an iteration, measured per launch pair's average:
+//   256 x 256 FP32, 8x32 tiles of one entry per thread: 5.0 us, latency (launch, the prologue's
+//     sums, one load, four stages, the block's sums); 7.2 in the stage-indexed kernel before.
+//   1024 x 1024 FP32: 13.3 us for 54 MB (6.6 us at the 8.2 TB/s of a cache-resident copy) with
+//     64x64 and 32x128 tiles, which leave one block per compute unit, a quarter of the work in the
+//     halo and 256 partials for the prologue; 15.7 with 16x32 on a persistent grid, 16.3 with 16x64;
+//     18.5 before.  About 4 us are vector instructions, 1 the prologue, 1 the launch.
+//   1024 x 1024 FP64: 23.3 us for 109 MB with 16x32 tiles of two entries per thread (several
+//     blocks per compute unit, one loading while another works), 24.7 with one entry, 26.4 32x32.
+//   512 x 512 FP64: 7.9 us with 32x32 tiles and 832 threads, 8.3 with 448, 8.6 with 16x32.
 int launch_eo_pf32(const Ctx &c, int TT, int TX, int nsys, const EoPfLaunch<float> &b) {
     switch (TT * 1000 + TX) {
     case 8032: return launch_tt<float, 8, 32, 320>(c, nsys, b);
@@ -326,18 +319,20 @@ int launch_eo_pf32(const Ctx &c, int TT, int TX, int nsys, const EoPfLaunch<floa
     case 4064: return launch_tt<float, 4, 64, 448>(c, nsys, b);
     case 2032: return launch_tt<float, 2, 32, 256>(c, nsys, b);
     case 32032: return launch_tt<float, 32, 32, 448>(c, nsys, b);
+    case 64064: return launch_tt<float, 64, 64, 704>(c, nsys, b);
+    case 32128: return launch_tt<float, 32, 128, 704>(c, nsys, b);
     default: return launch_tt<float, 16, 64, 448>(c, nsys, b);
     }
 }
 int launch_eo_pf64(const Ctx &c, int TT, int TX, int nsys, const EoPfLaunch<double> &b) {
     switch (TT * 1000 + TX) {
     case 8032: return launch_tt<double, 8, 32, 320>(c, nsys, b);
-    case 16032: return launch_tt<double, 16, 32, 512>(c, nsys, b);
+    case 16032: return launch_tt<double, 16, 32, 256>(c, nsys, b);
     case 16016: return launch_tt<double, 16, 16, 320>(c, nsys, b);
     case 4032: return launch_tt<double, 4, 32, 256>(c, nsys, b);
     case 2032: return launch_tt<double, 2, 32, 256>(c, nsys, b);
     case 4016: return launch_tt<double, 4, 16, 192>(c, nsys, b);
-    default: return launch_tt<double, 32, 32, 448>(c, nsys, b);
+    default: return launch_tt<double, 32, 32, 832>(c, nsys, b);
     }
 }
 

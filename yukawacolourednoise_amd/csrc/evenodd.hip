@@ -683,7 +683,8 @@ struct EoTileCfg {
 constexpr EoTileCfg kEoTiles64[] = {{8, 32, false}, {16, 16, false}, {4, 64, false}, {4, 32, false}, {2, 32, false}};
 constexpr EoTileCfg kEoTiles32[] = {{8, 32, false},  {16, 32, false}, {8, 64, false},  {16, 16, false},
                                     {4, 64, false},  {2, 32, false},  {32, 32, false}, {16, 64, false},
-                                    {8, 32, true},   {16, 32, true},  {16, 16, true},  {8, 64, true}};
+                                    {8, 32, true},   {16, 32, true},  {16, 16, true},  {8, 64, true},
+                                    {64, 64, false}, {32, 128, false}};
 // tiles of the pipelined FP64 iteration
 struct EoTile {
     int TT, TX;

@@ -573,6 +573,30 @@ struct EoPfLaunch {
 int launch_eo_pf32(const Ctx &c, int TT, int TX, int nsys, const EoPfLaunch<float> &b);
 int launch_eo_pf64(const Ctx &c, int TT, int TX, int nsys, const EoPfLaunch<double> &b);
 
+// blocks that the device holds of the kernel with the fewest of ks (persistent launches:
+// consecutive ones then leave the same number of partials)
+template <typename K>
+inline int resident_blocks(const K (&ks)[3], int threads) {
+    int dev = 0, cus = 0, m = 1 << 30;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+        return 8;
+    for (const K &k : ks) {
+        int per = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, reinterpret_cast<const void *>(k), threads, 0) !=
+            hipSuccess)
+            return 8;
+        m = std::min(m, per * cus);
+    }
+    return std::max(m, 8);
+}
+// the grid: as many blocks as are resident, or fewer where that evens out the tiles per block; a
+// multiple of 8, so that a block's tiles lie in one XCD's band of tiles
+inline int persistent_grid(int resident, int tiles) {
+    const int rounds = (tiles + resident - 1) / resident, g = (tiles + rounds - 1) / rounds;
+    return std::min(tiles, (g + 7) / 8 * 8);
+}
+
 // direction p_k (k >= -1) of a chunk of pipelined launches: the three buffers in rotation,
 // p_{-1} (the direction kept across the reliable update) in ps[0]
 inline float2 *pf_dir(const Ctx &c, int k) {

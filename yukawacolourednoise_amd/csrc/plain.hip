@@ -185,11 +185,15 @@ k_pl_pf(PlArgs A, const R *__restrict__ phi, CgState *st, const typename Vec2<R>
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
-// Tiles and the block sizes that their entries (with the halo) divide into with few idle threads.
+// Tiles and their block sizes.  Lattices that fill the chip want few waves per block, each with two
+// to four entries, so that several blocks share a compute unit and one loads while another works:
+// at 1024 x 1024 in FP64 8x32 takes 31.8 us with 256 threads and 36.1 with 448 (one entry each),
+// 16x32 32.3 and 40.9 with 384.  A persistent grid that prefetches the next tile was no faster
+// (32.4 at best).
 struct PlTile {
     int TT, TX, NT;
 };
-constexpr PlTile kPlTiles[] = {{4, 16, 192}, {8, 32, 448}, {16, 16, 448}, {16, 32, 384}, {32, 32, 448}, {8, 64, 448},
+constexpr PlTile kPlTiles[] = {{4, 16, 192}, {8, 32, 256}, {16, 16, 256}, {16, 32, 256}, {32, 32, 448}, {8, 64, 256},
                                {16, 64, 704}};
 constexpr int kNumPl = sizeof(kPlTiles) / sizeof(kPlTiles[0]);
 
@@ -249,11 +253,11 @@ static int launch_pl_any(Ctx &c, int ti, int nsys, bool dag1, int idx, int form,
     int nb = 0;
     switch (t.TT * 1000 + t.TX) {
     case 4016: nb = launch_pl_tt<R, 4, 16, 192>(c, nsys, dag1, idx, form, finMode, b); break;
-    case 8032: nb = launch_pl_tt<R, 8, 32, 448>(c, nsys, dag1, idx, form, finMode, b); break;
-    case 16016: nb = launch_pl_tt<R, 16, 16, 448>(c, nsys, dag1, idx, form, finMode, b); break;
-    case 16032: nb = launch_pl_tt<R, 16, 32, 384>(c, nsys, dag1, idx, form, finMode, b); break;
+    case 8032: nb = launch_pl_tt<R, 8, 32, 256>(c, nsys, dag1, idx, form, finMode, b); break;
+    case 16016: nb = launch_pl_tt<R, 16, 16, 256>(c, nsys, dag1, idx, form, finMode, b); break;
+    case 16032: nb = launch_pl_tt<R, 16, 32, 256>(c, nsys, dag1, idx, form, finMode, b); break;
     case 32032: nb = launch_pl_tt<R, 32, 32, 448>(c, nsys, dag1, idx, form, finMode, b); break;
-    case 8064: nb = launch_pl_tt<R, 8, 64, 448>(c, nsys, dag1, idx, form, finMode, b); break;
+    case 8064: nb = launch_pl_tt<R, 8, 64, 256>(c, nsys, dag1, idx, form, finMode, b); break;
     default: nb = launch_pl_tt<R, 16, 64, 704>(c, nsys, dag1, idx, form, finMode, b); break;
     }
     prof_after(c, PK_NORMAL_OP);
