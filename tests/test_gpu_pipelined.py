@@ -178,3 +178,31 @@ def test_large_even_odd_fp32_tiles(gpu, monkeypatch, tile, Nt, Nx, r, fin):
     dr, _ = O.fermion_drift(orc, phi, 3)
     assert st["converged"] == 1 and st["true_rel_resid"] <= 1e-10
     assert rel(d, dr) < 1e-8
+
+
+@pytest.mark.parametrize("Nt,Nx,r,vectors,scale", [(16, 16, 1.0, 1, 0.02), (32, 48, 0.7, 3, 0.0), (48, 16, 1.0, 2, 0.02),
+                                                   (64, 64, 1.0, 2, 5.0)])
+def test_flexible_iteration(gpu, Nt, Nx, r, vectors, scale):
+    """The flexible solver's two launches per iteration: a zero network (plain CG), random ones and
+    one so bad that it is switched off; chunks of 10 iterations; converged drifts of several noise
+    vectors as in test_every_tile.  An odd iteration cap is kept."""
+    Y = gpu
+    kw = dict(Nt=Nt, Nx=Nx, r=r, nNoise=vectors, cgTol=1e-10, cgTolMode=1)
+    phi = 1.0 + O.hot_start(Nt + Nx, Nt, Nx)
+    w = (scale * np.random.default_rng(3).standard_normal(4896)).astype(np.float32)
+    for cap in (20000, 13):
+        p, orc = mk(Y, cgMaxIter=cap, **kw)
+        p.cgPrecision = Y.YCN_CG_MIXED
+        p.precond = Y.YCN_PRECOND_CNN
+        p.reliableEvery = 10
+        with Y.Context(p) as c:
+            c.precond_set_weights(w)
+            c.set_field(phi)
+            d, st = c.fermion_force(3)
+        print(f"# {Nt}x{Nx} {scale} {cap}: {st}", flush=True)
+        if cap == 13:
+            assert st["iters"] == 13 and st["converged"] == 0 and np.all(np.isfinite(d))
+            continue
+        dr, _ = O.fermion_drift(orc, phi, 3)
+        assert st["converged"] == 1 and st["true_rel_resid"] <= 1e-10
+        assert rel(d, dr) < 1e-8

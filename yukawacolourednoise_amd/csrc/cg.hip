@@ -278,6 +278,7 @@ k_fin_mp_true(const double2 *__restrict__ part, int nb, CgState *__restrict__ st
             S.restartNext = 1;
         }
         S.true_prev = S.true_rel;
+        S.iter0 = S.iter;   // the next chunk's iterations count from here
     } else {
         S.beta = rrt / S.rr_prev;
     }
@@ -286,30 +287,10 @@ k_fin_mp_true(const double2 *__restrict__ part, int nb, CgState *__restrict__ st
     if (S.done) { S.done = 0; atomicAdd(active, 1); }
 }
 
-// flexible CG: alpha = <r, z> / Re <p', Ap> (real, the system seen as real 8V-vectors)
-__global__ void __launch_bounds__(kNT) k_fin_alpha_fcg(const double2 *__restrict__ part, int nb, CgState *__restrict__ st) {
-    __shared__ double2 lds[kNT / kWave];
-    const int sys = blockIdx.x;
-    const int skip = st[sys].done;   // loaded together with the partials
-    const double2 dot = fin_sum(part + (size_t)sys * nb, nb, lds);
-    if (skip || threadIdx.x) return;
-    CgState &S = st[sys];
-    if (!(dot.x > 0.0) || !isfinite(S.rz) || !(S.rz > 0.0)) {
-        // the preconditioned direction is not a descent direction: no step, and plain
-        // CG from the next reliable update on
-        S.alpha = make_double2(0.0, 0.0);
-        S.precOff = 1;
-        return;
-    }
-    S.alpha = make_double2(S.rz / dot.x, 0.0);
-}
-
-// flexible CG after z = CNN(r'): partials hold (<z, r'>, <z, Ap>).  Polak-Ribiere form
-// (Notay, SIAM J. Sci. Comput. 22 (2000)): beta = <z, r' - r> / <z_old, r> with
-// r = r' + alpha Ap, i.e. beta = -alpha <z, Ap> / rz_old.  MODE 0: inside the loop;
-// MODE 1: after a reliable update replaced r' by the true residual (rz_old is then the
-// value before the last iteration, rz_prev); MODE 2: restart (beta = 0).
-template <int MODE>
+// flexible CG outside the chunks, after z = CNN(r): partials hold (<z, r>, <z, Ap>).  Polak-Ribiere
+// form as in k_fcg_op.  START: the solve begins (beta = 0); else a reliable update has replaced r by
+// the true residual, and rz_old is the value before the last iteration, rz_prev.
+template <bool START>
 __global__ void __launch_bounds__(kNT) k_fin_fcg(const double2 *__restrict__ part, int nb, CgState *__restrict__ st) {
     __shared__ double2 lds[kNT / kWave];
     const int sys = blockIdx.x;
@@ -322,10 +303,8 @@ __global__ void __launch_bounds__(kNT) k_fin_fcg(const double2 *__restrict__ par
         S.beta = 0.0;
         return;
     }
-    const double rzOld = (MODE == 1) ? S.rz_prev : S.rz;
-    S.beta = (MODE == 2 || S.restartNext || !(rzOld > 0.0)) ? 0.0 : -S.alpha.x * tot.y / rzOld;
+    S.beta = (START || S.restartNext || !(S.rz_prev > 0.0)) ? 0.0 : -S.alpha.x * tot.y / S.rz_prev;
     S.restartNext = 0;
-    if (MODE != 1) S.rz_prev = S.rz;
     S.rz = tot.x;
 }
 
@@ -1161,6 +1140,9 @@ int mp_alloc(Ctx &c) {
         }
         int rc = eo_pf_alloc(c);
         if (rc) return rc;
+    } else if (c.p.precond == YCN_PRECOND_CNN) {   // the flexible solver's second residual buffer
+        YCN_HIP(hipMalloc(&c.pfA1, sizeof(float2) * n));
+        YCN_HIP(hipMemset(c.pfA1, 0, sizeof(float2) * n));
     }
     return YCN_OK;
 }
@@ -1346,26 +1328,6 @@ int spinor_slices(Ctx &c, const double2 *psi, double *out_dev) {
 // direction, and plain CG (identity preconditioner) once a reliable interval stalls.
 // The FP64 true residual with the plain operator decides convergence.
 // ===========================================================================
-static void launch_fcg_iteration(Ctx &c, int nsys, int mtype, int parity) {
-    constexpr int NC = kComplex;   // the network mixes real and imaginary channels
-    const float2 *pold = c.ps[parity];
-    float2 *pnew = c.ps[parity ^ 1];
-    prof_before(c, PK_NORMAL_OP, (double)nsys * c.V * (4 * NC * 8 + 4));
-    launch_fused<float, NC>(c, c.tile32, nsys, mtype != YCN_DAGGER, c.phis, c.cg_d, (const float2 *)c.zs, pold, pnew,
-                        c.Aps, c.partials);
-    prof_after(c, PK_NORMAL_OP);
-    const int nbF = fused_args(c, kTiles32[c.tile32].TT, kTiles32[c.tile32].TX).tilesPerSys;
-    hipLaunchKernelGGL(k_fin_alpha_fcg, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)c.partials, nbF, c.cg_d);
-    prof_before(c, PK_CG_UPDATE, (double)nsys * c.V * 6 * NC * 8);
-    hipLaunchKernelGGL(k_mp_update<NC>, site_grid(c, nsys), dim3(kNT), 0, c.stream, c.V, (const CgState *)c.cg_d, c.xs,
-                       c.rs, (const float2 *)pnew, (const float2 *)c.Aps, c.partials);
-    prof_after(c, PK_CG_UPDATE);
-    hipLaunchKernelGGL(k_fin_beta<true>, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)c.partials,
-                       site_blocks(c), c.cg_d, c.active);
-    const int nbC = cnn_apply(c, nsys, c.cg_d, c.rs, c.Aps, c.zs, c.partials);
-    hipLaunchKernelGGL(k_fin_fcg<0>, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)c.partials, nbC, c.cg_d);
-}
-
 int fcg_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, uint32_t streamBase, uint64_t step,
               SolveStats *st) {
     constexpr int NC = kComplex;
@@ -1394,9 +1356,9 @@ int fcg_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, uint32_t
     hipLaunchKernelGGL(k_fin_setup, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)c.partials, nb, c.cg_d,
                        c.active, c.p.cgTol, c.p.cgTolMode, maxIter, 0);
     // z = CNN(b), rz = <b, z>, p' = z on the first iteration
-    int nbC = cnn_apply(c, nsys, c.cg_d, c.rs, c.Aps, c.zs, c.partials);
+    int nbC = cnn_apply(c, nsys, c.rs, c.Aps, c.zs, c.partials);
     if (nbC < 0) return nbC;
-    hipLaunchKernelGGL(k_fin_fcg<2>, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)c.partials, nbC, c.cg_d);
+    hipLaunchKernelGGL(k_fin_fcg<true>, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)c.partials, nbC, c.cg_d);
     YCN_HIP(hipGetLastError());
     const int every = std::max(1, c.p.reliableEvery);
     const int nIt = every + (every & 1);
@@ -1406,8 +1368,9 @@ int fcg_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, uint32_t
     if (rc) return rc;
     while (active > 0 && launched < hardCap) {
         rc = run_chunk(c, nullptr, nsys, mtype, nIt, 2 /* flexible */, NC, c.tile32,
-                       [&](int i) { launch_fcg_iteration(c, nsys, mtype, i & 1); });
+                       [&](int i) { (void)fcg_iteration(c, nsys, i); });
         if (rc) return rc;
+        fcg_close(c, nsys, nIt);
         launched += nIt;
         hipLaunchKernelGGL(k_mp_accum<NC>, g, dim3(kNT), 0, c.stream, c.V, (const CgState *)c.cg_d, c.x, c.xs);
         hipLaunchKernelGGL((k_true_a<NC, false>), g, dim3(kNT), 0, c.stream, L, phi, (const double2 *)c.x, c.t);
@@ -1416,9 +1379,9 @@ int fcg_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, uint32_t
         const double refRate = (c.plainIters > 0 && c.p.cgTol > 0.0) ? std::log10(c.p.cgTol) / c.plainIters : 0.0;
         hipLaunchKernelGGL(k_fin_mp_true<true>, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)c.partials, nb,
                            c.cg_d, c.active, refRate);
-        nbC = cnn_apply(c, nsys, c.cg_d, c.rs, c.Aps, c.zs, c.partials);
+        nbC = cnn_apply(c, nsys, c.rs, c.Aps, c.zs, c.partials);
         if (nbC < 0) return nbC;
-        hipLaunchKernelGGL(k_fin_fcg<1>, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)c.partials, nbC,
+        hipLaunchKernelGGL(k_fin_fcg<false>, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)c.partials, nbC,
                            c.cg_d);
         YCN_HIP(hipGetLastError());
         rc = poll_active(c, active);

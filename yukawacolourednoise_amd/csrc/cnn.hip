@@ -33,6 +33,7 @@
 
 #include "cg_fused.hpp"
 #include "cnn_mfma.hpp"
+#include "pipelined.hpp"
 #include "ycn_device.hpp"
 #include "ycn_internal.hpp"
 
@@ -168,17 +169,33 @@ k_cnn_gates(int Nt, int Nx, const float *__restrict__ phis, float g, const float
     }
 }
 
+// UPD: the step of the flexible CG iteration before it (k_fcg_op): alpha = rz / <p, Ap> from the
+// operator's partials, by every block alike; x_s += alpha p and r' = r - alpha Ap, on the halo for
+// the network's input and on the tile also to memory; z = CNN(r') and the partials (<z, r'>,
+// <z, Ap>), |r'|^2.  Without a descent direction (the network can give one up) no step is taken and
+// the network is switched off.  The network's input is scaled by |r| where the chunk began: the
+// scale cancels, and bf16 keeps its relative precision.
+// UPD = false: z = CNN(r) and the partials (<z, r>, <z, Ap>).
+// What bounds it: the latency of three layers of MFMAs on one block of four waves per compute unit
+// (256 x 256: 256 blocks).  An iteration of the flexible solver took 35 us there in six launches
+// (operator, alpha, update, beta, network, rz) and takes 25 in the two.
+template <bool UPD>
 __global__ void __launch_bounds__(kCT)
-k_cnn_fused(int Nt, int Nx, int tilesX, int nNoise, float c0, const CgState *__restrict__ st,
+k_cnn_fused(int Nt, int Nx, int tilesX, int nNoise, float c0, CgState *__restrict__ st,
             const float2 *__restrict__ rs, const float2 *__restrict__ Ap, const _Float16 *__restrict__ gates,
             float2 *__restrict__ z, const bf16x8 *__restrict__ gf1, const bf16x8 *__restrict__ gf2,
-            const bf16x8 *__restrict__ gf3, double2 *__restrict__ part) {
+            const bf16x8 *__restrict__ gf3, double2 *__restrict__ part, FcgUpdate upd) {
     constexpr int W0 = 22, W1 = 20, W2 = 18, W3 = 16;
     __shared__ __attribute__((aligned(16))) __bf16 U0[W0 * W0 * 8];
     __shared__ __attribute__((aligned(16))) __bf16 U1[W1 * W1 * 16];
     __shared__ __attribute__((aligned(16))) __bf16 U2[W2 * W2 * 16];
-    __shared__ double2 red[kCT / kWave];
+    __shared__ double2 red2[UPD ? 1 : kCT / kWave];
+    __shared__ double red[3 * kCT / kWave];
     const int sys = blockIdx.y;
+    double opSum = 0.0;
+    if constexpr (UPD)
+        for (int k = threadIdx.x; k < upd.nbOp; k += kCT) opSum += upd.opPart[(size_t)sys * upd.nbOp + k];
+    const double rz = UPD ? st[sys].ab[upd.idx & 1].y : 0.0;
     if (st[sys].done) return;
     const int V = Nt * Nx;
     const size_t off = (size_t)sys * 4 * V;
@@ -188,32 +205,82 @@ k_cnn_fused(int Nt, int Nx, int tilesX, int nNoise, float c0, const CgState *__r
     const double s = sqrt(st[sys].rr / (8.0 * (double)V));
     const float inv = s > 0.0 ? (float)(1.0 / s) : 0.f, sf = (float)s;
     double2 acc = make_double2(0.0, 0.0);
-    if (st[sys].precOff) {
+    double rho = 0.0;
+    bool identity = st[sys].precOff;
+    float alpha = 0.f;
+    auto take_alpha = [&] {   // by all threads, after their first loads are issued
+        if constexpr (UPD) {
+            const double w = wave_sum(opSum);
+            if ((threadIdx.x & (kWave - 1)) == 0) red[threadIdx.x / kWave] = w;
+            __syncthreads();
+            double dot = red[0];
+#pragma unroll
+            for (int k = 1; k < kCT / kWave; ++k) dot += red[k];
+            const bool step = dot > 0.0 && isfinite(rz) && rz > 0.0;
+            const double al = step ? rz / dot : 0.0;
+            if (!step) identity = true;
+            alpha = (float)al;
+            if (blockIdx.x == 0 && threadIdx.x == 0) {
+                st[sys].ab[upd.idx & 1].x = al;
+                if (!step) st[sys].precOff = 1;
+            }
+        }
+    };
+    // r' of entry idx (component planes and site) and the x_s update there
+    struct RA {
+        float2 r[2], a[2], p[2], x[2];
+    };
+    auto load_ra = [&](RA &q, int h, size_t idx) {
+        q.r[h] = rs[idx];
+        q.a[h] = Ap[idx];
+        if constexpr (UPD) {
+            q.p[h] = upd.p[idx];
+            q.x[h] = upd.xs[idx];
+        }
+    };
+    auto step_at = [&](const RA &q, int h, size_t idx) {
+        const float2 r = q.r[h], a = q.a[h];
+        const float2 rn = make_float2(r.x - alpha * a.x, r.y - alpha * a.y);
+        if constexpr (UPD) {
+            const float2 p = q.p[h], x = q.x[h];
+            upd.rnew[idx] = rn;
+            upd.xs[idx] = make_float2(x.x + alpha * p.x, x.y + alpha * p.y);
+            rho += (double)(rn.x * rn.x + rn.y * rn.y);
+        }
+        return rn;
+    };
+    // a thread's inputs: entries of the tile with its 3-site halo
+    constexpr int L0 = (W0 * W0 + kCT - 1) / kCT;
+    float2 rv0[L0][4], av0[L0][4];
+#pragma unroll
+    for (int u = 0; u < L0; ++u) {
+        const int w = threadIdx.x + u * kCT;
+        if (w < W0 * W0) {
+            const int a = w / W0, b = w - a * W0;
+            const size_t gs = (size_t)wrapn(t0 - 3 + a, Nt) * Nx + wrapn(x0 - 3 + b, Nx);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                rv0[u][c] = rs[off + c * V + gs];
+                if (UPD) av0[u][c] = Ap[off + c * V + gs];
+            }
+        }
+    }
+    take_alpha();
+    if (identity) {
         // plain CG fallback: identity preconditioner z = r_s
         const int lt = threadIdx.x / 16, lx = threadIdx.x % 16;
         const size_t gs = (size_t)(t0 + lt) * Nx + x0 + lx;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            const float2 rv = rs[off + c * V + gs], av = Ap[off + c * V + gs];
+            RA q;
+            load_ra(q, 0, off + c * V + gs);
+            const float2 av = q.a[0], rv = step_at(q, 0, off + c * V + gs);
             z[off + c * V + gs] = rv;
             acc.x += (double)(rv.x * rv.x + rv.y * rv.y);
             acc.y += (double)(rv.x * av.x + rv.y * av.y);
         }
     } else {
         const _Float16 *gr = gates + (size_t)(sys / nNoise) * V * 32;
-        // all of a thread's loads are issued before the first conversion
-        constexpr int L0 = (W0 * W0 + kCT - 1) / kCT;
-        float2 rv0[L0][4];
-#pragma unroll
-        for (int u = 0; u < L0; ++u) {
-            const int w = threadIdx.x + u * kCT;
-            if (w < W0 * W0) {
-                const int a = w / W0, b = w - a * W0;
-                const size_t gs = (size_t)wrapn(t0 - 3 + a, Nt) * Nx + wrapn(x0 - 3 + b, Nx);
-#pragma unroll
-                for (int c = 0; c < 4; ++c) rv0[u][c] = rs[off + c * V + gs];
-            }
-        }
 #pragma unroll
         for (int u = 0; u < L0; ++u) {
             const int w = threadIdx.x + u * kCT;
@@ -221,8 +288,10 @@ k_cnn_fused(int Nt, int Nx, int tilesX, int nNoise, float c0, const CgState *__r
                 bf16x8 q;
 #pragma unroll
                 for (int c = 0; c < 4; ++c) {
-                    q[2 * c] = (__bf16)(rv0[u][c].x * inv);
-                    q[2 * c + 1] = (__bf16)(rv0[u][c].y * inv);
+                    float2 rv = rv0[u][c];
+                    if (UPD) rv = make_float2(rv.x - alpha * av0[u][c].x, rv.y - alpha * av0[u][c].y);
+                    q[2 * c] = (__bf16)(rv.x * inv);
+                    q[2 * c + 1] = (__bf16)(rv.y * inv);
                 }
                 *reinterpret_cast<bf16x8 *>(U0 + w * 8) = q;
             }
@@ -254,10 +323,7 @@ k_cnn_fused(int Nt, int Nx, int tilesX, int nNoise, float c0, const CgState *__r
             [&](int m, int kg, f32x4 v, h4 gt) { gated(U2, m, kg, v, gt); });
         __syncthreads();
         // output layer (8 channels: lanes kg = 0, 1 hold spinor components 2 kg, 2 kg + 1);
-        // r_s and Ap of the lane's two components are loaded before the group's MFMAs
-        struct RA {
-            float2 r[2], a[2];
-        };
+        // r_s and Ap (and p, x_s) of the lane's two components are loaded before the group's MFMAs
         conv_lds<16, W3, W2, ksteps(16)>(
             U2, gf3,
             [&](int m, int kg) {
@@ -266,11 +332,7 @@ k_cnn_fused(int Nt, int Nx, int tilesX, int nNoise, float c0, const CgState *__r
                     const int a = m / W3, b = m - a * W3;
                     const size_t gs = (size_t)(t0 + a) * Nx + x0 + b;
 #pragma unroll
-                    for (int h = 0; h < 2; ++h) {
-                        const size_t idx = off + (size_t)(2 * kg + h) * V + gs;
-                        q.r[h] = rs[idx];
-                        q.a[h] = Ap[idx];
-                    }
+                    for (int h = 0; h < 2; ++h) load_ra(q, h, off + (size_t)(2 * kg + h) * V + gs);
                 }
                 return q;
             },
@@ -281,7 +343,7 @@ k_cnn_fused(int Nt, int Nx, int tilesX, int nNoise, float c0, const CgState *__r
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     const size_t idx = off + (size_t)(2 * kg + h) * V + gs;
-                    const float2 rv = q.r[h], av = q.a[h];
+                    const float2 av = q.a[h], rv = step_at(q, h, idx);
                     const float2 zv = make_float2(c0 * rv.x + sf * v[2 * h], c0 * rv.y + sf * v[2 * h + 1]);
                     z[idx] = zv;
                     acc.x += (double)(zv.x * rv.x) + (double)(zv.y * rv.y);
@@ -289,8 +351,14 @@ k_cnn_fused(int Nt, int Nx, int tilesX, int nNoise, float c0, const CgState *__r
                 }
             });
     }
-    acc = block_sum2<kCT>(acc, red);
-    if (threadIdx.x == 0) part[(size_t)sys * gridDim.x + blockIdx.x] = acc;
+    const size_t blk = (size_t)sys * gridDim.x + blockIdx.x;
+    if constexpr (UPD) {
+        __syncthreads();   // every thread has read the sums in red
+        store_pf_partials<kCT>(part + 2 * blk, acc.x, acc.y, rho, red);
+    } else {
+        acc = block_sum2<kCT>(acc, red2);
+        if (threadIdx.x == 0) part[blk] = acc;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -577,16 +645,27 @@ int cnn_gates(Ctx &c, int nrep) {
     return YCN_OK;
 }
 
-int cnn_apply(Ctx &c, int nsys, const CgState *st, const float2 *rs, const float2 *Ap, float2 *z, double2 *part) {
+template <bool UPD>
+static int launch_cnn(Ctx &c, int nsys, const float2 *rs, const float2 *Ap, float2 *z, double2 *part,
+                      const FcgUpdate &u) {
     const int tilesX = c.p.Nx / 16, tiles = (c.p.Nt / 16) * tilesX;
-    // read r_s, Ap, the gates of both layers; write z
-    prof_before(c, PK_CNN, (double)nsys * c.V * 160.0);
-    hipLaunchKernelGGL(k_cnn_fused, dim3(tiles, nsys), dim3(kCT), 0, c.stream, c.p.Nt, c.p.Nx, tilesX, c.nNoise,
-                       (float)cnn_c0(c), st, rs, Ap, (const _Float16 *)c.cnnGates, z, (const bf16x8 *)c.cnnF1,
-                       (const bf16x8 *)c.cnnF2, (const bf16x8 *)c.cnnF3, part);
-    prof_after(c, PK_CNN);
+    // read r_s, Ap, the gates of both layers; write z (and read p, x_s, write r_s, x_s)
+    const int kind = UPD && c.profTarget == PK_CG_UPDATE ? PK_CG_UPDATE : PK_CNN;
+    prof_before(c, kind, (double)nsys * c.V * (UPD ? 288.0 : 160.0));
+    hipLaunchKernelGGL(k_cnn_fused<UPD>, dim3(tiles, nsys), dim3(kCT), 0, c.stream, c.p.Nt, c.p.Nx, tilesX, c.nNoise,
+                       (float)cnn_c0(c), c.cg_d, rs, Ap, (const _Float16 *)c.cnnGates, z, (const bf16x8 *)c.cnnF1,
+                       (const bf16x8 *)c.cnnF2, (const bf16x8 *)c.cnnF3, part, u);
+    prof_after(c, kind);
     YCN_HIP(hipGetLastError());
     return tiles;
+}
+
+int cnn_apply(Ctx &c, int nsys, const float2 *rs, const float2 *Ap, float2 *z, double2 *part) {
+    return launch_cnn<false>(c, nsys, rs, Ap, z, part, FcgUpdate{});
+}
+
+int cnn_update_apply(Ctx &c, int nsys, const float2 *r, const FcgUpdate &u) {
+    return launch_cnn<true>(c, nsys, r, c.Aps, c.zs, c.partials, u);
 }
 
 // activations for training at lattice volume V: x0[8V] y1[16V] gm1[16V] u1[16V]

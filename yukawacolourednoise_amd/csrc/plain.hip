@@ -23,6 +23,8 @@
 
 namespace ycn {
 
+constexpr int kFcgNT = 448;   // of k_fcg_op: one entry of the tile with its halo per thread
+
 struct PlArgs {
     int Nt, Nx, V, nNoise;
     double r, d0, g;
@@ -180,6 +182,159 @@ k_pl_pf(PlArgs A, const R *__restrict__ phi, CgState *st, const typename Vec2<R>
     else
         second(Q32);
     store_pf_partials<NT>(part + 2 * ((size_t)sys * gridDim.x + blockIdx.x), mu, nu, rho, red);
+}
+
+// ---------------------------------------------------------------------------
+// flexible CG: the operator's launch
+// ---------------------------------------------------------------------------
+// Iteration i of a chunk of the flexible solver (Polak-Ribiere form, Notay, SIAM J. Sci. Comput. 22
+// (2000)) is two launches: this one, p' = z + beta p and Ap, and the network's (k_cnn_fused), which
+// takes alpha, updates x_s and r and makes the next z.  Each finalizes the other in its prologue.
+// From iteration i - 1's <z, r'>, <z, Ap> and |r'|^2 every block derives the same
+// beta = <z, r' - r> / <z_old, r> = -alpha <z, Ap> / rz_old and the same pause (at the stop or the
+// drop after an even number of iterations, at the cap; a reliable update follows).  Block 0 records
+// rz in ab[i & 1].y for the network's launch, or the pause.
+struct FcgStep {
+    double beta, rz;
+    bool off, pause;
+};
+__device__ __forceinline__ FcgStep fcg_decide(const Pf3 &s, double2 prev, int iter, const PfHead &S) {
+    FcgStep d;
+    d.off = !isfinite(s.mu) || !isfinite(s.nu);   // switches the network off
+    d.beta = d.off || !(prev.y > 0.0) ? 0.0 : -prev.x * s.nu / prev.y;
+    d.rz = d.off ? prev.y : s.mu;
+    const bool stop = !(sqrt(s.rho) > S.stop) || s.rho < kReliableDrop * kReliableDrop * S.rrRel;
+    d.pause = iter >= S.maxIter || (stop && !(iter & 1));
+    return d;
+}
+// the state after iteration number `iter`, for the reliable update; rhoPrev: |r|^2 before it
+__device__ __forceinline__ void fcg_commit(CgState &S, const Pf3 &s, double2 prev, const FcgStep &d, int iter,
+                                           int *active) {
+    S.iter = iter;
+    S.rr = s.rho;
+    S.alpha = make_double2(prev.x, 0.0);
+    S.rz_prev = prev.y;
+    S.rz = d.rz;
+    if (d.off) S.precOff = 1;
+    if (d.pause) {
+        S.done = 1;
+        atomicSub(active, 1);
+    }
+}
+
+// A block owns a 16 x 16 tile of one flavour's complex spinor (D keeps flavours and is real, so
+// the two planes are a packed spinor of their own: grid.y = system and flavour).
+template <bool WR1>
+__global__ void __launch_bounds__(kFcgNT)
+k_fcg_op(PlArgs A, const float *__restrict__ phi, CgState *st, const float2 *__restrict__ z,
+         const float2 *__restrict__ pold, float2 *__restrict__ pnew, float2 *__restrict__ Ap,
+         double *__restrict__ part, int idx, const double2 *__restrict__ cnnPart, int nbCnn, int *active) {
+    constexpr int TT = 16, TX = 16, NT = kFcgNT, H = TT + 4, W = TX + 4, N = H * W, M0 = (N + NT - 1) / NT;
+    __shared__ SpLds<float, N> P, Q;
+    __shared__ double red[3 * NT / kWave], bc[1];
+    __shared__ int pause;
+    const int sys = blockIdx.y >> 1;
+    const PfHead hd = pf_head(st[sys]);
+    const double rz0 = st[sys].rz;
+    const double2 prev = st[sys].ab[(idx - 1) & 1];
+    PfParts<NT> parts;
+    const double2 *const pp = cnnPart + 2 * (size_t)sys * nbCnn;
+    if (idx) parts.load(pp, nbCnn);
+    if (hd.done) return;
+    const unsigned V = (unsigned)A.V;
+    const size_t off = (size_t)blockIdx.y * 2 * V;
+    z += off;
+    pold += off;
+    pnew += off;
+    Ap += off;
+    const float *ph = phi + (size_t)(sys / A.nNoise) * V;
+    int tile = blockIdx.x;
+    if (A.xcdRemap) tile = (tile % 8) * (A.tilesPerSys / 8) + tile / 8;
+    const int ty = tile / A.tilesX, t0 = ty * TT, x0 = (tile - ty * A.tilesX) * TX;
+    Sp<float> p[M0], q[M0];
+    float d[M0];
+    unsigned g[M0];
+    int place[M0];   // as in k_pl_pf
+#pragma unroll
+    for (int u = 0; u < M0; ++u) {
+        const int i = threadIdx.x + u * NT;
+        place[u] = 0;
+        if (i < N) {
+            const int row = i / W, col = i - row * W;
+            const int gt = wrapi(t0 - 2 + row, A.Nt), gx = wrapi(x0 - 2 + col, A.Nx);
+            g[u] = (unsigned)(gt * A.Nx + gx);
+            const bool in1 = row >= 1 && row < H - 1 && col >= 1 && col < W - 1;
+            const bool in2 = row >= 2 && row < H - 2 && col >= 2 && col < W - 2;
+            place[u] = (in1 ? 1 : 0) | (in2 ? 2 : 0) | (gt == A.Nt - 1 ? 4 : 0) | (gt == 0 ? 8 : 0);
+            q[u] = load_sp<float>(z, V, g[u]);
+            p[u] = load_sp<float>(pold, V, g[u]);
+            d[u] = at(ph, g[u]);
+        }
+    }
+    double betaD = hd.beta, rz = rz0;
+    if (idx) {
+        const Pf3 s = parts.sum(pp, nbCnn, red);
+        if (threadIdx.x == 0) {
+            const FcgStep f = fcg_decide(s, prev, hd.iter0 + idx, hd);
+            bc[0] = f.beta;
+            pause = f.pause;
+            rz = f.rz;
+            if (blockIdx.x == 0 && !(blockIdx.y & 1)) {
+                if (f.pause)
+                    fcg_commit(st[sys], s, prev, f, hd.iter0 + idx, active);
+                else if (f.off)
+                    st[sys].precOff = 1;
+            }
+        }
+        __syncthreads();
+        if (pause) return;
+        betaD = bc[0];
+    }
+    if (blockIdx.x == 0 && !(blockIdx.y & 1) && threadIdx.x == 0) st[sys].ab[idx & 1].y = rz;
+    const float beta = (float)betaD;
+#pragma unroll
+    for (int u = 0; u < M0; ++u) {
+        const int i = threadIdx.x + u * NT;
+        if (i < N) {
+            d[u] = (float)A.d0 + (float)A.g * d[u];
+            p[u] = axpy<float>(q[u], beta, p[u]);
+            P.set(i, p[u]);
+            if (place[u] & 2) store_sp<float>(pnew, V, g[u], p[u]);
+        }
+    }
+    __syncthreads();
+    double mu = 0.0;
+#pragma unroll
+    for (int u = 0; u < M0; ++u)
+        if (place[u] & 1) {
+            const int i = threadIdx.x + u * NT;
+            q[u] = pl_dirac<float, false, WR1>((float)A.r, P, i, W, place[u] & 4 ? -1.f : 1.f,
+                                               place[u] & 8 ? -1.f : 1.f, d[u], p[u]);
+            Q.set(i, q[u]);
+            if (place[u] & 2) mu += sq(q[u]);
+        }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < M0; ++u)
+        if (place[u] & 2)
+            store_sp<float>(Ap, V, g[u],
+                            pl_dirac<float, true, WR1>((float)A.r, Q, threadIdx.x + u * NT, W,
+                                                       place[u] & 4 ? -1.f : 1.f, place[u] & 8 ? -1.f : 1.f, d[u],
+                                                       q[u]));
+    const double v = block_sum3<NT>(mu, 0.0, 0.0, red);
+    if (threadIdx.x == 0) part[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = v;
+}
+
+// after the last of a chunk's n iterations: its state, for the reliable update
+__global__ void __launch_bounds__(kPfNT)
+k_fcg_close(const double2 *__restrict__ cnnPart, int nb, int n, CgState *__restrict__ st, int *__restrict__ active) {
+    __shared__ double red[3 * kPfNT / kWave];
+    CgState &S = st[blockIdx.x];
+    const PfHead hd = pf_head(S);
+    const Pf3 s = sum_pf_partials<kPfNT>(cnnPart + 2 * (size_t)blockIdx.x * nb, nb, red);
+    if (hd.done || threadIdx.x) return;
+    const double2 prev = S.ab[(n - 1) & 1];
+    fcg_commit(S, s, prev, fcg_decide(s, prev, hd.iter0 + n, hd), hd.iter0 + n, active);
 }
 
 // ---------------------------------------------------------------------------
@@ -417,6 +572,42 @@ void p64_close(Ctx &c, int nsys) {
     hipLaunchKernelGGL(k_p64_close<false>, dim3((c.V + kPfNT - 1) / kPfNT, nsys), dim3(kPfNT), 0, c.stream, c.V,
                        (const CgState *)c.cg_d, c.x, c.pv[0], (const double2 *)c.pv[1], c.r, (const double2 *)nullptr,
                        (const double2 *)nullptr);
+}
+
+// iteration idx of a chunk of the flexible solver (see k_fcg_op): r and the directions alternate
+// between two buffers, both ways starting from the first
+int fcg_iteration(Ctx &c, int nsys, int idx) {
+    PlArgs A;
+    A.Nt = c.p.Nt;
+    A.Nx = c.p.Nx;
+    A.V = c.V;
+    A.nNoise = c.nNoise;
+    A.r = c.p.r;
+    A.d0 = 2.0 * c.p.r + c.p.M;
+    A.g = c.p.g;
+    A.tilesX = c.p.Nx / 16;
+    A.tilesPerSys = (c.p.Nt / 16) * A.tilesX;
+    A.xcdRemap = A.tilesPerSys % 8 == 0 ? 1 : 0;
+    const int par = idx & 1, tiles = A.tilesPerSys;
+    double *const opPart = reinterpret_cast<double *>(c.partials + (size_t)2 * nsys * tiles);
+    prof_before(c, PK_NORMAL_OP, (double)nsys * c.V * (4 * 32 + 4));
+    auto *k = A.r == 1.0 ? &k_fcg_op<true> : &k_fcg_op<false>;
+    hipLaunchKernelGGL(k, dim3(tiles, 2 * nsys), dim3(kFcgNT), 0, c.stream, A, (const float *)c.phis, c.cg_d,
+                       (const float2 *)c.zs, (const float2 *)c.ps[par], c.ps[par ^ 1], c.Aps, opPart, idx,
+                       (const double2 *)c.partials, tiles, c.active);
+    prof_after(c, PK_NORMAL_OP);
+    FcgUpdate u;
+    u.rnew = par ? c.rs : c.pfA1;
+    u.p = c.ps[par ^ 1];
+    u.xs = c.xs;
+    u.opPart = opPart;
+    u.nbOp = 2 * tiles;
+    u.idx = idx;
+    return cnn_update_apply(c, nsys, par ? c.pfA1 : c.rs, u);
+}
+void fcg_close(Ctx &c, int nsys, int n) {
+    hipLaunchKernelGGL(k_fcg_close, dim3(nsys), dim3(kPfNT), 0, c.stream, (const double2 *)c.partials,
+                       (c.p.Nt / 16) * (c.p.Nx / 16), n, c.cg_d, c.active);
 }
 
 }  // namespace ycn
