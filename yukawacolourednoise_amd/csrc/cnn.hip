@@ -39,7 +39,8 @@
 
 namespace ycn {
 
-constexpr int kCT = 256;   // threads per CNN block (4 waves)
+constexpr int kCT = 256;    // threads per block of the training and gate kernels (4 waves)
+constexpr int kOneBlockTiles = 256;   // blocks that have a compute unit each
 
 __device__ __forceinline__ int wrapn(int a, int n) { return a < 0 ? a + n : (a >= n ? a - n : a); }
 
@@ -89,39 +90,38 @@ __global__ void k_make_frags(const float *__restrict__ W, bf16x8 *__restrict__ f
 // One layer on the LDS-resident tile: out[m][n] = sum_k in[site(m) + off(tap)][ci] W[k][n]
 // for the WOUT x WOUT output sites m (input array width WIN, one more site of halo on
 // each side).  The MFMA runs transposed, D[n][m] = sum_k W[k][n] A[m][k]: the weight
-// fragments are its first operand, the activations its second, so a lane ends with four
+// fragments B are its first operand, the activations its second, so a lane ends with four
 // consecutive channels 4 kg .. 4 kg + 3 of one site m = 16 g + col and stores them with
 // one access.  Each lane's tap offsets are fixed for the layer (kg picks them); padded K
 // steps load the centre tap (finite activations against zero weights) instead of
-// branching.  pre(m, kg) runs before a group's MFMAs (its global loads overlap them) and
-// store(m, kg, acc, pre's result) gets the four channels.
-template <int CIN, int WOUT, int WIN, int KS, typename Pre, typename Store>
-__device__ __forceinline__ void conv_lds(const __bf16 *__restrict__ in, const bf16x8 *__restrict__ frag, Pre pre,
-                                         Store store) {
-    constexpr int N = WOUT * WOUT;
-    constexpr int G = (N + 15) / 16;
+// branching.  Wave w of FW takes the groups of sites w, w + FW, ...; pre(round) runs before a group's MFMAs and
+// store(round, m, kg, acc, pre's result) gets the four channels.
+constexpr int conv_rounds(int wout, int fw) { return ((wout * wout + 15) / 16 + fw - 1) / fw; }
+template <int FW, int CIN, int WOUT, int WIN, int KS, typename Pre, typename Store>
+__device__ __forceinline__ void conv_lds(const __bf16 *__restrict__ in, const bf16x8 (&B)[KS], Pre pre, Store store) {
+    constexpr int N = WOUT * WOUT, G = (N + 15) / 16;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int kg = lane >> 4, col = lane & 15;
-    bf16x8 B[KS];   // this lane's weight fragments, held for all of the wave's site groups
     int toff[KS];   // LDS offset of this lane's tap and channel block from its site's corner
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-        B[ks] = frag[ks * 64 + lane];
         const int k0 = ks * 32 + kg * 8;
         const int tap = k0 / CIN, ci0 = k0 % CIN;
         toff[ks] = tap < 9 ? ((tap / 3) * WIN + tap % 3) * CIN + ci0 : (WIN + 1) * CIN;
     }
-    for (int g = wave; g < G; g += kCT / 64) {
-        const int m = g * 16 + col;
+#pragma unroll
+    for (int round = 0; round < conv_rounds(WOUT, FW); ++round) {
+        const int g = wave + round * FW, m = g * 16 + col;
+        if (g >= G) break;
         const int mc = m < N ? m : N - 1;
         const int a = mc / WOUT, b = mc - a * WOUT;
         const __bf16 *base = in + (a * WIN + b) * CIN;
-        const auto pl = pre(mc, kg);
+        const auto pl = pre(round);
         f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
             acc = mfma_bf16(B[ks], *reinterpret_cast<const bf16x8 *>(base + toff[ks]), acc);
-        if (m < N) store(m, kg, acc, pl);
+        if (m < N) store(round, m, kg, acc, pl);
     }
 }
 
@@ -176,187 +176,202 @@ k_cnn_gates(int Nt, int Nx, const float *__restrict__ phis, float g, const float
 // the network is switched off.  The network's input is scaled by |r| where the chunk began: the
 // scale cancels, and bf16 keeps its relative precision.
 // UPD = false: z = CNN(r) and the partials (<z, r>, <z, Ap>).
-// What bounds it: the latency of three layers of MFMAs on one block of four waves per compute unit
-// (256 x 256: 256 blocks).  An iteration of the flexible solver took 35 us there in six launches
-// (operator, alpha, update, beta, network, rz) and takes 25 in the two.
-template <bool UPD>
-__global__ void __launch_bounds__(kCT)
+// What bounds it where every block has a compute unit to itself (256 x 256: 256 blocks): latency, the
+// loads, three layers of a few MFMAs with a barrier each, the sums.  FW = 8 waves have 4, 3 and 2
+// groups of sites each, and everything that they read from memory (inputs, gates, weights, the
+// vectors of the update) is requested at the start.  On larger lattices other blocks cover the
+// latency and registers cost occupancy: FW = 4, each group's loads before its MFMAs.  An iteration
+// of the flexible solver: 256 x 256 19.9 us with 8 waves, 20.7 with 16, 23.0 with 4 loading late;
+// 512 x 512 52.3, 54.1 and 44.4; 1024 x 1024 276, 266 and 211.
+template <bool UPD, int FW>
+__global__ void __launch_bounds__(64 * FW)
 k_cnn_fused(int Nt, int Nx, int tilesX, int nNoise, float c0, CgState *__restrict__ st,
             const float2 *__restrict__ rs, const float2 *__restrict__ Ap, const _Float16 *__restrict__ gates,
             float2 *__restrict__ z, const bf16x8 *__restrict__ gf1, const bf16x8 *__restrict__ gf2,
             const bf16x8 *__restrict__ gf3, double2 *__restrict__ part, FcgUpdate upd) {
-    constexpr int W0 = 22, W1 = 20, W2 = 18, W3 = 16;
+    constexpr int W0 = 22, W1 = 20, W2 = 18, W3 = 16, kFT = 64 * FW;
+    constexpr int R1 = conv_rounds(W1, FW), R2 = conv_rounds(W2, FW), R3 = conv_rounds(W3, FW);
+    constexpr int E = 1024 / kFT;
+    constexpr bool EARLY = FW > 4;
+    typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+    typedef __bf16 b4 __attribute__((ext_vector_type(4)));
     __shared__ __attribute__((aligned(16))) __bf16 U0[W0 * W0 * 8];
     __shared__ __attribute__((aligned(16))) __bf16 U1[W1 * W1 * 16];
     __shared__ __attribute__((aligned(16))) __bf16 U2[W2 * W2 * 16];
-    __shared__ double2 red2[UPD ? 1 : kCT / kWave];
-    __shared__ double red[3 * kCT / kWave];
-    const int sys = blockIdx.y;
+    __shared__ double2 red2[UPD ? 1 : FW];
+    __shared__ double red[3 * FW];
+    const int sys = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     double opSum = 0.0;
     if constexpr (UPD)
-        for (int k = threadIdx.x; k < upd.nbOp; k += kCT) opSum += upd.opPart[(size_t)sys * upd.nbOp + k];
+        for (int k = tid; k < upd.nbOp; k += kFT) opSum += upd.opPart[(size_t)sys * upd.nbOp + k];
     const double rz = UPD ? st[sys].ab[upd.idx & 1].y : 0.0;
+    const double rr = st[sys].rr;
+    bool identity = st[sys].precOff;
     if (st[sys].done) return;
     const int V = Nt * Nx;
     const size_t off = (size_t)sys * 4 * V;
     const int tile = blockIdx.x;
     const int ty = tile / tilesX, tx = tile - ty * tilesX;
     const int t0 = ty * 16, x0 = tx * 16;
-    const double s = sqrt(st[sys].rr / (8.0 * (double)V));
-    const float inv = s > 0.0 ? (float)(1.0 / s) : 0.f, sf = (float)s;
-    double2 acc = make_double2(0.0, 0.0);
-    double rho = 0.0;
-    bool identity = st[sys].precOff;
-    float alpha = 0.f;
-    auto take_alpha = [&] {   // by all threads, after their first loads are issued
-        if constexpr (UPD) {
-            const double w = wave_sum(opSum);
-            if ((threadIdx.x & (kWave - 1)) == 0) red[threadIdx.x / kWave] = w;
-            __syncthreads();
-            double dot = red[0];
+
+    // inputs: entries of the tile with its 3-site halo, two of the four components each
+    float2 r0[E][2], a0[E][2];
+    auto entry = [&](int u, int &e, int &eh) {
+        e = (tid + u * kFT) & 511;
+        eh = (tid + u * kFT) >> 9;
+        return e < W0 * W0;
+    };
 #pragma unroll
-            for (int k = 1; k < kCT / kWave; ++k) dot += red[k];
-            const bool step = dot > 0.0 && isfinite(rz) && rz > 0.0;
-            const double al = step ? rz / dot : 0.0;
-            if (!step) identity = true;
-            alpha = (float)al;
-            if (blockIdx.x == 0 && threadIdx.x == 0) {
-                st[sys].ab[upd.idx & 1].x = al;
-                if (!step) st[sys].precOff = 1;
-            }
-        }
-    };
-    // r' of entry idx (component planes and site) and the x_s update there
-    struct RA {
-        float2 r[2], a[2], p[2], x[2];
-    };
-    auto load_ra = [&](RA &q, int h, size_t idx) {
-        q.r[h] = rs[idx];
-        q.a[h] = Ap[idx];
-        if constexpr (UPD) {
-            q.p[h] = upd.p[idx];
-            q.x[h] = upd.xs[idx];
-        }
-    };
-    auto step_at = [&](const RA &q, int h, size_t idx) {
-        const float2 r = q.r[h], a = q.a[h];
-        const float2 rn = make_float2(r.x - alpha * a.x, r.y - alpha * a.y);
-        if constexpr (UPD) {
-            const float2 p = q.p[h], x = q.x[h];
-            upd.rnew[idx] = rn;
-            upd.xs[idx] = make_float2(x.x + alpha * p.x, x.y + alpha * p.y);
-            rho += (double)(rn.x * rn.x + rn.y * rn.y);
-        }
-        return rn;
-    };
-    // a thread's inputs: entries of the tile with its 3-site halo
-    constexpr int L0 = (W0 * W0 + kCT - 1) / kCT;
-    float2 rv0[L0][4], av0[L0][4];
+    for (int u = 0; u < E; ++u) {
+        int e, eh;
+        if (!entry(u, e, eh)) continue;
+        const int a = e / W0, b = e - a * W0;
+        const size_t gs = (size_t)wrapn(t0 - 3 + a, Nt) * Nx + wrapn(x0 - 3 + b, Nx);
 #pragma unroll
-    for (int u = 0; u < L0; ++u) {
-        const int w = threadIdx.x + u * kCT;
-        if (w < W0 * W0) {
-            const int a = w / W0, b = w - a * W0;
-            const size_t gs = (size_t)wrapn(t0 - 3 + a, Nt) * Nx + wrapn(x0 - 3 + b, Nx);
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                rv0[u][c] = rs[off + c * V + gs];
-                if (UPD) av0[u][c] = Ap[off + c * V + gs];
-            }
+        for (int h = 0; h < 2; ++h) {
+            r0[u][h] = rs[off + (2 * eh + h) * V + gs];
+            if (UPD) a0[u][h] = Ap[off + (2 * eh + h) * V + gs];
         }
     }
-    take_alpha();
-    if (identity) {
-        // plain CG fallback: identity preconditioner z = r_s
-        const int lt = threadIdx.x / 16, lx = threadIdx.x % 16;
-        const size_t gs = (size_t)(t0 + lt) * Nx + x0 + lx;
+    // hidden layers: the lane's four gates of site m of a W x W array whose corner is lattice
+    // site (t0 - o, x0 - o): halves `half` .. half + 15 of the site's 32 in the per-solve array
+    const _Float16 *gr = gates + (size_t)(sys / nNoise) * V * 32;
+    const int kg = lane >> 4, col = lane & 15;
+    auto gate_of = [&](int W, int o, int half, int round) {
+        const int m = min((wave + round * FW) * 16 + col, W * W - 1), a = m / W, b = m - a * W;
+        const size_t gs = (size_t)wrapn(t0 - o + a, Nt) * Nx + wrapn(x0 - o + b, Nx);
+        return *reinterpret_cast<const h4 *>(gr + gs * 32 + half + 4 * kg);
+    };
+    h4 g1[R1], g2[R2];
+    bf16x8 B1[ksteps(8)], B2[ksteps(16)], B3[ksteps(16)];   // this lane's weight fragments
+    auto weights = [&](const bf16x8 *w, auto &B) {
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            RA q;
-            load_ra(q, 0, off + c * V + gs);
-            const float2 av = q.a[0], rv = step_at(q, 0, off + c * V + gs);
-            z[off + c * V + gs] = rv;
-            acc.x += (double)(rv.x * rv.x + rv.y * rv.y);
-            acc.y += (double)(rv.x * av.x + rv.y * av.y);
+        for (int k = 0; k < (int)(sizeof(B) / sizeof(B[0])); ++k) B[k] = w[k * 64 + lane];
+    };
+    if constexpr (EARLY) {
+#pragma unroll
+        for (int q = 0; q < R1; ++q) g1[q] = gate_of(W1, 2, 0, q);
+#pragma unroll
+        for (int q = 0; q < R2; ++q) g2[q] = gate_of(W2, 1, 16, q);
+        weights(gf1, B1);
+        weights(gf2, B2);
+        weights(gf3, B3);
+    }
+    // output layer: rows wave, wave + FW, ... of the tile, 8 channels: lanes kg = 0, 1 hold
+    // components 2 kg, 2 kg + 1 of site col
+    static_assert(W3 == 16 && 16 % FW == 0, "a group of sites is a row of the tile");
+    struct RA {
+        float2 r[2], a[2], p[2], x[2];
+    } ra[R3];
+    const size_t own = off + (size_t)(t0 + wave) * Nx + x0 + col;
+    auto load_own = [&](int q) {
+        RA v{};
+        if (kg < 2)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const size_t idx = own + (size_t)(2 * kg + h) * V + (size_t)(q * FW) * Nx;
+                v.r[h] = rs[idx];
+                v.a[h] = Ap[idx];
+                if constexpr (UPD) {
+                    v.p[h] = upd.p[idx];
+                    v.x[h] = upd.xs[idx];
+                }
+            }
+        return v;
+    };
+    if constexpr (EARLY)
+#pragma unroll
+        for (int q = 0; q < R3; ++q) ra[q] = load_own(q);
+
+    const double s = sqrt(rr / (8.0 * (double)V));
+    const float inv = s > 0.0 ? (float)(1.0 / s) : 0.f, sf = (float)s;
+    float alpha = 0.f;
+    if constexpr (UPD) {
+        const double w = wave_sum(opSum);
+        if (lane == 0) red[wave] = w;
+        __syncthreads();
+        const double dot = row_sum(col < FW ? red[col] : 0.0);
+        const bool step = dot > 0.0 && isfinite(rz) && rz > 0.0;
+        const double al = step ? rz / dot : 0.0;
+        if (!step) identity = true;
+        alpha = (float)al;
+        if (blockIdx.x == 0 && tid == 0) {
+            st[sys].ab[upd.idx & 1].x = al;
+            if (!step) st[sys].precOff = 1;
+        }
+    }
+    double2 acc = make_double2(0.0, 0.0);
+    double rho = 0.0;
+    // z of component 2 kg + h at the lane's own site, from r' there (and the x_s update)
+    auto finish = [&](const RA &v, int q, int h, float2 net) {
+        const size_t idx = own + (size_t)(2 * kg + h) * V + (size_t)(q * FW) * Nx;
+        const float2 av = v.a[h], rv = make_float2(v.r[h].x - alpha * av.x, v.r[h].y - alpha * av.y);
+        const float2 zv = identity ? rv : make_float2(c0 * rv.x + sf * net.x, c0 * rv.y + sf * net.y);
+        z[idx] = zv;
+        acc.x += (double)(zv.x * rv.x) + (double)(zv.y * rv.y);
+        acc.y += (double)(zv.x * av.x) + (double)(zv.y * av.y);
+        if constexpr (UPD) {
+            upd.rnew[idx] = rv;
+            upd.xs[idx] = make_float2(v.x[h].x + alpha * v.p[h].x, v.x[h].y + alpha * v.p[h].y);
+            rho += (double)(rv.x * rv.x + rv.y * rv.y);
+        }
+    };
+    if (identity) {   // plain CG fallback: identity preconditioner z = r_s
+#pragma unroll
+        for (int q = 0; q < R3; ++q) {
+            const RA v = EARLY ? ra[q] : load_own(q);
+            if (kg < 2)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) finish(v, q, h, make_float2(0.f, 0.f));
         }
     } else {
-        const _Float16 *gr = gates + (size_t)(sys / nNoise) * V * 32;
 #pragma unroll
-        for (int u = 0; u < L0; ++u) {
-            const int w = threadIdx.x + u * kCT;
-            if (w < W0 * W0) {
-                bf16x8 q;
+        for (int u = 0; u < E; ++u) {
+            int e, eh;
+            if (!entry(u, e, eh)) continue;
+            b4 q;
 #pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    float2 rv = rv0[u][c];
-                    if (UPD) rv = make_float2(rv.x - alpha * av0[u][c].x, rv.y - alpha * av0[u][c].y);
-                    q[2 * c] = (__bf16)(rv.x * inv);
-                    q[2 * c + 1] = (__bf16)(rv.y * inv);
-                }
-                *reinterpret_cast<bf16x8 *>(U0 + w * 8) = q;
+            for (int h = 0; h < 2; ++h) {
+                float2 rv = r0[u][h];
+                if (UPD) rv = make_float2(rv.x - alpha * a0[u][h].x, rv.y - alpha * a0[u][h].y);
+                q[2 * h] = (__bf16)(rv.x * inv);
+                q[2 * h + 1] = (__bf16)(rv.y * inv);
             }
+            *reinterpret_cast<b4 *>(U0 + e * 8 + 4 * eh) = q;
         }
         __syncthreads();
-        typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-        typedef __bf16 b4 __attribute__((ext_vector_type(4)));
-        // hidden layers: the lane's four gates of site m of a W x W array whose corner is
-        // lattice site (t0 - o, x0 - o), read from the per-solve gate array (halves
-        // `half` .. half + 15 of the site's 32) before the group's MFMAs; the four gated
-        // channels go to LDS with one 8-byte store
-        auto gate_of = [&](int W, int o, int half, int m, int kg) {
-            const int a = m / W, b = m - a * W;
-            const size_t gs = (size_t)wrapn(t0 - o + a, Nt) * Nx + wrapn(x0 - o + b, Nx);
-            return *reinterpret_cast<const h4 *>(gr + gs * 32 + half + 4 * kg);
-        };
-        auto gated = [&](__bf16 *U, int m, int kg, f32x4 v, h4 gt) {
+        // the four gated channels go to LDS with one 8-byte store
+        auto gated = [&](__bf16 *U, int m, int k, f32x4 v, h4 gt) {
             b4 o;
 #pragma unroll
             for (int i = 0; i < 4; ++i) o[i] = (__bf16)(v[i] * (float)gt[i]);
-            *reinterpret_cast<b4 *>(U + m * 16 + 4 * kg) = o;
+            *reinterpret_cast<b4 *>(U + m * 16 + 4 * k) = o;
         };
-        conv_lds<8, W1, W0, ksteps(8)>(
-            U0, gf1, [&](int m, int kg) { return gate_of(W1, 2, 0, m, kg); },
-            [&](int m, int kg, f32x4 v, h4 gt) { gated(U1, m, kg, v, gt); });
+        if constexpr (!EARLY) weights(gf1, B1);
+        conv_lds<FW, 8, W1, W0>(
+            U0, B1, [&](int q) { return EARLY ? g1[q] : gate_of(W1, 2, 0, q); },
+            [&](int, int m, int k, f32x4 v, h4 gt) { gated(U1, m, k, v, gt); });
         __syncthreads();
-        conv_lds<16, W2, W1, ksteps(16)>(
-            U1, gf2, [&](int m, int kg) { return gate_of(W2, 1, 16, m, kg); },
-            [&](int m, int kg, f32x4 v, h4 gt) { gated(U2, m, kg, v, gt); });
+        if constexpr (!EARLY) weights(gf2, B2);
+        conv_lds<FW, 16, W2, W1>(
+            U1, B2, [&](int q) { return EARLY ? g2[q] : gate_of(W2, 1, 16, q); },
+            [&](int, int m, int k, f32x4 v, h4 gt) { gated(U2, m, k, v, gt); });
         __syncthreads();
-        // output layer (8 channels: lanes kg = 0, 1 hold spinor components 2 kg, 2 kg + 1);
-        // r_s and Ap (and p, x_s) of the lane's two components are loaded before the group's MFMAs
-        conv_lds<16, W3, W2, ksteps(16)>(
-            U2, gf3,
-            [&](int m, int kg) {
-                RA q{};
-                if (kg < 2) {
-                    const int a = m / W3, b = m - a * W3;
-                    const size_t gs = (size_t)(t0 + a) * Nx + x0 + b;
+        if constexpr (!EARLY) weights(gf3, B3);
+        conv_lds<FW, 16, W3, W2>(
+            U2, B3, [&](int q) { return EARLY ? ra[q] : load_own(q); },
+            [&](int q, int, int k, f32x4 v, const RA &w) {
+                if (k >= 2) return;
 #pragma unroll
-                    for (int h = 0; h < 2; ++h) load_ra(q, h, off + (size_t)(2 * kg + h) * V + gs);
-                }
-                return q;
-            },
-            [&](int m, int kg, f32x4 v, const RA &q) {
-                if (kg >= 2) return;
-                const int a = m / W3, b = m - a * W3;
-                const size_t gs = (size_t)(t0 + a) * Nx + x0 + b;
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const size_t idx = off + (size_t)(2 * kg + h) * V + gs;
-                    const float2 av = q.a[h], rv = step_at(q, h, idx);
-                    const float2 zv = make_float2(c0 * rv.x + sf * v[2 * h], c0 * rv.y + sf * v[2 * h + 1]);
-                    z[idx] = zv;
-                    acc.x += (double)(zv.x * rv.x) + (double)(zv.y * rv.y);
-                    acc.y += (double)(zv.x * av.x) + (double)(zv.y * av.y);
-                }
+                for (int h = 0; h < 2; ++h) finish(w, q, h, make_float2(v[2 * h], v[2 * h + 1]));
             });
     }
     const size_t blk = (size_t)sys * gridDim.x + blockIdx.x;
     if constexpr (UPD) {
         __syncthreads();   // every thread has read the sums in red
-        store_pf_partials<kCT>(part + 2 * blk, acc.x, acc.y, rho, red);
+        store_pf_partials<kFT>(part + 2 * blk, acc.x, acc.y, rho, red);
     } else {
-        acc = block_sum2<kCT>(acc, red2);
+        acc = block_sum2<kFT>(acc, red2);
         if (threadIdx.x == 0) part[blk] = acc;
     }
 }
@@ -652,9 +667,16 @@ static int launch_cnn(Ctx &c, int nsys, const float2 *rs, const float2 *Ap, floa
     // read r_s, Ap, the gates of both layers; write z (and read p, x_s, write r_s, x_s)
     const int kind = UPD && c.profTarget == PK_CG_UPDATE ? PK_CG_UPDATE : PK_CNN;
     prof_before(c, kind, (double)nsys * c.V * (UPD ? 288.0 : 160.0));
-    hipLaunchKernelGGL(k_cnn_fused<UPD>, dim3(tiles, nsys), dim3(kCT), 0, c.stream, c.p.Nt, c.p.Nx, tilesX, c.nNoise,
-                       (float)cnn_c0(c), c.cg_d, rs, Ap, (const _Float16 *)c.cnnGates, z, (const bf16x8 *)c.cnnF1,
-                       (const bf16x8 *)c.cnnF2, (const bf16x8 *)c.cnnF3, part, u);
+    auto go = [&](auto fw) {
+        constexpr int FW = decltype(fw)::value;
+        hipLaunchKernelGGL((k_cnn_fused<UPD, FW>), dim3(tiles, nsys), dim3(64 * FW), 0, c.stream, c.p.Nt, c.p.Nx, tilesX,
+                           c.nNoise, (float)cnn_c0(c), c.cg_d, rs, Ap, (const _Float16 *)c.cnnGates, z,
+                           (const bf16x8 *)c.cnnF1, (const bf16x8 *)c.cnnF2, (const bf16x8 *)c.cnnF3, part, u);
+    };
+    if (tiles * nsys <= kOneBlockTiles)
+        go(std::integral_constant<int, 8>());
+    else
+        go(std::integral_constant<int, 4>());
     prof_after(c, kind);
     YCN_HIP(hipGetLastError());
     return tiles;
