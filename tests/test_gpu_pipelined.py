@@ -14,9 +14,9 @@ TILES = [(4, 16), (8, 32), (16, 16), (16, 32), (32, 32), (8, 64), (16, 64)]
 
 
 def extents(tile, scale):
-    """scale tiles each way; scale 0: two tiles and a part in time, one and a part in space."""
-    TT, TX = TILES[tile]
-    return (scale * TT, scale * TX) if scale else (2 * TT + 3, TX + 1)
+    """scale tiles each way; scale 0: two tiles and a part in time, one and a small part in space."""
+    TT, TX = (TILES + RC_TILES)[tile]
+    return (scale * TT, scale * TX) if scale else (2 * TT + 3, TX + (1 if tile < len(TILES) else 3))
 
 
 @pytest.mark.parametrize("fin", ["fused", "separate"])
@@ -74,8 +74,12 @@ def test_measured_correlator(gpu, monkeypatch):
     assert rel(corr, O.correlator(orc, phi)[0]) < 1e-9
 
 
+# the FP64 tiles that compute A p again instead of storing it
+RC_TILES = [(16, 32), (32, 32), (16, 64)]
+
+
 @pytest.mark.parametrize("fin", ["fused", "separate"])
-@pytest.mark.parametrize("tile", range(len(TILES)))
+@pytest.mark.parametrize("tile", range(len(TILES) + len(RC_TILES)))
 @pytest.mark.parametrize("scale,r,cap", [(1, 0.7, 13), (0, 1.0, 12), (0, 0.7, 1), (2, 1.0, 26)])
 def test_fp64_every_tile(gpu, monkeypatch, tile, fin, scale, r, cap):
     """Fixed iteration counts: the oracle's count, and its iterate to rounding."""
@@ -87,6 +91,8 @@ def test_fp64_every_tile(gpu, monkeypatch, tile, fin, scale, r, cap):
     p, orc = mk(Y, Nt=Nt, Nx=Nx, r=r, nNoise=2, cgTol=0.0, cgTolMode=0, cgMaxIter=cap)
     phi = 1.0 + O.hot_start(Nt + Nx, Nt, Nx)
     with Y.Context(p) as c:
+        name = "%dx%d%s " % ((TILES + RC_TILES)[tile] + ("r" if tile >= len(TILES) else "",))
+        assert name in c.tuning_report().split("fp64 pipelined tiles")[1]
         c.set_field(phi)
         d, st = c.fermion_force(3)
     dr, sr = O.fermion_drift(orc, phi, 3)

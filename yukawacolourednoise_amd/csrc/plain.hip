@@ -13,7 +13,7 @@
 // What bounds it: at 512 x 512 in FP32 the vectors stay in the caches and a launch is latency,
 // its chain of partial sums, loads, two stencil stages and a reduction.  At 1024 x 1024 in FP64
 // it moves 210 MB per launch out of the 256 MB last-level cache; an iteration takes 40 us there
-// against 68 us for the four launches.
+// against 68 us for the four launches, 35 without A p in memory (k_pl_rc).
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -184,6 +184,130 @@ k_pl_pf(PlArgs A, const R *__restrict__ phi, CgState *st, const typename Vec2<R>
     store_pf_partials<NT>(part + 2 * ((size_t)sys * gridDim.x + blockIdx.x), mu, nu, rho, red);
 }
 
+// The same launch (after the first of a phase) without A p in memory: p_{idx-1} is read with a
+// 4-site halo and A p_{idx-1} computed again, by the same operations that gave its alpha, on the
+// 2-site halo.  FP64 on lattices that fill the chip is bound by the last-level cache and has vector
+// instructions to spare: per site and launch p_{idx-2}, p_{idx-1}, p and phi (104 B) and every
+// other launch x (64 B more), against 168 and 232 B.  One array in LDS, two barriers per stage.
+// Per iteration, 1024 x 1024 in a solve: 35 us (16x32 tiles, 512 threads) against 38, for 136 MB
+// against 202; 512 x 512: 10.4 (32x32, 832 threads) against 11.4; at 256 x 256 the longer chain
+// costs more than the traffic, 6.4 against 5.6.
+template <typename R, int TT, int TX, int NT, bool DAG1, bool WR1, int XM>
+__global__ void __launch_bounds__(NT)
+k_pl_rc(PlArgs A, const R *__restrict__ phi, CgState *st, const typename Vec2<R>::T *__restrict__ pprev,
+        const typename Vec2<R>::T *__restrict__ pold, typename Vec2<R>::T *__restrict__ pnew,
+        typename Vec2<R>::T *__restrict__ xs, double2 *__restrict__ part, int finMode, int idx,
+        const double2 *__restrict__ prevPart, int *active) {
+    constexpr int H = TT + 8, W = TX + 8, N = H * W, M0 = (N + NT - 1) / NT;
+    __shared__ SpLds<R, N> P;
+    __shared__ double red[3 * NT / kWave], bc[2];
+    __shared__ int pause;
+    const int sys = blockIdx.y;
+    const PfHead hd = pf_head(st[sys]);
+    const double2 prev = st[sys].ab[(idx - 1) & 1];
+    PfParts<NT> parts;
+    if (finMode && idx) parts.load(prevPart + 2 * (size_t)sys * gridDim.x, (int)gridDim.x);
+    if (hd.done) return;
+    const unsigned V = (unsigned)A.V;
+    const size_t off = (size_t)sys * 2 * V;
+    pprev += off;
+    pold += off;
+    pnew += off;
+    xs += off;
+    const R *ph = phi + (size_t)(sys / A.nNoise) * V;
+    int tile = blockIdx.x;   // contiguous bands of tiles per XCD
+    if (A.xcdRemap) tile = (tile % 8) * (A.tilesPerSys / 8) + tile / 8;
+    const int ty = tile / A.tilesX, t0 = ty * TT, x0 = (tile - ty * A.tilesX) * TX;
+    const int rowEnd = min(TT, A.Nt - t0) + 4, colEnd = min(TX, A.Nx - x0) + 4;
+
+    // an entry's place: 1 = the tile's own; 2, 16, 32 = within the 1-, 2-, 3-site halo; 4, 8: the
+    // hops across the time boundary, forward and backward
+    Sp<R> p[M0], q[M0], x[M0];
+    R d[M0];
+    unsigned g[M0];
+    int place[M0];
+#pragma unroll
+    for (int u = 0; u < M0; ++u) {
+        const int i = threadIdx.x + u * NT;
+        place[u] = 0;
+        if (i < N) {
+            const int row = i / W, col = i - row * W;
+            const int gt = wrapi(t0 - 4 + row, A.Nt), gx = wrapi(x0 - 4 + col, A.Nx);
+            g[u] = (unsigned)(gt * A.Nx + gx);
+            auto in = [&](int h) { return row >= h && row < H - h && col >= h && col < W - h; };
+            const bool own = row >= 4 && row < rowEnd && col >= 4 && col < colEnd;
+            place[u] = (own ? 1 : 0) | (in(3) ? 2 : 0) | (in(2) ? 16 : 0) | (in(1) ? 32 : 0) |
+                       (gt == A.Nt - 1 ? 4 : 0) | (gt == 0 ? 8 : 0);
+            p[u] = load_sp<R>(pold, V, g[u]);
+            if (in(2)) q[u] = load_sp<R>(pprev, V, g[u]);
+            if (XM != 0 && own) x[u] = load_sp<R>(xs, V, g[u]);
+            d[u] = at(ph, g[u]);
+        }
+    }
+    double alphaD, betaD;
+    if (!p64_prologue<NT>(st, hd, sys, idx, finMode, parts, prevPart, active, red, bc, &pause, alphaD, betaD)) return;
+    if (blockIdx.x == 0 && threadIdx.x == 0) st[sys].ab[idx & 1] = make_double2(alphaD, betaD);
+    const R alpha = (R)alphaD, beta = (R)betaD, alphaPrev = (R)prev.x, betaPrev = (R)prev.y;
+    const R wr = (R)A.r;
+    auto dirac = [&](auto dag, int u, Sp<R> v) {
+        return pl_dirac<R, decltype(dag)::value, WR1>(wr, P, threadIdx.x + u * NT, W, place[u] & 4 ? (R)-1 : (R)1,
+                                                      place[u] & 8 ? (R)-1 : (R)1, d[u], v);
+    };
+    using First = std::integral_constant<bool, DAG1>;
+    using Second = std::integral_constant<bool, !DAG1>;
+    // v of the entries at `bit` into the array, once every thread has read what it holds
+    auto put = [&](int bit, const Sp<R> (&v)[M0]) {
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < M0; ++u)
+            if (place[u] & bit) P.set(threadIdx.x + u * NT, v[u]);
+        __syncthreads();
+    };
+
+    double rho = 0.0, mu = 0.0, nu = 0.0;
+#pragma unroll
+    for (int u = 0; u < M0; ++u) {
+        const int i = threadIdx.x + u * NT;
+        if (i < N) {
+            d[u] = (R)A.d0 + (R)A.g * d[u];
+            P.set(i, p[u]);
+            if (place[u] & 16) {
+                if (XM == 2 && (place[u] & 1))
+                    store_sp<R>(xs, V, g[u], axpy<R>(axpy<R>(x[u], alphaPrev, q[u]), alpha, p[u]));
+                q[u] = axpy<R>(p[u], -betaPrev, q[u]);   // r_{idx-1}
+            }
+        }
+    }
+    __syncthreads();
+    Sp<R> v[M0];
+#pragma unroll
+    for (int u = 0; u < M0; ++u)
+        if (place[u] & 32) v[u] = dirac(First(), u, p[u]);
+    put(32, v);
+#pragma unroll
+    for (int u = 0; u < M0; ++u)
+        if (place[u] & 16) {
+            const Sp<R> r = axpy<R>(q[u], -alpha, dirac(Second(), u, v[u]));
+            p[u] = axpy<R>(r, beta, p[u]);
+            if (place[u] & 1) {
+                rho += sq(r);
+                store_sp<R>(pnew, V, g[u], p[u]);
+            }
+        }
+    put(16, p);
+#pragma unroll
+    for (int u = 0; u < M0; ++u)
+        if (place[u] & 2) {
+            v[u] = dirac(First(), u, p[u]);
+            if (place[u] & 1) mu += sq(v[u]);
+        }
+    put(2, v);
+#pragma unroll
+    for (int u = 0; u < M0; ++u)
+        if (place[u] & 1) nu += sq(dirac(Second(), u, v[u]));
+    store_pf_partials<NT>(part + 2 * ((size_t)sys * gridDim.x + blockIdx.x), mu, nu, rho, red);
+}
+
 // ---------------------------------------------------------------------------
 // flexible CG: the operator's launch
 // ---------------------------------------------------------------------------
@@ -351,10 +475,17 @@ struct PlTile {
 constexpr PlTile kPlTiles[] = {{4, 16, 192}, {8, 32, 256}, {16, 16, 256}, {16, 32, 256}, {32, 32, 448}, {8, 64, 256},
                                {16, 64, 704}};
 constexpr int kNumPl = sizeof(kPlTiles) / sizeof(kPlTiles[0]);
+// FP64 only: tiles of k_pl_rc, numbered after those.  The entries per thread (two) matter more than
+// the tile: 16x32 with 960 threads takes 43.9 us at 1024 x 1024, with 256 35.1.
+constexpr PlTile kRcTiles[] = {{16, 32, 512}, {32, 32, 832}, {16, 64, 896}};
+constexpr int kNumRc = sizeof(kRcTiles) / sizeof(kRcTiles[0]);
+static PlTile pl_tile(int i) { return i < kNumPl ? kPlTiles[i] : kRcTiles[i - kNumPl]; }
 
 // a tile need not divide the lattice, but its halo may wrap around only once
-static bool pl_fits(const Ctx &c, PlTile t) {
-    auto ok = [](int n, int T) { return n >= 2 && (n % T == 0 || n > T); };
+static bool pl_fits(const Ctx &c, int i) {
+    const PlTile t = pl_tile(i);
+    const int halo = i < kNumPl ? 2 : 4;
+    auto ok = [&](int n, int T) { return n >= halo && (n % T == 0 || n > T + halo - 2); };
     return ok(c.p.Nt, t.TT) && ok(c.p.Nx, t.TX);
 }
 static int pl_blocks(const Ctx &c, PlTile t) {
@@ -369,10 +500,7 @@ struct PlPtrs {
     V2 *pnew, *Ap, *x;
 };
 
-// launch idx of a chunk; form 0: launch 0 of a phase (r read), 1: odd launches, 2: even ones;
-// returns the block partials per system
-template <typename R, int TT, int TX, int NT>
-static int launch_pl_tt(const Ctx &c, int nsys, bool dag1, int idx, int form, int finMode, const PlPtrs<R> &b) {
+static PlArgs pl_args(const Ctx &c, int TT, int TX) {
     PlArgs A;
     A.Nt = c.p.Nt;
     A.Nx = c.p.Nx;
@@ -382,8 +510,16 @@ static int launch_pl_tt(const Ctx &c, int nsys, bool dag1, int idx, int form, in
     A.d0 = 2.0 * c.p.r + c.p.M;
     A.g = c.p.g;
     A.tilesX = (c.p.Nx + TX - 1) / TX;
-    A.tilesPerSys = pl_blocks(c, {TT, TX, NT});
+    A.tilesPerSys = pl_blocks(c, {TT, TX, 0});
     A.xcdRemap = A.tilesPerSys % 8 == 0 ? 1 : 0;
+    return A;
+}
+
+// launch idx of a chunk; form 0: launch 0 of a phase (r read), 1: odd launches, 2: even ones;
+// returns the block partials per system
+template <typename R, int TT, int TX, int NT>
+static int launch_pl_tt(const Ctx &c, int nsys, bool dag1, int idx, int form, int finMode, const PlPtrs<R> &b) {
+    PlArgs A = pl_args(c, TT, TX);
     auto go = [&](auto dagTag, auto wrTag) {
         constexpr bool D = decltype(dagTag)::value, W1 = decltype(wrTag)::value;
         using K = decltype(&k_pl_pf<R, TT, TX, NT, D, W1, 0, 1>);
@@ -401,11 +537,44 @@ static int launch_pl_tt(const Ctx &c, int nsys, bool dag1, int idx, int form, in
     return A.tilesPerSys;
 }
 
+// k_pl_rc for the launches after a phase's first
+template <int TT, int TX, int NT>
+static int launch_rc_tt(const Ctx &c, int nsys, bool dag1, int idx, int form, int finMode, const PlPtrs<double> &b) {
+    if (form == 0) return launch_pl_tt<double, TT, TX, NT>(c, nsys, dag1, idx, form, finMode, b);
+    PlArgs A = pl_args(c, TT, TX);
+    auto go = [&](auto dagTag, auto wrTag) {
+        constexpr bool D = decltype(dagTag)::value, W1 = decltype(wrTag)::value;
+        auto *k = form == 1 ? &k_pl_rc<double, TT, TX, NT, D, W1, 2> : &k_pl_rc<double, TT, TX, NT, D, W1, 0>;
+        hipLaunchKernelGGL(k, dim3(A.tilesPerSys, nsys), dim3(NT), 0, c.stream, A, b.phi, c.cg_d, b.r, b.pold, b.pnew,
+                           b.x, c.pfSlot[idx & 1], finMode, idx, (const double2 *)c.pfSlot[~idx & 1], c.active);
+    };
+    const bool w1 = c.p.r == 1.0;
+    if (dag1)
+        w1 ? go(std::true_type(), std::true_type()) : go(std::true_type(), std::false_type());
+    else
+        w1 ? go(std::false_type(), std::true_type()) : go(std::false_type(), std::false_type());
+    return A.tilesPerSys;
+}
+
+static int launch_rc(const Ctx &c, int ti, int nsys, bool dag1, int idx, int form, int finMode,
+                     const PlPtrs<double> &b) {
+    switch (ti - kNumPl) {
+    case 0: return launch_rc_tt<16, 32, 512>(c, nsys, dag1, idx, form, finMode, b);
+    case 1: return launch_rc_tt<32, 32, 832>(c, nsys, dag1, idx, form, finMode, b);
+    default: return launch_rc_tt<16, 64, 896>(c, nsys, dag1, idx, form, finMode, b);
+    }
+}
+
 template <typename R>
 static int launch_pl_any(Ctx &c, int ti, int nsys, bool dag1, int idx, int form, int finMode, const PlPtrs<R> &b) {
-    const PlTile t = kPlTiles[ti];
-    prof_before(c, PK_NORMAL_OP, (double)nsys * c.V * ((idx & 1 ? 7 : 5) * 4 + 1) * sizeof(R));
+    const PlTile t = pl_tile(ti);
+    prof_before(c, PK_NORMAL_OP, (double)nsys * c.V * ((idx & 1 ? 7 : 5) * 4 - (ti < kNumPl ? 0 : 8) + 1) * sizeof(R));
     int nb = 0;
+    if (ti >= kNumPl) {
+        if constexpr (std::is_same<R, double>::value) nb = launch_rc(c, ti, nsys, dag1, idx, form, finMode, b);
+        prof_after(c, PK_NORMAL_OP);
+        return nb;
+    }
     switch (t.TT * 1000 + t.TX) {
     case 4016: nb = launch_pl_tt<R, 4, 16, 192>(c, nsys, dag1, idx, form, finMode, b); break;
     case 8032: nb = launch_pl_tt<R, 8, 32, 256>(c, nsys, dag1, idx, form, finMode, b); break;
@@ -457,8 +626,8 @@ static int launch_p64(Ctx &c, int ti, int nsys, const double *phi, bool dag1, in
 // third direction
 static int pl_alloc(Ctx &c, bool mixed) {
     size_t nb = 0;
-    for (const PlTile &t : kPlTiles)
-        if (pl_fits(c, t)) nb = std::max(nb, (size_t)pl_blocks(c, t));
+    for (int i = 0; i < kNumPl + kNumRc; ++i)
+        if (pl_fits(c, i)) nb = std::max(nb, (size_t)pl_blocks(c, pl_tile(i)));
     if (!nb || c.V >= (1 << 27)) return YCN_OK;   // 32-bit byte offsets into a system's two planes
     const size_t n = (size_t)c.nSys * kPacked * c.V;
     if (mixed)
@@ -486,17 +655,17 @@ int pl_autotune(Ctx &c) {
     const int rc = pl_alloc(c, mixed);
     if (rc || !c.pfSlot[1]) return rc;
     std::vector<double> us;
-    const int memoKey = mixed ? 2 : 3;
-    const bool memo = tune_lookup(memoKey, c, us) && us.size() == 2 * (size_t)kNumPl;
+    const int memoKey = mixed ? 2 : 3, n = mixed ? kNumPl : kNumPl + kNumRc;
+    const bool memo = tune_lookup(memoKey, c, us) && us.size() == 2 * (size_t)n;
     if (!memo) {
-        us.assign(2 * kNumPl, 1e30);
+        us.assign(2 * n, 1e30);
         hipEvent_t e0, e1;
         YCN_HIP(hipEventCreate(&e0));
         YCN_HIP(hipEventCreate(&e1));
         YCN_HIP(hipMemsetAsync(c.cg_d, 0, sizeof(CgState) * c.nSys, c.stream));
         const int reps = c.V >= (1 << 16) ? 10 : 4;
-        for (int i = 0; i < kNumPl; ++i) {
-            if (!pl_fits(c, kPlTiles[i])) continue;
+        for (int i = 0; i < n; ++i) {
+            if (!pl_fits(c, i)) continue;
             for (int m = 0; m < 2; ++m) {
                 auto launch = [&](int k) {
                     const int nb = mixed ? launch_pl(c, i, c.nSys, false, k, m ? 2 : 0)
@@ -529,9 +698,10 @@ int pl_autotune(Ctx &c) {
     int &tile = mixed ? c.tilePl : c.tileP64;
     c.tuneReport += mixed ? " | fp32 pipelined tiles (us/iteration, separate | prologue finalize):"
                           : " | fp64 pipelined tiles (us/iteration, separate | prologue finalize):";
-    for (int i = 0; i < kNumPl; ++i) {
-        if (!pl_fits(c, kPlTiles[i])) continue;
-        std::snprintf(line, sizeof line, " %dx%d %.1f|%.1f;", kPlTiles[i].TT, kPlTiles[i].TX, us[2 * i], us[2 * i + 1]);
+    for (int i = 0; i < n; ++i) {
+        if (!pl_fits(c, i)) continue;
+        std::snprintf(line, sizeof line, " %dx%d%s %.1f|%.1f;", pl_tile(i).TT, pl_tile(i).TX, i < kNumPl ? "" : "r",
+                      us[2 * i], us[2 * i + 1]);
         c.tuneReport += line;
         for (int m = 0; m < 2; ++m)
             if ((f < 0 || f == i) && us[2 * i + m] < best) {
@@ -552,7 +722,7 @@ int pl_iterations(Ctx &c, int nsys, int mtype, int n) {
         if (!c.eoFinFused) launch_fin_pf(c, nsys, nb, 1, c.pfSlot[i & 1]);
     });
     if (rc) return rc;
-    c.eoPfBlocks = pl_blocks(c, kPlTiles[c.tilePl]);
+    c.eoPfBlocks = pl_blocks(c, pl_tile(c.tilePl));
     if (c.eoFinFused) launch_fin_pf_chunk(c, nsys, n);
     return YCN_OK;
 }
@@ -577,17 +747,7 @@ void p64_close(Ctx &c, int nsys) {
 // iteration idx of a chunk of the flexible solver (see k_fcg_op): r and the directions alternate
 // between two buffers, both ways starting from the first
 int fcg_iteration(Ctx &c, int nsys, int idx) {
-    PlArgs A;
-    A.Nt = c.p.Nt;
-    A.Nx = c.p.Nx;
-    A.V = c.V;
-    A.nNoise = c.nNoise;
-    A.r = c.p.r;
-    A.d0 = 2.0 * c.p.r + c.p.M;
-    A.g = c.p.g;
-    A.tilesX = c.p.Nx / 16;
-    A.tilesPerSys = (c.p.Nt / 16) * A.tilesX;
-    A.xcdRemap = A.tilesPerSys % 8 == 0 ? 1 : 0;
+    PlArgs A = pl_args(c, 16, 16);
     const int par = idx & 1, tiles = A.tilesPerSys;
     double *const opPart = reinterpret_cast<double *>(c.partials + (size_t)2 * nsys * tiles);
     prof_before(c, PK_NORMAL_OP, (double)nsys * c.V * (4 * 32 + 4));
