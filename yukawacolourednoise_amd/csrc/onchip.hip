@@ -120,7 +120,8 @@ k_onchip_plain(OnchipArgs A, const double *__restrict__ phi, const uint64_t *__r
     int iter = 0, restarts = 0, converged = run ? 0 : 1;
     double beta = 0.0, trueRel = 0.0;
 
-    // w = D1 v through P and Q, leaving it in Q; o = D2 w
+    // w = D1 v through P and Q, leaving it in Q; o = D2 w; returns |w|^2, whose sum over the block
+    // shares the barrier that publishes w
     auto normal_op = [&](const double2 *v0, const double2 *v1, double2 *w0, double2 *w1, double2 *o0, double2 *o1) {
 #pragma unroll
         for (int k = 0; k < K; ++k) {
@@ -131,6 +132,7 @@ k_onchip_plain(OnchipArgs A, const double *__restrict__ phi, const uint64_t *__r
             }
         }
         __syncthreads();
+        double ww = 0.0;
 #pragma unroll
         for (int k = 0; k < K; ++k) {
             const int s = threadIdx.x + k * NT;
@@ -138,32 +140,29 @@ k_onchip_plain(OnchipArgs A, const double *__restrict__ phi, const uint64_t *__r
                 onchip_dirac<DAG1, WR1>(A, P, nb[k], d[k], v0[k], v1[k], w0[k], w1[k]);
                 Q[s] = w0[k];
                 Q[V + s] = w1[k];
+                ww += (w0[k].x * w0[k].x + w0[k].y * w0[k].y) + (w1[k].x * w1[k].x + w1[k].y * w1[k].y);
             }
         }
-        __syncthreads();
+        ww = onchip_sum(ww, red, turn);
 #pragma unroll
         for (int k = 0; k < K; ++k) {
             const int s = threadIdx.x + k * NT;
             o0[k] = o1[k] = make_double2(0.0, 0.0);
             if (s < V) onchip_dirac<!DAG1, WR1>(A, Q, nb[k], d[k], w0[k], w1[k], o0[k], o1[k]);
         }
+        return ww;
     };
 
     double2 w0[K], w1[K], a0[K], a1[K];
     for (;;) {
         while (run) {
-            double dot = 0.0;
+            const double inv = 1.0 / rr;   // ahead of the sum that beta waits for
 #pragma unroll
             for (int k = 0; k < K; ++k) {
                 p0[k] = make_double2(r0[k].x + beta * p0[k].x, r0[k].y + beta * p0[k].y);
                 p1[k] = make_double2(r1[k].x + beta * p1[k].x, r1[k].y + beta * p1[k].y);
             }
-            normal_op(p0, p1, w0, w1, a0, a1);
-#pragma unroll
-            for (int k = 0; k < K; ++k)
-                dot += (p0[k].x * a0[k].x + p0[k].y * a0[k].y) + (p1[k].x * a1[k].x + p1[k].y * a1[k].y);
-            dot = onchip_sum(dot, red, turn);
-            const double alpha = rr / dot;
+            const double alpha = rr / normal_op(p0, p1, w0, w1, a0, a1);   // <p, A p> = |D1 p|^2
             double rn = 0.0;
 #pragma unroll
             for (int k = 0; k < K; ++k) {
@@ -174,12 +173,12 @@ k_onchip_plain(OnchipArgs A, const double *__restrict__ phi, const uint64_t *__r
                 rn += (r0[k].x * r0[k].x + r0[k].y * r0[k].y) + (r1[k].x * r1[k].x + r1[k].y * r1[k].y);
             }
             rn = onchip_sum(rn, red, turn);
-            beta = rn / rr;
+            beta = rn * inv;
             rr = rn;
             ++iter;
-            if (iter >= A.maxIter || !(sqrt(rn) > stop)) {
+            if (iter >= A.maxIter || !(rn > stop * stop)) {
                 run = false;
-                converged = sqrt(rn) <= stop ? 1 : 0;
+                converged = rn <= stop * stop ? 1 : 0;
             }
         }
         // true residual |b - A x| / |b|; in relative mode restart from it while above tol

@@ -246,6 +246,7 @@ k_onchip_eo(OnchipEoArgs A, const double *__restrict__ phi, const uint64_t *__re
 
     for (;;) {
         while (run) {
+            const double inv = 1.0 / rr;   // ahead of the sum that beta waits for
             // p = r + beta p; U = A_o^-1 K p; v = S p; W = A_o^-1 H v; Ap = S^T v.  O is written
             // and E read between the same barriers, and the other way round, so one barrier
             // separates each stage from the next.
@@ -282,11 +283,11 @@ k_onchip_eo(OnchipEoArgs A, const double *__restrict__ phi, const uint64_t *__re
             }
             rho = onchip_sum(rho, red, turn);
             ++iter;
-            beta = rho / rr;
+            beta = rho * inv;
             rr = rho;
-            if (iter >= A.maxIter || !(sqrt(rho) > stop)) {
+            if (iter >= A.maxIter || !(rho > stop * stop)) {
                 run = false;
-                converged = sqrt(rho) <= stop ? 1 : 0;
+                converged = rho <= stop * stop ? 1 : 0;
             }
         }
         // true residual |b - S x| / |eta|; u = A_o^-1 K x is kept for the drift
