@@ -88,3 +88,24 @@ def test_onchip_even_odd_stopping(gpu, monkeypatch, mode, tol, cap):
         # the launched solver pauses after even numbers of iterations only
         assert abs(s1["iters"] - s0["iters"]) <= (2 if tol > 1e-16 else cap)
         assert rel(d1, d0) < 1e-7 and rel(c1, c0) < 1e-7
+
+
+@pytest.mark.parametrize("Nt,Nx,chains,eo,steps", [(8, 16, 1, 0, 70), (7, 32, 3, 0, 17), (32, 32, 2, 1, 33)])
+def test_run_equals_steps(gpu, Nt, Nx, chains, eo, steps):
+    """A run makes the noise of several steps in one launch (16 at most) and waits for up to 64:
+    the same fields as step by step, bit for bit (plain solver) or to the solver's tolerance
+    (even-odd: the starting thresholds are learned on the device or on the host)."""
+    Y = gpu
+    p, _ = mk(Y, Nt=Nt, Nx=Nx, nReplicas=chains, cgTol=1e-10, cgTolMode=1)
+    p.evenOdd = eo
+    out = []
+    for run in (True, False):
+        with Y.Context(p) as c:
+            c.hot_start(4)
+            if run:
+                c.langevin_run(5, steps)
+            else:
+                for k in range(steps):
+                    c.langevin_step(5 + k)
+            out.append(c.get_field())
+    assert np.array_equal(*out) if not eo else rel(*out) < 1e-7

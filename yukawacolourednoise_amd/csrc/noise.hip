@@ -397,8 +397,9 @@ k_noise_rows_inv(const double2 *__restrict__ spec, double *__restrict__ noise, i
 }
 
 // ---------------------------------------------------------------------------
-// the three passes of a small lattice by one block per replica, the spectrum in LDS
-// (buffers of `cap` entries): the same arithmetic in one launch
+// the three passes of a small lattice by one block per replica and step (step + blockIdx.y, the
+// fields one after the other), the spectrum in LDS (buffers of `cap` entries): the same arithmetic
+// in one launch
 // ---------------------------------------------------------------------------
 constexpr int kOneThreads = 512;
 constexpr int kOneLdsBytes = 81920;
@@ -411,6 +412,8 @@ k_noise_one(const double *__restrict__ xi, const uint64_t *__restrict__ seeds, u
         if (ctl->halt) return;
         step = ctl->step;
     }
+    step += blockIdx.y;
+    noise += (size_t)blockIdx.y * gridDim.x * Nt * Nx;
     const int rep = blockIdx.x, np = (Nt + 1) / 2, H = Nx / 2 + 1, rowX = fft_row(Nx), rowT = fft_row(Nt);
     double2 *a = lds, *b = lds + cap;
     load_rows(a, xi ? xi + (size_t)rep * Nt * Nx : nullptr, seeds[rep], step, 0, np, Nt, Nx);
@@ -624,7 +627,8 @@ int noise_generate(Ctx &c, uint64_t step, const double *xi_dev, double *out_dev)
 // column pass for a context's kernel timing
 static int launch_noise(hipStream_t s, int Nt, int Nx, int nRep, const double *xi_dev, const uint64_t *seeds,
                         uint64_t step, double2 *spec, const int *kmax, int kmaxAll, const FftPlan &planX,
-                        const FftPlan &planT, double *out_dev, Ctx *prof, const StepCtl *ctl = nullptr) {
+                        const FftPlan &planT, double *out_dev, Ctx *prof, const StepCtl *ctl = nullptr,
+                        int nsteps = 1) {
     const int H = Nx / 2 + 1, nk = kmaxAll + 1;   // columns up to the cutoff
     const double invV = 1.0 / ((double)Nt * (double)Nx);
     const int npairs = (Nt + 1) / 2;
@@ -635,10 +639,17 @@ static int launch_noise(hipStream_t s, int Nt, int Nx, int nRep, const double *x
     const size_t shOne = (size_t)2 * cap * sizeof(double2);
     if (shOne <= (size_t)kOneLdsBytes) {
         if (prof) prof_before(*prof, PK_NOISE_COLS, 40.0 * (double)nRep * Nt * Nx);
-        hipLaunchKernelGGL(k_noise_one, dim3(nRep), dim3(kOneThreads), shOne, s, xi_dev, seeds, step, kmax, nk, invV,
+        hipLaunchKernelGGL(k_noise_one, dim3(nRep, nsteps), dim3(kOneThreads), shOne, s, xi_dev, seeds, step, kmax, nk, invV,
                            out_dev, Nt, Nx, cap, planX, planT, ctl);
         if (prof) prof_after(*prof, PK_NOISE_COLS);
         return hipGetLastError() == hipSuccess ? YCN_OK : YCN_ERR_HIP;
+    }
+    if (nsteps > 1) {
+        for (int i = 0; i < nsteps; ++i)
+            if (launch_noise(s, Nt, Nx, nRep, xi_dev, seeds, step + i, spec, kmax, kmaxAll, planX, planT,
+                             out_dev + (size_t)i * nRep * Nt * Nx, prof, ctl))
+                return YCN_ERR_HIP;
+        return YCN_OK;
     }
     const int lx = lines_per_block(Nx, npairs * nRep, 1), lt = lines_per_block(Nt, nk * nRep, 2);
     dim3 g1((npairs + lx - 1) / lx, nRep), g2((nk + lt - 1) / lt, nRep);
@@ -658,6 +669,14 @@ static int launch_noise(hipStream_t s, int Nt, int Nx, int nRep, const double *x
 int noise_generate_on(Ctx &c, hipStream_t s, uint64_t step, const double *xi_dev, double *out_dev) {
     const int rc = launch_noise(s, c.p.Nt, c.p.Nx, c.nRep, xi_dev, (const uint64_t *)c.seed_d, step, c.spec,
                                 (const int *)c.kmax, c.kmaxAll, c.planX, c.planT, out_dev, &c);
+    if (rc) c.err = "coloured-noise kernel launch failed";
+    return rc;
+}
+
+// the fields of nsteps consecutive steps, one after the other
+int noise_generate_steps(Ctx &c, uint64_t step, int nsteps, double *out_dev) {
+    const int rc = launch_noise(c.stream, c.p.Nt, c.p.Nx, c.nRep, nullptr, (const uint64_t *)c.seed_d, step, c.spec,
+                                (const int *)c.kmax, c.kmaxAll, c.planX, c.planT, out_dev, &c, nullptr, nsteps);
     if (rc) c.err = "coloured-noise kernel launch failed";
     return rc;
 }

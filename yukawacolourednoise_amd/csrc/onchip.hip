@@ -399,11 +399,21 @@ bool onchip_steps(const Ctx &c) {
 }
 
 constexpr int kRunSlots = 64;   // steps in flight before the host waits for their reports
+// Steps whose noise one launch makes: a field takes one block 10 to 20 us (16 x 16 to 64 x 64), as
+// long as a whole launch of them does while the chip has compute units left, so a run of 16 steps
+// pays for one (32 x 32: 14 us of a 198 us step before).
+constexpr int kNoiseSteps = 16;
 
 static int run_init(Ctx &c) {
     if (!c.report) {
         YCN_HIP(hipHostMalloc((void **)&c.report, sizeof(StepReport) * kRunSlots * c.nRep, hipHostMallocDefault));
         for (int i = 0; i < kRunSlots * c.nRep; ++i) c.report[i].seq = 0;
+    }
+    // noise of several steps ahead, in at most 64 MiB
+    if (!c.noiseRun) {
+        const size_t one = (size_t)c.nRep * c.V, fit = ((size_t)64 << 20) / (sizeof(double) * one);
+        c.noiseSteps = (int)std::max<size_t>(1, std::min<size_t>(kNoiseSteps, fit));
+        YCN_HIP(hipMalloc(&c.noiseRun, sizeof(double) * one * c.noiseSteps));
     }
     if (c.p.evenOdd && !c.ratio) YCN_HIP(hipMalloc(&c.ratio, sizeof(double) * 2 * ((size_t)c.nSys + 1)));
     return YCN_OK;
@@ -412,6 +422,8 @@ static int run_init(Ctx &c) {
 void onchip_free(Ctx &c) {
     if (c.report) (void)hipHostFree(c.report);
     if (c.ratio) (void)hipFree(c.ratio);
+    if (c.noiseRun) (void)hipFree(c.noiseRun);
+    c.noiseRun = nullptr;
     c.report = nullptr;
     c.ratio = nullptr;
 }
@@ -446,11 +458,14 @@ int onchip_run(Ctx &c, uint64_t step0, int nsteps, SolveStats *tot, double *eps)
         for (int i = 0; i < seg; ++i) {
             const uint64_t step = step0 + (uint64_t)(done + i);
             double *in = c.phi[c.cur], *out = fixed ? c.phi[c.cur ^ 1] : in;
-            if ((rc = noise_generate(c, step, nullptr, c.noise))) return rc;                       // cn()
+            const int ahead = i % c.noiseSteps;
+            if (ahead == 0 && (rc = noise_generate_steps(c, step, std::min(seg - i, c.noiseSteps), c.noiseRun)))
+                return rc;                                                                          // cn()
+            const double *noise = c.noiseRun + (size_t)ahead * c.nRep * c.V;
             rc = c.p.evenOdd ? onchip_eo_force(c, in, 1u, step, i > 0) : onchip_force(c, in, 1u, step);
             if (rc) return rc;                                                                      // getForce(drift)
             hipLaunchKernelGGL(k_onchip_update, dim3(c.nRep), dim3(kOnchipThreads), 0, c.stream, (const double *)in, out,
-                               (const double *)c.drift, (const double *)c.noise, (const double *)c.m2_d,
+                               (const double *)c.drift, noise, (const double *)c.m2_d,
                                c.p.lambda / 6.0, c.p.Nt, c.p.Nx, c.epsBar, c.p.adaptive, c.step_d,
                                (const CgState *)c.cg_d, c.nNoise, c.report + (size_t)i * c.nRep, ++c.reportSeq);
             YCN_HIP(hipGetLastError());                                                             // kli.Run(kAll)

@@ -217,6 +217,8 @@ struct Ctx {
     double *ratio = nullptr;              // [2][nSys + 1]: need / stop0 of the last two on-chip even-odd solves, and
                                           // the threshold scale each started from
     int ratioTurn = 0;
+    double *noiseRun = nullptr;           // noise of noiseSteps consecutive on-chip steps
+    int noiseSteps = 1;
     bool onchip = false;                  // solves that fit one workgroup run in one launch (YCN_ONCHIP=0: never)
 
     // profiling
@@ -256,6 +258,7 @@ void noise_free(Ctx &c);
 int noise_generate(Ctx &c, uint64_t step, const double *xi_dev, double *out_dev);
 int noise_generate_on(Ctx &c, hipStream_t s, uint64_t step, const double *xi_dev, double *out_dev);
 // the noise of a graph-captured step: counter and halt flag from the control block
+int noise_generate_steps(Ctx &c, uint64_t step, int nsteps, double *out_dev);
 int noise_generate_ctl(Ctx &c, hipStream_t s, const StepCtl *ctl, double *out_dev);
 // the allocation-free entry point's scratch: address lookup on device dev (current),
 // and the message of the last failed call on this thread (nullptr if none)
