@@ -1032,7 +1032,7 @@ int stats_from_mirror(Ctx &c, int nsys, SolveStats *st) {
 int cg_solve(Ctx &c, const double *phi, int nsys, int mtype, SpinorForm form, bool gen, uint32_t streamBase,
              uint64_t step, SolveStats *st) {
     if (c.p.precond == YCN_PRECOND_CNN && mtype == YCN_DAGGER)
-        return fcg_solve(c, phi, nsys, mtype, gen, streamBase, step, st);
+        return fcg_solve(c, phi, nsys, mtype, form, gen, streamBase, step, st);
     // mixed precision where the FP32 tiles fit the lattice (with even-odd preconditioning
     // the fermion force may run mixed on shapes the plain FP32 tiles do not cover)
     const bool mixed = (c.p.cgPrecision == YCN_CG_MIXED && c.rs) || c.p.precond == YCN_PRECOND_CNN;
@@ -1328,9 +1328,10 @@ int spinor_slices(Ctx &c, const double2 *psi, double *out_dev) {
 // direction, and plain CG (identity preconditioner) once a reliable interval stalls.
 // The FP64 true residual with the plain operator decides convergence.
 // ===========================================================================
-int fcg_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, uint32_t streamBase, uint64_t step,
-              SolveStats *st) {
-    constexpr int NC = kComplex;
+template <int NC>
+static int fcg_solve_as(Ctx &c, const double *phi, int nsys, int mtype, bool gen, uint32_t streamBase, uint64_t step,
+                        SolveStats *st) {
+    constexpr SpinorForm form = (SpinorForm)NC;
     if (c.tile32 < 0 || !c.zs) {
         c.err = "the learned preconditioner needs Nt % 16 == 0 and Nx % 16 == 0";
         return YCN_ERR_UNSUPPORTED;
@@ -1356,7 +1357,7 @@ int fcg_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, uint32_t
     hipLaunchKernelGGL(k_fin_setup, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)c.partials, nb, c.cg_d,
                        c.active, c.p.cgTol, c.p.cgTolMode, maxIter, 0);
     // z = CNN(b), rz = <b, z>, p' = z on the first iteration
-    int nbC = cnn_apply(c, nsys, c.rs, c.Aps, c.zs, c.partials);
+    int nbC = cnn_apply(c, form, nsys, c.rs, c.Aps, c.zs, c.partials);
     if (nbC < 0) return nbC;
     hipLaunchKernelGGL(k_fin_fcg<true>, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)c.partials, nbC, c.cg_d);
     YCN_HIP(hipGetLastError());
@@ -1368,7 +1369,7 @@ int fcg_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, uint32_t
     if (rc) return rc;
     while (active > 0 && launched < hardCap) {
         rc = run_chunk(c, nullptr, nsys, mtype, nIt, 2 /* flexible */, NC, c.tile32,
-                       [&](int i) { (void)fcg_iteration(c, nsys, i); });
+                       [&](int i) { (void)fcg_iteration(c, form, nsys, i); });
         if (rc) return rc;
         fcg_close(c, nsys, nIt);
         launched += nIt;
@@ -1379,7 +1380,7 @@ int fcg_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, uint32_t
         const double refRate = (c.plainIters > 0 && c.p.cgTol > 0.0) ? std::log10(c.p.cgTol) / c.plainIters : 0.0;
         hipLaunchKernelGGL(k_fin_mp_true<true>, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)c.partials, nb,
                            c.cg_d, c.active, refRate);
-        nbC = cnn_apply(c, nsys, c.rs, c.Aps, c.zs, c.partials);
+        nbC = cnn_apply(c, form, nsys, c.rs, c.Aps, c.zs, c.partials);
         if (nbC < 0) return nbC;
         hipLaunchKernelGGL(k_fin_fcg<false>, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)c.partials, nbC,
                            c.cg_d);
@@ -1388,6 +1389,12 @@ int fcg_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, uint32_t
         if (rc) return rc;
     }
     return read_stats(c, nsys, st);
+}
+
+int fcg_solve(Ctx &c, const double *phi, int nsys, int mtype, SpinorForm form, bool gen, uint32_t streamBase,
+              uint64_t step, SolveStats *st) {
+    return form == kPacked ? fcg_solve_as<kPacked>(c, phi, nsys, mtype, gen, streamBase, step, st)
+                           : fcg_solve_as<kComplex>(c, phi, nsys, mtype, gen, streamBase, step, st);
 }
 
 // e = x_final - x_snapshot

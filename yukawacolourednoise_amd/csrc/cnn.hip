@@ -176,6 +176,9 @@ k_cnn_gates(int Nt, int Nx, const float *__restrict__ phis, float g, const float
 // the network is switched off.  The network's input is scaled by |r| where the chunk began: the
 // scale cancels, and bf16 keeps its relative precision.
 // UPD = false: z = CNN(r) and the partials (<z, r>, <z, Ap>).
+// NC = 2: r real, as the fermion force's is (packed real spinors), and z the real part of the
+// network's output, a linear map of real vectors like the network: its imaginary part is no part of
+// the solution, and half of every vector's traffic goes with it.  NC = 4: complex vectors.
 // What bounds it where every block has a compute unit to itself (256 x 256: 256 blocks): latency, the
 // loads, three layers of a few MFMAs with a barrier each, the sums.  FW = 8 waves have 4, 3 and 2
 // groups of sites each, and everything that they read from memory (inputs, gates, weights, the
@@ -183,7 +186,7 @@ k_cnn_gates(int Nt, int Nx, const float *__restrict__ phis, float g, const float
 // latency and registers cost occupancy: FW = 4, each group's loads before its MFMAs.  An iteration
 // of the flexible solver: 256 x 256 19.9 us with 8 waves, 20.7 with 16, 23.0 with 4 loading late;
 // 512 x 512 52.3, 54.1 and 44.4; 1024 x 1024 276, 266 and 211.
-template <bool UPD, int FW>
+template <bool UPD, int FW, int NC>
 __global__ void __launch_bounds__(64 * FW)
 k_cnn_fused(int Nt, int Nx, int tilesX, int nNoise, float c0, CgState *__restrict__ st,
             const float2 *__restrict__ rs, const float2 *__restrict__ Ap, const _Float16 *__restrict__ gates,
@@ -191,7 +194,8 @@ k_cnn_fused(int Nt, int Nx, int tilesX, int nNoise, float c0, CgState *__restric
             const bf16x8 *__restrict__ gf3, double2 *__restrict__ part, FcgUpdate upd) {
     constexpr int W0 = 22, W1 = 20, W2 = 18, W3 = 16, kFT = 64 * FW;
     constexpr int R1 = conv_rounds(W1, FW), R2 = conv_rounds(W2, FW), R3 = conv_rounds(W3, FW);
-    constexpr int E = 1024 / kFT;
+    constexpr bool REAL = NC == 2;   // packed real spinors: the imaginary channels are 0 and unused
+    constexpr int E = (REAL ? 512 : 1024) / kFT, HN = REAL ? 1 : 2;
     constexpr bool EARLY = FW > 4;
     typedef _Float16 h4 __attribute__((ext_vector_type(4)));
     typedef __bf16 b4 __attribute__((ext_vector_type(4)));
@@ -209,12 +213,12 @@ k_cnn_fused(int Nt, int Nx, int tilesX, int nNoise, float c0, CgState *__restric
     bool identity = st[sys].precOff;
     if (st[sys].done) return;
     const int V = Nt * Nx;
-    const size_t off = (size_t)sys * 4 * V;
+    const size_t off = (size_t)sys * NC * V;
     const int tile = blockIdx.x;
     const int ty = tile / tilesX, tx = tile - ty * tilesX;
     const int t0 = ty * 16, x0 = tx * 16;
 
-    // inputs: entries of the tile with its 3-site halo, two of the four components each
+    // inputs: entries of the tile with its 3-site halo, two planes each
     float2 r0[E][2], a0[E][2];
     auto entry = [&](int u, int &e, int &eh) {
         e = (tid + u * kFT) & 511;
@@ -258,18 +262,20 @@ k_cnn_fused(int Nt, int Nx, int tilesX, int nNoise, float c0, CgState *__restric
         weights(gf3, B3);
     }
     // output layer: rows wave, wave + FW, ... of the tile, 8 channels: lanes kg = 0, 1 hold
-    // components 2 kg, 2 kg + 1 of site col
+    // components 2 kg, 2 kg + 1 of site col (flavour kg, both spins), and finish these planes, or
+    // the packed plane of spin kg
     static_assert(W3 == 16 && 16 % FW == 0, "a group of sites is a row of the tile");
     struct RA {
-        float2 r[2], a[2], p[2], x[2];
+        float2 r[HN], a[HN], p[HN], x[HN];
     } ra[R3];
     const size_t own = off + (size_t)(t0 + wave) * Nx + x0 + col;
+    auto own_at = [&](int q, int h) { return own + (size_t)(HN * kg + h) * V + (size_t)(q * FW) * Nx; };
     auto load_own = [&](int q) {
         RA v{};
         if (kg < 2)
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const size_t idx = own + (size_t)(2 * kg + h) * V + (size_t)(q * FW) * Nx;
+            for (int h = 0; h < HN; ++h) {
+                const size_t idx = own_at(q, h);
                 v.r[h] = rs[idx];
                 v.a[h] = Ap[idx];
                 if constexpr (UPD) {
@@ -302,9 +308,9 @@ k_cnn_fused(int Nt, int Nx, int tilesX, int nNoise, float c0, CgState *__restric
     }
     double2 acc = make_double2(0.0, 0.0);
     double rho = 0.0;
-    // z of component 2 kg + h at the lane's own site, from r' there (and the x_s update)
+    // z of plane HN kg + h at the lane's own site, from r' there (and the x_s update)
     auto finish = [&](const RA &v, int q, int h, float2 net) {
-        const size_t idx = own + (size_t)(2 * kg + h) * V + (size_t)(q * FW) * Nx;
+        const size_t idx = own_at(q, h);
         const float2 av = v.a[h], rv = make_float2(v.r[h].x - alpha * av.x, v.r[h].y - alpha * av.y);
         const float2 zv = identity ? rv : make_float2(c0 * rv.x + sf * net.x, c0 * rv.y + sf * net.y);
         z[idx] = zv;
@@ -322,22 +328,29 @@ k_cnn_fused(int Nt, int Nx, int tilesX, int nNoise, float c0, CgState *__restric
             const RA v = EARLY ? ra[q] : load_own(q);
             if (kg < 2)
 #pragma unroll
-                for (int h = 0; h < 2; ++h) finish(v, q, h, make_float2(0.f, 0.f));
+                for (int h = 0; h < HN; ++h) finish(v, q, h, make_float2(0.f, 0.f));
         }
     } else {
 #pragma unroll
         for (int u = 0; u < E; ++u) {
             int e, eh;
             if (!entry(u, e, eh)) continue;
-            b4 q;
+            b4 q[2];   // four channels each: of flavours 0 and 1 (REAL), or the entry's half eh
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 float2 rv = r0[u][h];
                 if (UPD) rv = make_float2(rv.x - alpha * a0[u][h].x, rv.y - alpha * a0[u][h].y);
-                q[2 * h] = (__bf16)(rv.x * inv);
-                q[2 * h + 1] = (__bf16)(rv.y * inv);
+                if constexpr (REAL) {
+                    q[0][2 * h] = (__bf16)(rv.x * inv);
+                    q[1][2 * h] = (__bf16)(rv.y * inv);
+                    q[0][2 * h + 1] = q[1][2 * h + 1] = (__bf16)0.f;
+                } else {
+                    q[0][2 * h] = (__bf16)(rv.x * inv);
+                    q[0][2 * h + 1] = (__bf16)(rv.y * inv);
+                }
             }
-            *reinterpret_cast<b4 *>(U0 + e * 8 + 4 * eh) = q;
+            *reinterpret_cast<b4 *>(U0 + e * 8 + 4 * eh) = q[0];
+            if constexpr (REAL) *reinterpret_cast<b4 *>(U0 + e * 8 + 4) = q[1];
         }
         __syncthreads();
         // the four gated channels go to LDS with one 8-byte store
@@ -361,9 +374,15 @@ k_cnn_fused(int Nt, int Nx, int tilesX, int nNoise, float c0, CgState *__restric
         conv_lds<FW, 16, W3, W2>(
             U2, B3, [&](int q) { return EARLY ? ra[q] : load_own(q); },
             [&](int q, int, int k, f32x4 v, const RA &w) {
-                if (k >= 2) return;
+                if constexpr (REAL) {
+                    // the real parts of both spins of flavour k to both flavours of spin k
+                    const auto f = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[0]), __float_as_uint(v[2]),
+                                                                    false, false);
+                    if (k < 2) finish(w, q, 0, make_float2(__uint_as_float(f[0]), __uint_as_float(f[1])));
+                } else if (k < 2) {
 #pragma unroll
-                for (int h = 0; h < 2; ++h) finish(w, q, h, make_float2(v[2 * h], v[2 * h + 1]));
+                    for (int h = 0; h < HN; ++h) finish(w, q, h, make_float2(v[2 * h], v[2 * h + 1]));
+                }
             });
     }
     const size_t blk = (size_t)sys * gridDim.x + blockIdx.x;
@@ -661,33 +680,37 @@ int cnn_gates(Ctx &c, int nrep) {
 }
 
 template <bool UPD>
-static int launch_cnn(Ctx &c, int nsys, const float2 *rs, const float2 *Ap, float2 *z, double2 *part,
+static int launch_cnn(Ctx &c, SpinorForm form, int nsys, const float2 *rs, const float2 *Ap, float2 *z, double2 *part,
                       const FcgUpdate &u) {
     const int tilesX = c.p.Nx / 16, tiles = (c.p.Nt / 16) * tilesX;
     // read r_s, Ap, the gates of both layers; write z (and read p, x_s, write r_s, x_s)
     const int kind = UPD && c.profTarget == PK_CG_UPDATE ? PK_CG_UPDATE : PK_CNN;
-    prof_before(c, kind, (double)nsys * c.V * (UPD ? 288.0 : 160.0));
-    auto go = [&](auto fw) {
-        constexpr int FW = decltype(fw)::value;
-        hipLaunchKernelGGL((k_cnn_fused<UPD, FW>), dim3(tiles, nsys), dim3(64 * FW), 0, c.stream, c.p.Nt, c.p.Nx, tilesX,
-                           c.nNoise, (float)cnn_c0(c), c.cg_d, rs, Ap, (const _Float16 *)c.cnnGates, z,
+    prof_before(c, kind, (double)nsys * c.V * (64.0 + (UPD ? 7 : 3) * 8 * (int)form));
+    auto go = [&](auto fw, auto nc) {
+        constexpr int FW = decltype(fw)::value, NC = decltype(nc)::value;
+        hipLaunchKernelGGL((k_cnn_fused<UPD, FW, NC>), dim3(tiles, nsys), dim3(64 * FW), 0, c.stream, c.p.Nt, c.p.Nx,
+                           tilesX, c.nNoise, (float)cnn_c0(c), c.cg_d, rs, Ap, (const _Float16 *)c.cnnGates, z,
                            (const bf16x8 *)c.cnnF1, (const bf16x8 *)c.cnnF2, (const bf16x8 *)c.cnnF3, part, u);
     };
+    using W8 = std::integral_constant<int, 8>;
+    using W4 = std::integral_constant<int, 4>;
+    using Real = std::integral_constant<int, kPacked>;
+    using Cplx = std::integral_constant<int, kComplex>;
     if (tiles * nsys <= kOneBlockTiles)
-        go(std::integral_constant<int, 8>());
+        form == kPacked ? go(W8(), Real()) : go(W8(), Cplx());
     else
-        go(std::integral_constant<int, 4>());
+        form == kPacked ? go(W4(), Real()) : go(W4(), Cplx());
     prof_after(c, kind);
     YCN_HIP(hipGetLastError());
     return tiles;
 }
 
-int cnn_apply(Ctx &c, int nsys, const float2 *rs, const float2 *Ap, float2 *z, double2 *part) {
-    return launch_cnn<false>(c, nsys, rs, Ap, z, part, FcgUpdate{});
+int cnn_apply(Ctx &c, SpinorForm form, int nsys, const float2 *rs, const float2 *Ap, float2 *z, double2 *part) {
+    return launch_cnn<false>(c, form, nsys, rs, Ap, z, part, FcgUpdate{});
 }
 
-int cnn_update_apply(Ctx &c, int nsys, const float2 *r, const FcgUpdate &u) {
-    return launch_cnn<true>(c, nsys, r, c.Aps, c.zs, c.partials, u);
+int cnn_update_apply(Ctx &c, SpinorForm form, int nsys, const float2 *r, const FcgUpdate &u) {
+    return launch_cnn<true>(c, form, nsys, r, c.Aps, c.zs, c.partials, u);
 }
 
 // activations for training at lattice volume V: x0[8V] y1[16V] gm1[16V] u1[16V]

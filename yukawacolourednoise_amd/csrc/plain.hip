@@ -346,9 +346,10 @@ __device__ __forceinline__ void fcg_commit(CgState &S, const Pf3 &s, double2 pre
     }
 }
 
-// A block owns a 16 x 16 tile of one flavour's complex spinor (D keeps flavours and is real, so
-// the two planes are a packed spinor of their own: grid.y = system and flavour).
-template <bool WR1>
+// A block owns a 16 x 16 tile of one packed spinor: the system's (FL = 1), or one flavour's complex
+// spinor (FL = 2: D keeps flavours and is real, so its two planes are like a packed spinor's:
+// grid.y = system and flavour).
+template <bool WR1, int FL>
 __global__ void __launch_bounds__(kFcgNT)
 k_fcg_op(PlArgs A, const float *__restrict__ phi, CgState *st, const float2 *__restrict__ z,
          const float2 *__restrict__ pold, float2 *__restrict__ pnew, float2 *__restrict__ Ap,
@@ -357,7 +358,7 @@ k_fcg_op(PlArgs A, const float *__restrict__ phi, CgState *st, const float2 *__r
     __shared__ SpLds<float, N> P, Q;
     __shared__ double red[3 * NT / kWave], bc[1];
     __shared__ int pause;
-    const int sys = blockIdx.y >> 1;
+    const int sys = blockIdx.y / FL;
     const PfHead hd = pf_head(st[sys]);
     const double rz0 = st[sys].rz;
     const double2 prev = st[sys].ab[(idx - 1) & 1];
@@ -403,7 +404,7 @@ k_fcg_op(PlArgs A, const float *__restrict__ phi, CgState *st, const float2 *__r
             bc[0] = f.beta;
             pause = f.pause;
             rz = f.rz;
-            if (blockIdx.x == 0 && !(blockIdx.y & 1)) {
+            if (blockIdx.x == 0 && blockIdx.y % FL == 0) {
                 if (f.pause)
                     fcg_commit(st[sys], s, prev, f, hd.iter0 + idx, active);
                 else if (f.off)
@@ -414,7 +415,7 @@ k_fcg_op(PlArgs A, const float *__restrict__ phi, CgState *st, const float2 *__r
         if (pause) return;
         betaD = bc[0];
     }
-    if (blockIdx.x == 0 && !(blockIdx.y & 1) && threadIdx.x == 0) st[sys].ab[idx & 1].y = rz;
+    if (blockIdx.x == 0 && blockIdx.y % FL == 0 && threadIdx.x == 0) st[sys].ab[idx & 1].y = rz;
     const float beta = (float)betaD;
 #pragma unroll
     for (int u = 0; u < M0; ++u) {
@@ -746,13 +747,15 @@ void p64_close(Ctx &c, int nsys) {
 
 // iteration idx of a chunk of the flexible solver (see k_fcg_op): r and the directions alternate
 // between two buffers, both ways starting from the first
-int fcg_iteration(Ctx &c, int nsys, int idx) {
+int fcg_iteration(Ctx &c, SpinorForm form, int nsys, int idx) {
     PlArgs A = pl_args(c, 16, 16);
     const int par = idx & 1, tiles = A.tilesPerSys;
     double *const opPart = reinterpret_cast<double *>(c.partials + (size_t)2 * nsys * tiles);
-    prof_before(c, PK_NORMAL_OP, (double)nsys * c.V * (4 * 32 + 4));
-    auto *k = A.r == 1.0 ? &k_fcg_op<true> : &k_fcg_op<false>;
-    hipLaunchKernelGGL(k, dim3(tiles, 2 * nsys), dim3(kFcgNT), 0, c.stream, A, (const float *)c.phis, c.cg_d,
+    const int fl = form == kPacked ? 1 : 2;
+    prof_before(c, PK_NORMAL_OP, (double)nsys * c.V * (4 * 16 * fl + 4));
+    auto *k = form == kPacked ? (A.r == 1.0 ? &k_fcg_op<true, 1> : &k_fcg_op<false, 1>)
+                              : (A.r == 1.0 ? &k_fcg_op<true, 2> : &k_fcg_op<false, 2>);
+    hipLaunchKernelGGL(k, dim3(tiles, fl * nsys), dim3(kFcgNT), 0, c.stream, A, (const float *)c.phis, c.cg_d,
                        (const float2 *)c.zs, (const float2 *)c.ps[par], c.ps[par ^ 1], c.Aps, opPart, idx,
                        (const double2 *)c.partials, tiles, c.active);
     prof_after(c, PK_NORMAL_OP);
@@ -761,9 +764,9 @@ int fcg_iteration(Ctx &c, int nsys, int idx) {
     u.p = c.ps[par ^ 1];
     u.xs = c.xs;
     u.opPart = opPart;
-    u.nbOp = 2 * tiles;
+    u.nbOp = fl * tiles;
     u.idx = idx;
-    return cnn_update_apply(c, nsys, par ? c.pfA1 : c.rs, u);
+    return cnn_update_apply(c, form, nsys, par ? c.pfA1 : c.rs, u);
 }
 void fcg_close(Ctx &c, int nsys, int n) {
     hipLaunchKernelGGL(k_fcg_close, dim3(nsys), dim3(kPfNT), 0, c.stream, (const double2 *)c.partials,

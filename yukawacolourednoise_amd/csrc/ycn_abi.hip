@@ -439,12 +439,10 @@ static int force_impl(Ctx &c, uint64_t step, uint32_t streamBase, SolveStats *st
         const int rc = onchip_force(c, c.phi[c.cur], streamBase, step);
         return rc ? rc : read_stats(c, c.nSys, st);
     }
-    // eta and D are real: packed real vectors, except where the network mixes in imaginary
-    // channels
-    const SpinorForm form = c.p.precond == YCN_PRECOND_CNN ? kComplex : kPacked;
-    int rc = cg_solve(c, c.phi[c.cur], c.nSys, YCN_DAGGER, form, true, streamBase, step, st);
+    // eta and D are real: packed real vectors
+    int rc = cg_solve(c, c.phi[c.cur], c.nSys, YCN_DAGGER, kPacked, true, streamBase, step, st);
     if (rc) return rc;
-    return fermion_drift(c, c.phi[c.cur], form, c.drift);
+    return fermion_drift(c, c.phi[c.cur], kPacked, c.drift);
 }
 
 int ycn_fermion_force(ycn_ctx *ctx, uint64_t step, double *drift, ycn_cg_stats *stats) {
@@ -668,7 +666,7 @@ int ycn_precond_apply(ycn_ctx *ctx, const double *r, double *z) {
     YCN_HIP(hipMemcpyAsync(c.cg_d, &S, sizeof(CgState), hipMemcpyHostToDevice, c.stream));
     if ((rc = field_to_f32(c, c.phi[c.cur], c.phis))) return rc;   // the gates read the field
     if ((rc = cnn_gates(c, 1))) return rc;
-    rc = cnn_apply(c, 1, c.rs, c.Aps, c.zs, c.partials);
+    rc = cnn_apply(c, kComplex, 1, c.rs, c.Aps, c.zs, c.partials);
     if (rc < 0) return rc;
     if ((rc = spinor_to_f64(c, c.zs, c.t, 1))) return rc;
     if ((rc = soa_to_aos(c, c.t, (double *)aos.p, 1))) return rc;

@@ -310,7 +310,7 @@ int cnn_get_grad(Ctx &c, float *g);
 // launches the fused CNN on nsys systems; returns the number of partials per system
 // the field gates of the first nrep replicas from c.phis (before cnn_apply, once per field)
 int cnn_gates(Ctx &c, int nrep);
-int cnn_apply(Ctx &c, int nsys, const float2 *rs, const float2 *Ap, float2 *z, double2 *part);
+int cnn_apply(Ctx &c, SpinorForm form, int nsys, const float2 *rs, const float2 *Ap, float2 *z, double2 *part);
 // a flexible CG iteration: the step that the network's launch takes before it (plain.hip)
 struct FcgUpdate {
     float2 *rnew;
@@ -319,13 +319,13 @@ struct FcgUpdate {
     const double *opPart;   // the operator's partials of <p, Ap>, nbOp per system
     int nbOp, idx;
 };
-int cnn_update_apply(Ctx &c, int nsys, const float2 *r, const FcgUpdate &u);
-int fcg_iteration(Ctx &c, int nsys, int idx);
+int cnn_update_apply(Ctx &c, SpinorForm form, int nsys, const float2 *r, const FcgUpdate &u);
+int fcg_iteration(Ctx &c, SpinorForm form, int nsys, int idx);
 void fcg_close(Ctx &c, int nsys, int n);
 int cnn_train_step(Ctx &c, const double2 *r, const double2 *e, const float *phis, float lr, double *loss,
                    bool update);
 // flexible CG with the CNN and the online training driver (cg.hip)
-int fcg_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, uint32_t streamBase, uint64_t step,
+int fcg_solve(Ctx &c, const double *phi, int nsys, int mtype, SpinorForm form, bool gen, uint32_t streamBase, uint64_t step,
               SolveStats *st);
 int train_preconditioner(Ctx &c, uint64_t step0, int nsteps, int pairsPerSolve, float lr, int *pairsUsed);
 
