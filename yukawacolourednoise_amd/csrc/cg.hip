@@ -1246,11 +1246,12 @@ static int mp_solve(Ctx &c, const double *phi, int nsys, int mtype, bool gen, ui
         return pf_loop(c, nsys, 0, st, [&](int n) -> int {
             const int rcc = pl_iterations(c, nsys, mtype, n);
             if (rcc) return rcc;
-            hipLaunchKernelGGL(k_pf_reliable, g, dim3(kNT), 0, c.stream, c.V, (const CgState *)c.cg_d, c.x, c.xs,
+            const PfChunkEnd end = pf_chunk_end(c, n);
+            hipLaunchKernelGGL(k_pf_reliable, g, dim3(kNT), 0, c.stream, c.V, end.n, (const CgState *)c.cg_d, c.x, c.xs,
                                (const float2 *)c.ps[1], (const float2 *)c.pfP2, c.ps[0]);
             launch_true_residual<NC>(c, L, phi, nsys, mtype);
             hipLaunchKernelGGL(k_fin_pf_true, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)c.partials,
-                               (const double2 *)c.partials, nb, c.cg_d, c.active);
+                               (const double2 *)c.partials, nb, c.cg_d, c.active, end);
             YCN_HIP(hipGetLastError());
             return YCN_OK;
         });

@@ -1125,12 +1125,12 @@ static int eo_mixed_chunk(Ctx &c, const double *phi, int nsys, int n, bool graph
                                  [&](int i) { launch_eo_pf_iteration(c, nsys, i); });
         if (rc) return rc;
     }
-    if (c.eoFinFused) launch_fin_pf_chunk(c, nsys, n);
-    hipLaunchKernelGGL(k_pf_reliable, gH, dim3(kNT), 0, c.stream, Vh, (const CgState *)c.cg_d, c.x, c.xs,
+    const PfChunkEnd end = pf_chunk_end(c, n);
+    hipLaunchKernelGGL(k_pf_reliable, gH, dim3(kNT), 0, c.stream, Vh, end.n, (const CgState *)c.cg_d, c.x, c.xs,
                        (const float2 *)c.ps[1], (const float2 *)c.pfP2, c.ps[0]);
     const int nbR = launch_eo_ru(c, nsys, phi, c.x, B.b, c.r, c.rs, partRu, partRu2);
     hipLaunchKernelGGL(k_fin_pf_true, dim3(nsys), dim3(kNT), 0, c.stream, (const double2 *)partRu,
-                       (const double2 *)partRu2, nbR, c.cg_d, c.active);
+                       (const double2 *)partRu2, nbR, c.cg_d, c.active, end);
     YCN_HIP(hipGetLastError());
     return YCN_OK;
 }

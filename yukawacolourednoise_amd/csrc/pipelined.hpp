@@ -414,30 +414,6 @@ k_fin_pf_wave(const double2 *__restrict__ part, int nb, int nsys, CgState *__res
     pf_commit(S, s, active, commit);
 }
 
-// Finalize at the end of a chunk of n launches that finalized each other in their
-// prologues (finMode 1): launch n - 1's partials in slotLast, launch n - 2's in slotPrev.
-// Systems that paused inside the chunk already hold their state.
-template <int NT>
-__global__ void __launch_bounds__(NT)
-k_fin_pf_chunk(const double2 *__restrict__ slotLast, const double2 *__restrict__ slotPrev, int nb, int n,
-               CgState *__restrict__ st, int *__restrict__ active) {
-    __shared__ double red[3 * NT / kWave];
-    CgState &S = st[blockIdx.x];
-    if (S.done) return;
-    const Pf3 s = sum_pf_partials<NT>(slotLast + 2 * (size_t)blockIdx.x * nb, nb, red);
-    __syncthreads();
-    const Pf3 before = sum_pf_partials<NT>(slotPrev + 2 * (size_t)blockIdx.x * nb, nb, red);
-    if (threadIdx.x) return;
-    S.iter = S.iter0 + n;
-    const PfStep d = pf_decide(s, S.iter, pf_head(S));
-    S.rr_prev = before.rho;
-    S.rr = s.rho;
-    if (d.stop) {
-        S.done = 1;
-        atomicSub(active, 1);
-    }
-}
-
 // one wave per system for few partials, 1024 threads once a system has more partials
 // than four rounds of 256 threads cover
 inline void launch_fin_pf(Ctx &c, int nsys, int nb, int commit, const double2 *part) {
@@ -459,13 +435,14 @@ inline void launch_fin_pf(Ctx &c, int nsys, int nb, int commit, const double2 *p
 // launch) the even launch's deferred term alpha_{m-1} p_{m-2} is added too, with the alpha
 // it recorded in ab.
 [[maybe_unused]] static __global__ void __launch_bounds__(kPfNT)
-k_pf_reliable(int n, const CgState *__restrict__ st, double2 *__restrict__ x, float2 *__restrict__ xs,
+k_pf_reliable(int n, int chunk, const CgState *__restrict__ st, double2 *__restrict__ x, float2 *__restrict__ xs,
               const float2 *__restrict__ p1, const float2 *__restrict__ p2, float2 *__restrict__ p0) {
     const int sys = blockIdx.y;
     if (st[sys].final_) return;
     const int s = blockIdx.x * kPfNT + threadIdx.x;
     if (s >= n) return;
-    const int m = st[sys].iter - st[sys].iter0, slot = m >= 1 ? (m - 1) % 3 : 0;
+    // (a chunk of prologue-finalized launches that no stop has ended is still to be recorded)
+    const int m = chunk && !st[sys].done ? chunk : st[sys].iter - st[sys].iter0, slot = m >= 1 ? (m - 1) % 3 : 0;
     const float2 *src = slot == 1 ? p1 : slot == 2 ? p2 : p0;
     const double a = (m & 1) ? st[sys].ab[(m - 1) & 1].x : 0.0;
     const size_t off = (size_t)sys * 2 * n;
@@ -483,19 +460,49 @@ k_pf_reliable(int n, const CgState *__restrict__ st, double2 *__restrict__ x, fl
     }
 }
 
-// after the reliable update of the pipelined iteration: partRes = |b_e - S x_e|^2 and
+// What ends a chunk of n launches that finalized each other in their prologues: launch n - 1's
+// partials in slot 1, launch n - 2's in slot 0 (n is even), nb per system.  n = 0: a finalize launch
+// followed each.
+struct PfChunkEnd {
+    int n, nb;
+    const double2 *last, *before;
+};
+inline PfChunkEnd pf_chunk_end(const Ctx &c, int n) {
+    if (!c.eoFinFused) return {0, 0, nullptr, nullptr};
+    return {n, c.eoPfBlocks, c.pfSlot[1], c.pfSlot[0]};
+}
+
+// The decision that ends a chunk, and the one after its reliable update, one block per system.  The
+// first takes the place of a prologue after launch n - 1 (end.n > 0; systems that paused inside the
+// chunk already hold their state).  Reliable update: partRes = |b_e - S x_e|^2 and
 // partN = |S^T (b_e - S x_e)|^2 (the new normal residual).  Converged on the system residual, or resume with alpha = 0 (r already is the true
 // residual) and beta = |r_true|^2 / |r_prev|^2 (the direction is kept)
 [[maybe_unused]] static __global__ void __launch_bounds__(kPfNT)
 k_fin_pf_true(const double2 *__restrict__ partRes, const double2 *__restrict__ partN, int nb,
-                 CgState *__restrict__ st, int *__restrict__ active) {
+                 CgState *__restrict__ st, int *__restrict__ active, PfChunkEnd end) {
     __shared__ double2 lds0[kPfNT / kWave], lds1[kPfNT / kWave];
+    __shared__ double red[2][3 * kPfNT / kWave];
     const int sys = blockIdx.x;
-    const int skip = st[sys].final_;
+    const int skip = st[sys].final_, paused = st[sys].done;
+    if (skip) return;
+    Pf3 s{}, before{};
+    if (end.n && !paused) {
+        s = sum_pf_partials<kPfNT>(end.last + 2 * (size_t)sys * end.nb, end.nb, red[0]);
+        before = sum_pf_partials<kPfNT>(end.before + 2 * (size_t)sys * end.nb, end.nb, red[1]);
+    }
     const double2 res = pf_fin_sum(partRes + (size_t)sys * nb, nb, lds0);
     const double2 rn = pf_fin_sum(partN + (size_t)sys * nb, nb, lds1);
-    if (skip || threadIdx.x) return;
+    if (threadIdx.x) return;
     CgState &S = st[sys];
+    if (end.n && !paused) {
+        S.iter = S.iter0 + end.n;
+        S.rr_prev = before.rho;
+        S.rr = s.rho;
+        if (pf_decide(s, S.iter, pf_head(S)).stop) {
+            S.done = 1;
+            atomicSub(active, 1);
+        }
+    }
     S.true_rel = S.enorm2 > 0.0 ? sqrt(res.x / S.enorm2) : sqrt(res.x);
     S.restarts += 1;
     if (S.nRu < kMaxRounds) S.ruIter[S.nRu] = S.iter;
@@ -602,12 +609,6 @@ inline int persistent_grid(int resident, int tiles) {
 inline float2 *pf_dir(const Ctx &c, int k) {
     float2 *const rot[3] = {c.ps[0], c.ps[1], c.pfP2};
     return rot[(k + 1) % 3];
-}
-
-// after a chunk of n prologue-finalized launches (n even: launch n - 1 wrote slot 1)
-inline void launch_fin_pf_chunk(Ctx &c, int nsys, int n) {
-    hipLaunchKernelGGL(k_fin_pf_chunk<kPfNT>, dim3(nsys), dim3(kPfNT), 0, c.stream, (const double2 *)c.pfSlot[(n - 1) & 1],
-                       (const double2 *)c.pfSlot[n & 1], c.eoPfBlocks, n, c.cg_d, c.active);
 }
 
 // Length of the next chunk: the reliable-update interval until the predicted iteration

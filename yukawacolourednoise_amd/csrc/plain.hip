@@ -724,7 +724,6 @@ int pl_iterations(Ctx &c, int nsys, int mtype, int n) {
     });
     if (rc) return rc;
     c.eoPfBlocks = pl_blocks(c, pl_tile(c.tilePl));
-    if (c.eoFinFused) launch_fin_pf_chunk(c, nsys, n);
     return YCN_OK;
 }
 
