@@ -33,3 +33,11 @@ def test_generated_field(gpu, Nt, Nx):
     with Y.Context(p) as c:
         got = c.coloured_noise(2 ** 33 + 1)
     assert rel(got, O.coloured_noise(orc, 2 ** 33 + 1)) < RTOL
+
+
+@pytest.mark.parametrize("Nt,Nx,s,chains", [(40, 48, 1.0, 1), (96, 160, 0.7, 2), (128, 256, 0.5, 1), (512, 64, 1.0, 1),
+                                            (6, 1024, 0.4, 3), (320, 2048, 0.3, 1), (1536, 34, 1.0, 1)])
+def test_powers_of_two(gpu, Nt, Nx, s, chains):
+    """Every split of a power of two 2^3 ... 2^11 into radix-8 and radix-4 passes, alone and with an
+    odd factor, with blocks of 64 to 512 threads."""
+    test_filter_plans(gpu, Nt, Nx, s, chains)

@@ -1,7 +1,7 @@
 // noise.hip -- coloured noise on gfx950 (replaces ColouredNoise,
 // code/src/colouredNoise.cpp:16-29,40-67,138-178, and its cuFFT D2Z/Z2D calls).
 //
-// Mixed-radix Stockham FFTs in LDS (radix 16, 8, 4, 2, 3, 5 and 7 butterflies in registers,
+// Mixed-radix Stockham FFTs in LDS (radix 8, 4, 2, 3, 5 and 7 butterflies in registers,
 // any other prime by a direct DFT), in three passes:
 //   rows_fwd : Philox N(0,1) field generated in registers, rows t and t+1 packed as
 //              z = xi_t + i xi_{t+1}, forward FFT along x, untangled into the two
@@ -17,11 +17,15 @@
 // Algorithmic HBM traffic ~ 8 (rows_fwd write) + 16 (cols r/w) + 8 + 8 (rows_inv)
 // = 40 bytes per site.
 //
-// What bounds it is latency: at 1024 x 1024 a pass holds 512 lines of 1024 points, four
-// waves per CU at 8 points per thread, and each FFT pass is an LDS round trip, a barrier and
-// a twiddle load.  So the passes are few (1024 = 16 x 8 x 8), index divisions are
-// multiplications, LDS rows are padded against the power-of-two strides of the first pass,
-// and a launch has as many blocks as lines allow.
+// What bounds it is latency: at 1024 x 1024 a pass holds 512 lines of 1024 points, four to eight
+// waves per CU, and each FFT pass is a chain of an LDS read, a twiddle load, a butterfly, an LDS
+// write and a barrier.  So butterflies are of radix 8 and 4, whose instructions spread over the
+// block's lanes (a radix-16 one is 660 instructions of one lane, and 64 of them hold a line of
+// 1024), a thread requests all it needs from memory before it waits, blocks have a thread per two
+// points, index divisions are multiplications and LDS rows are padded against power-of-two strides.
+// A field into a device buffer, before these choices (radix 16, eight points per thread, a load at a
+// time) and with them: 1024 x 1024 50.0 -> 43.6 us (columns 18, rows forward 13, rows inverse 9),
+// 512 x 512 36.9 -> 27.8, 256 x 256 42.3 -> 24.8, four of 256 x 480 45.9 -> 30.7.
 #include <math.h>
 
 #include <algorithm>
@@ -34,6 +38,11 @@
 namespace ycn {
 
 constexpr int kFftThreads = 256;
+constexpr int kLineThreads = 512;   // most threads of a block of the line passes
+// The launches never fill a SIMD with more than four waves: registers for loads in flight instead
+// (left to itself the compiler keeps to 62 of 128 and waits for each load: 512 x 512 34.9 us a
+// field against 27.8)
+#define YCN_FOUR_WAVES __attribute__((amdgpu_waves_per_eu(4, 4)))
 constexpr int kFftLdsBytes = 73760;  // two padded ping-pong buffers per block (one line of 2048)
 
 // ---------------------------------------------------------------------------
@@ -98,28 +107,6 @@ __device__ __forceinline__ void dft(double2 (&v)[R]) {
         }
 #pragma unroll
         for (int k = 0; k < 8; ++k) v[k] = o[k];
-    } else if constexpr (R == 16) {
-        // 4 x 4: columns, twiddles exp(-2 pi i n k / 16), rows
-        constexpr double h = 0.70710678118654752440, c = 0.92387953251128675613, d = 0.38268343236508977173;
-#pragma unroll
-        for (int n = 0; n < 4; ++n) dft4<INV>(v[n], v[n + 4], v[n + 8], v[n + 12]);
-        v[5] = twid<INV>(v[5], make_double2(c, -d));
-        v[9] = twid<INV>(v[9], make_double2(h, -h));
-        v[13] = twid<INV>(v[13], make_double2(d, -c));
-        v[6] = twid<INV>(v[6], make_double2(h, -h));
-        v[10] = rot<INV>(v[10]);
-        v[14] = twid<INV>(v[14], make_double2(-h, -h));
-        v[7] = twid<INV>(v[7], make_double2(d, -c));
-        v[11] = twid<INV>(v[11], make_double2(-h, -h));
-        v[15] = twid<INV>(v[15], make_double2(-c, d));
-#pragma unroll
-        for (int k = 0; k < 4; ++k) dft4<INV>(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
-        // X[k1 + 4 k2] sits at v[4 k1 + k2]: transpose
-        double2 o[16];
-#pragma unroll
-        for (int k = 0; k < 16; ++k) o[k] = v[4 * (k & 3) + (k >> 2)];
-#pragma unroll
-        for (int k = 0; k < 16; ++k) v[k] = o[k];
     } else {
         // odd prime: pairs q, R - q
         constexpr int M = (R - 1) / 2;
@@ -213,7 +200,6 @@ __device__ double2 *lds_fft(double2 *a, double2 *b, int lines, const FftPlan &P)
     for (int f = 0; f < P.nf; ++f) {
         const FftPass &F = P.pass[f];
         switch (F.R) {
-        case 16: fft_pass<16, INV>(a, b, lines, row, F, P.tw); break;
         case 8: fft_pass<8, INV>(a, b, lines, row, F, P.tw); break;
         case 4: fft_pass<4, INV>(a, b, lines, row, F, P.tw); break;
         case 2: fft_pass<2, INV>(a, b, lines, row, F, P.tw); break;
@@ -271,6 +257,29 @@ __device__ __forceinline__ void load_rows(double2 *a, const double *__restrict__
     }
 }
 
+// use(w, get(w)) for every w < n that is this thread's; U values are requested before any is used,
+// so that a thread waits for memory once per U
+template <int U, typename T, typename Get, typename Use>
+__device__ __forceinline__ void batched(int n, Get get, Use use) {
+    for (int base = threadIdx.x; base < n; base += U * blockDim.x) {
+        T v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int w = base + u * blockDim.x;
+            if (w < n) v[u] = get(w);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int w = base + u * blockDim.x;
+            if (w < n) use(w, v[u]);
+        }
+    }
+}
+
+struct RowPair {
+    double2 A, B;
+};
+
 // the half spectra of rows t0, t0 + 1 at column k from their packed transform (a line)
 __device__ __forceinline__ void untangle(const double2 *line, int k, int Nx, double2 &A, double2 &B) {
     // A = (Z_k + conj Z_-k)/2 ; B = (Z_k - conj Z_-k)/(2i)
@@ -290,7 +299,7 @@ __device__ __forceinline__ void retangle(double2 *line, int k, int Nx, double2 A
 // pass 1: Philox field + forward row FFTs (two rows per complex transform)
 // grid: (ceil(Nt / (2*lpb)), nRep)
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(kFftThreads)
+__global__ void __launch_bounds__(kLineThreads) YCN_FOUR_WAVES
 k_noise_rows_fwd(const double *__restrict__ xi, const uint64_t *__restrict__ seeds, uint64_t step,
                  double2 *__restrict__ spec, int Nt, int Nx, int H, int nk, int lpb, FftPlan P, const StepCtl *ctl) {
     extern __shared__ double2 lds[];
@@ -323,7 +332,7 @@ k_noise_rows_fwd(const double *__restrict__ xi, const uint64_t *__restrict__ see
 // grid: (ceil(nk / lpb), nRep).  Neighbouring column groups share the cache lines of their
 // rows, so blocks are handed to the 8 XCDs in contiguous bands of groups.
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(kFftThreads)
+__global__ void __launch_bounds__(kLineThreads) YCN_FOUR_WAVES
 k_noise_cols(double2 *__restrict__ spec, const int *__restrict__ kmax, int nk, double invV, int Nt, int H, int lpb,
              FftPlan P, const StepCtl *ctl) {
     extern __shared__ double2 lds[];
@@ -338,18 +347,26 @@ k_noise_cols(double2 *__restrict__ spec, const int *__restrict__ kmax, int nk, d
     const int nl = min(lpb, nk - k0);
     double2 *s = spec + (size_t)rep * Nt * H;
     const float inv = 1.0f / (float)lpb;
-    for (int w = threadIdx.x; w < lpb * Nt; w += blockDim.x) {
-        const int t = fast_div(w, inv), l = w - t * lpb;
-        a[l * row + fft_at(t)] = (l < nl) ? s[(size_t)t * H + k0 + l] : make_double2(0.0, 0.0);
-    }
+    batched<8, double2>(
+        lpb * Nt,
+        [&](int w) {
+            const int t = fast_div(w, inv), l = w - t * lpb;
+            return l < nl ? s[(size_t)t * H + k0 + l] : make_double2(0.0, 0.0);
+        },
+        [&](int w, double2 v) {
+            const int t = fast_div(w, inv), l = w - t * lpb;
+            a[l * row + fft_at(t)] = v;
+        });
     __syncthreads();
     double2 *res = lds_fft<false>(a, b, lpb, P);
     double2 *oth = (res == a) ? b : a;
-    for (int w = threadIdx.x; w < lpb * Nt; w += blockDim.x) {
-        const int kt = fast_div(w, inv), l = w - kt * lpb;
-        const int at = l * row + fft_at(kt);
-        res[at] = cscl((k0 + l <= kmax[kt]) ? invV : 0.0, res[at]);
-    }
+    batched<8, int>(
+        lpb * Nt, [&](int w) { return kmax[fast_div(w, inv)]; },
+        [&](int w, int km) {
+            const int kt = fast_div(w, inv), l = w - kt * lpb;
+            const int at = l * row + fft_at(kt);
+            res[at] = cscl(k0 + l <= km ? invV : 0.0, res[at]);
+        });
     __syncthreads();
     const double2 *fin = lds_fft<true>(res, oth, lpb, P);
     for (int w = threadIdx.x; w < lpb * Nt; w += blockDim.x) {
@@ -361,7 +378,7 @@ k_noise_cols(double2 *__restrict__ spec, const int *__restrict__ kmax, int nk, d
 // ---------------------------------------------------------------------------
 // pass 3: inverse row FFTs (C2R), two rows per complex transform
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(kFftThreads)
+__global__ void __launch_bounds__(kLineThreads) YCN_FOUR_WAVES
 k_noise_rows_inv(const double2 *__restrict__ spec, double *__restrict__ noise, int Nt, int Nx, int H, int nk, int lpb,
                  FftPlan P, const StepCtl *ctl) {
     extern __shared__ double2 lds[];
@@ -372,16 +389,22 @@ k_noise_rows_inv(const double2 *__restrict__ spec, double *__restrict__ noise, i
     const int pair0 = blockIdx.x * lpb;
     const double2 *s = spec + (size_t)rep * Nt * H;
     const float inv = 1.0f / (float)H;
-    for (int w = threadIdx.x; w < lpb * H; w += blockDim.x) {
-        const int l = fast_div(w, inv), k = w - l * H;
-        const int t0 = 2 * (pair0 + l);
-        double2 A = make_double2(0.0, 0.0), B = A;
-        if (t0 < Nt && k < nk) {
-            A = s[(size_t)t0 * H + k];
-            if (t0 + 1 < Nt) B = s[(size_t)(t0 + 1) * H + k];
-        }
-        retangle(a + l * row, k, Nx, A, B);
-    }
+    batched<4, RowPair>(
+        lpb * H,
+        [&](int w) {
+            const int l = fast_div(w, inv), k = w - l * H;
+            const int t0 = 2 * (pair0 + l);
+            RowPair v = {make_double2(0.0, 0.0), make_double2(0.0, 0.0)};
+            if (t0 < Nt && k < nk) {
+                v.A = s[(size_t)t0 * H + k];
+                if (t0 + 1 < Nt) v.B = s[(size_t)(t0 + 1) * H + k];
+            }
+            return v;
+        },
+        [&](int w, RowPair v) {
+            const int l = fast_div(w, inv), k = w - l * H;
+            retangle(a + l * row, k, Nx, v.A, v.B);
+        });
     __syncthreads();
     const double2 *res = lds_fft<true>(a, b, lpb, P);
     double *o = noise + (size_t)rep * Nt * Nx;
@@ -403,7 +426,7 @@ k_noise_rows_inv(const double2 *__restrict__ spec, double *__restrict__ noise, i
 // ---------------------------------------------------------------------------
 constexpr int kOneThreads = 512;
 constexpr int kOneLdsBytes = 81920;
-__global__ void __launch_bounds__(kOneThreads)
+__global__ void __launch_bounds__(kOneThreads) YCN_FOUR_WAVES
 k_noise_one(const double *__restrict__ xi, const uint64_t *__restrict__ seeds, uint64_t step,
             const int *__restrict__ kmax, int nk, double invV, double *__restrict__ noise, int Nt, int Nx, int cap,
             FftPlan PX, FftPlan PT, const StepCtl *ctl) {
@@ -473,10 +496,10 @@ __global__ void __launch_bounds__(kFftThreads) k_twiddles(double2 *__restrict__ 
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
-// Passes of a transform of length n, its power of two first.  Long lines: as few passes as
-// radix 16 and 8 give (1024 = 16 x 8 x 8).  Lines of up to 32: radix 4, since a short line's
-// radix-16 butterfly is 660 instructions of one thread while the block's others idle (16 x 16:
-// 13.5 -> 10.0 us a field; 64 x 64 prefers 8 x 8, 22.5 us against 23.3).  Then 3, 5, 7 and the other odd primes (direct DFTs).  false if more
+// Passes of a transform of length n, its power of two first: radix 8 with one or two of radix 4, or
+// radix 4 alone for lines of up to 32, where a radix-8 butterfly leaves most lanes idle (256 x 256:
+// 26.0 us a field with radix 4 alone, 24.8 so, 35.7 with radix 16; 512 x 512 31.2, 27.8, 28.3;
+// 64 x 64 23.3, 20.3, 20.4).  Then 3, 5, 7 and the other odd primes (direct DFTs).  false if more
 // than kMaxFactors are needed.
 static bool factor_plan(int n, FftPlan &P) {
     P.n = n;
@@ -502,13 +525,10 @@ static bool factor_plan(int n, FftPlan &P) {
     if (n <= 32 || e <= 2) {
         for (; e >= 2; e -= 2) put(4);
         if (e) put(2);
-    } else if (e == 5) {
-        put(8);
-        put(4);
     } else {
-        // passes of 3 and 4 bits: p = ceil(e / 4) passes, the first e - 3 p of them radix 16
-        const int p = (e + 3) / 4, wide = e - 3 * p;
-        for (int k = 0; k < p; ++k) put(k < wide ? 16 : 8);
+        int fours = e % 3 == 1 ? 2 : e % 3 == 2 ? 1 : 0;   // 2^e = 8 ... 8 x 4 ... 4
+        for (e -= 2 * fours; e > 0; e -= 3) put(8);
+        for (; fours > 0; --fours) put(4);
     }
     for (int q = 3; m > 1; q += 2)
         while (m % q == 0) {
@@ -578,9 +598,10 @@ static int lines_per_block(int n, int lines, int least) {
     const int most = std::max(1, kFftLdsBytes / (2 * (int)sizeof(double2) * fft_row(n)));
     return std::min(most, std::max(least, lines / 512));
 }
-// threads of such a block: eight points each, the register butterflies' usual share
+// threads of such a block: two points each, so that the generation, the loads and the stores are
+// short chains; the radix-8 butterflies then leave half of the lanes idle
 static int fft_threads(int points) {
-    return std::min(kFftThreads, std::max(kWave, (points / 8 + kWave - 1) / kWave * kWave));
+    return std::min(kLineThreads, std::max(kWave, (points / 2 + kWave - 1) / kWave * kWave));
 }
 // entries of one LDS buffer of the one-block form
 static int one_block_entries(int Nt, int Nx, int nk) {
