@@ -173,7 +173,8 @@ __device__ __forceinline__ void fft_pass(const double2 *a, double2 *b, int lines
 
 // any other prime factor: one thread per output, a direct sum of R terms
 template <bool INV>
-__device__ void fft_pass_prime(const double2 *a, double2 *b, int lines, const FftPlan &P, const FftPass &F) {
+__device__ void fft_pass_prime(const double2 *a, double2 *b, int lines, const FftPlan &P, const FftPass &F,
+                               const double2 *__restrict__ tw) {
     const int n = P.n, R = F.R, Ns = F.Ns, nb = F.nb, tstride = F.tstride, row = fft_row(n);
     for (int w = threadIdx.x; w < n * lines; w += blockDim.x) {
         const int line = w / n, o = w - line * n;
@@ -187,7 +188,7 @@ __device__ void fft_pass_prime(const double2 *a, double2 *b, int lines, const Ff
         for (int q = 1; q < R; ++q) {
             e += step;
             if (e >= n) e -= n;
-            acc = cadd(acc, twid<INV>(in[fft_at(j + q * nb)], P.tw[e]));
+            acc = cadd(acc, twid<INV>(in[fft_at(j + q * nb)], tw[e]));
         }
         b[line * row + fft_at(o)] = acc;
     }
@@ -195,18 +196,18 @@ __device__ void fft_pass_prime(const double2 *a, double2 *b, int lines, const Ff
 
 // transforms a (barrier before and after); returns the buffer holding the result (a or b)
 template <bool INV>
-__device__ double2 *lds_fft(double2 *a, double2 *b, int lines, const FftPlan &P) {
+__device__ __forceinline__ double2 *lds_fft(double2 *a, double2 *b, int lines, const FftPlan &P, const double2 *tw) {
     const int row = fft_row(P.n);
     for (int f = 0; f < P.nf; ++f) {
         const FftPass &F = P.pass[f];
         switch (F.R) {
-        case 8: fft_pass<8, INV>(a, b, lines, row, F, P.tw); break;
-        case 4: fft_pass<4, INV>(a, b, lines, row, F, P.tw); break;
-        case 2: fft_pass<2, INV>(a, b, lines, row, F, P.tw); break;
-        case 3: fft_pass<3, INV>(a, b, lines, row, F, P.tw); break;
-        case 5: fft_pass<5, INV>(a, b, lines, row, F, P.tw); break;
-        case 7: fft_pass<7, INV>(a, b, lines, row, F, P.tw); break;
-        default: fft_pass_prime<INV>(a, b, lines, P, F); break;
+        case 8: fft_pass<8, INV>(a, b, lines, row, F, tw); break;
+        case 4: fft_pass<4, INV>(a, b, lines, row, F, tw); break;
+        case 2: fft_pass<2, INV>(a, b, lines, row, F, tw); break;
+        case 3: fft_pass<3, INV>(a, b, lines, row, F, tw); break;
+        case 5: fft_pass<5, INV>(a, b, lines, row, F, tw); break;
+        case 7: fft_pass<7, INV>(a, b, lines, row, F, tw); break;
+        default: fft_pass_prime<INV>(a, b, lines, P, F, tw); break;
         }
         __syncthreads();
         double2 *tmp = a;
@@ -214,6 +215,10 @@ __device__ double2 *lds_fft(double2 *a, double2 *b, int lines, const FftPlan &P)
         b = tmp;
     }
     return a;
+}
+template <bool INV>
+__device__ __forceinline__ double2 *lds_fft(double2 *a, double2 *b, int lines, const FftPlan &P) {
+    return lds_fft<INV>(a, b, lines, P, P.tw);
 }
 
 // Row pairs pair0 .. pair0 + np - 1 of the white field into the LDS lines a: from xi, or
@@ -426,6 +431,8 @@ k_noise_rows_inv(const double2 *__restrict__ spec, double *__restrict__ noise, i
 // ---------------------------------------------------------------------------
 constexpr int kOneThreads = 512;
 constexpr int kOneLdsBytes = 81920;
+// TW: with the twiddle tables behind the buffers, one entry per thread
+template <bool TW>
 __global__ void __launch_bounds__(kOneThreads) YCN_FOUR_WAVES
 k_noise_one(const double *__restrict__ xi, const uint64_t *__restrict__ seeds, uint64_t step,
             const int *__restrict__ kmax, int nk, double invV, double *__restrict__ noise, int Nt, int Nx, int cap,
@@ -439,30 +446,46 @@ k_noise_one(const double *__restrict__ xi, const uint64_t *__restrict__ seeds, u
     noise += (size_t)blockIdx.y * gridDim.x * Nt * Nx;
     const int rep = blockIdx.x, np = (Nt + 1) / 2, H = Nx / 2 + 1, rowX = fft_row(Nx), rowT = fft_row(Nt);
     double2 *a = lds, *b = lds + cap;
+    const double2 *twX = PX.tw, *twT = PT.tw;
+    double2 wx, wt;
+    if constexpr (TW) {   // requested here, in LDS once the field is made
+        if ((int)threadIdx.x < Nx) wx = PX.tw[threadIdx.x];
+        if ((int)threadIdx.x < Nt) wt = PT.tw[threadIdx.x];
+    }
     load_rows(a, xi ? xi + (size_t)rep * Nt * Nx : nullptr, seeds[rep], step, 0, np, Nt, Nx);
+    if constexpr (TW) {
+        double2 *const w = lds + 2 * cap;
+        if ((int)threadIdx.x < Nx) w[threadIdx.x] = wx;
+        if ((int)threadIdx.x < Nt) w[Nx + threadIdx.x] = wt;
+        twX = w;
+        twT = w + Nx;
+    }
     __syncthreads();
-    double2 *res = lds_fft<false>(a, b, np, PX);
+    double2 *res = lds_fft<false>(a, b, np, PX, twX);
     double2 *oth = (res == a) ? b : a;
+    const float invK = 1.0f / (float)nk, invT = 1.0f / (float)Nt, invH = 1.0f / (float)H, invX = 1.0f / (float)Nx;
     for (int w = threadIdx.x; w < np * nk; w += blockDim.x) {
-        const int l = w / nk, k = w - l * nk;
+        const int l = fast_div(w, invK), k = w - l * nk;
         double2 A, B;
         untangle(res + l * rowX, k, Nx, A, B);
         oth[k * rowT + fft_at(2 * l)] = A;
         if (2 * l + 1 < Nt) oth[k * rowT + fft_at(2 * l + 1)] = B;
     }
     __syncthreads();
-    double2 *col = lds_fft<false>(oth, res, nk, PT);
+    double2 *col = lds_fft<false>(oth, res, nk, PT, twT);
     oth = (col == oth) ? res : oth;
-    for (int w = threadIdx.x; w < nk * Nt; w += blockDim.x) {
-        const int k = w / Nt, kt = w - k * Nt;
-        const int at = k * rowT + fft_at(kt);
-        col[at] = cscl((k <= kmax[kt]) ? invV : 0.0, col[at]);
-    }
+    batched<4, int>(
+        nk * Nt, [&](int w) { return kmax[w - fast_div(w, invT) * Nt]; },
+        [&](int w, int km) {
+            const int k = fast_div(w, invT), kt = w - k * Nt;
+            const int at = k * rowT + fft_at(kt);
+            col[at] = cscl((k <= km) ? invV : 0.0, col[at]);
+        });
     __syncthreads();
-    double2 *fin = lds_fft<true>(col, oth, nk, PT);
+    double2 *fin = lds_fft<true>(col, oth, nk, PT, twT);
     oth = (fin == a) ? b : a;
     for (int w = threadIdx.x; w < np * H; w += blockDim.x) {
-        const int l = w / H, k = w - l * H;
+        const int l = fast_div(w, invH), k = w - l * H;
         double2 A = make_double2(0.0, 0.0), B = A;
         if (k < nk) {
             A = fin[k * rowT + fft_at(2 * l)];
@@ -471,10 +494,10 @@ k_noise_one(const double *__restrict__ xi, const uint64_t *__restrict__ seeds, u
         retangle(oth + l * rowX, k, Nx, A, B);
     }
     __syncthreads();
-    const double2 *out = lds_fft<true>(oth, fin, np, PX);
+    const double2 *out = lds_fft<true>(oth, fin, np, PX, twX);
     double *o = noise + (size_t)rep * Nt * Nx;
     for (int w = threadIdx.x; w < np * Nx; w += blockDim.x) {
-        const int l = w / Nx, x = w - l * Nx;
+        const int l = fast_div(w, invX), x = w - l * Nx;
         const double2 z = out[l * rowX + fft_at(x)];
         o[(size_t)(2 * l) * Nx + x] = z.x;
         if (2 * l + 1 < Nt) o[(size_t)(2 * l + 1) * Nx + x] = z.y;
@@ -660,8 +683,13 @@ static int launch_noise(hipStream_t s, int Nt, int Nx, int nRep, const double *x
     const size_t shOne = (size_t)2 * cap * sizeof(double2);
     if (shOne <= (size_t)kOneLdsBytes) {
         if (prof) prof_before(*prof, PK_NOISE_COLS, 40.0 * (double)nRep * Nt * Nx);
-        hipLaunchKernelGGL(k_noise_one, dim3(nRep, nsteps), dim3(kOneThreads), shOne, s, xi_dev, seeds, step, kmax, nk, invV,
-                           out_dev, Nt, Nx, cap, planX, planT, ctl);
+        // its twiddles in LDS too, where they leave room for a second block (a pass then waits for
+        // LDS instead of the caches: 12 of 45 x 50 19.6 -> 18.5 us, 5 of 64 x 64 20.6 -> 19.4)
+        const size_t shTw = shOne + (size_t)(Nx + Nt) * sizeof(double2);
+        const bool tw = shTw <= (size_t)kOneLdsBytes && std::max(Nx, Nt) <= kOneThreads;
+        hipLaunchKernelGGL(tw ? &k_noise_one<true> : &k_noise_one<false>, dim3(nRep, nsteps), dim3(kOneThreads),
+                           tw ? shTw : shOne, s, xi_dev, seeds, step, kmax, nk, invV, out_dev, Nt, Nx, cap, planX,
+                           planT, ctl);
         if (prof) prof_after(*prof, PK_NOISE_COLS);
         return hipGetLastError() == hipSuccess ? YCN_OK : YCN_ERR_HIP;
     }
