@@ -1283,23 +1283,30 @@ static std::vector<int> eo_main_chunks(const Ctx &c, int pred) {
 // The chunk schedule of a captured step: one chunk per reliable update of the previous
 // solve (its longest system), each as long as that solve's round (the iterations between
 // two reliable updates: up to a pause for the residual drop, to the stop, or to the end of
-// an eager chunk) plus 2, rounded up to a multiple of 8 (so that consecutive solves mostly
-// share one schedule and its captured graphs), then `tail` chunks of 8.  A
+// an eager chunk) plus 2, rounded up to a multiple of 4, then `tail` chunks of 8.  The last
+// schedule stays while it covers that with at most 7 launches to spare per round, so that
+// consecutive solves mostly share one and its captured graphs.  (A launch after the systems have
+// paused costs about 2 us: of the 56 of a 256 x 256 step with multiples of 8, 18 did.)  A
 // round of this solve that ends a little later than the previous one's ends at the chunk
 // boundary instead and the rest moves to the next round; a solve that needs more than
 // the schedule holds halts the run.
 constexpr int kTailRound = 8;
-static std::vector<int> eo_schedule(const Ctx &c, int tail) {
+static std::vector<int> eo_schedule(Ctx &c, int tail) {
     std::vector<int> v;
     if (c.eoRounds.empty()) {
         v = eo_main_chunks(c, c.eoPredIters);
     } else {
         int prev = 0, total = 0;
+        bool keep = c.eoRoundChunks.size() == c.eoRounds.size();
         for (int r : c.eoRounds) {
-            v.push_back(std::max(8, (r - prev + 2 + 7) / 8 * 8));
-            total += v.back();
+            const int need = std::max(4, r - prev + 2);
+            if (keep) keep = need <= c.eoRoundChunks[v.size()] && c.eoRoundChunks[v.size()] <= need + 7;
+            v.push_back((need + 3) / 4 * 4);
             prev = r;
         }
+        if (keep) v = c.eoRoundChunks;
+        c.eoRoundChunks = v;
+        for (int n : v) total += n;
         // a solve with more reliable updates than CgState records ends after its last
         // recorded round: chunks of the reliable-update interval up to its iteration count
         if (prev < c.eoPredIters) {
@@ -1373,7 +1380,7 @@ static int eo_step_graph(Ctx &c, int parity, const std::vector<int> &chunks, hip
 }
 
 // While a segment runs on the GPU the host would only wait: it captures the schedules
-// the next segment most likely needs, the current one with one chunk 8 launches shorter
+// the next segment most likely needs, the current one with one chunk 4 launches shorter
 // or longer (the rounds of consecutive solves move by a few iterations), for both field
 // buffers, at most kPrecapture new ones per segment.  They go in at the cache's old end,
 // so that they are evicted before anything the running segment uses.
@@ -1382,8 +1389,8 @@ static int eo_precapture(Ctx &c, const std::vector<int> &chunks, int nTail, bool
     int made = 0;
     const size_t nMain = chunks.size() - (size_t)nTail;
     for (size_t i = 0; i < nMain && made < kPrecapture; ++i)
-        for (int d : {-8, 8}) {
-            if (chunks[i] + d < 8) continue;
+        for (int d : {-4, 4}) {
+            if (chunks[i] + d < 4) continue;
             std::vector<int> v = chunks;
             v[i] += d;
             for (int par = 0; par < (bothParities ? 2 : 1) && made < kPrecapture; ++par) {

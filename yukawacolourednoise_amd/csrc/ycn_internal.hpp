@@ -151,6 +151,7 @@ struct Ctx {
     CgState *cg_h = nullptr;              // pinned host mirror of the CG states
     hipEvent_t pollEv = nullptr;          // spin-waited by the solvers' polls
     int eoPredIters = 0;                  // iterations of the last even-odd mixed solve (chunk predictor)
+    std::vector<int> eoRoundChunks;       // captured steps: the last schedule's chunk per round
     std::vector<int> eoRounds;            // iteration counts at that solve's reliable updates (its longest system)
     double eoStopScale = 1.0;             // starting threshold of even-odd solves / tol |r_0| (relative mode)
     int maxBlocks = 0;
