@@ -287,7 +287,7 @@ class Context:
         return st.as_dict()
 
     def host_syncs(self):
-        """(host waits on the context's work since creation, captured steps the host
+        """(host waits on the context's work since creation, enqueued steps the host
         finished)"""
         n, h = C.c_int64(), C.c_int64()
         self._check(lib.ycn_host_syncs(self._h, C.byref(n), C.byref(h)))

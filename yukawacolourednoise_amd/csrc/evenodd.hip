@@ -1241,12 +1241,15 @@ int eo_drift(Ctx &c, const double *phi, double *drift, const StepCtl *ctl) {
 }
 
 // ---------------------------------------------------------------------------
-// graph-captured Langevin steps
+// Langevin steps without a host wait
 // ---------------------------------------------------------------------------
-// A step replays one captured graph -- the solve's setup, a fixed chunk schedule of the
-// pipelined FP32 iteration with its reliable updates, k_step_check and the drift --
-// between k_step_begin and the coloured noise before it and the update after it, with no
-// host wait.  The schedule repeats the previous solve's rounds (eo_schedule), then `tail`
+// A step is k_step_begin, the coloured noise, the solve -- its setup, a fixed chunk schedule
+// of the pipelined FP32 iteration with its reliable updates, k_step_check -- the drift and
+// the update, all enqueued.  The solve and the drift may also be a captured graph
+// (c.stepCapture), but a replay leaves longer gaps between its kernels than a stream does:
+// sixteen steps at 1024 x 1024 38.4 ms replayed and 36.9 enqueued, 512 x 512 near the chiral
+// point 19.1 and 17.9, 256 x 256 5.43 and 5.14, 128 x 96 11.28 and 11.20; enqueueing keeps
+// the host busy instead (about 100 launches per step).  The schedule repeats the previous solve's rounds (eo_schedule), then `tail`
 // chunks of 8.  A solve that needs more than the schedule holds halts the run
 // (k_step_check): the later steps' kernels return at once except their chunk schedules,
 // which keep iterating the halted solve (its FP32 and FP64 fields stay in c.phis and
@@ -1257,7 +1260,7 @@ int eo_drift(Ctx &c, const double *phi, double *drift, const StepCtl *ctl) {
 // four segments without one.  The field ping-pongs between the context's two buffers with
 // a fixed step size and is updated in place with an adaptive one, so each schedule has at
 // most two executables (one per field buffer).
-constexpr int kStepSegment = 16;   // captured steps between two reads of the control block
+constexpr int kStepSegment = 16;   // steps between two reads of the control block
 constexpr int kMaxTail = 8;
 constexpr size_t kMaxStepGraphs = 48;
 
@@ -1280,7 +1283,7 @@ static std::vector<int> eo_main_chunks(const Ctx &c, int pred) {
     return v;
 }
 
-// The chunk schedule of a captured step: one chunk per reliable update of the previous
+// The chunk schedule of a step: one chunk per reliable update of the previous
 // solve (its longest system), each as long as that solve's round (the iterations between
 // two reliable updates: up to a pause for the residual drop, to the stop, or to the end of
 // an eager chunk) plus 2, rounded up to a multiple of 4, then `tail` chunks of 8.  The last
@@ -1322,13 +1325,11 @@ static std::vector<int> eo_schedule(Ctx &c, int tail) {
     return v;
 }
 
-// the captured part of a step: the solve's setup, its chunk schedule, k_step_check and
-// the drift (the step's noise and update are launched around it by eo_enqueue_step)
-static int eo_capture_step(Ctx &c, int parity, const std::vector<int> &chunks, hipGraphExec_t *out) {
+// a step's solve and drift: the setup, the chunk schedule, k_step_check and the drift (the step's
+// noise and update are launched around it by eo_enqueue_step)
+static int eo_step_body(Ctx &c, int parity, const std::vector<int> &chunks) {
     const double *phiIn = c.phi[parity];
     const int nsys = c.nSys;
-    hipGraph_t g = nullptr;
-    YCN_HIP(hipStreamBeginCapture(c.stream, hipStreamCaptureModeThreadLocal));
     int rc = eo_setup(c, phiIn, nsys, true, 1u, 0, true, c.ctl_d);
     for (int n : chunks)
         if (!rc) rc = eo_mixed_chunk(c, c.phiSolve, nsys, n, true);
@@ -1337,6 +1338,12 @@ static int eo_capture_step(Ctx &c, int parity, const std::vector<int> &chunks, h
                            c.p.cgTolMode == YCN_TOL_REL_TRUE ? 1 : 0);
         rc = eo_drift(c, phiIn, c.drift, c.ctl_d);   // fDrift.getForce(drift)
     }
+    return rc;
+}
+static int eo_capture_step(Ctx &c, int parity, const std::vector<int> &chunks, hipGraphExec_t *out) {
+    hipGraph_t g = nullptr;
+    YCN_HIP(hipStreamBeginCapture(c.stream, hipStreamCaptureModeThreadLocal));
+    int rc = eo_step_body(c, parity, chunks);
     const hipError_t le = hipGetLastError();
     const hipError_t ee = hipStreamEndCapture(c.stream, &g);
     if (rc || le != hipSuccess || ee != hipSuccess) {
@@ -1410,12 +1417,12 @@ static int eo_precapture(Ctx &c, const std::vector<int> &chunks, int nTail, bool
     return YCN_OK;
 }
 
-// One captured step on the context stream, no host wait: k_step_begin, the coloured
+// One step on the context stream, no host wait: k_step_begin, the coloured
 // noise (on the noise stream beside the solve when the context has it, as a single step
-// does: a graph with a second branch measured slower), the captured solve and drift, then
+// does: a graph with a second branch measured slower), the solve and drift (a captured graph where ex is given), then
 // the update once the noise is there.  The noise reads the copy of the halt flag and
 // counter k_step_begin made, so the solve's check kernel cannot change them under it.
-static int eo_enqueue_step(Ctx &c, int parity, hipGraphExec_t ex) {
+static int eo_enqueue_step(Ctx &c, int parity, hipGraphExec_t ex, const std::vector<int> &chunks) {
     const bool fixed = c.p.adaptive == 0;
     double *phiIn = c.phi[parity], *phiOut = fixed ? c.phi[parity ^ 1] : c.phi[parity];
     StepCtl *ctlNoise = c.ctl_d + 1;
@@ -1433,7 +1440,10 @@ static int eo_enqueue_step(Ctx &c, int parity, hipGraphExec_t ex) {
         rc = noise_generate_ctl(c, c.stream, ctlNoise, c.noise);   // cn()
         if (rc) return rc;
     }
-    YCN_HIP(hipGraphLaunch(ex, c.stream));   // fDrift.getForce(drift)
+    if (ex)
+        YCN_HIP(hipGraphLaunch(ex, c.stream));   // fDrift.getForce(drift)
+    else if ((rc = eo_step_body(c, parity, chunks)))
+        return rc;
     if (side) YCN_HIP(hipStreamWaitEvent(c.stream, c.evNoise, 0));
     return bosonic_update_gated(c, fixed ? 1 : 0, phiIn, phiOut, &c.ctl_d->halt);   // kli.Run(kAll)
 }
@@ -1471,14 +1481,14 @@ int eo_graph_run(Ctx &c, uint64_t step0, int nsteps, SolveStats *tot) {
         const std::vector<int> chunks = eo_schedule(c, c.stepTail);
         const int p0 = c.cur;
         hipGraphExec_t ex[2] = {nullptr, nullptr};
-        if ((rc = eo_step_graph(c, p0, chunks, &ex[p0]))) return rc;
-        if (fixed && seg > 1 && (rc = eo_step_graph(c, p0 ^ 1, chunks, &ex[p0 ^ 1]))) return rc;
+        if (c.stepCapture && (rc = eo_step_graph(c, p0, chunks, &ex[p0]))) return rc;
+        if (c.stepCapture && fixed && seg > 1 && (rc = eo_step_graph(c, p0 ^ 1, chunks, &ex[p0 ^ 1]))) return rc;
         for (int i = 0; i < seg; ++i) {
             const int parity = fixed ? p0 ^ (i & 1) : p0;
-            if ((rc = eo_enqueue_step(c, parity, ex[parity]))) return rc;
+            if ((rc = eo_enqueue_step(c, parity, ex[parity], chunks))) return rc;
         }
         YCN_HIP(hipMemcpyAsync(c.ctl_h, c.ctl_d, sizeof(StepCtl), hipMemcpyDeviceToHost, c.stream));
-        if ((rc = eo_precapture(c, chunks, c.stepTail, fixed))) return rc;
+        if (c.stepCapture && (rc = eo_precapture(c, chunks, c.stepTail, fixed))) return rc;
         if ((rc = spin_sync(c))) return rc;
         if (!h.halt) {
             c.cur = fixed ? p0 ^ (seg & 1) : p0;

@@ -257,9 +257,13 @@ int ycn_create(const ycn_params *p, ycn_ctx **out) {
         c.useGraphs = std::atoi(gr) != 0;
     else if (std::getenv("ROCP_TOOL_LIBRARIES"))
         c.useGraphs = false;
-    // YCN_STEP_GRAPHS=0 keeps ycn_langevin_run on single eagerly launched steps (with
-    // captured CG chunks) where it would replay whole captured steps; results are identical
-    if (const char *sg = std::getenv("YCN_STEP_GRAPHS")) c.stepGraphsOn = std::atoi(sg) != 0;
+    // YCN_STEP_GRAPHS=0 keeps ycn_langevin_run on single polled steps (with captured CG chunks)
+    // where it would enqueue whole steps without a host wait, 1 replays their solves as captured
+    // graphs (for hosts too slow to launch a kernel every few us); results are identical
+    if (const char *sg = std::getenv("YCN_STEP_GRAPHS")) {
+        c.stepGraphsOn = std::atoi(sg) != 0;
+        c.stepCapture = c.stepGraphsOn;
+    }
     if ((rc = onchip_init(c))) return bail(rc);
     if ((rc = cg_autotune(c))) return bail(rc);
     if ((rc = pl_autotune(c))) return bail(rc);

@@ -200,7 +200,8 @@ struct Ctx {
         hipGraphExec_t exec;
     };
     std::vector<StepGraph> stepGraphs;
-    bool stepGraphsOn = true;             // YCN_STEP_GRAPHS=0: every step launches eagerly
+    bool stepGraphsOn = true;             // YCN_STEP_GRAPHS=0: every step is polled by the host
+    bool stepCapture = false;             // YCN_STEP_GRAPHS=1: a step's solve is a captured graph
     int stepTail = 1, stepClean = 0;      // tail rounds of the schedule; clean segments since a halt
     int64_t hostSyncs = 0;                // host waits on the context's work since creation
     int64_t haltedSteps = 0;              // captured steps finished by the host
