@@ -143,3 +143,28 @@ def test_many_reliable_updates_per_solve(gpu, monkeypatch):
     assert e < 1e-9, e
     assert hg <= 2, hg
     assert wg < we
+
+
+@pytest.mark.parametrize("n,reps,adaptive,nsteps", [(128, 2, 0, 40), (96, 1, 1, 35)])
+def test_replayed_steps_match_enqueued_steps(gpu, monkeypatch, n, reps, adaptive, nsteps):
+    """YCN_STEP_GRAPHS=1 replays each step's solve as a captured graph instead of enqueueing it: the
+    same field (1e-9, the bar above) from as many host waits."""
+    Y = gpu
+    hot = np.random.default_rng(n).uniform(-1.0, 1.0, (reps, n, n))
+    out = []
+    for replay in (False, True):
+        p, _ = mk(Y, Nt=n, Nx=n, nReplicas=reps, adaptive=adaptive, **C3)
+        p.cgPrecision, p.evenOdd = Y.YCN_CG_MIXED, 1
+        with monkeypatch.context() as m:
+            if replay:
+                m.setenv("YCN_STEP_GRAPHS", "1")
+            else:
+                m.delenv("YCN_STEP_GRAPHS", raising=False)
+            c = Y.Context(p)
+        with c:
+            c.set_replicas(np.full(reps, C3["m2"]), np.arange(11, 11 + reps, dtype=np.uint64))
+            out.append(_run(c, [hot], nsteps))
+    (fe, se, we, he), (fg, sg, wg, hg) = out
+    assert se["converged"] == 1 and sg["converged"] == 1
+    assert l2rel(fg, fe) < 1e-9
+    assert (wg, hg) == (we, he)
