@@ -97,15 +97,37 @@ void tune_store(int kind, const Ctx &c, const std::vector<double> &t) {
 
 }  // namespace ycn
 
-#define CHECK_CTX(ctx)                                  \
-    do {                                                \
-        if (!(ctx)) return YCN_ERR_INVALID;             \
-    } while (0)
-
 static int fail(Ctx &c, int code, const std::string &msg) {
     c.err = msg;
     return code;
 }
+
+// The context's device is the current one while an entry point runs, and the caller's again
+// afterwards: buffers, events and streams made inside a call (the first step's, a measurement's)
+// belong to the current device, and a thread may hold contexts on several.
+class DeviceScope {
+public:
+    explicit DeviceScope(int device) {
+        int now = -1;
+        failed_ = hipGetDevice(&now) != hipSuccess || (now != device && hipSetDevice(device) != hipSuccess);
+        if (!failed_ && now != device) caller_ = now;
+    }
+    ~DeviceScope() {
+        if (caller_ >= 0) (void)hipSetDevice(caller_);
+    }
+    DeviceScope(const DeviceScope &) = delete;
+    DeviceScope &operator=(const DeviceScope &) = delete;
+    bool failed() const { return failed_; }
+
+private:
+    int caller_ = -1;
+    bool failed_ = false;
+};
+
+#define CHECK_CTX(ctx)                              \
+    if (!(ctx)) return YCN_ERR_INVALID;             \
+    const DeviceScope deviceScope((ctx)->p.device); \
+    if (deviceScope.failed()) return fail(*(ctx), YCN_ERR_HIP, "the context's device cannot be made current")
 
 // Copy a host array into a temporary device buffer owned by the caller of this helper.
 struct DevTmp {
@@ -471,8 +493,7 @@ int ycn_fermion_force(ycn_ctx *ctx, uint64_t step, double *drift, ycn_cg_stats *
 // 1024^2), for a cause not yet found; such contexts never create it.
 static int step_impl(Ctx &c, uint64_t step, SolveStats *st) {
     if (c.noiseSide && !c.noiseStream) {
-        if (hipSetDevice(c.p.device) != hipSuccess ||
-            hipStreamCreateWithFlags(&c.noiseStream, hipStreamNonBlocking) != hipSuccess ||
+        if (hipStreamCreateWithFlags(&c.noiseStream, hipStreamNonBlocking) != hipSuccess ||
             hipEventCreateWithFlags(&c.evMain, hipEventDisableTiming) != hipSuccess ||
             hipEventCreateWithFlags(&c.evNoise, hipEventDisableTiming) != hipSuccess) {
             // the side stream is only an overlap: without it the noise stays on the
