@@ -91,6 +91,34 @@ def test_entry_points_use_the_contexts_device(stub, params):
         assert restored, name
 
 
+# ---- the one-workgroup even-odd solve: no two of its buffers are the same memory ---------------
+def onchip_buffers(hip, params):
+    """the buffers of every such launch of a force and of a measurement's propagator"""
+    import yukawacolourednoise_amd as Y
+    hip.stub_watch(b"k_onchip_eo", 13)
+    # k_onchip_eo's arguments after its structure
+    names = ["phi", "seeds", "streamBase", "step", "eta", "b", "drift", "out", "st", "ratioIn", "ratioOut", "nsys"]
+    with Y.Context(Y.default_params(evenOdd=1, **params)) as c:
+        hip.stub_clear()
+        for call in (lambda: c.fermion_force(0), lambda: c.measure(0, 1)):
+            try:
+                call()
+            except Y.YcnError as e:   # nothing ran: no solve converges
+                assert e.code == Y.abi.YCN_ERR_NOT_CONVERGED
+        launches = [x.split()[3:] for x in hip.stub_record().decode().splitlines() if "k_onchip_eo" in x]
+    return [dict(zip(names, map(int, x))) for x in launches]
+
+
+@pytest.mark.parametrize("params", [dict(Nt=16, Nx=16), dict(Nt=64, Nx=64, nReplicas=2, nNoise=3)])
+def test_onchip_even_odd_buffers_are_distinct(stub, params):
+    launches = child(stub, "onchip_buffers", **params)
+    assert sum(x["out"] != 0 for x in launches) == 1   # the propagator's
+    assert len(launches) > 1
+    for x in launches:
+        buffers = [x[k] for k in ("phi", "eta", "b", "drift", "out", "st") if x[k]]
+        assert len(set(buffers)) == len(buffers), x
+
+
 if __name__ == "__main__":
     sys.path.insert(0, ROOT)
     print(json.dumps(globals()[sys.argv[2]](open_stub(sys.argv[1]), json.loads(sys.argv[3]))))

@@ -355,9 +355,10 @@ bool onchip_eo(const Ctx &c) {
     return c.onchip && c.p.evenOdd && eo_available(c) && c.V / 2 <= kOnchipEoSites && c.profTarget == PK_NONE;
 }
 
+// bg: scratch for b_e; no two of bg, drift and out may be the same memory
 template <bool GEN, bool PROP>
-static int launch_eo(Ctx &c, const double *phi, int nsys, uint32_t streamBase, uint64_t step, double *drift,
-                     double2 *out, const double *ratioIn, double *ratioOut) {
+static int launch_eo(Ctx &c, const double *phi, int nsys, uint32_t streamBase, uint64_t step, double2 *bg,
+                     double *drift, double2 *out, const double *ratioIn, double *ratioOut) {
     OnchipEoArgs A;
     A.Nt = c.p.Nt;
     A.Nx = c.p.Nx;
@@ -381,7 +382,8 @@ static int launch_eo(Ctx &c, const double *phi, int nsys, uint32_t streamBase, u
         constexpr int KK = decltype(kTag)::value;
         auto *k = A.r == 1.0 ? &k_onchip_eo<KK, true, GEN, PROP> : &k_onchip_eo<KK, false, GEN, PROP>;
         hipLaunchKernelGGL(k, dim3(nsys), dim3(threads), 2 * EoLds<KK>::bytes, c.stream, A, phi,
-                           (const uint64_t *)c.seed_d, streamBase, step, c.eta, c.t, drift, out, c.cg_d, ratioIn, ratioOut, nsys);
+                           (const uint64_t *)c.seed_d, streamBase, step, c.eta, bg, drift, out, c.cg_d, ratioIn, ratioOut,
+                           nsys);
     };
     if (K == 1)
         go(std::integral_constant<int, 1>());
@@ -400,12 +402,13 @@ int onchip_eo_force(Ctx &c, const double *phi, uint32_t streamBase, uint64_t ste
         c.ratioTurn ^= 1;
         out = c.ratio + row * c.ratioTurn;
     }
-    const int rc = launch_eo<true, false>(c, phi, c.nSys, streamBase, step, onchip_share(c), nullptr, in, out);
+    const int rc = launch_eo<true, false>(c, phi, c.nSys, streamBase, step, c.t, onchip_share(c), nullptr, in, out);
     return rc ? rc : onchip_mean(c);
 }
 
 int onchip_eo_propagator(Ctx &c, const double *phi, double2 *out) {
-    return launch_eo<false, true>(c, phi, 1, 0, 0, nullptr, out, nullptr, nullptr);
+    // (b_e in Ap: the measurement's out is t)
+    return launch_eo<false, true>(c, phi, 1, 0, 0, c.Ap, nullptr, out, nullptr, nullptr);
 }
 
 }  // namespace ycn
