@@ -652,7 +652,7 @@ int pl_autotune(Ctx &c) {
     c.tilePl = c.tileP64 = -1;
     if (c.p.evenOdd || c.p.precond != YCN_PRECOND_NONE || onchip_plain(c)) return YCN_OK;
     const bool mixed = c.p.cgPrecision == YCN_CG_MIXED;
-    if (!mixed && std::getenv("YCN_TILE")) return YCN_OK;   // a forced tile of the unpipelined iteration
+    if (std::getenv(mixed ? "YCN_TILE32" : "YCN_TILE")) return YCN_OK;   // a forced tile of the unpipelined iteration
     const int rc = pl_alloc(c, mixed);
     if (rc || !c.pfSlot[1]) return rc;
     std::vector<double> us;
