@@ -18,6 +18,27 @@ def context(Y, mixed, **kw):
     return Y.Context(p), orc
 
 
+@pytest.mark.parametrize("mixed", [True, False])
+def test_update_kernel_is_timed(gpu, mixed):
+    """"cg_update": the solve under it runs the iteration that has an update kernel, reads x, r, p
+    and Ap and writes x and r (packed spinors, two planes), and gives the same drift."""
+    Y = gpu
+    phi = 1.0 + O.hot_start(4, NT, NX)
+    c, orc = context(Y, mixed)
+    with c:
+        c.set_field(phi)
+        d0, _ = c.fermion_force(2)
+        c.profile_begin("cg_update")
+        d, st = c.fermion_force(2)
+        ms, n, b = c.profile_end()
+        d1, _ = c.fermion_force(2)
+    print(f"# {n} launches for {st['iters']} iterations, {b} bytes", flush=True)
+    assert n >= st["iters"] and ms > 0.0
+    assert b == NT * NX * 6 * 2 * (8 if mixed else 16)
+    dr, _ = O.fermion_drift(orc, phi, 2)
+    assert st["converged"] == 1 and max(rel(x, dr) for x in (d0, d, d1)) < 1e-8
+
+
 @pytest.mark.parametrize("tile", [0, 2, 5])
 def test_forced_fp32_tile_runs(gpu, monkeypatch, tile):
     """YCN_TILE32: the fused normal operator, which reads r, p and phi and writes p and Ap, runs in

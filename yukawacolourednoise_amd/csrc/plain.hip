@@ -643,7 +643,8 @@ static int pl_alloc(Ctx &c, bool mixed) {
     return YCN_OK;
 }
 
-bool pl_available(const Ctx &c) { return c.tilePl >= 0; }
+// (neither has an update kernel of its own to time)
+bool pl_available(const Ctx &c) { return c.tilePl >= 0 && c.profTarget != PK_CG_UPDATE; }
 bool p64_available(const Ctx &c) { return c.tileP64 >= 0 && c.profTarget != PK_CG_UPDATE; }
 
 // The pipelined iteration of the context's precision: times every tile that fits, with either
