@@ -39,6 +39,19 @@ def test_update_kernel_is_timed(gpu, mixed):
     assert st["converged"] == 1 and max(rel(x, dr) for x in (d0, d, d1)) < 1e-8
 
 
+def test_measured_dirac_application_is_timed(gpu):
+    """"dirac": the propagator of a measurement ends with one application, D^dag on a packed spinor."""
+    Y = gpu
+    c, _ = context(Y, False)
+    with c:
+        c.set_field(1.0 + O.hot_start(4, NT, NX))
+        c.profile_begin("dirac")
+        c.measure(0, 1)
+        ms, n, b = c.profile_end()
+    assert n == 1 and ms > 0.0
+    assert b == NT * NX * (2 * 2 * 16 + 8)
+
+
 @pytest.mark.parametrize("tile", [0, 2, 5])
 def test_forced_fp32_tile_runs(gpu, monkeypatch, tile):
     """YCN_TILE32: the fused normal operator, which reads r, p and phi and writes p and Ap, runs in

@@ -789,16 +789,21 @@ int set_int(Ctx &c, int *ptr, int v) {
     return YCN_OK;
 }
 
-int dirac_apply(Ctx &c, const double *phi_dev, const double2 *in, double2 *out, int nsys, int dagger) {
+template <int NC>
+static int dirac_apply_as(Ctx &c, const double *phi_dev, const double2 *in, double2 *out, int nsys, int dagger) {
     const LatticeArgs L = largs(c);
-    prof_before(c, PK_DIRAC, (double)nsys * c.V * (2 * 64 + 8));
+    prof_before(c, PK_DIRAC, (double)nsys * c.V * (2 * 16 * NC + 8));
     if (dagger)
-        hipLaunchKernelGGL((k_dirac<4, true>), site_grid(c, nsys), dim3(kNT), 0, c.stream, L, phi_dev, in, out);
+        hipLaunchKernelGGL((k_dirac<NC, true>), site_grid(c, nsys), dim3(kNT), 0, c.stream, L, phi_dev, in, out);
     else
-        hipLaunchKernelGGL((k_dirac<4, false>), site_grid(c, nsys), dim3(kNT), 0, c.stream, L, phi_dev, in, out);
+        hipLaunchKernelGGL((k_dirac<NC, false>), site_grid(c, nsys), dim3(kNT), 0, c.stream, L, phi_dev, in, out);
     prof_after(c, PK_DIRAC);
     YCN_HIP(hipGetLastError());
     return YCN_OK;
+}
+
+int dirac_apply(Ctx &c, const double *phi_dev, const double2 *in, double2 *out, int nsys, int dagger) {
+    return dirac_apply_as<kComplex>(c, phi_dev, in, out, nsys, dagger);
 }
 
 // p' = r + beta p_old, Ap = A p' and the partials of <p', Ap>: the fused LDS kernel
@@ -1303,10 +1308,7 @@ int plain_propagator(Ctx &c, const double *phi, double2 *out, SolveStats *st) {
     c.lastIters = last;
     c.eoRounds = rounds;
     if (rc) return rc;
-    const LatticeArgs L = largs(c);
-    hipLaunchKernelGGL((k_dirac<2, true>), site_grid(c, 1), dim3(kNT), 0, c.stream, L, phi, (const double2 *)c.x, out);
-    YCN_HIP(hipGetLastError());
-    return YCN_OK;
+    return dirac_apply_as<kPacked>(c, phi, c.x, out, 1, 1);
 }
 
 // the measurement's source (1, 1, 0, 0) at site 0, packed, in c.eta
