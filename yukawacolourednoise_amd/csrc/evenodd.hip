@@ -984,11 +984,11 @@ int eo_autotune(Ctx &c) {
                 }
         }
     }
-    if (c.tileEo32 >= 0) {
+    if (c.tileEoP64 >= 0)
+        tune_report_choice(c, "fp64", kEoTilesP64[c.tileEoP64].TT, kEoTilesP64[c.tileEoP64].TX, "");
+    if (c.tileEo32 >= 0 && c.p.cgPrecision == YCN_CG_MIXED) {
         const EoTileCfg t = kEoTiles32[c.tileEo32];
-        std::snprintf(line, sizeof line, " | fp32 pipelined iteration: %dx%d%s, %s finalize", t.TT, t.TX,
-                      t.persist ? "p" : "", c.eoFinFused ? "prologue" : "separate");
-        c.tuneReport += line;
+        tune_report_choice(c, "fp32", t.TT, t.TX, t.persist ? "p" : "");
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);

@@ -713,6 +713,10 @@ int pl_autotune(Ctx &c) {
             }
     }
     if (const char *fin = std::getenv("YCN_PL_FIN")) c.eoFinFused = std::strcmp(fin, "fused") == 0;
+    if (tile >= 0) {
+        const PlTile t = pl_tile(tile);
+        tune_report_choice(c, mixed ? "fp32" : "fp64", t.TT, t.TX, tile < kNumPl ? "" : "r");
+    }
     return YCN_OK;
 }
 

@@ -84,6 +84,12 @@ bool tune_lookup(int kind, const Ctx &c, std::vector<double> &t) {
     return false;
 }
 
+// the end of the report: the pipelined iteration that the context runs
+void tune_report_choice(Ctx &c, const char *precision, int TT, int TX, const char *form) {
+    c.tuneReport += std::string(" | ") + precision + " pipelined iteration: " + std::to_string(TT) + "x" +
+                    std::to_string(TX) + form + ", " + (c.eoFinFused ? "prologue" : "separate") + " finalize";
+}
+
 void tune_store(int kind, const Ctx &c, const std::vector<double> &t) {
     const TuneKey k = tune_key(kind, c);
     std::lock_guard<std::mutex> lock(g_tuneMutex);

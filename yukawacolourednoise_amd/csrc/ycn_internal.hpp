@@ -252,6 +252,7 @@ void prof_chunk_end(Ctx &c, int slot);
 // autotuner timing memo (ycn_abi.hip): kind 0 = normal-operator tiles, 1 = even-odd
 bool tune_lookup(int kind, const Ctx &c, std::vector<double> &t);
 void tune_store(int kind, const Ctx &c, const std::vector<double> &t);
+void tune_report_choice(Ctx &c, const char *precision, int TT, int TX, const char *form);
 
 // noise.hip
 int noise_init(Ctx &c);
