@@ -210,8 +210,7 @@ def run_method(Y, ctx, size, method, phi0, step0, steps, warmup, profile_kernel,
     ctx.set_field(phi0)
     step = step0
     # warm-up through the same entry point as the timed steps: a first single step (it
-    # sizes the solver's chunk schedule), then a run, which captures the step graphs the
-    # timed run replays
+    # sizes the solver's chunk schedule), then a run like the timed one
     for _ in range(min(warmup, 1)):
         ctx.langevin_step(step)
         step += 1

@@ -69,8 +69,8 @@ typedef struct {
     double cgTol;          /* default 1e-8 (params.h:14)                                */
     int cgTolMode;         /* YCN_TOL_*; default absolute recursive (CGsolver.cu:107)   */
     int cgMaxIter;         /* default 1000 (params.h:15)                                */
-    int cgPrecision;       /* YCN_CG_* (mixed: any lattice; the fused FP32 tiles where  */
-                           /* one divides it, an FP32 two-stencil pair elsewhere)       */
+    int cgPrecision;       /* YCN_CG_* (mixed: any lattice; solves that one workgroup   */
+                           /* holds, see ycn_fermion_force, are FP64 in either)         */
     int reliableEvery;     /* mixed precision: FP64 reliable update period (50)         */
     int precond;           /* YCN_PRECOND_*                                             */
     int device;            /* HIP device ordinal                                        */
@@ -117,7 +117,8 @@ void ycn_destroy(ycn_ctx *ctx);
 const char *ycn_last_error(const ycn_ctx *ctx);
 int ycn_abi_version(void);
 /* Stencil-tile autotuner result of ycn_create: the measured time per launch of the
- * fused normal operator for each tile shape that divides the lattice, and the choice.
+ * fused normal operator and of the pipelined iteration for each tile shape that the
+ * lattice takes, and at its end the pipelined iteration that the context runs.
  * No reference counterpart (the reference sizes launches with
  * cudaOccupancyMaxPotentialBlockSize, code/src/device_info.h:18-66). */
 const char *ycn_tuning_report(const ycn_ctx *ctx);
@@ -173,7 +174,10 @@ int ycn_cg_solve(ycn_ctx *ctx, const double *phi, const double *b, double *x, in
 
 /* FermionicDrift::getForce (code/src/FermionicDrift.cu:57-80): eta_j (stream 1+j,
  * counter = step), CG on D^dag D, chi = D y, drift = -g Re sum conj(chi) eta (x s^2
- * in rescaled mode), averaged over nNoise.  drift (nReplicas*V) copied out if non-NULL. */
+ * in rescaled mode), averaged over nNoise.  drift (nReplicas*V) copied out if non-NULL.
+ * Systems of up to 2048 sites (with evenOdd: 2048 even sites) are solved by one workgroup
+ * each, in FP64 whatever cgPrecision asks for; not with the learned preconditioner, nor
+ * while a kernel is profiled. */
 int ycn_fermion_force(ycn_ctx *ctx, uint64_t step, double *drift, ycn_cg_stats *stats);
 
 /* One full Langevin step (main.cu:305-315 = cn(); getForce(); kli.Run(kAll)):
@@ -182,19 +186,21 @@ int ycn_langevin_step(ycn_ctx *ctx, uint64_t step, double *eps, ycn_cg_stats *st
 /* nsteps steps starting at counter step0 (the loop of main.cu:300-502 between two
  * exports, which synchronises and copies eps to the host every step: main.cu:305-315,
  * FermionicDrift.cu:61-78).  The step sizes and the Langevin time stay on the device.
- * With even-odd preconditioning and mixed precision every step after the context's
- * first solve is enqueued whole (noise, solve setup, a fixed chunk schedule sized from
- * the previous solve, drift, update; with YCN_STEP_GRAPHS=1 in the environment its solve
- * is a captured graph): the host waits once per segment of up to 16 steps and never
- * inside a step; a step whose solve outlasts its
- * schedule is finished by the host at the end of the segment.  Other configurations
- * poll CG convergence inside each step.  Results are the same either way.
+ * Steps whose solves one workgroup holds (see ycn_fermion_force) are enqueued whole,
+ * with any of these solvers: the host waits once per 64 steps and polls nothing.
+ * With even-odd preconditioning and mixed precision on larger lattices every step after
+ * the context's first solve is enqueued whole (noise, solve setup, a fixed chunk schedule
+ * sized from the previous solve, drift, update; with YCN_STEP_GRAPHS=1 in the environment
+ * its solve is a captured graph): the host waits once per segment of up to 16 steps and
+ * never inside a step; a step whose solve outlasts its schedule is finished by the host
+ * at the end of the segment.  Other configurations poll CG convergence inside each step.
+ * Results are the same either way.
  * stats (optional) receives the totals: iters = sum over steps of the per-step max,
  * iters_mean = mean per solve. */
 int ycn_langevin_run(ycn_ctx *ctx, uint64_t step0, int nsteps, ycn_cg_stats *stats);
 
 /* Host waits on the context's work since its creation (the CG solvers' convergence
- * polls, the reads of the enqueued steps' control block) and the enqueued steps the
+ * polls, the reads of the enqueued steps' reports) and the enqueued steps the
  * host had to finish; either pointer may be NULL.  No counterpart in the reference:
  * it is how a caller sees how often the host synchronises inside its Langevin runs. */
 int ycn_host_syncs(ycn_ctx *ctx, int64_t *syncs, int64_t *halted_steps);
@@ -252,7 +258,9 @@ int ycn_precond_train(ycn_ctx *ctx, uint64_t step0, int nsteps, int pairsPerSolv
 
 /* Kernel timing with HIP events on the context stream (for roofline figures):
  * between begin and end every launch of the named kernel is bracketed by events
- * (iteration chunks are then launched one kernel at a time, not as graph replays);
+ * (iteration chunks are then launched one kernel at a time, not as graph replays; no
+ * solve is held by one workgroup; and under "cg_update" the plain solvers and the FP64
+ * even-odd one run their unpipelined iterations, which have an update kernel);
  * end returns the summed duration and count of the launches that did work (launches
  * shorter than a quarter of the 90th percentile exited at once for converged systems and
  * are left out) and the algorithmic bytes moved per launch (averaged over the launches: the

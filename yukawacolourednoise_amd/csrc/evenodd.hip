@@ -15,12 +15,14 @@
 // (x >> 1).  Needs even Nt and Nx.  All vectors are packed real spinors (ycn_device.hpp):
 // planes [sys][c][Vh], c the spin, each entry (flavour 0, flavour 1).
 //
-// FP64: one CG iteration = k_eo_normal_fused (p' = r + beta p, v = S p', Ap = S^T v,
-// |v|^2: four half-lattice hops through LDS) + the BLAS-1 update on Vh sites: 5S + P
-// bytes per site of the full lattice, against 10S + P for the unpreconditioned
-// iteration.  Mixed precision: one launch per pipelined FP32 iteration (52 B per site),
-// its finalize in the next launch's prologue or a separate kernel, and FP64 reliable
-// updates whose residual b - S x and S^T of it take one fused launch.
+// An iteration is one launch of the pipelined kernel (eo_pipelined.hip), in FP64 (104 B per
+// site of the full lattice) or for mixed precision in FP32 (52 B), its finalize in the next
+// launch's prologue or a separate kernel; mixed precision adds FP64 reliable updates whose
+// residual b - S x and S^T of it take one launch of k_eo_normal_fused.  That kernel's other
+// form (p' = r + beta p, v = S p', Ap = S^T v, |v|^2: four half-lattice hops through LDS) with
+// the BLAS-1 update is the unpipelined FP64 iteration: where a tile of it is forced or the
+// update kernel is timed.  Systems of up to 2048 even sites solve in one workgroup
+// (onchip_eo.hip).
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
@@ -45,7 +47,7 @@ struct EoArgs {
     double r, M, g;
     int tilesX, tilesPerSys, xcdRemap;
     float invNt, invNx;              // 1 / Nt, 1 / Nx in single precision (wrapf)
-    // graph-captured steps (else null): the setup, drift kernels return at once while
+    // enqueued steps (else null): the setup, drift kernels return at once while
     // *halt is set, and k_eo_eta takes its noise counter from *stepPtr
     const int *halt;
     const uint64_t *stepPtr;
@@ -296,7 +298,7 @@ k_fin_eo_setup(const double2 *__restrict__ partE, int nbE, const double2 *__rest
                CgState *__restrict__ st, int *__restrict__ active, double tol, int mode, int maxIter, int maxRestarts,
                double stopScale, const StepCtl *__restrict__ ctl) {
     __shared__ double2 lds0[kNT / kWave], lds1[kNT / kWave];
-    if (ctl) {   // graph-captured step: nothing while halted; the threshold learned on the device
+    if (ctl) {   // enqueued step: nothing while halted; the threshold learned on the device
         if (ctl->halt) return;
         stopScale = ctl->stopScale;
     }
@@ -616,7 +618,7 @@ k_eo_normal_fused(EoArgs A, const double *__restrict__ phi, CgState *st, const d
     }
 }
 
-// graph-captured Langevin steps: start of a step.  The count of active systems of its
+// enqueued Langevin steps: start of a step.  The count of active systems of its
 // solve, and the halt flag and counter the step's coloured noise reads, copied into a
 // second block (noise): the noise runs on a branch of the graph beside the solve, whose
 // check kernel may change the first block while the noise kernels run.
@@ -628,7 +630,7 @@ __global__ void k_step_begin(const StepCtl *__restrict__ ctl, StepCtl *__restric
     noise->step = ctl->step;
 }
 
-// graph-captured Langevin steps: after the step's chunk schedule.  Every system final:
+// enqueued Langevin steps: after the step's chunk schedule.  Every system final:
 // the step's statistics into the control block, the next solve's starting threshold
 // (relative mode: 0.9 times the largest ratio need / stop0 the systems reported, as
 // eo_learn_stop_scale does on the host) and the next step's counter.  A system still
@@ -1047,7 +1049,7 @@ static bool eo_mixed(const Ctx &c) {
 
 // Setup of a solve: eta (from the Philox streams when gen) and u_o = A_o^-1 eta_o,
 // b_e = eta_e - K_eo u_o, r = S^T b (FP32 copy when mixed), x and the directions cleared,
-// the FP32 copy of the field (mixed) and the per-system state.  ctl (a graph-captured
+// the FP32 copy of the field (mixed) and the per-system state.  ctl (an enqueued
 // step, else null): every launch returns at once while ctl->halt is set, the noise
 // counter is ctl->step and the starting threshold ctl->stopScale.
 static int eo_setup(Ctx &c, const double *phi, int nsys, bool gen, uint32_t streamBase, uint64_t step, bool mixed,
@@ -1061,7 +1063,7 @@ static int eo_setup(Ctx &c, const double *phi, int nsys, bool gen, uint32_t stre
     const int nbF = gF.x, nbH = gH.x;
     double2 *partE = c.partials, *partH = c.partials + (size_t)nsys * nbF;
     const EoBufs B = eo_bufs(c, nsys);
-    if (!ctl) {   // (a captured step sets the count in k_step_begin)
+    if (!ctl) {   // (an enqueued step sets the count in k_step_begin)
         const int rc = set_int(c, c.active, nsys);
         if (rc) return rc;
     }
@@ -1091,7 +1093,7 @@ static int eo_setup(Ctx &c, const double *phi, int nsys, bool gen, uint32_t stre
                        zero);
     if (mixed) {
         const int nrepUsed = (nsys + c.nNoise - 1) / c.nNoise;
-        // a captured step also keeps the FP64 field its solve reads in c.phiSolve: the
+        // an enqueued step also keeps the FP64 field its solve reads in c.phiSolve: the
         // reliable updates of a halted solve that later steps' chunks run read it there
         const int rc = to_f32_n(c, phi, c.phis, (int64_t)std::min(nrepUsed, c.nRep) * c.V,
                                 ctl ? &ctl->halt : nullptr, ctl ? c.phiSolve : nullptr);
@@ -1118,7 +1120,7 @@ static int eo_mixed_chunk(Ctx &c, const double *phi, int nsys, int n, bool graph
         c.err = "internal: a chunk of the pipelined iteration has an odd number of launches";
         return YCN_ERR_INVALID;
     }
-    if (graphed) {   // already inside a capture: the launches themselves
+    if (graphed) {   // a whole step is enqueued or captured: the launches themselves
         for (int i = 0; i < n; ++i) launch_eo_pf_iteration(c, nsys, i);
     } else {
         const int rc = run_chunk(c, nullptr, nsys, YCN_DAGGER, n, 4, kPacked, c.tileEo32,
@@ -1135,7 +1137,7 @@ static int eo_mixed_chunk(Ctx &c, const double *phi, int nsys, int n, bool graph
     return YCN_OK;
 }
 
-// The pipelined FP32 solve from the state the setup (or an unfinished captured solve) left,
+// The pipelined FP32 solve from the state the setup (or an unfinished enqueued solve) left,
 // until every system is final; itDone: iterations already done.
 static int eo_mixed_loop(Ctx &c, const double *phi, int nsys, int itDone, SolveStats *st) {
     const int rc = pf_loop(c, nsys, itDone, st, [&](int n) { return eo_mixed_chunk(c, phi, nsys, n, false); });
@@ -1503,7 +1505,7 @@ int eo_graph_run(Ctx &c, uint64_t step0, int nsteps, SolveStats *tot) {
             // update, eagerly; the field it started from is the one that step read
             const uint64_t first = step0 + (uint64_t)done;
             if (h.haltStep < first || h.haltStep >= first + (uint64_t)seg) {
-                c.err = "captured steps: the control block names a step outside the segment";
+                c.err = "enqueued steps: the control block names a step outside the segment";
                 return YCN_ERR_HIP;
             }
             const int k = (int)(h.haltStep - first);
@@ -1533,7 +1535,7 @@ int eo_graph_run(Ctx &c, uint64_t step0, int nsteps, SolveStats *tot) {
         c.eoStopScale = h.stopScale;
     }
     c.lastIters = std::max(kGraphIters, c.eoPredIters);
-    // the captured steps' figures (the last read of the block holds them all)
+    // the enqueued steps' figures (the last read of the block holds them all)
     SolveStats dev;
     dev.iters_max = (int)h.itersMaxSum;
     dev.iters_mean = h.itersMeanSum;

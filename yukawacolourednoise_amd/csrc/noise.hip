@@ -308,7 +308,7 @@ __global__ void __launch_bounds__(kLineThreads) YCN_FOUR_WAVES
 k_noise_rows_fwd(const double *__restrict__ xi, const uint64_t *__restrict__ seeds, uint64_t step,
                  double2 *__restrict__ spec, int Nt, int Nx, int H, int nk, int lpb, FftPlan P, const StepCtl *ctl) {
     extern __shared__ double2 lds[];
-    if (ctl) {   // a graph-captured step: counter from the control block, nothing while halted
+    if (ctl) {   // an enqueued step: counter from the control block, nothing while halted
         if (ctl->halt) return;
         step = ctl->step;
     }

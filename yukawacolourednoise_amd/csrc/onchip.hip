@@ -9,9 +9,9 @@
 // round, and nothing but eta touches memory until the end.  Vectors are packed real
 // spinors (ycn_device.hpp).
 //
-// What bounds an iteration is LDS traffic and the chain of four barriers: at 32 x 32 about
-// 256 KB of LDS reads and writes per iteration, 2 000 cycles at 128 B per cycle.  Langevin
-// steps in FP64, launched iterations against this with the step around it: 16 x 16
+// What bounds an iteration is LDS traffic and the chain of three barriers (p; D p with the
+// first sum; the second sum): at 32 x 32 about 256 KB of LDS reads and writes per iteration,
+// 2 000 cycles at 128 B per cycle.  Langevin steps in FP64, launched iterations against this with the step around it: 16 x 16
 // 950 -> 107 us, 7 x 32 (no tile divides it) 1 060 -> 102 us, 32 x 32 1 250 -> 186 us.
 #include <algorithm>
 #include <cstdlib>

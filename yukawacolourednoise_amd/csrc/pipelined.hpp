@@ -1,6 +1,6 @@
-// pipelined.hpp -- the parts that the pipelined FP32 iterations share (plain.hip, evenodd.hip):
-// finalize kernels, the stop decision, the reliable update's accumulation and decision, and the
-// host loop over chunks of launches.
+// pipelined.hpp -- the parts that the pipelined iterations share (plain.hip, eo_pipelined.hip,
+// evenodd.hip): finalize kernels and stop decisions of both precisions, the FP32 ones' reliable
+// update and host loop over chunks of launches, the FP64 ones' close.
 #pragma once
 #include <algorithm>
 #include <type_traits>
@@ -625,7 +625,7 @@ inline int pf_chunk_len(const Ctx &c, int pred, int itDone) {
 // the eager loop polls once it is within this many iterations of the prediction
 inline int pf_poll_margin(int pred) { return std::max(8, pred / 8); }
 
-// The pipelined FP32 solve from the state the setup (or an unfinished captured solve)
+// The pipelined FP32 solve from the state the setup (or an unfinished enqueued solve)
 // left, until every system is final, polling the systems only where they may have
 // converged; itDone: iterations already done (the chunk lengths count from there).
 // The summary goes to *st, the iteration count and the starting threshold of the next

@@ -556,9 +556,10 @@ int ycn_langevin_step(ycn_ctx *ctx, uint64_t step, double *eps, ycn_cg_stats *st
     return st.converged ? YCN_OK : YCN_ERR_NOT_CONVERGED;
 }
 
-// With the even-odd mixed solver (and graphs on, no kernel profiled) the steps after the
-// context's first solve replay captured whole steps: no host wait inside a step, one per
-// segment of steps (eo_graph_run); every other configuration runs single steps.
+// Steps whose solves one workgroup holds, and with the even-odd mixed solver (graphs on, no
+// kernel profiled) the steps after the context's first solve, are enqueued whole: no host
+// wait inside a step, one per segment of steps (onchip_run, eo_graph_run); every other
+// configuration runs single steps.
 int ycn_langevin_run(ycn_ctx *ctx, uint64_t step0, int nsteps, ycn_cg_stats *stats) {
     CHECK_CTX(ctx);
     if (nsteps < 0) return YCN_ERR_INVALID;

@@ -220,7 +220,7 @@ __device__ __forceinline__ void eta_site(const uint64_t *seeds, uint32_t streamB
 // two planes per system, plane s = (flavour 0, flavour 1) of spin s as the two members of a
 // V2, so the complex form's kernels run on it with NC = 2 planes instead of 4: half the
 // bytes, LDS and arithmetic, and the same products and sums.  The complex form (NC = 4)
-// stays for complex right-hand sides and the learned preconditioner.
+// stays for complex right-hand sides and the training of the learned preconditioner.
 // ---------------------------------------------------------------------------
 template <int NC>
 __device__ __forceinline__ void eta_planes(const uint64_t *seeds, uint32_t streamBase, uint64_t step, int sys,

@@ -79,10 +79,10 @@ struct StepState {
     int pad;
 };
 
-// Control block of graph-captured Langevin steps (device resident).  Every kernel of a
-// captured step outside the CG iteration chunks returns at once while `halt` is set; the
+// Control block of Langevin steps that are enqueued whole (device resident).  Every kernel of
+// such a step outside the CG iteration chunks returns at once while `halt` is set; the
 // step's check kernel sets it when the step's solve did not reach its stopping rule within
-// the captured chunk schedule, so that the later steps of the run leave the state as it
+// the step's chunk schedule, so that the later steps of the run leave the state as it
 // is (their chunk kernels keep iterating the unfinished solve) and the host finishes that
 // step when it reads the block at the end of the segment of steps.
 struct StepCtl {
@@ -151,7 +151,7 @@ struct Ctx {
     CgState *cg_h = nullptr;              // pinned host mirror of the CG states
     hipEvent_t pollEv = nullptr;          // spin-waited by the solvers' polls
     int eoPredIters = 0;                  // iterations of the last even-odd mixed solve (chunk predictor)
-    std::vector<int> eoRoundChunks;       // captured steps: the last schedule's chunk per round
+    std::vector<int> eoRoundChunks;       // enqueued steps: the last schedule's chunk per round
     std::vector<int> eoRounds;            // iteration counts at that solve's reliable updates (its longest system)
     double eoStopScale = 1.0;             // starting threshold of even-odd solves / tol |r_0| (relative mode)
     int maxBlocks = 0;
@@ -167,8 +167,8 @@ struct Ctx {
 
     // mixed precision: [nSys][4][V] float2
     float2 *rs = nullptr, *ps[2] = {nullptr, nullptr}, *Aps = nullptr, *xs = nullptr;
-    // pipelined even-odd FP32 iteration ([nSys][4][V/2]): the second Ap buffer, and the third
-    // direction buffer (the directions rotate through ps[0], ps[1], pfP2)
+    // pipelined FP32 iterations (packed, [nSys][2][V], even-odd V/2): the second Ap buffer (learned
+    // preconditioner: [nSys][4][V], the second residual buffer), and the third direction buffer (the directions rotate through ps[0], ps[1], pfP2)
     float2 *pfA1 = nullptr, *pfP2 = nullptr;
     double2 *pfSlot[2] = {nullptr, nullptr};   // block partials of prologue-finalized launches
     int tilePl = -1, tileP64 = -1;        // tiles of the plain pipelined FP32 and FP64 iterations (-1: not available)
@@ -190,10 +190,11 @@ struct Ctx {
     double trainLossFirst = 0, trainLossLast = 0;
     int trainPairs = 0;
 
-    // graph-captured Langevin steps (even-odd mixed precision): control block, its pinned
-    // mirror, and one executable per (chunk schedule, field parity)
+    // enqueued Langevin steps (even-odd mixed precision): control block, its pinned mirror, and
+    // where their solves are replayed as captured graphs one executable per (chunk schedule,
+    // field parity)
     StepCtl *ctl_d = nullptr, *ctl_h = nullptr;
-    double *phiSolve = nullptr;           // the field of the captured step's solve (FP64)
+    double *phiSolve = nullptr;           // the field of the enqueued step's solve (FP64)
     struct StepGraph {
         std::vector<int> chunks;   // launches of each chunk of the schedule
         int parity;                // field buffer the step reads
@@ -204,7 +205,7 @@ struct Ctx {
     bool stepCapture = false;             // YCN_STEP_GRAPHS=1: a step's solve is a captured graph
     int stepTail = 1, stepClean = 0;      // tail rounds of the schedule; clean segments since a halt
     int64_t hostSyncs = 0;                // host waits on the context's work since creation
-    int64_t haltedSteps = 0;              // captured steps finished by the host
+    int64_t haltedSteps = 0;              // enqueued steps finished by the host
 
     // captured CG iteration chunks: key -> executable graph
     struct GraphEntry {
@@ -260,8 +261,9 @@ void noise_free(Ctx &c);
 // xi == nullptr: Philox field of (seeds, stream 0, step); else filter xi (device, nRep*V)
 int noise_generate(Ctx &c, uint64_t step, const double *xi_dev, double *out_dev);
 int noise_generate_on(Ctx &c, hipStream_t s, uint64_t step, const double *xi_dev, double *out_dev);
-// the noise of a graph-captured step: counter and halt flag from the control block
+// the fields of nsteps consecutive steps, one after the other
 int noise_generate_steps(Ctx &c, uint64_t step, int nsteps, double *out_dev);
+// the noise of an enqueued step: counter and halt flag from the control block
 int noise_generate_ctl(Ctx &c, hipStream_t s, const StepCtl *ctl, double *out_dev);
 // the allocation-free entry point's scratch: address lookup on device dev (current),
 // and the message of the last failed call on this thread (nullptr if none)
@@ -279,7 +281,7 @@ enum SpinorForm { kComplex = 4, kPacked = 2 };
 int cg_alloc(Ctx &c);
 void cg_free(Ctx &c);
 int cg_autotune(Ctx &c);
-// mixed precision (cg_mixed.hip)
+// mixed precision
 int mp_alloc(Ctx &c);
 void mp_free(Ctx &c);
 int dirac_apply(Ctx &c, const double *phi_dev, const double2 *in, double2 *out, int nsys, int dagger);
@@ -294,7 +296,7 @@ int plain_propagator(Ctx &c, const double *phi, double2 *out, SolveStats *st);
 // correlator / trace helpers
 int spinor_slices(Ctx &c, const double2 *psi, double *out_dev);
 
-// pipelined FP32 iteration of the plain mixed solver (plain.hip)
+// pipelined iterations of the plain solvers (plain.hip)
 int pl_autotune(Ctx &c);
 bool pl_available(const Ctx &c);
 int pl_iterations(Ctx &c, int nsys, int mtype, int n);
@@ -334,7 +336,7 @@ int train_preconditioner(Ctx &c, uint64_t step0, int nsteps, int pairsPerSolve, 
 
 // update.hip
 int bosonic_update(Ctx &c, int fixedEps);
-// the update of a graph-captured step: phi_in -> phi_out (fixed eps; adaptive: in place
+// the update of an enqueued step: phi_in -> phi_out (fixed eps; adaptive: in place
 // on phi_in), no-op while *halt is set; leaves c.cur alone
 int bosonic_update_gated(Ctx &c, int fixedEps, double *phi_in, double *phi_out, const int *halt);
 int field_slices(Ctx &c, int rep, double *slices_dev, double *sums_dev);
@@ -380,12 +382,11 @@ bool eo_available(const Ctx &c);
 int eo_pf_alloc(Ctx &c);
 int eo_autotune(Ctx &c);
 int eo_solve(Ctx &c, const double *phi, int nsys, bool gen, uint32_t streamBase, uint64_t step, SolveStats *st);
-// ctl (graph-captured steps, else null): the drift kernel returns at once while halted
+// ctl (enqueued steps, else null): the drift kernel returns at once while halted
 int eo_drift(Ctx &c, const double *phi, double *drift, const StepCtl *ctl = nullptr);
-// Langevin steps as graph-captured steps (even-odd mixed precision): eligible when the
-// context runs that solver with graphs on and no kernel profiled.  eo_graph_run does
-// nsteps steps from counter step0 with one host wait per segment of captured steps and
-// adds each step's figures to *tot the way a run of single steps sums them (iters_max,
+// Langevin steps enqueued whole (even-odd mixed precision): eligible when the context
+// runs that solver with graphs on and no kernel profiled.  eo_graph_run does nsteps steps
+// from counter step0 with one host wait per segment of enqueued steps and adds each step's figures to *tot the way a run of single steps sums them (iters_max,
 // restarts and iters_mean summed, converged and-ed, rr_max and true_rel_max maxed).
 bool eo_graph_eligible(const Ctx &c);
 int eo_graph_run(Ctx &c, uint64_t step0, int nsteps, SolveStats *tot);
